@@ -535,7 +535,6 @@ __device__ __forceinline__ void push_found_n(const bool (&claim)[K], const int32
 // Claims stay exact (the same wave-combined atomics), so the reach set and
 // the found counts are those of a level-synchronous traversal; only the
 // level at which a vertex is expanded changes.  All lanes call it.
-template <bool BW>
 __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root, const int32_t* __restrict__ beg,
                                              const int32_t* __restrict__ adj, const uint64_t* __restrict__ allow,
                                              uint64_t* vis, uint64_t* qout, int32_t* qn_out, HubStage& hs,
@@ -608,11 +607,6 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
 // flat).
 constexpr int kLocalPerWave = 8;
 
-// Top-down: edges per lane per step.  One measured fastest: two let their
-// load chains overlap, but the registers they hold push the kernel into
-// spills on other paths.
-constexpr int kTK = 1;
-
 // Per-direction state of the joint traversal (the same in every block).
 struct Dir {
     int mode;         // 0 top-down, 1 bottom-up, 2 top-down to exhaustion
@@ -632,24 +626,24 @@ struct Dir {
 // giant SCC is fvis & bvis either way (a path from v to the pivot lies in
 // the forward set when v does), and the two directions then need not wait
 // for each other.
-template <bool BW>
-__device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int32_t root, int64_t& my_found, int64_t& fedges) {
+__device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_t root, int64_t& my_found,
+                                           int64_t& fedges) {
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
-    const int32_t* beg = BW ? a.bwb : a.fwb;  // expansion (top-down) direction
-    const int32_t* adj = BW ? a.bwa : a.fwa;
-    const int32_t* rbeg = BW ? a.fwb : a.bwb;  // bottom-up scans the reverse direction
-    const int32_t* radj = BW ? a.fwa : a.bwa;
-    const int32_t* rfirst = BW ? a.fw_first : a.bw_first;
+    const bool bw = dir != 0;
+    const int32_t* beg = bw ? a.bwb : a.fwb;  // expansion (top-down) direction
+    const int32_t* adj = bw ? a.bwa : a.fwa;
+    const int32_t* rbeg = bw ? a.fwb : a.bwb;  // bottom-up scans the reverse direction
+    const int32_t* radj = bw ? a.fwa : a.bwa;
+    const int32_t* rfirst = bw ? a.fw_first : a.bw_first;
     const uint64_t* allow = a.act;
-    uint64_t* vis = BW ? a.bvis : a.fvis;
-    uint64_t* snap = BW ? a.snapb : a.snap;
-    uint64_t* q0 = BW ? a.qb0 : a.q0;
-    uint64_t* q1 = BW ? a.qb1 : a.q1;
-    HubItem* h0 = BW ? a.hb0 : a.h0;
-    HubItem* h1 = BW ? a.hb1 : a.h1;
+    uint64_t* vis = bw ? a.bvis : a.fvis;
+    uint64_t* snap = bw ? a.snapb : a.snap;
+    uint64_t* q0 = bw ? a.qb0 : a.q0;
+    uint64_t* q1 = bw ? a.qb1 : a.q1;
+    HubItem* h0 = bw ? a.hb0 : a.h0;
+    HubItem* h1 = bw ? a.hb1 : a.h1;
     GiantState* gs = a.gs;
-    const int dir = BW ? 1 : 0;
     PairQueue pq{c.stage(), 0};    // top-down: staged next-level entries
     WaveQueue wq{c.stage32(), 0};  // bottom-up: the same LDS, parked misses (ids)
     HubStage hs{sm.hv[c.wave], sm.hs[c.wave], sm.hd[c.wave], 0};
@@ -702,89 +696,56 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int32_t root, i
         // the backward direction's tiles start half the grid away, so that
         // when both directions' levels are small (fewer tiles than blocks)
         // they run on different blocks at the same time
-        const int64_t b0 = BW ? ((int64_t)c.b + c.G / 2) % c.G : c.b;
+        const int64_t b0 = bw ? ((int64_t)c.b + c.G / 2) % c.G : c.b;
         for (int64_t u = b0; u < ntiles + nh; u += c.G) {
-            if (u < ntiles) {
-                // a tile: queue entries on threads 0..tile-1
+            // a tile: queue entries on threads 0..tile-1; a hub item is a
+            // tile of one entry on thread 0
+            const bool hub = u >= ntiles;
+            int32_t st = 0, dg = 0;
+            if (!hub) {
                 const int64_t i = u * tile + c.tid;
-                int32_t st = 0, dg = 0;
                 if (c.tid < tile && i < n) {
                     const uint64_t q = load_agent(&qin[i]);
                     st = qentry_start(q);
                     dg = qentry_degree(q);
                 }
-                int excl, total;
-                block_excl_scan<kW>(dg, excl, total, sm.tmp);
-                sm.off[c.tid] = excl;
-                sm.start[c.tid] = st;
-                if (c.tid == 0) c.edges_td += total;
-                __syncthreads();
-                for (int eb = 0; eb < total; eb += kGBlock * kTK) {
-                    // lane owns edges eb + k * kGBlock + tid; the source of
-                    // edge e is the last j with off[j] <= e (off[0] = 0,
-                    // non-decreasing), found by a fixed-depth search
-                    int e[kTK], pos[kTK];
-#pragma unroll
-                    for (int k = 0; k < kTK; ++k) {
-                        e[k] = eb + k * kGBlock + c.tid;
-                        pos[k] = 0;
-                    }
-#pragma unroll
-                    for (int sp = kGBlock / 2; sp > 0; sp >>= 1) {
-#pragma unroll
-                        for (int k = 0; k < kTK; ++k)
-                            if (sm.off[pos[k] + sp] <= e[k]) pos[k] += sp;
-                    }
-                    bool want[kTK];
-                    int32_t w[kTK];
-#pragma unroll
-                    for (int k = 0; k < kTK; ++k) {
-                        w[k] = 0;
-                        if (e[k] < total) w[k] = adj[sm.start[pos[k]] + (e[k] - sm.off[pos[k]])];
-                    }
-#pragma unroll
-                    for (int k = 0; k < kTK; ++k) want[k] = e[k] < total && w[k] != root;
-                    bool claim[kTK];
-                    int32_t s0[kTK], d[kTK];
-                    claim_with_degree<kTK>(want, w, allow, vis, beg, claim, s0, d);
-#pragma unroll
-                    for (int k = 0; k < kTK; ++k) {
-                        my_found += claim[k];
-                    }
-                    push_found_n<kTK>(claim, w, s0, d, pq, qout, qn_out, hs, hout, hn_out, fedges);
-                }
-                __syncthreads();
-            } else {
-                int32_t v, s0;
+            } else if (c.tid == 0) {
+                int32_t v = root;
                 if (L == 0 && !multi) {
-                    v = root;
-                    s0 = beg[root] + (int32_t)(u - ntiles) * rchunk;
+                    st = beg[root] + (int32_t)(u - ntiles) * rchunk;
                 } else {
                     v = load_agent(&hin[u - ntiles].v);
-                    s0 = load_agent(&hin[u - ntiles].start);
+                    st = load_agent(&hin[u - ntiles].start);
                 }
-                const int32_t e1 = min(s0 + (L == 0 && !multi ? rchunk : kGiantChunk), beg[v + 1]);
-                if (c.tid == 0) c.edges_td += e1 - s0;
-                for (int32_t eb = s0; eb < e1; eb += kGBlock * kTK) {
-                    bool want[kTK];
-                    int32_t w[kTK];
-#pragma unroll
-                    for (int k = 0; k < kTK; ++k) {
-                        const int32_t e = eb + k * kGBlock + c.tid;
-                        w[k] = e < e1 ? adj[e] : 0;
-                    }
-#pragma unroll
-                    for (int k = 0; k < kTK; ++k) want[k] = eb + k * kGBlock + c.tid < e1 && w[k] != root;
-                    bool claim[kTK];
-                    int32_t ws[kTK], wd[kTK];
-                    claim_with_degree<kTK>(want, w, allow, vis, beg, claim, ws, wd);
-#pragma unroll
-                    for (int k = 0; k < kTK; ++k) {
-                        my_found += claim[k];
-                    }
-                    push_found_n<kTK>(claim, w, ws, wd, pq, qout, qn_out, hs, hout, hn_out, fedges);
-                }
+                dg = min(rchunk, beg[v + 1] - st);
             }
+            int excl, total;
+            block_excl_scan<kW>(dg, excl, total, sm.tmp);
+            sm.off[c.tid] = excl;
+            sm.start[c.tid] = st;
+            if (c.tid == 0) c.edges_td += total;
+            __syncthreads();
+            for (int eb = 0; eb < total; eb += kGBlock) {
+                // the source of edge e is the last j with off[j] <= e
+                // (off[0] = 0, non-decreasing), found by a fixed-depth
+                // search; a hub item's is its one entry
+                const int e = eb + c.tid;
+                int pos = 0;
+                if (!hub) {
+#pragma unroll
+                    for (int sp = kGBlock / 2; sp > 0; sp >>= 1)
+                        if (sm.off[pos + sp] <= e) pos += sp;
+                }
+                int32_t w[1] = {0};
+                if (e < total) w[0] = adj[sm.start[pos] + (e - sm.off[pos])];
+                const bool want[1] = {e < total && w[0] != root};
+                bool claim[1];
+                int32_t s0[1], dw[1];
+                claim_with_degree<1>(want, w, allow, vis, beg, claim, s0, dw);
+                my_found += claim[0];
+                push_found_n<1>(claim, w, s0, dw, pq, qout, qn_out, hs, hout, hn_out, fedges);
+            }
+            __syncthreads();
         }
         // in place: in top-down to exhaustion, and in any later top-down
         // level whose input gives every wave at least kLocalPerWave
@@ -793,7 +754,7 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int32_t root, i
         // growing region alone: levels of up to 256-65536 entries
         // expanded so took the 4096^2 grid from 5.09 to 5.8-6.5 ms.
         if (a.td_local > 0 && (mode == 2 || (L > 0 && nh == 0 && n >= kLocalPerWave * total_waves)))
-            expand_local<BW>(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found,
+            expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found,
                              a.td_local);
         block_flush_both(c, pq, qout, qn_out, hs, hout, hn_out);
     } else {
@@ -876,36 +837,36 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int32_t root, i
             int64_t pw = 0;
             uint64_t pm = 0;
             while (busy) {
-                int js[kU];
-#pragma unroll
-                for (int u = 0; u < kU; ++u) {
-                    js[u] = busy ? __ffsll((unsigned long long)busy) - 1 : -1;
-                    busy &= busy ? busy - 1 : 0;
-                }
+                uint64_t group = 0;  // the kU words worked on, as lanes of wl / lcand
                 int32_t f[kU];
-                int64_t ws[kU];  // word of group member u (wave-uniform)
 #pragma unroll
                 for (int u = 0; u < kU; ++u) {
                     f[u] = -1;
-                    ws[u] = js[u] >= 0 ? lane_get(wl, js[u]) : 0;
-                    if (js[u] >= 0 && ((lane_get(lcand, js[u]) >> c.lane) & 1ull))
-                        f[u] = rfirst[ws[u] * 64 + c.lane];
+                    if (busy) {
+                        const int l = __ffsll((unsigned long long)busy) - 1;
+                        busy &= busy - 1;
+                        group |= 1ull << l;
+                        if ((lane_get(lcand, l) >> c.lane) & 1ull) f[u] = rfirst[lane_get(wl, l) * 64 + c.lane];
+                    }
                 }
                 if (pm) atomicOr(reinterpret_cast<unsigned long long*>(vis + pw), (unsigned long long)pm);
                 pm = 0;
-                uint32_t hits = 0;
-#pragma unroll
-                for (int u = 0; u < kU; ++u) hits |= (f[u] >= 0 && bit_of(vis, f[u])) ? 1u << u : 0u;
+                uint32_t hits = 0, listed = 0;  // bit u: first neighbour visited / list not empty
 #pragma unroll
                 for (int u = 0; u < kU; ++u) {
-                    if (js[u] < 0) continue;
-                    const uint64_t cm = lane_get(lcand, js[u]);
-                    const int64_t w = ws[u];
-                    const int32_t v = (int32_t)(w * 64 + c.lane);
+                    listed |= f[u] >= 0 ? 1u << u : 0u;
+                    hits |= (f[u] >= 0 && bit_of(vis, f[u])) ? 1u << u : 0u;
+                }
+                // rolled, so that the miss scan is in the code once
+#pragma unroll 1
+                for (int u = 0; group; ++u, group &= group - 1) {
+                    const int l = __ffsll((unsigned long long)group) - 1;
+                    const uint64_t cm = lane_get(lcand, l);
+                    const int64_t w = lane_get(wl, l);
                     const bool is_c = (cm >> c.lane) & 1ull;
-                    const bool hit = is_c && ((hits >> u) & 1u);
+                    const bool hit = (hits >> u) & 1u;  // f is -1 unless a candidate
                     scanned += is_c;
-                    park_misses(is_c && !hit && f[u] >= 0, v);
+                    park_misses(!hit && ((listed >> u) & 1u), (int32_t)(w * 64 + c.lane));
                     // found bits are set within the level: later probes
                     // already see them
                     const uint64_t fm = __ballot(hit);
@@ -923,26 +884,31 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int32_t root, i
             // candidates, kS at a time, and sets its found bits at once
             uint64_t mine = dense ? 0ull : lcand, fm_lane = 0;
             while (__ballot(mine != 0)) {
-                int32_t v[kS], f[kS];
+                uint64_t group = mine;  // its lowest kS bits are this step's candidates
+                int32_t f[kS];
 #pragma unroll
                 for (int k = 0; k < kS; ++k) {
-                    v[k] = -1;
+                    f[k] = -1;
                     if (mine) {
-                        v[k] = (int32_t)(wl * 64 + __ffsll((unsigned long long)mine) - 1);
+                        f[k] = rfirst[wl * 64 + __ffsll((unsigned long long)mine) - 1];
                         mine &= mine - 1;
                     }
                 }
-#pragma unroll
-                for (int k = 0; k < kS; ++k) f[k] = v[k] >= 0 ? rfirst[v[k]] : -1;
-                bool hit[kS];
-#pragma unroll
-                for (int k = 0; k < kS; ++k) hit[k] = f[k] >= 0 && bit_of(vis, f[k]);
+                uint32_t hits = 0, listed = 0;
 #pragma unroll
                 for (int k = 0; k < kS; ++k) {
-                    scanned += v[k] >= 0;
-                    park_misses(v[k] >= 0 && !hit[k] && f[k] >= 0, v[k]);
-                    if (hit[k]) {
-                        fm_lane |= 1ull << (v[k] & 63);
+                    listed |= f[k] >= 0 ? 1u << k : 0u;
+                    hits |= (f[k] >= 0 && bit_of(vis, f[k])) ? 1u << k : 0u;
+                }
+#pragma unroll 1
+                for (int k = 0; k < kS; ++k) {
+                    const int bit = __ffsll((unsigned long long)group) - 1;  // -1: none left
+                    group &= group ? group - 1 : 0;
+                    const bool hit = (hits >> k) & 1u;
+                    scanned += bit >= 0;
+                    park_misses(!hit && ((listed >> k) & 1u), (int32_t)(wl * 64 + bit));
+                    if (hit) {
+                        fm_lane |= 1ull << bit;
                         my_found += 1;
                     }
                 }
@@ -965,17 +931,16 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int32_t root, i
 // The gather of a direction that switches from bottom-up back to top-down:
 // the last level's finds (vis & ~snap) become the next level's queue and hub
 // items.  Each wave loads 64 words at once, then expands the non-empty ones.
-template <bool BW>
-__device__ __forceinline__ void gather_finds(Ctx& c, const Dir& d) {
+__device__ __forceinline__ void gather_finds(Ctx& c, const Dir& d, int dir) {
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
     GiantState* gs = a.gs;
-    const int dir = BW ? 1 : 0;
-    const int32_t* beg = BW ? a.bwb : a.fwb;
-    const uint64_t* vis = BW ? a.bvis : a.fvis;
-    const uint64_t* snap = BW ? a.snapb : a.snap;
-    uint64_t* q_next = (d.L & 1) ? (BW ? a.qb1 : a.q1) : (BW ? a.qb0 : a.q0);
-    HubItem* h_next = (d.L & 1) ? (BW ? a.hb1 : a.h1) : (BW ? a.hb0 : a.h0);
+    const bool bw = dir != 0;
+    const int32_t* beg = bw ? a.bwb : a.fwb;
+    const uint64_t* vis = bw ? a.bvis : a.fvis;
+    const uint64_t* snap = bw ? a.snapb : a.snap;
+    uint64_t* q_next = (d.L & 1) ? (bw ? a.qb1 : a.q1) : (bw ? a.qb0 : a.q0);
+    HubItem* h_next = (d.L & 1) ? (bw ? a.hb1 : a.h1) : (bw ? a.hb0 : a.h0);
     int32_t* qn_next = &gs->qn[dir][d.L % 3].v;
     int32_t* hn_next = &gs->hn[dir][d.L % 3].v;
     PairQueue wq{c.stage(), 0};
@@ -1045,8 +1010,11 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
     while (f.live || b.live) {
         if (f.gather || b.gather) {
             // the visited bits were made exact after the level's barrier
-            if (f.gather) gather_finds<false>(c, f);
-            if (b.gather) gather_finds<true>(c, b);
+#pragma unroll 1
+            for (int dir = 0; dir < 2; ++dir) {
+                const Dir d = dir ? b : f;
+                if (d.gather) gather_finds(c, d, dir);
+            }
             f.gather = b.gather = false;
             // the top-down level reads the queues coherently and visited bits
             // only as hints: no L2 invalidation
@@ -1056,14 +1024,28 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
         const int64_t edges0 = c.edges_td + c.edges_bu;  // thread 0's are the block's
         const bool tr = a.trace != 0;
         const int64_t tl0 = tr ? (int64_t)wall_clock64() : 0;
-        int64_t ff = 0, fe = 0, bf = 0, be = 0;  // per thread: found, pushed work / scanned entries
-        if (f.live) level_work<false>(c, f, root, ff, fe);
-        if (b.live) level_work<true>(c, b, root, bf, be);
+        // per thread and direction: found (high 32 bits), pushed work or
+        // scanned entries (low).  One copy of the level's code serves both
+        // directions: the instruction cache (64 KB for two CUs) does not
+        // hold two, and a small level is bound by its first pass over the
+        // code.
+        int64_t pf = 0, pb = 0;
+#pragma unroll 1
+        for (int dir = 0; dir < 2; ++dir) {
+            const Dir d = dir ? b : f;
+            if (!d.live) continue;
+            int64_t found = 0, edges = 0;
+            level_work(c, d, dir, root, found, edges);
+            const int64_t pk = (found << 32) + edges;
+            if (dir) pb = pk;
+            else pf = pk;
+        }
         // ---- level totals: every block computes the same sums.  One sum per
         // direction carries the level's finds (high 32 bits) and the next
         // level's exact work or the scan (low 32 bits: at most E < 2^31, so no
         // carry), both reduced in one block round
-        int64_t pf = wave_sum((ff << 32) + fe), pb = wave_sum((bf << 32) + be);
+        pf = wave_sum(pf);
+        pb = wave_sum(pb);
         if (c.lane == 0) {
             sm.red[c.wave] = pf;
             sm.red2[c.wave] = pb;
