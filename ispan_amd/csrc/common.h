@@ -61,20 +61,12 @@ struct alignas(128) GLine {
     int32_t pad[31];
 };
 
-// Reduction carried by one grid barrier: three sums and a max over keys
-// (identity 0 for all four).
-struct alignas(128) RLine {
-    int64_t sum[3];
-    int64_t key;
-    int64_t pad[12];
-};
+// Bytes of grid-barrier records (GiantArgs::bar) per block.
+constexpr int kBarBytesPerBlock = 128;
 
-// Device state of one k_giant launch; zeroed before every launch.
+// Device state of one k_giant launch, which clears it itself.
 constexpr int kLevelTrace = 1024;
 struct GiantState {
-    GLine sub[32];      // barrier arrival counters (two-level barrier)
-    GLine top;
-    GLine gen;          // barrier generation
     GLine qn[2][3];     // [direction][level % 3] queue lengths
     GLine hn[2][3];     // [direction][level % 3] hub work items
     GLine err;          // 1 barrier timeout, 2 level cap, 4 queue count out of range
@@ -89,9 +81,7 @@ struct GiantState {
     int64_t bw_reach;     // vertices the backward traversal reached (the giant and what reaches it)
     int64_t unlabelled;   // with unl_checked: vertices the kernel left at -1 (its final check)
     int64_t unl_checked;  // 1: the kernel labelled everything it was given and counted `unlabelled`
-    RLine gacc[32];     // barrier reductions: per arrival group
-    RLine tacc;         // barrier reductions: over groups
-    RLine res[2];       // barrier reductions: result of generation g in res[g & 1]
+    int64_t bar_next;     // GiantArgs::bar_base of the next launch on these barrier records
     // blocks' start and first-barrier arrival clocks: min, max of each
     int64_t t_start[2], t_arrive[2];
     // per level of each direction (first kLevelTrace levels): end time,
@@ -111,9 +101,6 @@ struct GiantState {
     // with GiantArgs::trace: latest clock of any block after the post
     // phase's count pass, its barrier, and the labels and active queue
     int64_t post_cp[3];
-    // the launch that last cleared this state (GiantArgs::epoch); never
-    // cleared itself, and 0 when the state is allocated
-    int64_t epoch;
 };
 constexpr size_t kGiantStateHead = offsetof(GiantState, lv_ts);
 
@@ -142,7 +129,8 @@ struct GiantArgs {
     HubItem* hb1;
     int32_t* fq;              // active queue after the giant phase
     GiantState* gs;
-    int64_t* part;            // kGiantSlots x grid partial counts
+    uint64_t* bar;            // grid-barrier records, kBarBytesPerBlock per block, zero when allocated
+    uint32_t bar_base;        // barriers these records have seen (GiantState::bar_next of the last launch)
     int32_t* fq_n_out;        // receives the active queue length
     int64_t hub_cap;          // capacity of h0 / h1
     // after the giant (when rest != 0): trim-1 sweeps, size-2/3 patterns,
@@ -175,14 +163,11 @@ struct GiantArgs {
     uint64_t* ckey;           // colouring: (priority, colour) per vertex
     int32_t* aux;             // colouring: smallest member per SCC root
     // set by launch_giant: block 0 clears `state_words` words of gs and
-    // `ctl_words` of ctl, then publishes `epoch` (unique per launch, never 0)
-    // in gs->epoch; the other blocks start once they read it
+    // `ctl_words` of ctl
     Ctl* ctl;
-    int64_t epoch;
     int32_t state_words, ctl_words;
 };
 
-constexpr int kGiantSlots = 16;
 constexpr int kGiantHubDeg = 512;   // degree from which a claimed vertex is split into work items
 constexpr int kGiantChunk = 8192;   // edges per work item
 // A vertex of degree d >= kGiantHubDeg becomes ceil(d / kGiantChunk) <=
@@ -195,8 +180,7 @@ int giant_max_blocks_per_cu();
 int64_t giant_bu_mult(int grid);
 // records `before` (when given), then launches k_giant cooperatively; the
 // kernel clears a.gs and ctl itself (a kernel queued in front of a
-// cooperative launch costs a cross-queue wait).  gs->epoch must not hold an
-// epoch of this process that is still to come: 0 at allocation does.
+// cooperative launch costs a cross-queue wait).
 hipError_t launch_giant(const GiantArgs& a, Ctl* ctl, int grid, hipStream_t s, hipEvent_t before);
 // after launch_giant on the same stream, for a.wcc_mode 1 or 2 when the giant
 // phase left active vertices: the WCC by label propagation, or the colouring

@@ -4,14 +4,13 @@
 // 944-1248) and the relabelling of what they found, with grid-wide barriers
 // between levels instead of host round trips.
 //
-// Every block runs the same control flow: after each barrier all blocks sum
-// the same per-block partial counts and take the same top-down/bottom-up
-// decision, so every block passes the same barriers.  Data written by other
+// Every block runs the same control flow: each barrier gives all blocks the
+// same totals, they take the same top-down/bottom-up decision, so every block
+// passes the same barriers.  Data written by other
 // blocks before a barrier is read with plain loads after a barrier that
 // invalidates the caches, and with device-coherent loads after one that does
 // not; device-coherent loads are also kept for what other blocks change
 // during the same phase.
-#include <atomic>
 #include "common.h"
 #include "device_util.h"
 
@@ -21,15 +20,12 @@ using namespace dev;
 namespace {
 
 constexpr int kSpinCap = 1 << 24;  // barrier wait bound (~1 s); beyond it the kernel aborts
-constexpr int kBarGroups = 32;     // arrival counters of the two-level barrier
+constexpr int kBarWords = 8;       // payload words a barrier can carry per block
+static_assert(kBarWords * 2 * 8 == kBarBytesPerBlock, "two record buffers of 8-byte words");
 // One 1024-thread block per CU: every block invalidates its caches after a
 // barrier, so fewer, larger blocks make the barrier cheaper.
 constexpr int kGBlock = 1024;
 constexpr int kW = kGBlock / kWave;
-
-// Partial-count slots: part[slot * grid + block].
-enum Slot { kPivP, kPivI, kSurv, kPost, kEdgeTD, kEdgeBU, kFoundTD, kFoundBU, kGiantN };
-static_assert(kGiantN < kGiantSlots, "slot count");
 
 struct Smem {
     int32_t off[kGBlock];    // top-down tile: exclusive degree prefix, first edge
@@ -37,11 +33,10 @@ struct Smem {
     int tmp[kW];
     int64_t red[kW];
     int64_t red2[kW];
-    int64_t rres[4];  // reduction result of the last barrier
     int32_t bi[kW];
-    int ok;
-    int32_t nbar;   // barriers this block has arrived at in this launch
-    int32_t gbase;  // barrier generation when this launch started
+    alignas(16) uint32_t bv[kBarWords][kW];  // a barrier's payload per wave
+    int64_t tot[2][kBarWords];               // its totals over the grid, per reading wave
+    int ok[2];
     int32_t wcnt[2][kW];    // block flushes: per-wave counts and bases of up to two counters
     int32_t wbase[2][kW];
     int32_t hv[kW][kWave];  // per-wave staged hub vertices: id, first edge, degree
@@ -62,16 +57,11 @@ struct Ctx {
     const GiantArgs& a;
     int G, b, tid, lane, wave;
     Smem& sm;
-    int64_t edges_td, edges_bu, found_td, found_bu;  // work counters (thread 0's are the block's)
+    uint32_t nbar;  // barriers this launch has passed (the same in every block)
+    int64_t edges_td, edges_bu, found_td, found_bu;  // work counters of this wave (wave-uniform)
     // this wave's staging, as 8-byte entries or as ids
     __device__ uint64_t* stage() const { return stage_lds + wave * kPairCap; }
     __device__ int32_t* stage32() const { return reinterpret_cast<int32_t*>(stage()); }
-};
-
-// Values a block contributes to the reduction a barrier carries: two sums
-// and a max over non-negative keys (0 contributes nothing).
-struct Red {
-    int64_t s0, s1, s2, key;
 };
 
 // Waits until every vector-memory access this wave has issued (loads,
@@ -83,120 +73,227 @@ struct Red {
 // share one L1; at agent scope it also writes back the whole L2.)
 __device__ __forceinline__ void wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmcnt(0), others unchanged
 
-// Two-level grid barrier: blocks arrive on one of 32 counters, the last of
-// each group arrives on the top counter, the last overall bumps `gen`.
+// Grid barrier that carries a payload.  Every block publishes one record, NW
+// (4 or 8) 8-byte words of {tag, 32-bit value}, and wave 0 of every block
+// reads every block's record until all of them bear this barrier's tag: one
+// store and one read across the chip, with nothing passed on in between.
+// What the blocks contribute comes with the arrival itself, so a reduction
+// costs no further round trip.  A counter tree (32 group counters, a top
+// counter, a generation word) needs three dependent atomics, and carried
+// sums add an exchange and an add at each of its levels; same box, 256 blocks
+// of 1024 threads, back to back: 4.2 us with 2 sums and 5.3 us with 4, against
+// 2.1 us with 4 words and 2.8 us with 8 here.
+//
+// Lane l of the reading wave takes word l % NW of record l / NW, then the
+// same of the next 64 / NW records, so a load instruction covers 512
+// consecutive bytes; one record a lane takes 3.1 and 4.4 us instead.  A lane
+// has 16 loads in flight (more spill), so with 8 words the records of 256
+// blocks take two waves, or two rounds of one wave where the barrier also
+// acquires: only one wave may do that (four at once: 8.9 us a barrier).
+//
+// Tags: each barrier's is one more than the last, counted on over the
+// launches on one state (GiantArgs::bar_base), so no record left from before
+// bears it, and the records need no clearing.  Consecutive barriers use the
+// two record buffers in turn: a block writes a buffer again only after a
+// barrier that every block reached after reading it.
 //
 // Memory protocol: everything a block writes for other blocks is written
 // device-coherently (atomics or st_agent), so arriving needs no L2
 // writeback.  It does need every one of those writes to have completed
-// before the arrival, and they are issued by all 16 waves while only thread
-// 0 arrives: so every wave waits for its own accesses (wait_vm) before the
-// block barrier, and thread 0 waits again before each of its arrival
-// atomics (its reduction atomics and counter resets precede them).  The
-// last block's reduction results and counter resets likewise complete
-// before it bumps `gen`.  A block that sees `gen` move therefore sees every
-// write made before the barrier, once it invalidates its L1 and its XCC's
-// L2 (device-scope acquire) or reads the data with device-coherent loads.
-//
-// With RED, each block's `in` is folded in on the way: into its group's
-// accumulator before arriving, the group total into the top accumulator by
-// the group's last arriver, the grand total published by the last block
-// before it bumps `gen`; every block gets the same `out`.
+// before the record is written, and they are issued by all 16 waves while
+// only wave 0 writes the record: so every wave waits for its own accesses
+// (wait_vm) before the block barrier.  A block that reads a record of this
+// tag therefore sees every write its block made before the barrier, once it
+// invalidates its L1 and its XCC's L2 (device-scope acquire) or reads the
+// data with device-coherent loads.
 //
 // ACQ: after the wait, invalidate this CU's L1 and this XCC's L2 (agent
 // acquire), so that plain loads see what other blocks wrote before the
 // barrier.  Without it only coherent loads and atomics may read such data
 // (and loads that tolerate stale values).
 //
-// Returns false (and flags an error) if a wait exceeds kSpinCap.
+// src() gives lane w < NW of wave 0 the block's word w, after the block
+// barrier; fold.take(record, value) is called in the reading waves for every
+// word of every record (lanes as above), then fold.finish() once per wave.
 //
-// USE: which of s0, s1, s2, key (bits 0-3) the barrier carries (the same in
-// every block); the others read back as 0.
-template <bool RED = false, bool ACQ = true>
-__device__ __forceinline__ bool gsync(GiantState* gs, int G, Smem& sm, int32_t* dbg, Red in = Red{0, 0, 0, 0},
-                                      Red* out = nullptr, int use = 15) {
-    using ull = unsigned long long;
+// Returns false (and flags an error) if the wait exceeds kSpinCap.
+template <int NW, bool ACQ, class Src, class Fold>
+__device__ __forceinline__ bool gsync_with(Ctx& c, Src src, Fold& fold) {
+    static_assert(NW == 4 || NW == 8, "record size");
+    constexpr int kReaders = ACQ ? 1 : NW / 4;  // reading waves
+    Smem& sm = c.sm;
+    const uint32_t nb = ++c.nbar;
     wait_vm();  // this wave's writes for other blocks have completed
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (c.wave < kReaders) {
+        const uint32_t tag = c.a.bar_base + nb;
+        uint64_t* rec = c.a.bar + (int64_t)(tag & 1) * c.G * kBarWords;
+        if (c.wave == 0) {
+            const uint32_t mine = src();  // by every lane
+            if (c.lane < NW) st_agent(&rec[c.b * NW + c.lane], ((uint64_t)tag << 32) | mine);
+        }
+        if (c.tid == 0) {  // diagnostics: barriers arrived at, and passed
+            c.a.dbg[c.b] = (int32_t)nb;
+            c.a.dbg[c.G + c.b] = (int32_t)nb - 1;
+        }
+        constexpr int K = 16;  // loads a lane has in flight
+        const int words = c.G * NW;
         int ok = 1;
-        // gen is gbase when the launch starts and each barrier bumps it once,
-        // so at this block's nb-th barrier it reads gbase + nb - 1: no load
-        // needed
-        const int32_t nb = ++sm.nbar;
-        const int32_t g0 = sm.gbase + nb - 1;
-        const int grp = blockIdx.x % kBarGroups;
-        const int ngrp = min(kBarGroups, G);
-        const int gsize = (G - grp + kBarGroups - 1) / kBarGroups;
-        RLine& ga = gs->gacc[grp];
-        if (RED) {
-            if (in.s0) atomicAdd(reinterpret_cast<ull*>(&ga.sum[0]), (ull)in.s0);
-            if (in.s1) atomicAdd(reinterpret_cast<ull*>(&ga.sum[1]), (ull)in.s1);
-            if (in.s2) atomicAdd(reinterpret_cast<ull*>(&ga.sum[2]), (ull)in.s2);
-            if (in.key) atomicMax(reinterpret_cast<ull*>(&ga.key), (ull)in.key);
-        }
-        wait_vm();  // the group accumulator holds this block's values before it arrives
-        bool last = false;
-        const int arrived = atomicAdd(&gs->sub[grp].v, 1);
-        // diagnostics, stored while the arrival is in flight: barriers arrived
-        // at, and passed (this block's previous one)
-        dbg[blockIdx.x] = nb;
-        dbg[G + blockIdx.x] = nb - 1;
-        if (arrived == gsize - 1) {
-            st_agent(&gs->sub[grp].v, 0);
-            if (RED) {
-                const ull a0 = (use & 1) ? atomicExch(reinterpret_cast<ull*>(&ga.sum[0]), 0ull) : 0ull;
-                const ull a1 = (use & 2) ? atomicExch(reinterpret_cast<ull*>(&ga.sum[1]), 0ull) : 0ull;
-                const ull a2 = (use & 4) ? atomicExch(reinterpret_cast<ull*>(&ga.sum[2]), 0ull) : 0ull;
-                const ull ak = (use & 8) ? atomicExch(reinterpret_cast<ull*>(&ga.key), 0ull) : 0ull;
-                if (a0) atomicAdd(reinterpret_cast<ull*>(&gs->tacc.sum[0]), a0);
-                if (a1) atomicAdd(reinterpret_cast<ull*>(&gs->tacc.sum[1]), a1);
-                if (a2) atomicAdd(reinterpret_cast<ull*>(&gs->tacc.sum[2]), a2);
-                if (ak) atomicMax(reinterpret_cast<ull*>(&gs->tacc.key), ak);
+        for (int base = c.wave * K * kWave; base < words && ok; base += kReaders * K * kWave) {
+            uint64_t x[K];
+            uint32_t todo = 0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                x[k] = 0;
+                todo |= base + k * kWave + c.lane < words ? 1u << k : 0u;
             }
-            wait_vm();  // the group counter's reset and the group's totals precede the top arrival
-            if (atomicAdd(&gs->top.v, 1) == ngrp - 1) {
-                st_agent(&gs->top.v, 0);
-                if (RED) {
-                    RLine& r = gs->res[(g0 + 1) & 1];
-                    if (use & 1) st_agent(&r.sum[0], (int64_t)atomicExch(reinterpret_cast<ull*>(&gs->tacc.sum[0]), 0ull));
-                    if (use & 2) st_agent(&r.sum[1], (int64_t)atomicExch(reinterpret_cast<ull*>(&gs->tacc.sum[1]), 0ull));
-                    if (use & 4) st_agent(&r.sum[2], (int64_t)atomicExch(reinterpret_cast<ull*>(&gs->tacc.sum[2]), 0ull));
-                    if (use & 8) st_agent(&r.key, (int64_t)atomicExch(reinterpret_cast<ull*>(&gs->tacc.key), 0ull));
-                }
-                last = true;
-            }
-        }
-        if (last) {
-            wait_vm();  // the top counter's reset and the results precede the new generation
-            atomicAdd(&gs->gen.v, 1);
-        } else {
             int spins = 0;
-            while (load_agent(&gs->gen.v) == g0) {
-                __builtin_amdgcn_s_sleep(2);
+            while (true) {
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if ((todo >> k) & 1u) x[k] = load_agent(&rec[base + k * kWave + c.lane]);
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if ((uint32_t)(x[k] >> 32) == tag) todo &= ~(1u << k);
+                if (!__ballot(todo != 0)) break;
+                __builtin_amdgcn_s_sleep(1);
                 if (++spins > kSpinCap) {
-                    atomicOr(&gs->err.v, 1);
+                    if (c.lane == 0) atomicOr(&c.a.gs->err.v, 1);
                     ok = 0;
                     break;
                 }
             }
+#pragma unroll
+            for (int k = 0; k < K; ++k) fold.take((base + k * kWave + c.lane) / NW, (uint32_t)x[k]);
         }
+        fold.finish(sm, c.wave);
         if (ACQ) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // this CU's L1 and this XCC's L2
         else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        if (RED && ok) {
-            const RLine& r = gs->res[(g0 + 1) & 1];
-            sm.rres[0] = (use & 1) ? load_agent(&r.sum[0]) : 0;
-            sm.rres[1] = (use & 2) ? load_agent(&r.sum[1]) : 0;
-            sm.rres[2] = (use & 4) ? load_agent(&r.sum[2]) : 0;
-            sm.rres[3] = (use & 8) ? load_agent(&r.key) : 0;
-        }
-        sm.ok = ok && load_agent(&gs->err.v) == 0;
+        if (c.lane == 0) sm.ok[c.wave] = ok;
     }
     __syncthreads();
-    if (RED && out) *out = Red{sm.rres[0], sm.rres[1], sm.rres[2], sm.rres[3]};
-    __syncthreads();
-    return sm.ok;
+    return __builtin_amdgcn_readfirstlane(kReaders == 1 ? sm.ok[0] : (sm.ok[0] & sm.ok[1]));
 }
+
+// The payload as each wave stages it: word w's value of this wave, the same
+// in every lane.
+template <int NW>
+__device__ __forceinline__ void stage_words(Ctx& c, const uint32_t (&v)[NW]) {
+    uint32_t x = v[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) x = c.lane == w ? v[w] : x;
+    if (c.lane < NW) c.sm.bv[c.lane][c.wave] = x;
+}
+
+// Sum of word lane % kBarWords over the waves.
+__device__ __forceinline__ uint32_t staged_sum(const Smem& sm, int lane) {
+    uint32_t s = 0;
+#pragma unroll
+    for (int i = 0; i < kW; ++i) s += sm.bv[lane & (kBarWords - 1)][i];
+    return s;
+}
+
+// Folds the lanes that hold the same word (lane % NW), op over them; every
+// lane gets its word's result.
+template <int NW, class T, class Op>
+__device__ __forceinline__ T fold_lanes(T s, Op op) {
+#pragma unroll
+    for (int d = NW; d < kWave; d <<= 1) s = op(s, (T)__shfl_xor(s, d, kWave));
+    return s;
+}
+
+// Totals of every word into sm.tot.
+template <int NW>
+struct SumFold {
+    uint64_t s = 0;
+    __device__ void take(int, uint32_t x) { s += x; }
+    __device__ void finish(Smem& sm, int wave) {
+        s = fold_lanes<NW>(s, [](uint64_t p, uint64_t q) { return p + q; });
+        if (lane_id() < NW) sm.tot[wave][lane_id()] = (int64_t)s;
+    }
+};
+
+// Barrier whose payload is summed: v holds each wave's values (the same in
+// every lane); out receives the totals.
+template <int NW, bool ACQ>
+__device__ __forceinline__ bool gsync_sum(Ctx& c, const uint32_t (&v)[NW], int64_t (&out)[NW]) {
+    stage_words<NW>(c, v);
+    SumFold<NW> f;
+    if (!gsync_with<NW, ACQ>(c, [&c]() { return staged_sum(c.sm, c.lane); }, f)) return false;
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+        out[w] = lane_get((NW == 8 && !ACQ) ? c.sm.tot[0][w] + c.sm.tot[1][w] : c.sm.tot[0][w], 0);
+    return true;
+}
+
+struct NoFold {
+    __device__ void take(int, uint32_t) {}
+    __device__ void finish(Smem&, int) {}
+};
+
+// Barrier without a payload.
+template <bool ACQ = true>
+__device__ __forceinline__ bool gsync(Ctx& c) {
+    NoFold f;
+    return gsync_with<4, ACQ>(c, []() { return 0u; }, f);
+}
+
+// The largest (product, -id) over the records of {product high, product low,
+// id, survivors}, and the survivors' sum, into sm.tot[0][0..2].
+struct PivotFold {
+    int64_t bestp = 0;
+    int32_t besti = INT32_MAX;
+    uint64_t surv = 0;
+    __device__ void take(int, uint32_t x) {
+        // the four words of a record lie in the four lanes of a quad
+        const int32_t y = (int32_t)x;
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, y, 0x00, 0xF, 0xF, false);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, y, 0x55, 0xF, 0xF, false);
+        const int32_t id = __builtin_amdgcn_update_dpp(0, y, 0xAA, 0xF, 0xF, false);
+        const int64_t p = (int64_t)(((uint64_t)hi << 32) | lo);
+        if (pivot_better(p, id, bestp, besti)) {
+            bestp = p;
+            besti = id;
+        }
+        surv += x;  // of lanes 3, 7, ..: the others' sums are not used
+    }
+    __device__ void finish(Smem& sm, int) {
+#pragma unroll
+        for (int d = 4; d < kWave; d <<= 1) {
+            const int64_t op = __shfl_xor(bestp, d, kWave);
+            const int32_t oi = __shfl_xor(besti, d, kWave);
+            if (pivot_better(op, oi, bestp, besti)) {
+                bestp = op;
+                besti = oi;
+            }
+        }
+        surv = fold_lanes<4>(surv, [](uint64_t p, uint64_t q) { return p + q; });
+        if (lane_id() == 3) {
+            sm.tot[0][0] = bestp;
+            sm.tot[0][1] = besti;
+            sm.tot[0][2] = (int64_t)surv;
+        }
+    }
+};
+
+// Totals of every word but word 2, whose largest value is taken, into
+// sm.tot[0][0..6], and into sm.tot[0][7] the sum of word 0 over the blocks before
+// this one (word 7 carries nothing).
+struct PostFold {
+    int b;
+    uint64_t s = 0, pre = 0;
+    __device__ void take(int rec, uint32_t x) {
+        s = (lane_id() & 7) == 2 ? max(s, (uint64_t)x) : s + x;
+        pre += rec < b ? x : 0u;
+    }
+    __device__ void finish(Smem& sm, int) {
+        const bool mx = (lane_id() & 7) == 2;
+        s = fold_lanes<8>(s, [mx](uint64_t p, uint64_t q) { return mx ? max(p, q) : p + q; });
+        pre = fold_lanes<8>(pre, [](uint64_t p, uint64_t q) { return p + q; });
+        if (lane_id() < 7) sm.tot[0][lane_id()] = (int64_t)s;
+        if (lane_id() == 0) sm.tot[0][7] = (int64_t)pre;
+    }
+};
 
 // Sum of a per-thread value over the block (every thread gets it).
 __device__ __forceinline__ int64_t block_sum(int64_t x, Smem& sm) {
@@ -210,21 +307,14 @@ __device__ __forceinline__ int64_t block_sum(int64_t x, Smem& sm) {
     return x;
 }
 
-// Sum / minimum of one partial slot over all blocks (every block computes
-// the same value).
-__device__ __forceinline__ int64_t sum_slot(const int64_t* part, int slot, int G, Smem& sm) {
-    int64_t x = 0;
-    for (int i = threadIdx.x; i < G; i += kGBlock) x += load_agent(&part[(int64_t)slot * G + i]);
-    return block_sum(x, sm);
-}
-
 // Per-wave staging of hub vertices in LDS; a flush turns them into
 // kGiantChunk-edge work items with one atomic for the whole batch.
 struct HubStage {
     int32_t* v;
     int32_t* s;
     int32_t* d;
-    int n;  // wave-uniform fill
+    int n;              // wave-uniform fill
+    uint32_t sent = 0;  // work items written so far (wave-uniform)
 };
 
 __device__ __forceinline__ void hub_flush(HubStage& hs, HubItem* hout, int32_t* hn_out) {
@@ -241,6 +331,7 @@ __device__ __forceinline__ void hub_flush(HubStage& hs, HubItem* hout, int32_t* 
     int base = 0;
     if (lane == kWave - 1) base = atomicAdd(hn_out, incl);
     base = lane_get(base, kWave - 1) + incl - nch;
+    hs.sent += (uint32_t)lane_get(incl, kWave - 1);
     for (int k = 0; k < nch; ++k) {
         st_agent(&hout[base + k].v, v);
         st_agent(&hout[base + k].start, s0 + k * kGiantChunk);
@@ -317,30 +408,6 @@ __device__ __forceinline__ void block_flush(Ctx& c, WaveQueue& wq, int32_t* gq, 
     wave_sync();
 }
 
-// block_flush of the queue and of the staged hub vertices (as work items)
-// with one reservation round.
-__device__ __forceinline__ void block_flush_both(Ctx& c, WaveQueue& wq, int32_t* gq, int32_t* gcount, HubStage& hs,
-                                                 HubItem* hout, int32_t* hn_out) {
-    int32_t v = 0, s0 = 0, nch = 0;
-    if (c.lane < hs.n) {
-        v = hs.v[c.lane];
-        s0 = hs.s[c.lane];
-        nch = (hs.d[c.lane] + kGiantChunk - 1) / kGiantChunk;
-    }
-    const int incl = wave_incl_scan(nch);
-    int qb, hb;
-    block_reserve2(c, wq.n, gcount, lane_get(incl, kWave - 1), hn_out, qb, hb);
-    for (int i = c.lane; i < wq.n; i += kWave) st_agent(&gq[qb + i], wq.buf[i]);
-    hb += incl - nch;
-    for (int k = 0; k < nch; ++k) {
-        st_agent(&hout[hb + k].v, v);
-        st_agent(&hout[hb + k].start, s0 + k * kGiantChunk);
-    }
-    wq.n = 0;
-    hs.n = 0;
-    wave_sync();
-}
-
 // A top-down queue entry: a vertex's first edge (high half) and degree (low
 // half), which is all a top-down level needs to walk the vertex's list, so
 // it loads no offsets; the claim that queues a vertex has just loaded them.
@@ -353,7 +420,8 @@ __device__ __forceinline__ int32_t qentry_degree(uint64_t e) { return (int32_t)(
 // A wave's staged top-down queue entries (in LDS) and its fill.
 struct PairQueue {
     uint64_t* buf;
-    int n;  // wave-uniform
+    int n;              // wave-uniform
+    uint32_t sent = 0;  // entries written to the next level's queue so far (wave-uniform)
 };
 
 __device__ __forceinline__ void pq_flush(PairQueue& pq, uint64_t* gq, int32_t* gcount) {
@@ -363,6 +431,7 @@ __device__ __forceinline__ void pq_flush(PairQueue& pq, uint64_t* gq, int32_t* g
     if (lane_id() == 0) base = atomicAdd(gcount, pq.n);
     base = lane_get(base, 0);
     for (int i = lane_id(); i < pq.n; i += kWave) st_agent(&gq[base + i], pq.buf[i]);
+    pq.sent += (uint32_t)pq.n;
     pq.n = 0;
     wave_sync();
 }
@@ -376,7 +445,8 @@ __device__ __forceinline__ void pq_push(PairQueue& pq, bool pred, uint64_t e, ui
     pq.n += c;
 }
 
-// block_flush_both for top-down queue entries.
+// The end-of-level flush of the queue and of the staged hub vertices (as work
+// items), with one reservation round.
 __device__ __forceinline__ void block_flush_both(Ctx& c, PairQueue& pq, uint64_t* gq, int32_t* gcount, HubStage& hs,
                                                  HubItem* hout, int32_t* hn_out) {
     int32_t v = 0, s0 = 0, nch = 0;
@@ -394,6 +464,8 @@ __device__ __forceinline__ void block_flush_both(Ctx& c, PairQueue& pq, uint64_t
         st_agent(&hout[hb + k].v, v);
         st_agent(&hout[hb + k].start, s0 + k * kGiantChunk);
     }
+    pq.sent += (uint32_t)pq.n;
+    hs.sent += (uint32_t)lane_get(incl, kWave - 1);
     pq.n = 0;
     hs.n = 0;
     wave_sync();
@@ -415,7 +487,7 @@ __device__ __forceinline__ void push_next(bool claim, int32_t w, const int32_t* 
     pq_push(pq, claim && d > 0 && d < kGiantHubDeg, qentry(s0, d), qout, qn_out);
 }
 
-// The acquire gsync<.., true> performs, for a block that passed a barrier
+// The acquire of a barrier with ACQ, for a block that passed a barrier
 // without it.
 __device__ __forceinline__ void block_acquire() {
     if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -585,6 +657,7 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
                 int base = 0;
                 if (c.lane == 0) base = atomicAdd(qn_out, cnt);
                 base = lane_get(base, 0);
+                wq.sent += (uint32_t)cnt;
                 if (keep) st_agent(&qout[base + __popcll(m & lanemask_lt())], qentry(s0[0], d[0]));
             }
         }
@@ -596,6 +669,7 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
         if (c.lane == 0) base = atomicAdd(qn_out, left);
         base = lane_get(base, 0);
         for (int i = c.lane; i < left; i += kWave) st_agent(&qout[base + i], buf[(head + i) & mask]);
+        wq.sent += (uint32_t)left;
     }
     wq.n = 0;
     wave_sync();
@@ -614,20 +688,26 @@ struct Dir {
     int64_t visited;  // vertices claimed, the roots excluded
     bool live;        // still traversing
     bool gather;      // its last level was bottom-up and its next is top-down
+    int64_t nq, nh;   // next level's queue entries and hub work items
+};
+
+// What a wave's part of a level came to: per-thread counts and wave-uniform
+// queue totals.
+struct Level {
+    int found;          // vertices this thread claimed
+    int edges;          // out-degree sum of what it pushed (top-down), entries it scanned (bottom-up)
+    uint32_t nq, nh;    // queue entries and work items this wave wrote for the next level
 };
 
 // One level of one direction: top-down over the level's queue and hub items
 // (then, where it applies, in place), or bottom-up over the candidate
-// bitmap.  my_found (per thread) counts the vertices claimed; fedges, the
-// out-degree sum of what was pushed for the next level (top-down) or the
-// adjacency entries scanned (bottom-up).  Forward: from the pivot along
+// bitmap.  Forward: from the pivot along
 // out-edges, claiming active vertices into fvis.  Backward: along in-edges,
 // claiming active vertices into bvis, not only those of the forward set: the
 // giant SCC is fvis & bvis either way (a path from v to the pivot lies in
 // the forward set when v does), and the two directions then need not wait
 // for each other.
-__device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_t root, int64_t& my_found,
-                                           int64_t& fedges) {
+__device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_t root, Level& lv) {
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
     const bool bw = dir != 0;
@@ -653,8 +733,7 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
     const int64_t gwave = (int64_t)c.b * kW + c.wave;
     auto is_vis = [vis](int32_t u, int32_t) { return bit_of(vis, u); };
     const bool multi = a.n_roots > 0;
-    my_found = 0;
-    fedges = 0;
+    int64_t my_found = 0, fedges = 0;
     const uint64_t* qin = (L & 1) ? q1 : q0;
     uint64_t* qout = (L & 1) ? q0 : q1;
     const HubItem* hin = (L & 1) ? h1 : h0;
@@ -678,14 +757,15 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
             rchunk = min(rchunk, kGiantChunk);
             nh = (rdeg + rchunk - 1) / rchunk;
         } else {
-            n = load_agent(&gs->qn[dir][L % 3].v);
-            nh = load_agent(&gs->hn[dir][L % 3].v);
+            n = d.nq;
+            nh = d.nh;
             if (n < 0 || n > a.V || nh < 0 || nh > a.hub_cap) {  // cannot happen with exact claims
                 if (c.tid == 0) atomicOr(&gs->err.v, 4);
                 n = 0;
                 nh = 0;
             }
         }
+        if (n == 0 && nh == 0) return;
         static_assert((kGBlock & (kGBlock - 1)) == 0, "tile size");
         // entries per tile: a power of two from 64 to kGBlock, the
         // smallest that needs no more tiles than blocks, so a small
@@ -723,7 +803,7 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
             block_excl_scan<kW>(dg, excl, total, sm.tmp);
             sm.off[c.tid] = excl;
             sm.start[c.tid] = st;
-            if (c.tid == 0) c.edges_td += total;
+            if (c.wave == 0) c.edges_td += total;
             __syncthreads();
             for (int eb = 0; eb < total; eb += kGBlock) {
                 // the source of edge e is the last j with off[j] <= e
@@ -757,6 +837,7 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
             expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found,
                              a.td_local);
         block_flush_both(c, pq, qout, qn_out, hs, hout, hn_out);
+        lv = Level{(int)my_found, (int)fedges, pq.sent, hs.sent};
     } else {
         // ---- bottom-up over the candidate bitmap, one wave per group of
         // kU consecutive 64-vertex words; only that wave writes those
@@ -924,14 +1005,14 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
         if (tr && c.tid == 0)
             atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_cp[dir][L][2]),
                       (unsigned long long)((int64_t)wall_clock64() - tl0));
-        fedges = scanned;  // bottom-up pushes nothing: the low half of the level sum counts the scan
+        lv = Level{(int)my_found, scanned, 0, 0};  // bottom-up pushes nothing
     }
 }
 
 // The gather of a direction that switches from bottom-up back to top-down:
 // the last level's finds (vis & ~snap) become the next level's queue and hub
 // items.  Each wave loads 64 words at once, then expands the non-empty ones.
-__device__ __forceinline__ void gather_finds(Ctx& c, const Dir& d, int dir) {
+__device__ __forceinline__ void gather_finds(Ctx& c, const Dir& d, int dir, uint32_t& nq, uint32_t& nh) {
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
     GiantState* gs = a.gs;
@@ -962,6 +1043,8 @@ __device__ __forceinline__ void gather_finds(Ctx& c, const Dir& d, int dir) {
         }
     }
     block_flush_both(c, wq, q_next, qn_next, hs, h_next, hn_next);
+    nq = wq.sent;
+    nh = hs.sent;
 }
 
 // The giant's traversals: forward and backward in the same levels, one grid
@@ -978,13 +1061,14 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
     GiantState* gs = a.gs;
-    f = Dir{0, 0, 0, true, false};
-    b = Dir{0, 0, 0, true, false};
+    f = Dir{0, 0, 0, true, false, 0, 0};
+    b = Dir{0, 0, 0, true, false, 0, 0};
     *seeded_out = 1;
     if (a.n_roots > 0) {
         // level-0 input of both directions: every graph's root, marked
         // visited, queued or split into hub items like any claimed vertex
-        int64_t seeded = 0;
+        int seeded = 0;
+        uint32_t cnt[4];
         for (int dir = 0; dir < 2; ++dir) {
             PairQueue wq{c.stage(), 0};
             HubStage hs{sm.hv[c.wave], sm.hs[c.wave], sm.hd[c.wave], 0};
@@ -1002,114 +1086,128 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
                 push_next(ok, r, beg, wq, q0, &gs->qn[dir][0].v, hs, h0, &gs->hn[dir][0].v, unused);
             }
             block_flush_both(c, wq, q0, &gs->qn[dir][0].v, hs, h0, &gs->hn[dir][0].v);
+            cnt[2 * dir] = wq.sent;
+            cnt[2 * dir + 1] = hs.sent;
         }
-        Red r;
-        if (!gsync<true>(gs, c.G, sm, a.dbg, Red{block_sum(seeded, sm), 0, 0, 0}, &r, 1)) return false;
-        *seeded_out = r.s0;
+        int64_t r[8];
+        if (!gsync_sum<8, true>(c, {(uint32_t)wave_sum(seeded), 0, cnt[0], cnt[1], 0, 0, cnt[2], cnt[3]}, r))
+            return false;
+        *seeded_out = r[0];
+        f.nq = r[2];
+        f.nh = r[3];
+        b.nq = r[6];
+        b.nh = r[7];
     }
     while (f.live || b.live) {
         if (f.gather || b.gather) {
             // the visited bits were made exact after the level's barrier
+            uint32_t fq = 0, fh = 0, bq = 0, bh = 0;
 #pragma unroll 1
             for (int dir = 0; dir < 2; ++dir) {
                 const Dir d = dir ? b : f;
-                if (d.gather) gather_finds(c, d, dir);
+                uint32_t nq = 0, nh = 0;
+                if (d.gather) gather_finds(c, d, dir, nq, nh);
+                if (dir) {
+                    bq = nq;
+                    bh = nh;
+                } else {
+                    fq = nq;
+                    fh = nh;
+                }
             }
-            f.gather = b.gather = false;
             // the top-down level reads the queues coherently and visited bits
             // only as hints: no L2 invalidation
-            if (!gsync<false, false>(gs, c.G, sm, a.dbg)) return false;
+            int64_t r[4];
+            if (!gsync_sum<4, false>(c, {fq, fh, bq, bh}, r)) return false;
+            if (f.gather) {
+                f.nq = r[0];
+                f.nh = r[1];
+            }
+            if (b.gather) {
+                b.nq = r[2];
+                b.nh = r[3];
+            }
+            f.gather = b.gather = false;
         }
         const bool tdf = f.mode != 1, tdb = b.mode != 1;
         const int64_t edges0 = c.edges_td + c.edges_bu;  // thread 0's are the block's
         const bool tr = a.trace != 0;
         const int64_t tl0 = tr ? (int64_t)wall_clock64() : 0;
-        // per thread and direction: found (high 32 bits), pushed work or
-        // scanned entries (low).  One copy of the level's code serves both
-        // directions: the instruction cache (64 KB for two CUs) does not
-        // hold two, and a small level is bound by its first pass over the
-        // code.
-        int64_t pf = 0, pb = 0;
+        // One copy of the level's code serves both directions: the
+        // instruction cache (64 KB for two CUs) does not hold two.
+        Level lf{0, 0, 0, 0}, lb{0, 0, 0, 0};
 #pragma unroll 1
         for (int dir = 0; dir < 2; ++dir) {
             const Dir d = dir ? b : f;
             if (!d.live) continue;
-            int64_t found = 0, edges = 0;
-            level_work(c, d, dir, root, found, edges);
-            const int64_t pk = (found << 32) + edges;
-            if (dir) pb = pk;
-            else pf = pk;
+            Level lv{0, 0, 0, 0};
+            level_work(c, d, dir, root, lv);
+            lv.found = wave_sum(lv.found);
+            lv.edges = wave_sum(lv.edges);
+            if (dir) lb = lv;
+            else lf = lv;
         }
-        // ---- level totals: every block computes the same sums.  One sum per
-        // direction carries the level's finds (high 32 bits) and the next
-        // level's exact work or the scan (low 32 bits: at most E < 2^31, so no
-        // carry), both reduced in one block round
-        pf = wave_sum(pf);
-        pb = wave_sum(pb);
-        if (c.lane == 0) {
-            sm.red[c.wave] = pf;
-            sm.red2[c.wave] = pb;
-        }
-        __syncthreads();
-        pf = lane_get(row_incl(sm.red[c.lane & 15], (int64_t)0, [](int64_t x, int64_t y) { return x + y; }), 15);
-        pb = lane_get(row_incl(sm.red2[c.lane & 15], (int64_t)0, [](int64_t x, int64_t y) { return x + y; }), 15);
-        __syncthreads();
-        auto block_counts = [&](const Dir& d, int64_t pk, bool td, int dir) {
-            const int64_t blk = (int64_t)((uint64_t)pk >> 32);
+        // this wave's part of the work counters
+        auto wave_counts = [&](const Dir& d, const Level& lv, bool td, int dir) {
             if (td) {
-                c.found_td += blk;
+                c.found_td += (uint32_t)lv.found;
             } else {
-                const int64_t bscan = pk & 0xffffffffll;
-                c.found_bu += blk;
-                c.edges_bu += bscan;
-                if (tr && d.L < kLevelTrace && c.tid == 0) {
-                    atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_cp[dir][d.L][0]), (unsigned long long)bscan);
-                    if (dir == 0 && c.b < 1024 && gs->bu1_scan[c.b] == 0) {
-                        gs->bu1_scan[c.b] = bscan + 1;
-                        gs->bu1_work[c.b] = (int64_t)wall_clock64() - tl0;
+                c.found_bu += (uint32_t)lv.found;
+                c.edges_bu += (uint32_t)lv.edges;
+            }
+            if (tr && d.L < kLevelTrace) {
+                const int64_t scan = c.edges_td + c.edges_bu - edges0;
+                if (c.lane == 0)
+                    atomicAdd(reinterpret_cast<unsigned long long*>(&gs->lv_edges[dir][d.L]),
+                              (unsigned long long)(td ? scan : (int64_t)(uint32_t)lv.edges));
+                if (c.tid == 0) {  // wave 0 of each block
+                    if (!td)
+                        atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_cp[dir][d.L][0]),
+                                  (unsigned long long)(uint32_t)lv.edges);
+                    const unsigned long long wt = (unsigned long long)((int64_t)wall_clock64() - tl0);
+                    atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_wmax[dir][d.L]), wt);
+                    atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_wmin[dir][d.L]), ~wt);
+                    if (!td && dir == 0 && c.b < 1024 && gs->bu1_scan[c.b] == 0) {
+                        gs->bu1_scan[c.b] = (uint32_t)lv.edges + 1;
+                        gs->bu1_work[c.b] = (int64_t)wt;
                     }
                 }
             }
-            if (tr && d.L < kLevelTrace && c.tid == 0) {
-                const unsigned long long wt = (unsigned long long)((int64_t)wall_clock64() - tl0);
-                atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_wmax[dir][d.L]), wt);
-                atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_wmin[dir][d.L]), ~wt);
-            }
             // counters of level L+2: last read at the start of level L-1,
-            // first written in level L+1 (reset here, where the store overlaps
-            // the barrier's own atomics)
+            // first written in level L+1 (reset here, before the barrier)
             if (c.b == 0 && c.tid == 0) {
                 __hip_atomic_store(&gs->qn[dir][(d.L + 2) % 3].v, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(&gs->hn[dir][(d.L + 2) % 3].v, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         };
-        if (f.live) block_counts(f, pf, tdf, 0);
-        if (b.live) block_counts(b, pb, tdb, 1);
+        if (f.live) wave_counts(f, lf, tdf, 0);
+        if (b.live) wave_counts(b, lb, tdb, 1);
         // Top-down levels read what other blocks wrote in the level before
         // through coherent loads (queue entries, hub items, counts), a
         // candidate bitmap that is fixed during the traversal, and visited
         // bits only as a hint for the claim atomics: their barriers skip the
         // L2 invalidation (the acquire below catches up where needed).
-        Red r;
-        if (!gsync<true, false>(gs, c.G, sm, a.dbg, Red{pf, pb, tr ? c.edges_td + c.edges_bu - edges0 : 0, 0}, &r,
-                                3 | (tr ? 4 : 0)))
+        int64_t r[8];
+        if (!gsync_sum<8, false>(c,
+                                 {(uint32_t)lf.found, (uint32_t)lf.edges, lf.nq, lf.nh, (uint32_t)lb.found,
+                                  (uint32_t)lb.edges, lb.nq, lb.nh},
+                                 r))
             return false;
         // per direction: the level's totals, the end test and the switches
         bool acquire = false, failed = false;
-        auto decide = [&](Dir& d, int64_t pk, bool td, int dir) {
-            const int64_t found = (int64_t)((uint64_t)pk >> 32);
-            const int64_t next_edges = pk & 0xffffffffll;  // top-down levels: exact work of the next level
+        auto decide = [&](Dir& d, int64_t found, int64_t next_edges, int64_t nq, int64_t nh, bool td, int dir) {
+            // next_edges: top-down levels, the exact work of the next level
+            d.nq = nq;
+            d.nh = nh;
             if (c.b == 0 && c.tid == 0 && d.L < kLevelTrace) {
                 gs->lv_ts[dir][d.L] = wall_clock64();
                 gs->lv_found[dir][d.L] = found;
-                gs->lv_edges[dir][d.L] = r.s2;
                 gs->lv_mode[dir][d.L] = td ? 0 : 1;
             }
             d.visited += found;
             ++d.L;
             if (found == 0 ||
-                (td && a.td_local > 0 &&  // the waves may have expanded everything they found
-                 load_agent(&gs->qn[dir][d.L % 3].v) == 0 && load_agent(&gs->hn[dir][d.L % 3].v) == 0)) {
+                (td && a.td_local > 0 && nq == 0 && nh == 0)) {  // the waves expanded everything they found
                 d.live = false;
                 acquire = true;  // what follows reads the visited bits exactly
                 if (dir == 0 && c.b == 0 && c.tid == 0) gs->ts[2] = wall_clock64();  // the forward one's end
@@ -1132,8 +1230,8 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
                 d.gather = true;
             }
         };
-        if (f.live) decide(f, r.s0, tdf, 0);
-        if (b.live) decide(b, r.s1, tdb, 1);
+        if (f.live) decide(f, r[0], r[1], r[2], r[3], tdf, 0);
+        if (b.live) decide(b, r[4], r[5], r[6], r[7], tdb, 1);
         if (failed) return false;
         if (acquire) block_acquire();
     }
@@ -1144,16 +1242,17 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
 
 // One trim-1 sweep (trim_1_from_fq_gfq, src/trim_1_gfq.h:365-458) over
 // fin[0, n): act is updated in place, survivors are pushed to fout.
-// Returns the number this block trimmed.
+// trimmed and kept: this wave's counts (the same in every lane).
 // With lo >= 0 the block sweeps only fin[lo, lo + n), entries it wrote
 // itself, so no barrier has to make other blocks' entries visible first.
-__device__ __forceinline__ int64_t trim_sweep(Ctx& c, const int32_t* fin, int64_t n, int32_t* fout, int32_t* fcount,
-                                              int64_t lo = -1) {
+__device__ __forceinline__ void trim_sweep(Ctx& c, const int32_t* fin, int64_t n, int32_t* fout, int32_t* fcount,
+                                           int64_t lo, int& trimmed, int& kept) {
     const GiantArgs& a = c.a;
     WaveQueue wq{c.stage32(), 0};
     const uint64_t* act = a.act;
     auto live = [act](int32_t w, int32_t self) { return w != self && bit_of(act, w); };
-    int trimmed = 0, scanned = 0;
+    int scanned = 0;
+    trimmed = kept = 0;
     const bool local = lo >= 0;
     const int64_t first = local ? c.wave * kWave : (int64_t)c.b * kGBlock + c.wave * kWave;
     const int64_t step = local ? kGBlock : (int64_t)c.G * kGBlock;
@@ -1173,12 +1272,12 @@ __device__ __forceinline__ int64_t trim_sweep(Ctx& c, const int32_t* fin, int64_
         if (trim) {
             st_agent(&a.lab[v], v);
             atomicAnd(reinterpret_cast<unsigned long long*>(a.act + (v >> 6)), ~(1ull << (v & 63)));
-            ++trimmed;
         }
+        trimmed += __popcll(__ballot(trim));
+        kept += __popcll(__ballot(alive && !trim));
         wq_push<true>(wq, alive && !trim, v, fout, fcount);
     }
     block_flush(c, wq, fout, fcount);
-    return block_sum(trimmed, c.sm);
 }
 
 __device__ __forceinline__ int32_t uf_root_g(int32_t* parent, int32_t v) {
@@ -1205,7 +1304,7 @@ __device__ __forceinline__ bool lp_wcc(Ctx& c, const int32_t* q, int64_t n, int6
     const int64_t gt = (int64_t)c.b * kGBlock + c.tid;
     int32_t* col = a.parent;
     for (int64_t i = gt; i < n; i += nthreads) st_agent(&col[q[i]], q[i]);
-    if (!gsync(a.gs, c.G, c.sm, a.dbg)) return false;
+    if (!gsync(c)) return false;
     for (rounds = 1;; ++rounds) {
         int changed = 0;
         for (int64_t i = gt; i < n; i += nthreads) {
@@ -1232,9 +1331,9 @@ __device__ __forceinline__ bool lp_wcc(Ctx& c, const int32_t* q, int64_t n, int6
                 ++changed;
             }
         }
-        Red r;
-        if (!gsync<true>(a.gs, c.G, c.sm, a.dbg, Red{block_sum(changed, c.sm), 0, 0, 0}, &r, 1)) return false;
-        if (r.s0 == 0) return true;
+        int64_t r[4];
+        if (!gsync_sum<4, true>(c, {(uint32_t)wave_sum(changed), 0, 0, 0}, r)) return false;
+        if (r[0] == 0) return true;
         if (rounds > (int64_t)a.V + 2) {
             if (c.tid == 0) atomicOr(&a.gs->err.v, 2);
             return false;
@@ -1285,7 +1384,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
             st_agent(&a.ckey[v], ((uint64_t)(uint32_t)load_agent(&a.parent[v]) << 32) | (uint32_t)v);
             st_agent(&a.stamp[v], -1);
         }
-        if (!gsync(gs, c.G, c.sm, a.dbg)) return false;
+        if (!gsync(c)) return false;
         for (int64_t it = 0;; ++it) {  // largest key among the vertices that reach v
             int changed = 0;
             for (int64_t i = gt; i < n; i += nthreads) {
@@ -1306,9 +1405,9 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
                     ++changed;
                 }
             }
-            Red r;
-            if (!gsync<true>(gs, c.G, c.sm, a.dbg, Red{block_sum(changed, c.sm), 0, 0, 0}, &r, 1)) return false;
-            if (r.s0 == 0) break;
+            int64_t r[4];
+            if (!gsync_sum<4, true>(c, {(uint32_t)wave_sum(changed), 0, 0, 0}, r)) return false;
+            if (r[0] == 0) break;
             if (it > (int64_t)a.V + 2) {
                 if (c.tid == 0) atomicOr(&gs->err.v, 2);
                 return false;
@@ -1321,7 +1420,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
                 st_agent(&a.aux[v], v);
             }
         }
-        if (!gsync(gs, c.G, c.sm, a.dbg)) return false;
+        if (!gsync(c)) return false;
         for (int64_t it = 0;; ++it) {  // v joins its colour's SCC through an out-neighbour in it
             int changed = 0;
             for (int64_t i = gt; i < n; i += nthreads) {
@@ -1337,9 +1436,9 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
                     }
                 }
             }
-            Red r;
-            if (!gsync<true>(gs, c.G, c.sm, a.dbg, Red{block_sum(changed, c.sm), 0, 0, 0}, &r, 1)) return false;
-            if (r.s0 == 0) break;
+            int64_t r[4];
+            if (!gsync_sum<4, true>(c, {(uint32_t)wave_sum(changed), 0, 0, 0}, r)) return false;
+            if (r[0] == 0) break;
             if (it > (int64_t)a.V + 2) {
                 if (c.tid == 0) atomicOr(&gs->err.v, 2);
                 return false;
@@ -1350,7 +1449,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
             const int32_t r = load_agent(&a.stamp[v]);
             if (r >= 0 && r != v) atomicMin(&a.aux[r], v);
         }
-        if (!gsync(gs, c.G, c.sm, a.dbg)) return false;
+        if (!gsync(c)) return false;
         // label the SCCs found, take them out of the active set, queue the rest
         WaveQueue wq{c.stage32(), 0};
         int found = 0;
@@ -1369,9 +1468,9 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
             wq_push<true>(wq, i < n && r < 0, v, qn, cnt);
         }
         block_flush(c, wq, qn, cnt);
-        Red r;
-        if (!gsync<true>(gs, c.G, c.sm, a.dbg, Red{block_sum(found, c.sm), 0, 0, 0}, &r, 1)) return false;
-        sccs += r.s0;
+        int64_t r[4];
+        if (!gsync_sum<4, true>(c, {(uint32_t)wave_sum(found), 0, 0, 0}, r)) return false;
+        sccs += r[0];
         n = load_agent(cnt);
         cur ^= 1;
         ++s;
@@ -1401,18 +1500,18 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
     int it = 0;
     const int64_t nthreads = (int64_t)c.G * kGBlock;
     const int64_t gt = (int64_t)c.b * kGBlock + c.tid;
-    // Sweep s pushes into fqn[s % 3]; all blocks read it after the barrier.
-    // It clears fqn[(s + 1) % 3] for the next sweep: that counter was last read
-    // after sweep s - 2, i.e. before the barrier that ended sweep s - 1.
+    // Sweep s pushes at fqn[s % 3]; what it kept is summed by its barrier.
+    // It clears fqn[(s + 1) % 3] for the next sweep: that counter was last
+    // used in sweep s - 2, before the barrier that ended it.
     auto sweep = [&]() -> bool {
         if (c.b == 0 && c.tid == 0)
             __hip_atomic_store(&gs->fqn[(s + 1) % 3].v, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int64_t t = s == 0 ? trim_sweep(c, buf(cur), own_n, buf(cur ^ 1), &gs->fqn[s % 3].v, own_lo)
-                                 : trim_sweep(c, buf(cur), n, buf(cur ^ 1), &gs->fqn[s % 3].v);
-        Red r;
-        if (!gsync<true>(gs, c.G, c.sm, a.dbg, Red{t, 0, 0, 0}, &r, 1)) return false;
-        trim1 += r.s0;
-        n = load_agent(&gs->fqn[s % 3].v);
+        int t, kept;
+        trim_sweep(c, buf(cur), s == 0 ? own_n : n, buf(cur ^ 1), &gs->fqn[s % 3].v, s == 0 ? own_lo : -1, t, kept);
+        int64_t r[4];
+        if (!gsync_sum<4, true>(c, {(uint32_t)t, (uint32_t)kept, 0, 0}, r)) return false;
+        trim1 += r[0];
+        n = r[1];
         cur ^= 1;
         ++s;
         return true;
@@ -1426,7 +1525,7 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
         ++it;
     }
     bool wcc = false;
-    if (n > 0 && s == 0 && !gsync(gs, c.G, c.sm, a.dbg)) return false;  // no sweep: the queue's barrier
+    if (n > 0 && s == 0 && !gsync(c)) return false;  // no sweep: the queue's barrier
     if (n > 0) {
         // P8-P10: pattern detection against the current act, then commit.
         // Over the active queue (trim_*_from_fq, src/trim_2_3.h:146-283,
@@ -1474,7 +1573,7 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
             for (int j = 0; j < nl; ++j)
                 pattern_check<true>(a.fwb, a.fwa, a.bwb, a.bwa, a.lab, a.stamp, a.act, lq[j]);
         }
-        if (!gsync(gs, c.G, c.sm, a.dbg)) return false;
+        if (!gsync(c)) return false;
         int c2 = 0, c3 = 0;
         each_active([&](int32_t v) {
             if (a.lab[v] >= 0) {
@@ -1483,11 +1582,10 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
                 else ++c3;
             }
         });
-        const int64_t b2 = block_sum(c2, c.sm), b3 = block_sum(c3, c.sm);
-        Red r;
-        if (!gsync<true>(gs, c.G, c.sm, a.dbg, Red{b2, b3, 0, 0}, &r, 3)) return false;
-        p2 = r.s0;
-        p3 = r.s1;
+        int64_t r[4];
+        if (!gsync_sum<4, true>(c, {(uint32_t)wave_sum(c2), (uint32_t)wave_sum(c3), 0, 0}, r)) return false;
+        p2 = r[0];
+        p3 = r[1];
         // P11: one more trim-1 sweep
         if (!sweep()) return false;
         // (wcc_mode 1 and 2 run in k_tail, launched when something is left)
@@ -1498,7 +1596,7 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
                 const int32_t v = g[i];
                 st_agent(&a.parent[v], v);
             }
-            if (!gsync(gs, c.G, c.sm, a.dbg)) return false;
+            if (!gsync(c)) return false;
             for (int64_t i = gt; i < n; i += nthreads) {
                 const int32_t v = g[i];
                 for (int32_t k = a.fwb[v]; k < a.fwb[v + 1]; ++k) {
@@ -1518,7 +1616,7 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
                     }
                 }
             }
-            if (!gsync(gs, c.G, c.sm, a.dbg)) return false;
+            if (!gsync(c)) return false;
             for (int64_t i = gt; i < n; i += nthreads) {
                 const int32_t v = g[i];
                 st_agent(&a.parent[v], uf_root_g(a.parent, v));
@@ -1542,59 +1640,26 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
 
 }  // namespace
 
-// Start of a k_giant launch: block 0 clears the state and the control block
-// (device-coherent stores, completed before the epoch is published); the
-// other blocks wait, bounded, for the launch's epoch and then acquire.
-// Returns false after a timed-out wait.
-__device__ __forceinline__ bool launch_start(const GiantArgs& a, Smem& sm) {
-    GiantState* gs = a.gs;
-    if (blockIdx.x == 0) {
-        int64_t* p = reinterpret_cast<int64_t*>(gs);
-        for (int i = threadIdx.x; i < a.state_words; i += kGBlock) st_agent(&p[i], (int64_t)0);
-        int64_t* q = reinterpret_cast<int64_t*>(a.ctl);
-        for (int i = threadIdx.x; i < a.ctl_words; i += kGBlock) st_agent(&q[i], (int64_t)0);
-        wait_vm();
-        __syncthreads();
-        if (threadIdx.x == 0) st_agent(&gs->epoch, a.epoch);
-        return true;
-    }
-    if (threadIdx.x == 0) {
-        int ok = 1, spins = 0;
-        while (load_agent(&gs->epoch) != a.epoch) {
-            __builtin_amdgcn_s_sleep(2);
-            if (++spins > kSpinCap) {
-                atomicOr(&gs->err.v, 1);
-                ok = 0;
-                break;
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        sm.ok = ok;
-    }
-    __syncthreads();
-    return sm.ok;
-}
-
 __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
     __shared__ Smem sm;
-    if (threadIdx.x == 0) {
-        a.dbg[blockIdx.x] = 0;
-        a.dbg[gridDim.x + blockIdx.x] = 0;
-        sm.nbar = 0;
-        sm.gbase = 0;  // block 0 clears the state (gen included) before any block starts
-    }
-    if (!launch_start(a, sm)) return;
-    Ctx c{a, (int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, lane_id(), wave_id(), sm, 0, 0, 0, 0};
+    Ctx c{a, (int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, lane_id(), wave_id(), sm, 0, 0, 0, 0, 0};
     GiantState* gs = a.gs;
+    // Block 0 clears the state and the control block.  No other block writes
+    // either before the first barrier (whose records are not part of them),
+    // so none has to wait for it.
+    if (c.b == 0) {
+        int64_t* p = reinterpret_cast<int64_t*>(gs);
+        for (int i = c.tid; i < a.state_words; i += kGBlock) st_agent(&p[i], (int64_t)0);
+        int64_t* q = reinterpret_cast<int64_t*>(a.ctl);
+        for (int i = c.tid; i < a.ctl_words; i += kGBlock) st_agent(&q[i], (int64_t)0);
+        wait_vm();
+        __syncthreads();
+    }
     const int64_t total_waves = (int64_t)c.G * kW;
     const int64_t gwave = (int64_t)c.b * kW + c.wave;
     const bool stamp = c.b == 0 && c.tid == 0;  // phase timestamps (constant-rate clock)
     if (stamp) gs->ts[0] = wall_clock64();
-    if (c.tid == 0) {  // launch ramp: when each block started
-        const unsigned long long t = wall_clock64();
-        atomicMax(reinterpret_cast<unsigned long long*>(&gs->t_start[0]), ~t);  // min as max of ~t (state starts at 0)
-        atomicMax(reinterpret_cast<unsigned long long*>(&gs->t_start[1]), t);
-    }
+    const unsigned long long t_begin = a.trace ? wall_clock64() : 0;  // launch ramp: when each block started
 
     // ---- phase A: trim-1-first (raw degree 0 either way), act bitmap,
     // cleared traversal bitmaps, pivot = largest out*in (lowest id on ties).
@@ -1676,57 +1741,45 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
             besti = oi;
         }
     }
+    surv = wave_sum(surv);
     if (c.lane == 0) {
         sm.red2[c.wave] = bestp;
         sm.bi[c.wave] = besti;
+        sm.red[c.wave] = surv;
     }
-    const int64_t surv_blk = block_sum(surv, sm);
-    if (c.tid == 0) {
-        for (int w = 1; w < kW; ++w)
-            if (pivot_better(sm.red2[w], sm.bi[w], bestp, besti)) {
-                bestp = sm.red2[w];
-                besti = sm.bi[w];
-            }
-        st_agent(&a.part[(int64_t)kPivP * c.G + c.b], (int64_t)(bestp));
-        st_agent(&a.part[(int64_t)kPivI * c.G + c.b], (int64_t)(besti));
-        st_agent(&a.part[(int64_t)kSurv * c.G + c.b], (int64_t)(surv_blk));
-        const unsigned long long t = wall_clock64();  // trim-1-first done in this block
-        atomicMax(reinterpret_cast<unsigned long long*>(&gs->t_arrive[0]), ~t);
-        atomicMax(reinterpret_cast<unsigned long long*>(&gs->t_arrive[1]), t);
-    }
-    if (!gsync(gs, c.G, sm, a.dbg)) return;
-    // every block reduces the pivot candidates and the survivor count
-    bestp = 0;
-    besti = INT32_MAX;
-    for (int i = c.tid; i < c.G; i += kGBlock) {
-        const int64_t p = load_agent(&a.part[(int64_t)kPivP * c.G + i]);
-        const int32_t id = (int32_t)load_agent(&a.part[(int64_t)kPivI * c.G + i]);
-        if (pivot_better(p, id, bestp, besti)) {
-            bestp = p;
-            besti = id;
-        }
-    }
+    const unsigned long long t_arrive = a.trace ? wall_clock64() : 0;
+    // the barrier carries each block's candidate and survivor count
+    PivotFold pf;
+    const bool go = gsync_with<4, true>(
+        c,
+        [&]() {
+            int64_t p = sm.red2[c.lane & 15];
+            int32_t id = sm.bi[c.lane & 15];
+            const int64_t n = row_incl(sm.red[c.lane & 15], (int64_t)0, [](int64_t x, int64_t y) { return x + y; });
 #pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) {
-        const int64_t op = __shfl_xor(bestp, d, kWave);
-        const int32_t oi = __shfl_xor(besti, d, kWave);
-        if (pivot_better(op, oi, bestp, besti)) {
-            bestp = op;
-            besti = oi;
-        }
+            for (int d = kW / 2; d > 0; d >>= 1) {
+                const int64_t op = __shfl_xor(p, d, kWave);
+                const int32_t oi = __shfl_xor(id, d, kWave);
+                if (pivot_better(op, oi, p, id)) {
+                    p = op;
+                    id = oi;
+                }
+            }
+            const uint32_t nn = (uint32_t)lane_get(n, kW - 1);
+            return c.lane == 0 ? (uint32_t)((uint64_t)p >> 32) : c.lane == 1 ? (uint32_t)p : c.lane == 2 ? (uint32_t)id : nn;
+        },
+        pf);
+    if (!go) return;
+    bestp = lane_get(sm.tot[0][0], 0);
+    besti = (int32_t)lane_get(sm.tot[0][1], 0);
+    const int64_t fq0 = lane_get(sm.tot[0][2], 0);
+    if (a.trace && c.tid == 0) {  // min as max of ~t (the state starts at 0)
+        using ull = unsigned long long;
+        atomicMax(reinterpret_cast<ull*>(&gs->t_start[0]), ~t_begin);
+        atomicMax(reinterpret_cast<ull*>(&gs->t_start[1]), t_begin);
+        atomicMax(reinterpret_cast<ull*>(&gs->t_arrive[0]), ~t_arrive);
+        atomicMax(reinterpret_cast<ull*>(&gs->t_arrive[1]), t_arrive);
     }
-    if (c.lane == 0) {
-        sm.red2[c.wave] = bestp;
-        sm.bi[c.wave] = besti;
-    }
-    __syncthreads();
-    for (int w = 0; w < kW; ++w)
-        if (pivot_better(sm.red2[w], sm.bi[w], bestp, besti)) {
-            bestp = sm.red2[w];
-            besti = sm.bi[w];
-        }
-    __syncthreads();
-    const int64_t fq0 = sum_slot(a.part, kSurv, c.G, sm);
     const int32_t root = (a.n_roots == 0 && bestp > 0 && besti < a.V) ? besti : -1;
     if (stamp) gs->ts[1] = wall_clock64();
 
@@ -1775,29 +1828,26 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
         gcnt += __popcll(g);
         if (want_min && g && w <= (root >> 6)) mn = min(mn, (int32_t)(w * 64 + __ffsll((unsigned long long)g) - 1));
     }
-    const int64_t cnt_blk = block_sum(cnt, sm), giant_blk = block_sum(gcnt, sm);
-    if (want_min) {
-        mn = wave_min(mn);
-        if (c.lane == 0) sm.tmp[c.wave] = mn;
-        __syncthreads();
-        mn = lane_get(row_incl(sm.tmp[c.lane & 15], INT32_MAX, [](int32_t x, int32_t y) { return min(x, y); }), 15);
-        __syncthreads();
-    }
+    const int wmn = wave_min(mn);
+    const uint32_t key = wmn < INT32_MAX ? (uint32_t)(INT32_MAX - wmn) : 0u;
     if (a.trace && c.tid == 0) atomicMax((unsigned long long*)&gs->post_cp[0], (unsigned long long)wall_clock64());
-    if (c.tid == 0) {
-        st_agent(&a.part[(int64_t)kPost * c.G + c.b], (int64_t)(cnt_blk));
-        st_agent(&a.part[(int64_t)kGiantN * c.G + c.b], (int64_t)(giant_blk));
-        st_agent(&a.part[(int64_t)kEdgeTD * c.G + c.b], (int64_t)(c.edges_td));
-        st_agent(&a.part[(int64_t)kEdgeBU * c.G + c.b], (int64_t)(c.edges_bu));
-        st_agent(&a.part[(int64_t)kFoundTD * c.G + c.b], (int64_t)(c.found_td));
-        st_agent(&a.part[(int64_t)kFoundBU * c.G + c.b], (int64_t)(c.found_bu));
-    }
+    stage_words<8>(c, {(uint32_t)wave_sum((int)cnt), (uint32_t)wave_sum((int)gcnt), key, (uint32_t)c.edges_td,
+                       (uint32_t)c.edges_bu, (uint32_t)c.found_td, (uint32_t)c.found_bu, 0});
     {
-        Red r;
-        if (!gsync<true>(gs, c.G, sm, a.dbg, Red{0, 0, 0, mn < INT32_MAX ? (int64_t)INT32_MAX - mn : 0}, &r, 8))
-            return;
-        if (want_min) gmin = (int32_t)((int64_t)INT32_MAX - r.key);
+        PostFold f{c.b};
+        auto src = [&]() {
+            if (c.lane != 2) return staged_sum(sm, c.lane);
+            uint32_t k = 0;
+            for (int i = 0; i < kW; ++i) k = max(k, sm.bv[2][i]);
+            return k;
+        };
+        if (!gsync_with<8, true>(c, src, f)) return;
     }
+    if (want_min) gmin = (int32_t)((int64_t)INT32_MAX - lane_get(sm.tot[0][2], 0));
+    int64_t off = lane_get(sm.tot[0][7], 0);  // active vertices of the blocks before this one
+    const int64_t tot = lane_get(sm.tot[0][0], 0);
+    const int64_t giant = lane_get(sm.tot[0][1], 0);
+    const int64_t w0 = sm.tot[0][3], w1 = sm.tot[0][4], w2 = sm.tot[0][5], w3 = sm.tot[0][6];
     if (a.trace && c.tid == 0) atomicMax((unsigned long long*)&gs->post_cp[1], (unsigned long long)wall_clock64());
     // the labels: one word per lane, the wave loads 64 words at once (its own
     // block's, narrowed above), then writes them four words at a time, four
@@ -1835,18 +1885,6 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
             }
         }
     }
-    // exclusive prefix of the block counts, then an ordered block-local scan
-    int64_t off, tot;
-    {
-        int64_t x0 = 0, xt = 0;
-        for (int i = c.tid; i < c.G; i += kGBlock) {
-            const int64_t x = load_agent(&a.part[(int64_t)kPost * c.G + i]);
-            xt += x;
-            if (i < c.b) x0 += x;
-        }
-        off = block_sum(x0, sm);
-        tot = block_sum(xt, sm);
-    }
     // this block's slice of the queue, the active vertices of its own words.
     // The first trim sweep takes it alone (no barrier before it): a sweep
     // clears act bits only of the vertices it sweeps, so no block's sweep
@@ -1868,9 +1906,6 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
     }
     if (a.trace && c.tid == 0) atomicMax((unsigned long long*)&gs->post_cp[2], (unsigned long long)wall_clock64());
     if (c.b == 0) {
-        const int64_t w0 = sum_slot(a.part, kEdgeTD, c.G, sm), w1 = sum_slot(a.part, kEdgeBU, c.G, sm);
-        const int64_t w2 = sum_slot(a.part, kFoundTD, c.G, sm), w3 = sum_slot(a.part, kFoundBU, c.G, sm);
-        const int64_t giant = sum_slot(a.part, kGiantN, c.G, sm);
         if (c.tid == 0) {
             gs->root = root;
             gs->fq0 = fq0;
@@ -1915,24 +1950,17 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
         }
         if (stamp) gs->ts[5] = wall_clock64();
     }
+    if (stamp) gs->bar_next = a.bar_base + c.nbar;
 }
 
 __global__ __launch_bounds__(kGBlock) void k_tail(const GiantArgs a) {
     __shared__ Smem sm;
     GiantState* gs = a.gs;
-    if (threadIdx.x == 0) {
-        a.dbg[blockIdx.x] = 0;
-        a.dbg[gridDim.x + blockIdx.x] = 0;
-        sm.nbar = 0;
-        sm.gbase = gs->gen.v;  // barrier generations continue from k_giant's
-        sm.ok = gs->err.v == 0;
-    }
-    __syncthreads();
-    if (!sm.ok) return;  // k_giant failed; the host reports its error
+    if (gs->err.v != 0) return;  // k_giant failed; the host reports its error
     const int64_t n = gs->n_final;
     int cur = (int)gs->final_sel;
     if (n == 0) return;
-    Ctx c{a, (int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, lane_id(), wave_id(), sm, 0, 0, 0, 0};
+    Ctx c{a, (int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, lane_id(), wave_id(), sm, 0, 0, 0, 0, 0};
     const bool lead = c.b == 0 && c.tid == 0;
     int64_t rounds = 0, sccs = 0;
     if (a.wcc_mode == 1) {  // P12 by label propagation: parent = smallest id of the WCC
@@ -1951,7 +1979,10 @@ __global__ __launch_bounds__(kGBlock) void k_tail(const GiantArgs a) {
             a.fq_n_ctl[cur] = 0;
         }
     }
-    if (lead) gs->ts[5] = wall_clock64();
+    if (lead) {
+        gs->bar_next = a.bar_base + c.nbar;
+        gs->ts[5] = wall_clock64();
+    }
 }
 
 __global__ void k_zero_i64(int64_t* p, int64_t n) {
@@ -1992,15 +2023,12 @@ int64_t giant_bu_mult(int grid) {
 }
 
 hipError_t launch_giant(const GiantArgs& a, Ctl* ctl, int grid, hipStream_t s, hipEvent_t before) {
-    static_assert(kGiantStateHead % 8 == 0 && sizeof(Ctl) % 8 == 0 && offsetof(GiantState, epoch) % 8 == 0,
-                  "state sizes");
-    static std::atomic<int64_t> epochs{0};
+    static_assert(kGiantStateHead % 8 == 0 && sizeof(Ctl) % 8 == 0 && sizeof(GiantState) % 8 == 0, "state sizes");
     hipError_t e;
     if (before && (e = hipEventRecord(before, s)) != hipSuccess) return e;
     GiantArgs copy = a;
     copy.ctl = ctl;
-    copy.epoch = ++epochs;
-    copy.state_words = (int32_t)((a.trace ? offsetof(GiantState, epoch) : kGiantStateHead) / 8);
+    copy.state_words = (int32_t)((a.trace ? sizeof(GiantState) : kGiantStateHead) / 8);
     copy.ctl_words = (int32_t)(sizeof(Ctl) / 8);
     void* args[] = {&copy};
     return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_giant), dim3(grid), dim3(kGBlock), args,

@@ -75,10 +75,11 @@ struct ispan_ctx {
     HubItem* gh[2] = {nullptr, nullptr};   // forward hub work items
     HubItem* ghb[2] = {nullptr, nullptr};  // backward
     uint64_t* snapb = nullptr;             // backward bottom-up snapshot
-    int64_t* gpart = nullptr;
     int32_t* gdbg = nullptr;
     GiantState* gstate = nullptr;
     GiantState* h_gstate = nullptr;  // pinned
+    uint64_t* bar = nullptr;         // grid-barrier records (GiantArgs::bar) and how many barriers they have seen
+    uint32_t bar_base = 0;
     hipEvent_t ev[16] = {};
     bool have_solution = false;
     // batched solves: consecutive graphs grouped so that each group's
@@ -168,7 +169,6 @@ void free_solve_buffers(ispan_ctx* ctx) {
     dfree(ctx->ghb[0]);
     dfree(ctx->ghb[1]);
     dfree(ctx->snapb);
-    dfree(ctx->gpart);
     dfree(ctx->gdbg);
     if (ctx->sort_tmp) (void)hipFree(ctx->sort_tmp);
     ctx->sort_tmp = nullptr;
@@ -258,7 +258,6 @@ int ensure_buffers(ispan_ctx* ctx, int32_t V, int64_t E) {
         CK(hipMalloc(&ctx->ghb[i], (size_t)giant_hub_capacity(E) * sizeof(HubItem)));
     }
     CK(hipMalloc(&ctx->snapb, nw * 8));
-    CK(hipMalloc(&ctx->gpart, (size_t)kGiantSlots * std::max(ctx->coop_grid, 1) * 8));
     CK(hipMalloc(&ctx->gdbg, (size_t)2 * std::max(ctx->coop_grid, 1) * 4));
     size_t bytes = 0;
     CK(rocprim::radix_sort_keys(nullptr, bytes, ctx->keys, ctx->keys_alt, (size_t)nv, 0, 64, ctx->stream));
@@ -471,7 +470,8 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
         ga.hb1 = ctx->ghb[1];
         ga.fq = ctx->fq[1];
         ga.gs = ctx->gstate;
-        ga.part = ctx->gpart;
+        ga.bar = ctx->bar;
+        ga.bar_base = ctx->bar_base;
         ga.fq_n_out = &ctx->ctl->fq_n[1];
         ga.hub_cap = giant_hub_capacity(E);
         ga.alpha = P->alpha;
@@ -520,6 +520,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
             // by the readbacks of later launches.
             CK(hipStreamSynchronize(s));
             ++syncs;
+            ctx->bar_base = (uint32_t)ctx->h_gstate->bar_next;
             *ctx->h_ctl = Ctl{};
             ctx->h_ctl->unlabelled = (int32_t)ctx->h_gstate->unlabelled;
             bool tail = false;
@@ -528,15 +529,21 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
                 // active vertices are left: the WCC by label propagation, or
                 // the colouring SCC method, on the device (one more launch
                 // and wait, as the mice phase would take)
+                ga.bar_base = ctx->bar_base;
                 CK(launch_tail(ga, ctx->coop_grid, s));
                 CK(hipMemcpyAsync(ctx->h_gstate, ctx->gstate,
                                   ctx->level_trace ? sizeof(GiantState) : kGiantStateHead, hipMemcpyDeviceToHost, s));
                 CK(launch_fill_i32(&ctx->ctl->unlabelled, 0, 1, 1, s));
                 CK(launch_count_unlabelled(ctx->lab, V, ctx->batch_sel, ctx->ctl, G, s));
                 if ((rc = readback(ctx, &syncs))) return rc;
+                ctx->bar_base = (uint32_t)ctx->h_gstate->bar_next;
             }
             const GiantState& gs = *ctx->h_gstate;
             if (gs.err.v) {
+                // the blocks stopped at different barriers: start the records over
+                ctx->bar_base = 0;
+                CK(launch_fill_i32(reinterpret_cast<int32_t*>(ctx->bar), 0,
+                                   (int64_t)kBarBytesPerBlock / 4 * ctx->coop_grid, 1, s));
                 if (gs.err.v & 1) {  // where did the blocks stop?
                     std::vector<int32_t> d((size_t)2 * ctx->coop_grid);
                     if (hipMemcpy(d.data(), ctx->gdbg, d.size() * 4, hipMemcpyDeviceToHost) == hipSuccess) {
@@ -549,7 +556,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
                             zero += d[b] == 0;
                         }
                         fprintf(stderr, "[ispan] barrier timeout: grid %d, arrived min %d max %d (blocks at 0: %d), "
-                                "passed min %d max %d, gen %d\n", ctx->coop_grid, amin, amax, zero, pmin, pmax, gs.gen.v);
+                                "passed min %d max %d\n", ctx->coop_grid, amin, amax, zero, pmin, pmax);
                     }
                 }
                 ctx->err = gs.err.v & 1   ? "giant phase: grid barrier timed out"
@@ -781,10 +788,20 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
         // k_mice left this rest alone: the colouring method labels it
         GiantArgs gc = ga_tail;
         gc.wcc_mode = 2;
+        gc.bar_base = ctx->bar_base;
         CK(launch_tail(gc, ctx->coop_grid, s));
+        CK(hipMemcpyAsync(ctx->h_gstate, ctx->gstate, kGiantStateHead, hipMemcpyDeviceToHost, s));
         CK(launch_fill_i32(&ctx->ctl->unlabelled, 0, 1, 1, s));
         CK(launch_count_unlabelled(ctx->lab, V, ctx->batch_sel, ctx->ctl, G, s));
         if ((rc = readback(ctx, &syncs))) return rc;
+        ctx->bar_base = (uint32_t)ctx->h_gstate->bar_next;
+        if (ctx->h_gstate->err.v) {
+            ctx->bar_base = 0;
+            CK(launch_fill_i32(reinterpret_cast<int32_t*>(ctx->bar), 0,
+                               (int64_t)kBarBytesPerBlock / 4 * ctx->coop_grid, 1, s));
+            ctx->err = "colouring method: grid barrier timed out or round cap exceeded";
+            return ctx->h_gstate->err.v & 2 ? ISPAN_ERR_ITER : ISPAN_ERR_HIP;
+        }
         local.coloured = local.mice;
         local.mice = 0;
     }
@@ -961,8 +978,11 @@ int ispan_ctx_create(ispan_ctx** out, int device) {
         if (const char* env = getenv("ISPAN_LEVEL_TRACE")) ctx->level_trace = atoi(env) != 0;
     }
     if (hipMalloc(&ctx->gstate, sizeof(GiantState)) != hipSuccess) return fail(ISPAN_ERR_NOMEM);
-    // epoch 0: no launch of this process has cleared it (the kernel clears the rest)
-    if (hipMemset(ctx->gstate, 0, sizeof(GiantState)) != hipSuccess) return fail(ISPAN_ERR_HIP);
+    {
+        const size_t bytes = (size_t)kBarBytesPerBlock * std::max(ctx->coop_grid, 1);
+        if (hipMalloc(&ctx->bar, bytes) != hipSuccess) return fail(ISPAN_ERR_NOMEM);
+        if (hipMemset(ctx->bar, 0, bytes) != hipSuccess) return fail(ISPAN_ERR_HIP);
+    }
     if (hipHostMalloc(&ctx->h_gstate, sizeof(GiantState), hipHostMallocDefault) != hipSuccess)
         return fail(ISPAN_ERR_NOMEM);
     if (hipMalloc(&ctx->ctl, sizeof(Ctl)) != hipSuccess) return fail(ISPAN_ERR_NOMEM);
@@ -982,6 +1002,7 @@ int ispan_ctx_destroy(ispan_ctx* ctx) {
     free_workspace(ctx);
     dfree(ctx->ctl);
     dfree(ctx->gstate);
+    dfree(ctx->bar);
     dfree(ctx->hist);
     if (ctx->h_ctl) (void)hipHostFree(ctx->h_ctl);
     if (ctx->h_gstate) (void)hipHostFree(ctx->h_gstate);
@@ -1779,7 +1800,6 @@ size_t carve_solve_state(ispan_ctx* c, unsigned char* base, int32_t V, int64_t E
         take(c->ghb[i], (size_t)giant_hub_capacity(E) * sizeof(HubItem));
     }
     take(c->snapb, nw * 8);
-    take(c->gpart, (size_t)kGiantSlots * std::max(c->coop_grid, 1) * 8);
     take(c->gdbg, (size_t)2 * std::max(c->coop_grid, 1) * 4);
     unsigned char* st = nullptr;
     take(st, sort_bytes + 256);
@@ -1787,6 +1807,7 @@ size_t carve_solve_state(ispan_ctx* c, unsigned char* base, int32_t V, int64_t E
     c->sort_tmp_bytes = sort_bytes + 256;
     take(c->ctl, sizeof(Ctl));
     take(c->gstate, sizeof(GiantState));
+    take(c->bar, (size_t)kBarBytesPerBlock * std::max(c->coop_grid, 1));
     take(c->fw_first, (size_t)std::max(V, 1) * 4);
     take(c->bw_first, (size_t)std::max(V, 1) * 4);
     return off;
@@ -1836,9 +1857,10 @@ int ispan_scc_detection_noalloc(int32_t V, int64_t E, const int32_t* d_fw_beg, c
     c.bwa = d_bw_adj;
     if ((rc = check_bound(&c, &P))) return rc;
     if (V > 0) {
-        // the kernel's state sits wherever this call's layout puts it: its
-        // epoch word must not hold a value a launch is still to publish
-        if (launch_fill_i32(reinterpret_cast<int32_t*>(&c.gstate->epoch), 0, 2, 1, c.stream) != hipSuccess ||
+        // the barrier records sit wherever this call's layout puts them: they
+        // must not hold a tag a barrier is still to use
+        if (launch_fill_i32(reinterpret_cast<int32_t*>(c.bar), 0, (int64_t)kBarBytesPerBlock / 4 * c.coop_grid, 32,
+                            c.stream) != hipSuccess ||
             launch_first(c.fwb, c.fwa, V, c.fw_first, c.grid, c.stream) != hipSuccess ||
             launch_first(c.bwb, c.bwa, V, c.bw_first, c.grid, c.stream) != hipSuccess)
             return ISPAN_ERR_HIP;
