@@ -7,6 +7,8 @@
 //   bvis[W]  uint64  bit v: reached by the backward traversal inside fvis
 // The bitmaps are 2 MB each at V = 2^24, so the random probes of the
 // traversals stay in L2/MALL while adjacency is streamed from HBM.
+#include <algorithm>
+
 #include "common.h"
 #include "device_util.h"
 
@@ -765,68 +767,156 @@ __global__ __launch_bounds__(kBlock) void k_check_csr(const int32_t* __restrict_
 // Extends get_scc_result (src/load_print.cpp:24-60), which tallies SCC
 // sizes in a std::map but prints only count classes.
 //
-// size[lab[v]] += 1 over canonical labels.  A wave takes 64 consecutive
-// vertices; lanes that share a label add together (one leader per round,
-// up to kSizeRounds rounds), the rest one atomic each, so a label carried by
-// a third of the vertices (R-MAT's giant) costs one atomic per wave step
-// instead of one per vertex.
-constexpr int kSizeRounds = 4;
-__global__ __launch_bounds__(kBlock) void k_scc_sizes(const int32_t* __restrict__ lab, int32_t V, int32_t* size) {
-    const int lane = lane_id();
-    const int64_t waves = (int64_t)gridDim.x * (kBlock / kWave);
-    for (int64_t base = ((int64_t)blockIdx.x * (kBlock / kWave) + wave_id()) * kWave; base < V;
-         base += waves * kWave) {
-        const int64_t v = base + lane;
-        const int32_t l = v < V ? lab[v] : -1;
-        bool todo = v < V;
-        for (int r = 0; r < kSizeRounds; ++r) {
-            const uint64_t m = __ballot(todo);
-            if (!m) break;
-            const int lead = __ffsll((unsigned long long)m) - 1;
-            const int32_t L = lane_get(l, lead);
-            const uint64_t same = __ballot(todo && l == L);
-            if (lane == lead) atomicAdd(&size[L], __popcll(same));
-            if (l == L) todo = false;
+// Canonical labels: the vertex whose label is its own id is its SCC's
+// smallest, so every size starts at 1 with a plain store there, and only the
+// other vertices of an SCC are counted by atomics.
+constexpr int kHistGrid = 512;  // blocks: each ends with one atomic per common address
+
+// Four consecutive labels from v (16-byte load; entries past V are -1).
+__device__ __forceinline__ int4 load4(const int32_t* __restrict__ p, int64_t v, int32_t V) {
+    if (v + 3 < V) return *reinterpret_cast<const int4*>(p + v);
+    return int4{v < V ? p[v] : -1, v + 1 < V ? p[v + 1] : -1, v + 2 < V ? p[v + 2] : -1, -1};
+}
+
+__global__ __launch_bounds__(kBlock) void k_size_roots(const int32_t* __restrict__ lab, int32_t V, int32_t* size,
+                                                       int64_t* out) {
+    if (blockIdx.x == 0 && threadIdx.x < kHistSlots) out[threadIdx.x] = 0;
+    for (int64_t v = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * 4; v < V; v += (int64_t)gridDim.x * kBlock * 4) {
+        const int4 l = load4(lab, v, V);
+        const int4 r{l.x == v, l.y == v + 1, l.z == v + 2, l.w == v + 3};
+        if (v + 3 < V) {
+            *reinterpret_cast<int4*>(size + v) = r;
+        } else {
+            size[v] = r.x;
+            if (v + 1 < V) size[v + 1] = r.y;
+            if (v + 2 < V) size[v + 2] = r.z;
         }
-        if (todo) atomicAdd(&size[l], 1);
+    }
+}
+
+// size[lab[v]] += 1 for every vertex that is not its SCC's smallest.  Atomics
+// on one address run one after the other over the whole chip (11 ns each), so
+// the giant's label, which most such vertices carry, must not cost one per
+// wave step: each thread counts on while the label stays the same, then the
+// block's waves and at last the block add up what they hold of one label.
+// 2 M vertices (R-MAT, edge factor 16): sizes and bins together 629 -> 31 us
+// against a wave's combined atomic per step and a cleared size array.
+__global__ __launch_bounds__(kBlock) void k_scc_sizes(const int32_t* __restrict__ lab, int32_t V, int32_t* size) {
+    constexpr int NW = kBlock / kWave;
+    __shared__ int32_t s_lab[NW];
+    __shared__ int s_cnt[NW];
+    int32_t cur = -1;  // this thread's current label and how often it met it
+    int cnt = 0;
+    auto meet = [&](int32_t l, int64_t v) {
+        if (l < 0 || l == v) return;
+        if (l != cur) {
+            if (cnt) atomicAdd(&size[cur], cnt);
+            cur = l;
+            cnt = 0;
+        }
+        ++cnt;
+    };
+    for (int64_t v = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * 4; v < V; v += (int64_t)gridDim.x * kBlock * 4) {
+        const int4 l = load4(lab, v, V);
+        meet(l.x, v);
+        meet(l.y, v + 1);
+        meet(l.z, v + 2);
+        meet(l.w, v + 3);
+    }
+    // the wave: add up the label of the first lane that holds one, a few
+    // times; what is left goes out by itself, the first label to the block
+    const int lane = lane_id();
+    int32_t wl = -1;
+    int wc = 0;
+    for (int r = 0; r < 3; ++r) {
+        const uint64_t m = __ballot(cnt > 0);
+        if (!m) break;
+        const int32_t L = lane_get(cur, __ffsll((unsigned long long)m) - 1);
+        const int total = wave_sum(cnt > 0 && cur == L ? cnt : 0);
+        if (cur == L) cnt = 0;
+        if (total > wc) {  // the most frequent one waits for the block
+            if (wc && lane == 0) atomicAdd(&size[wl], wc);
+            wl = L;
+            wc = total;
+        } else if (lane == 0) {
+            atomicAdd(&size[L], total);
+        }
+    }
+    if (cnt > 0) atomicAdd(&size[cur], cnt);
+    if (lane == 0) {
+        s_lab[wave_id()] = wl;
+        s_cnt[wave_id()] = wc;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 0; i < NW; ++i) {
+            int c = s_cnt[i];
+            if (!c) continue;
+            for (int k = i + 1; k < NW; ++k)
+                if (s_lab[k] == s_lab[i]) {
+                    c += s_cnt[k];
+                    s_cnt[k] = 0;
+                }
+            atomicAdd(&size[s_lab[i]], c);
+        }
     }
 }
 
 // Log2 bins of the SCC sizes (bin k: sizes in [2^k, 2^(k+1))), per block in
 // LDS, plus the largest size, the counts of sizes 1, 2, 3 and the SCC
 // count: out[0..63] bins, out[64] largest, out[65..67] sizes 1-3, out[68]
-// total.
+// total.  Sizes up to 3, nearly all of them, are counted in registers (one
+// LDS bin for all of a wave's lanes took 292 us at 2 M vertices).
 __global__ __launch_bounds__(kBlock) void k_scc_hist(const int32_t* __restrict__ size, int32_t V, int64_t* out) {
+    constexpr int NW = kBlock / kWave;
     __shared__ int s_bin[64];
+    __shared__ int s_part[5][NW];
     if (threadIdx.x < 64) s_bin[threadIdx.x] = 0;
     __syncthreads();
     int largest = 0, c1 = 0, c2 = 0, c3 = 0, tot = 0;
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += (int64_t)gridDim.x * blockDim.x) {
-        const int c = size[v];
-        if (c <= 0) continue;
-        atomicAdd(&s_bin[31 - __clz(c)], 1);
-        largest = max(largest, c);
+    auto meet = [&](int c) {
+        if (c <= 0) return;
         c1 += c == 1;
         c2 += c == 2;
         c3 += c == 3;
         ++tot;
+        if (c > 3) atomicAdd(&s_bin[31 - __clz(c)], 1);
+        largest = max(largest, c);
+    };
+    for (int64_t v = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * 4; v < V; v += (int64_t)gridDim.x * kBlock * 4) {
+        const int4 c = load4(size, v, V);
+        meet(c.x);
+        meet(c.y);
+        meet(c.z);
+        meet(c.w);
     }
     c1 = wave_sum(c1);
     c2 = wave_sum(c2);
     c3 = wave_sum(c3);
     tot = wave_sum(tot);
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) largest = max(largest, __shfl_xor(largest, d, kWave));
+    largest = -wave_min(-largest);
     if (lane_id() == 0) {
-        if (largest) atomicMax(reinterpret_cast<unsigned long long*>(&out[64]), (unsigned long long)largest);
-        if (c1) atomicAdd(reinterpret_cast<unsigned long long*>(&out[65]), (unsigned long long)c1);
-        if (c2) atomicAdd(reinterpret_cast<unsigned long long*>(&out[66]), (unsigned long long)c2);
-        if (c3) atomicAdd(reinterpret_cast<unsigned long long*>(&out[67]), (unsigned long long)c3);
-        if (tot) atomicAdd(reinterpret_cast<unsigned long long*>(&out[68]), (unsigned long long)tot);
+        const int w = wave_id();
+        s_part[0][w] = c1;
+        s_part[1][w] = c2;
+        s_part[2][w] = c3;
+        s_part[3][w] = tot;
+        s_part[4][w] = largest;
     }
     __syncthreads();
-    if (threadIdx.x < 64 && s_bin[threadIdx.x])
-        atomicAdd(reinterpret_cast<unsigned long long*>(&out[threadIdx.x]), (unsigned long long)s_bin[threadIdx.x]);
+    if (threadIdx.x < 64) {
+        int x[5] = {0, 0, 0, 0, 0};
+        for (int w = 0; w < NW; ++w) {
+            for (int k = 0; k < 4; ++k) x[k] += s_part[k][w];
+            x[4] = max(x[4], s_part[4][w]);
+        }
+        const int t = threadIdx.x;
+        const int bin = s_bin[t] + (t == 0 ? x[0] : t == 1 ? x[1] + x[2] : 0);
+        if (bin) atomicAdd(reinterpret_cast<unsigned long long*>(&out[t]), (unsigned long long)bin);
+        const int y = t == 0 ? x[4] : t < 4 ? x[t - 1] : t == 4 ? x[3] : 0;  // out[64..68]
+        if (t == 0 && y) atomicMax(reinterpret_cast<unsigned long long*>(&out[64]), (unsigned long long)y);
+        else if (t > 0 && t < 5 && y) atomicAdd(reinterpret_cast<unsigned long long*>(&out[64 + t]), (unsigned long long)y);
+    }
 }
 
 // ------------------------------------------------------------- launchers
@@ -960,10 +1050,10 @@ hipError_t launch_stats(const int32_t* fwb, const int32_t* bwb, const int32_t* l
     LAUNCH(k_stats, grid, fwb, bwb, lab, fvis, bvis, V, ctl);
 }
 
-hipError_t launch_scc_histogram(const int32_t* lab, int32_t V, int32_t* size, int64_t* out, int grid, hipStream_t s) {
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid), dim3(kBlock), 0, s, size, 0, (int64_t)V);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(kBlock), 0, s, reinterpret_cast<int32_t*>(out), 0,
-                       (int64_t)kHistSlots * 2);
+hipError_t launch_scc_histogram(const int32_t* lab, int32_t V, int32_t* size, int64_t* out, hipStream_t s) {
+    static_assert(kHistSlots <= kBlock, "one thread clears one slot");
+    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(kHistGrid, ((int64_t)V + 4 * kBlock - 1) / (4 * kBlock)));
+    hipLaunchKernelGGL(k_size_roots, dim3(grid), dim3(kBlock), 0, s, lab, V, size, out);
     hipLaunchKernelGGL(k_scc_sizes, dim3(grid), dim3(kBlock), 0, s, lab, V, size);
     LAUNCH(k_scc_hist, grid, size, V, out);
 }

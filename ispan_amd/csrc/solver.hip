@@ -1956,7 +1956,7 @@ int ispan_scc_histogram(ispan_ctx* ctx, int64_t* bins, int32_t n_bins, ispan_sum
         CK(hipSetDevice(ctx->device));
         if (!ctx->hist) CK(hipMalloc(&ctx->hist, sizeof(h)));
         // the mice queue buffer (int32[V + 1]) holds the sizes: the solve is over
-        CK(launch_scc_histogram(ctx->lab, ctx->V, ctx->qbuf, ctx->hist, ctx->grid, ctx->stream));
+        CK(launch_scc_histogram(ctx->lab, ctx->V, ctx->qbuf, ctx->hist, ctx->stream));
         CK(hipMemcpyAsync(h, ctx->hist, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
         CK(hipStreamSynchronize(ctx->stream));
     }

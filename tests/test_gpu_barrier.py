@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 GRAPHS = {
     "no_edges": lambda: O.build_csr(70, np.zeros(0, np.int32), np.zeros(0, np.int32)),  # no traversal
     "toy": lambda: G.toy_graph()[0],
-    "rmat": lambda: O.rmat(1000, 8.0, 3),
+    "rmat": lambda: O.rmat(10, 8.0, 3),
     "grid": lambda: O.grid(60, 0.5, 2),          # many levels
     "cycles": lambda: G.cycles_graph(5),         # patterns, WCC and mice
     "chain": lambda: G.cycle_chain(500, 7),      # a second cooperative launch (colouring)
