@@ -1,9 +1,9 @@
 // Device-side producers of the iSpan CSR layout: seeded synthetic edge
 // lists (R-MAT, lattice) and an edge-list -> CSR-pair builder (sort, drop
-// self-loops, deduplicate, offsets by binary search, transpose).  This is
+// self-loops, deduplicate, offsets, transpose).  This is
 // the format producer of graph_converter/txt_to_bin_{fw,bw}_int.cpp
 // (:31-217), which does not deduplicate; here both directions are built in
-// one pass over sorted 64-bit (src,dst) keys.
+// one pass over sorted (src,dst) keys.
 //
 // Randomness is a counter hash of (seed, draw index), so the edge multiset
 // depends on nothing but the parameters.
@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <string>
+#include <type_traits>
 
 #include "common.h"
 
@@ -37,13 +38,27 @@ uint64_t stream_base(uint64_t seed, uint64_t tag) {
     return mix64(seed * 0x632BE59BD9B4E019ull + tag * 0xD1B54A32D192ED03ull + 1ull);
 }
 
-constexpr uint64_t kNoEdge = ~0ull;
+// A directed edge as one sort key: src above the low `bits` bits, dst in
+// them, bits = id_bits(V).  An absent edge is any self-loop, (0, 0) where
+// there is nothing to keep: self-loops are dropped after the sort, so absent
+// edges need no value outside the 2 * bits bits that are sorted.
+int id_bits(int64_t V) {
+    int b = 1;
+    while (b < 31 && ((int64_t)1 << b) < V) ++b;
+    return b;
+}
+
+template <class K>
+__device__ __forceinline__ K edge_key(uint32_t s, uint32_t d, int bits) {
+    return (K)(((K)s << bits) | (K)d);
+}
 
 // R-MAT draw e: at each of `scale` bit levels (most significant first) a
 // 32-bit draw picks the quadrant: r < t1 (0,0), r < t2 (0,1), r < t3 (1,0),
 // else (1,1).  Two levels share one 64-bit hash.
-__global__ void k_rmat(int32_t V, int scale, int64_t m, uint32_t t1, uint32_t t2, uint32_t t3, uint64_t base,
-                       uint64_t* keys) {
+template <class K>
+__global__ void k_rmat(int32_t V, int scale, int64_t m, uint32_t t1, uint32_t t2, uint32_t t3, uint64_t base, int bits,
+                       K* keys) {
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m; e += (int64_t)gridDim.x * blockDim.x) {
         uint32_t s = 0, d = 0;
         uint64_t h = 0;
@@ -55,13 +70,14 @@ __global__ void k_rmat(int32_t V, int scale, int64_t m, uint32_t t1, uint32_t t2
             s |= sb << (scale - 1 - k);
             d |= db << (scale - 1 - k);
         }
-        keys[e] = (s < (uint32_t)V && d < (uint32_t)V && s != d) ? (((uint64_t)s << 32) | d) : kNoEdge;
+        keys[e] = (s < (uint32_t)V && d < (uint32_t)V) ? edge_key<K>(s, d, bits) : (K)0;
     }
 }
 
 // n x n lattice: draw i < L covers lattice edge i (horizontal edges first,
 // row-major), slots 2i and 2i+1; then L/100 uniform random directed edges.
-__global__ void k_grid(int32_t n, uint32_t tb, uint64_t b1, uint64_t b2, uint64_t* keys) {
+template <class K>
+__global__ void k_grid(int32_t n, uint32_t tb, uint64_t b1, uint64_t b2, int bits, K* keys) {
     const int64_t H = (int64_t)n * (n - 1), L = 2 * H, R = L / 100;
     const uint64_t V = (uint64_t)n * (uint64_t)n;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < L + R;
@@ -79,52 +95,160 @@ __global__ void k_grid(int32_t n, uint32_t tb, uint64_t b1, uint64_t b2, uint64_
                 v = u + n;
             }
             const uint64_t h = mix64(b1 ^ (uint64_t)i);
-            const uint64_t uv = ((uint64_t)u << 32) | (uint64_t)v, vu = ((uint64_t)v << 32) | (uint64_t)u;
+            const K uv = edge_key<K>((uint32_t)u, (uint32_t)v, bits), vu = edge_key<K>((uint32_t)v, (uint32_t)u, bits);
             if ((uint32_t)h < tb) {
                 keys[2 * i] = uv;
                 keys[2 * i + 1] = vu;
             } else {
                 keys[2 * i] = (h >> 63) == 0 ? uv : vu;
-                keys[2 * i + 1] = kNoEdge;
+                keys[2 * i + 1] = 0;
             }
         } else {
             const int64_t k = i - L;
             const uint64_t h = mix64(b2 ^ (uint64_t)k);
             const uint64_t s = ((h & 0xffffffffull) * V) >> 32, d = ((h >> 32) * V) >> 32;
-            keys[2 * L + k] = s != d ? ((s << 32) | d) : kNoEdge;
+            keys[2 * L + k] = edge_key<K>((uint32_t)s, (uint32_t)d, bits);
         }
     }
 }
 
+template <class K>
 __global__ void k_pack(const int32_t* __restrict__ src, const int32_t* __restrict__ dst, int64_t m, int32_t V,
-                       uint64_t* keys, int32_t* bad) {
+                       int bits, K* __restrict__ keys, int32_t* bad) {
+    int wrong = 0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
         const int32_t s = src[i], d = dst[i];
-        if (s < 0 || s >= V || d < 0 || d >= V) {
-            atomicAdd(bad, 1);
-            keys[i] = kNoEdge;
-        } else {
-            keys[i] = s != d ? (((uint64_t)(uint32_t)s << 32) | (uint32_t)d) : kNoEdge;
+        const bool ok = s >= 0 && s < V && d >= 0 && d < V;
+        wrong |= !ok;
+        keys[i] = ok ? edge_key<K>((uint32_t)s, (uint32_t)d, bits) : (K)0;
+    }
+    if (wrong) atomicOr(bad, 1);
+}
+
+// Row offsets come with a pass over the keys in row order: where a key's row
+// is larger than the one before it, the rows in between and its own begin at
+// its position.  (A binary search per row, bounded per 256 or 1024 rows, was
+// bound by its scattered probes: 60 us for 2^20 rows over 16 M keys, twice a
+// build.)  A lane writes up to kLaneRows rows itself, the wave the rest of a
+// gap, and a gap of more than kGapRows rows is cut into pieces that k_gaps
+// fills, one block each, so that a hole in the ids does not hold up one wave.
+constexpr int kLaneRows = 4;
+constexpr int kGapRows = 4096;
+struct Gap {
+    int32_t lo, n, pos;
+};
+struct Rows {
+    int32_t* beg;
+    Gap* gaps;        // gap_capacity(V) entries
+    int32_t* n_gaps;  // zero before the pass
+};
+// Pieces are full but for one per gap, and a gap has more than kGapRows rows.
+int64_t gap_capacity(int64_t V) { return 2 * (V / kGapRows) + 2; }
+
+// beg[r0 + 1 .. r1] = pos, for every lane's own r0, r1, pos (r1 <= r0: none).
+// All 64 lanes call it.
+__device__ __forceinline__ void begin_rows(const Rows& R, int32_t r0, int32_t r1, int32_t pos) {
+    const int lane = threadIdx.x & 63;
+    const int32_t n = r1 - r0;
+#pragma unroll
+    for (int k = 0; k < kLaneRows; ++k)
+        if (k < n) R.beg[r0 + 1 + k] = pos;
+    uint64_t more = __ballot(n > kLaneRows);
+    while (more) {
+        const int l = __ffsll((unsigned long long)more) - 1;
+        more &= more - 1;
+        const int32_t lo = __builtin_amdgcn_readlane(r0, l) + 1 + kLaneRows, hi = __builtin_amdgcn_readlane(r1, l);
+        const int32_t p = __builtin_amdgcn_readlane(pos, l);
+        if (hi - lo < kGapRows) {
+            for (int32_t v = lo + lane; v <= hi; v += 64) R.beg[v] = p;
+        } else if (lane == 0) {
+            const int32_t pieces = (int32_t)(((int64_t)hi - lo + kGapRows) / kGapRows);
+            const int32_t at = atomicAdd(R.n_gaps, pieces);
+            for (int32_t k = 0; k < pieces; ++k)
+                R.gaps[at + k] = Gap{lo + k * kGapRows, min(kGapRows, hi - lo + 1 - k * kGapRows), p};
         }
     }
 }
 
-// adj[i] = low word; beg[v] = first i with key >= v<<32 (binary search).
-__global__ void k_csr_from_keys(const uint64_t* __restrict__ keys, int64_t E, int32_t V, int32_t* beg,
-                                int32_t* adj) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    for (int64_t i = t; i < E; i += stride) adj[i] = (int32_t)(uint32_t)keys[i];
-    for (int64_t v = t; v <= V; v += stride) {
-        const uint64_t key = (uint64_t)v << 32;
-        int64_t lo = 0, hi = E;
-        while (lo < hi) {
-            const int64_t mid = (lo + hi) >> 1;
-            if (keys[mid] < key) lo = mid + 1;
-            else hi = mid;
-        }
-        beg[v] = (int32_t)lo;
+__global__ void k_gaps(Rows R) {
+    const int32_t n = *R.n_gaps;
+    for (int32_t g = blockIdx.x; g < n; g += gridDim.x) {
+        const Gap x = R.gaps[g];
+        for (int32_t k = threadIdx.x; k < x.n; k += blockDim.x) R.beg[x.lo + k] = x.pos;
     }
+}
+
+// Sorted keys -> kept keys (the first of equal ones, no self-loops).  A wave
+// owns kKeepChunk consecutive keys; k_keep_count counts what each keeps, and
+// after a prefix sum over the chunks k_keep writes them in order, with their
+// low halves as the adjacency, and the row offsets.  Bound by memory: two
+// reads of the keys and one write.
+constexpr int kKeepChunk = 1024;
+constexpr int kKeepWaves = 4;
+
+// f(valid, key, keep, previous key) for the 64 keys of every step.
+template <class K, class F>
+__device__ __forceinline__ void each_key(const K* __restrict__ keys, int64_t m, int bits, int64_t chunk, F&& f) {
+    const int lane = threadIdx.x & 63;
+    const K low = ((K)1 << bits) - 1;
+    const int64_t i0 = chunk * kKeepChunk, i1 = min(i0 + kKeepChunk, m);
+    for (int64_t ib = i0; ib < i1; ib += 64) {
+        const int64_t i = ib + lane;
+        const bool valid = i < i1;
+        const K k = valid ? keys[i] : 0, before = valid && i > 0 ? keys[i - 1] : 0;
+        f(i, valid, k, valid && (K)(k >> bits) != (k & low) && (i == 0 || before != k), before);
+    }
+}
+
+template <class K>
+__global__ __launch_bounds__(64 * kKeepWaves) void k_keep_count(const K* __restrict__ keys, int64_t m, int bits,
+                                                                int64_t chunks, int32_t* __restrict__ counts) {
+    for (int64_t c = (int64_t)blockIdx.x * kKeepWaves + threadIdx.x / 64; c < chunks; c += (int64_t)gridDim.x * kKeepWaves) {
+        int n = 0;
+        each_key<K>(keys, m, bits, c, [&](int64_t, bool, K, bool keep, K) { n += __popcll(__ballot(keep)); });
+        if ((threadIdx.x & 63) == 0) counts[c] = n;
+    }
+}
+
+template <class K>
+__global__ __launch_bounds__(64 * kKeepWaves) void k_keep(const K* __restrict__ keys, int64_t m, int bits,
+                                                          int64_t chunks, const int64_t* __restrict__ start,
+                                                          K* __restrict__ kept, int32_t* __restrict__ adj, Rows R,
+                                                          int32_t V) {
+    const int lane = threadIdx.x & 63;
+    const K low = ((K)1 << bits) - 1;
+    for (int64_t c = (int64_t)blockIdx.x * kKeepWaves + threadIdx.x / 64; c < chunks; c += (int64_t)gridDim.x * kKeepWaves) {
+        int64_t p = start[c];
+        each_key<K>(keys, m, bits, c, [&](int64_t i, bool valid, K k, bool keep, K before) {
+            const uint64_t mask = __ballot(keep);
+            const int64_t q = p + __popcll(mask & ((1ull << lane) - 1));
+            if (keep) {
+                kept[q] = k;
+                adj[q] = (int32_t)(k & low);
+            }
+            const int32_t row = (int32_t)(k >> bits);
+            begin_rows(R, i == 0 ? -1 : (int32_t)(before >> bits), valid ? row : -1, (int32_t)q);
+            p += __popcll(mask);
+            const bool last = i == m - 1;  // the rows after the last key's
+            if (__ballot(last)) begin_rows(R, row, last ? V : -1, (int32_t)p);
+        });
+    }
+}
+
+// Kept keys in (dst, src) order -> the transposed rows.
+template <class K>
+__global__ __launch_bounds__(64 * kKeepWaves) void k_transposed(const K* __restrict__ keys, int64_t E, int bits,
+                                                                int64_t chunks, int32_t* __restrict__ adj, Rows R,
+                                                                int32_t V) {
+    const K low = ((K)1 << bits) - 1;
+    for (int64_t c = (int64_t)blockIdx.x * kKeepWaves + threadIdx.x / 64; c < chunks; c += (int64_t)gridDim.x * kKeepWaves)
+        each_key<K>(keys, E, bits, c, [&](int64_t i, bool valid, K k, bool, K before) {
+            if (valid) adj[i] = (int32_t)(k >> bits);
+            const int32_t row = (int32_t)(k & low);
+            begin_rows(R, i == 0 ? -1 : (int32_t)(before & low), valid ? row : -1, (int32_t)i);
+            const bool last = i == E - 1;
+            if (__ballot(last)) begin_rows(R, row, last ? V : -1, (int32_t)E);
+        });
 }
 
 __global__ void k_widen_keys(const uint32_t* __restrict__ k, int64_t m, uint64_t* out) {
@@ -146,17 +270,6 @@ __global__ void k_beg_from_keys(const uint64_t* __restrict__ keys, int64_t m, in
     }
 }
 
-__global__ void k_swap_halves(const uint64_t* __restrict__ in, int64_t E, uint64_t* out) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < E; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint64_t k = in[i];
-        out[i] = (k << 32) | (k >> 32);
-    }
-}
-
-struct NotSentinel {
-    __device__ bool operator()(uint64_t k) const { return k != kNoEdge; }
-};
-
 #define GK(call)                                                             \
     do {                                                                     \
         hipError_t e_ = (call);                                              \
@@ -171,35 +284,51 @@ constexpr int kGrid = 4096;
 
 }  // namespace
 
-// keys[0, m) (kNoEdge = absent) -> CSR pair.  keys is clobbered.
-int csr_from_keys(hipStream_t s, int32_t V, int64_t m, uint64_t* keys, int32_t** fwb, int32_t** fwa, int32_t** bwb,
+// keys[0, m) (edge_key form) -> CSR pair.  keys is clobbered.  Only the
+// 2 * bits bits of a key are sorted, in 32-bit keys when they fit (V <= 65536);
+// the kept keys, then in (src, dst) order, are sorted by dst alone for the
+// transposed rows: the sort is stable, so each row stays in src order.  At
+// 2^20 vertices that is 5 + 3 radix passes instead of the 8 + 8 of full 64-bit
+// keys.
+template <class K>
+int csr_from_keys(hipStream_t s, int32_t V, int64_t m, K* keys, int32_t** fwb, int32_t** fwa, int32_t** bwb,
                   int32_t** bwa, int64_t* E_out, std::string& err) {
     int rc = 0;
-    uint64_t* sorted = nullptr;
+    const int bits = id_bits(V);
+    const int64_t chunks = (m + kKeepChunk - 1) / kKeepChunk;
+    const int keep_grid = (int)std::max<int64_t>(1, std::min<int64_t>(kGrid, (chunks + kKeepWaves - 1) / kKeepWaves));
+    const int64_t gap_bytes = gap_capacity(V) * (int64_t)sizeof(Gap);
+    K* alt = nullptr;
     void* tmp = nullptr;
+    int32_t* counts = nullptr;
+    int64_t* start = nullptr;  // first kept position of every chunk, then their total
     size_t tmp_bytes = 0, b1 = 0, b2 = 0;
-    int64_t* d_count = nullptr;
     int64_t E = 0;
+    char* gaps = nullptr;  // two counters, then the gaps of one direction
+    rocprim::double_buffer<K> buf(keys, keys);
     *fwb = *fwa = *bwb = *bwa = nullptr;
-    GK(hipMalloc(&sorted, (size_t)std::max<int64_t>(m, 1) * 8));
-    GK(hipMalloc(&d_count, 8));
-    GK(rocprim::radix_sort_keys(nullptr, b1, keys, sorted, (size_t)m, 0, 64, s));
-    GK(rocprim::unique(nullptr, b2, sorted, keys, d_count, (size_t)m, rocprim::equal_to<uint64_t>(), s));
-    tmp_bytes = std::max(b1, b2) + 256;
-    GK(hipMalloc(&tmp, tmp_bytes));
+    GK(hipMalloc(&alt, (size_t)std::max<int64_t>(m, 1) * sizeof(K)));
+    GK(hipMalloc(&start, (size_t)(chunks + 1) * 8));
+    GK(hipMalloc(&counts, (size_t)(chunks + 1) * 4));
+    GK(hipMalloc(&gaps, (size_t)gap_bytes + 16));
+    buf = rocprim::double_buffer<K>(keys, alt);
     if (m > 0) {
-        b1 = tmp_bytes;
-        GK(rocprim::radix_sort_keys(tmp, b1, keys, sorted, (size_t)m, 0, 64, s));
-        b2 = tmp_bytes;
-        GK(rocprim::unique(tmp, b2, sorted, keys, d_count, (size_t)m, rocprim::equal_to<uint64_t>(), s));
-        GK(hipMemcpyAsync(&E, d_count, 8, hipMemcpyDeviceToHost, s));
+        GK(rocprim::radix_sort_keys(nullptr, b1, buf, (size_t)m, 0, 2 * bits, s));
+        GK(rocprim::exclusive_scan(nullptr, b2, counts, start, (int64_t)0, (size_t)chunks + 1,
+                                   rocprim::plus<int64_t>(), s));
+        tmp_bytes = std::max(b1, b2) + 256;
+        GK(hipMalloc(&tmp, tmp_bytes));
+        b1 = b2 = tmp_bytes;
+        GK(rocprim::radix_sort_keys(tmp, b1, buf, (size_t)m, 0, 2 * bits, s));
+        hipLaunchKernelGGL(k_keep_count<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), m, bits,
+                           chunks, counts);
+        GK(hipGetLastError());
+        // one entry more than chunks: the last start is the total (the last
+        // count is not read into it)
+        GK(rocprim::exclusive_scan(tmp, b2, counts, start, (int64_t)0, (size_t)chunks + 1, rocprim::plus<int64_t>(),
+                                   s));
+        GK(hipMemcpyAsync(&E, start + chunks, 8, hipMemcpyDeviceToHost, s));
         GK(hipStreamSynchronize(s));
-        // the sentinel sorts last: drop it if present
-        if (E > 0) {
-            uint64_t last = 0;
-            GK(hipMemcpy(&last, keys + E - 1, 8, hipMemcpyDeviceToHost));
-            if (last == kNoEdge) --E;
-        }
     }
     if (E > INT32_MAX) {
         err = "edge count exceeds int32";
@@ -210,22 +339,43 @@ int csr_from_keys(hipStream_t s, int32_t V, int64_t m, uint64_t* keys, int32_t**
     GK(hipMalloc(bwb, ((size_t)V + 1) * 4));
     GK(hipMalloc(fwa, (size_t)std::max<int64_t>(E, 1) * 4));
     GK(hipMalloc(bwa, (size_t)std::max<int64_t>(E, 1) * 4));
-    hipLaunchKernelGGL(k_csr_from_keys, dim3(kGrid), dim3(256), 0, s, keys, E, V, *fwb, *fwa);
-    GK(hipGetLastError());
     if (E > 0) {
-        hipLaunchKernelGGL(k_swap_halves, dim3(kGrid), dim3(256), 0, s, keys, E, sorted);
+        K* kept = buf.alternate();
+        int32_t* n_gaps = reinterpret_cast<int32_t*>(gaps);
+        Rows R{*fwb, reinterpret_cast<Gap*>(gaps + 16), n_gaps};
+        GK(launch_fill_i32(n_gaps, 0, 2, 1, s));
+        hipLaunchKernelGGL(k_keep<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), m, bits, chunks,
+                           start, kept, *fwa, R, V);
         GK(hipGetLastError());
+        hipLaunchKernelGGL(k_gaps, dim3(256), dim3(256), 0, s, R);
+        GK(hipGetLastError());
+        buf = rocprim::double_buffer<K>(kept, buf.current());
+        // fewer keys can take another of the sort's methods, with more scratch
+        GK(rocprim::radix_sort_keys(nullptr, b1, buf, (size_t)E, 0, bits, s));
+        if (b1 > tmp_bytes) {
+            (void)hipFree(tmp);
+            tmp = nullptr;
+            GK(hipMalloc(&tmp, b1));
+            tmp_bytes = b1;
+        }
         b1 = tmp_bytes;
-        GK(rocprim::radix_sort_keys(tmp, b1, sorted, keys, (size_t)E, 0, 64, s));
+        GK(rocprim::radix_sort_keys(tmp, b1, buf, (size_t)E, 0, bits, s));
+        R.beg = *bwb;
+        R.n_gaps = n_gaps + 1;
+        hipLaunchKernelGGL(k_transposed<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), E, bits,
+                           (E + kKeepChunk - 1) / kKeepChunk, *bwa, R, V);
+        GK(hipGetLastError());
+        hipLaunchKernelGGL(k_gaps, dim3(256), dim3(256), 0, s, R);
+        GK(hipGetLastError());
+    } else {
+        GK(launch_fill_i32(*fwb, 0, (int64_t)V + 1, kGrid, s));
+        GK(launch_fill_i32(*bwb, 0, (int64_t)V + 1, kGrid, s));
     }
-    hipLaunchKernelGGL(k_csr_from_keys, dim3(kGrid), dim3(256), 0, s, keys, E, V, *bwb, *bwa);
-    GK(hipGetLastError());
     GK(hipStreamSynchronize(s));
     *E_out = E;
 done:
-    if (sorted) (void)hipFree(sorted);
-    if (tmp) (void)hipFree(tmp);
-    if (d_count) (void)hipFree(d_count);
+    for (void* p : {(void*)alt, tmp, (void*)counts, (void*)start, (void*)gaps})
+        if (p) (void)hipFree(p);
     if (rc) {
         for (int32_t** p : {fwb, fwa, bwb, bwa}) {
             if (*p) (void)hipFree(*p);
@@ -279,6 +429,34 @@ done:
     return rc;
 }
 
+// The key buffer of m edges over V vertices and, on it, `fill` (which writes
+// the keys) and csr_from_keys.
+template <class Fill>
+int csr_from_filled(hipStream_t s, int32_t V, int64_t m, Fill&& fill, int32_t** fwb, int32_t** fwa, int32_t** bwb,
+                    int32_t** bwa, int64_t* E, std::string& err) {
+    void* keys = nullptr;
+    int rc = 0;
+    const bool narrow = 2 * id_bits(V) <= 32;
+    GK(hipMalloc(&keys, (size_t)std::max<int64_t>(m, 1) * (narrow ? 4 : 8)));
+    if (narrow) {
+        rc = fill(static_cast<uint32_t*>(keys));
+        if (!rc) rc = csr_from_keys(s, V, m, static_cast<uint32_t*>(keys), fwb, fwa, bwb, bwa, E, err);
+    } else {
+        rc = fill(static_cast<uint64_t*>(keys));
+        if (!rc) rc = csr_from_keys(s, V, m, static_cast<uint64_t*>(keys), fwb, fwa, bwb, bwa, E, err);
+    }
+done:
+    if (keys) (void)hipFree(keys);
+    return rc;
+}
+
+int launched(std::string& err) {
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return 0;
+    err = std::string("kernel launch: ") + hipGetErrorString(e);
+    return e == hipErrorOutOfMemory ? -3 : -4;
+}
+
 int gen_rmat_device(hipStream_t s, int32_t V, double ef, double a, double b, double c, uint64_t seed, int32_t** fwb,
                     int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
     if (V <= 0 || ef < 0 || a < 0 || b < 0 || c < 0 || a + b + c > 1.0) return -1;
@@ -287,15 +465,13 @@ int gen_rmat_device(hipStream_t s, int32_t V, double ef, double a, double b, dou
     const int64_t m = llround(ef * (double)V);
     const double S = 4294967296.0;
     const uint32_t t1 = (uint32_t)(a * S), t2 = (uint32_t)((a + b) * S), t3 = (uint32_t)((a + b + c) * S);
-    uint64_t* keys = nullptr;
-    int rc = 0;
-    GK(hipMalloc(&keys, (size_t)std::max<int64_t>(m, 1) * 8));
-    hipLaunchKernelGGL(k_rmat, dim3(kGrid), dim3(256), 0, s, V, scale, m, t1, t2, t3, stream_base(seed, 1), keys);
-    GK(hipGetLastError());
-    rc = csr_from_keys(s, V, m, keys, fwb, fwa, bwb, bwa, E, err);
-done:
-    if (keys) (void)hipFree(keys);
-    return rc;
+    auto fill = [&](auto* keys) {
+        using K = std::remove_pointer_t<decltype(keys)>;
+        hipLaunchKernelGGL(k_rmat<K>, dim3(kGrid), dim3(256), 0, s, V, scale, m, t1, t2, t3, stream_base(seed, 1),
+                           id_bits(V), keys);
+        return launched(err);
+    };
+    return csr_from_filled(s, V, m, fill, fwb, fwa, bwb, bwa, E, err);
 }
 
 int gen_grid_device(hipStream_t s, int32_t n, double p_bidir, uint64_t seed, int32_t** fwb, int32_t** fwa,
@@ -303,42 +479,42 @@ int gen_grid_device(hipStream_t s, int32_t n, double p_bidir, uint64_t seed, int
     if (n < 2 || (int64_t)n * n > INT32_MAX || p_bidir < 0 || p_bidir > 1) return -1;
     const int64_t L = 2 * (int64_t)n * (n - 1), R = L / 100, m = 2 * L + R;
     const uint32_t tb = (uint32_t)(p_bidir * 4294967296.0);
-    uint64_t* keys = nullptr;
-    int rc = 0;
-    GK(hipMalloc(&keys, (size_t)m * 8));
-    hipLaunchKernelGGL(k_grid, dim3(kGrid), dim3(256), 0, s, n, tb, stream_base(seed, 2), stream_base(seed, 3),
-                       keys);
-    GK(hipGetLastError());
-    rc = csr_from_keys(s, n * n, m, keys, fwb, fwa, bwb, bwa, E, err);
-done:
-    if (keys) (void)hipFree(keys);
-    return rc;
+    auto fill = [&](auto* keys) {
+        using K = std::remove_pointer_t<decltype(keys)>;
+        hipLaunchKernelGGL(k_grid<K>, dim3(kGrid), dim3(256), 0, s, n, tb, stream_base(seed, 2), stream_base(seed, 3),
+                           id_bits((int64_t)n * n), keys);
+        return launched(err);
+    };
+    return csr_from_filled(s, n * n, m, fill, fwb, fwa, bwb, bwa, E, err);
 }
 
 int build_csr_device(hipStream_t s, int32_t V, int64_t m, const int32_t* src, const int32_t* dst, int32_t** fwb,
                      int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
     if (V < 0 || m < 0) return -1;
-    uint64_t* keys = nullptr;
     int32_t* d_bad = nullptr;
     int32_t bad = 0;
     int rc = 0;
-    GK(hipMalloc(&keys, (size_t)std::max<int64_t>(m, 1) * 8));
+    auto fill = [&](auto* keys) {
+        using K = std::remove_pointer_t<decltype(keys)>;
+        if (m > 0) {
+            hipLaunchKernelGGL(k_pack<K>, dim3(kGrid), dim3(256), 0, s, src, dst, m, V, id_bits(V), keys, d_bad);
+            if (int e = launched(err)) return e;
+        }
+        if (hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess) {
+            err = "reading the edge check failed";
+            return -4;
+        }
+        if (bad) {
+            err = "edge endpoint outside [0, V)";
+            return -2;
+        }
+        return 0;
+    };
     GK(hipMalloc(&d_bad, 4));
     GK(hipMemsetAsync(d_bad, 0, 4, s));
-    if (m > 0) {
-        hipLaunchKernelGGL(k_pack, dim3(kGrid), dim3(256), 0, s, src, dst, m, V, keys, d_bad);
-        GK(hipGetLastError());
-    }
-    GK(hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, s));
-    GK(hipStreamSynchronize(s));
-    if (bad) {
-        err = "edge endpoint outside [0, V)";
-        rc = -2;
-        goto done;
-    }
-    rc = csr_from_keys(s, V, m, keys, fwb, fwa, bwb, bwa, E, err);
+    rc = csr_from_filled(s, V, m, fill, fwb, fwa, bwb, bwa, E, err);
 done:
-    if (keys) (void)hipFree(keys);
     if (d_bad) (void)hipFree(d_bad);
     return rc;
 }
