@@ -55,6 +55,28 @@ struct HubItem {
     int32_t start;  // first edge offset of this chunk
 };
 
+// Device memory that is kept from one use to the next and grows when a use
+// needs more (its contents do not survive that).
+struct Workspace {
+    void* p = nullptr;
+    size_t cap = 0;
+    hipError_t ensure(size_t bytes) {
+        if (p && bytes <= cap) return hipSuccess;
+        release();
+        const hipError_t e = hipMalloc(&p, bytes);
+        if (e == hipSuccess) cap = bytes;
+        else p = nullptr;
+        return e;
+    }
+    void release() {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        cap = 0;
+    }
+};
+// A graph builder's scratch beyond this is given back when the call ends.
+constexpr size_t kKeepScratch = (size_t)1 << 30;
+
 // ---- cooperative giant-phase kernel (giant.hip) --------------------------
 struct alignas(128) GLine {
     int32_t v;
@@ -289,11 +311,17 @@ hipError_t launch_check_csr(const int32_t* beg, const int32_t* adj, int32_t V, i
 
 // ---- graph building (gen.hip).  Return 0, -1 bad argument, -2 bad edge,
 // -3 out of memory, -4 HIP error (message in err).
-int gen_rmat_device(hipStream_t s, int32_t V, double ef, double a, double b, double c, uint64_t seed, int32_t** fwb,
+// m keeps the keys and counts, sort the sort's own scratch; both belong to
+// the caller, who makes one call on them at a time.
+struct GenScratch {
+    Workspace& m;
+    Workspace& sort;
+};
+int gen_rmat_device(hipStream_t s, GenScratch& w, int32_t V, double ef, double a, double b, double c, uint64_t seed, int32_t** fwb,
                     int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err);
-int gen_grid_device(hipStream_t s, int32_t n, double p_bidir, uint64_t seed, int32_t** fwb, int32_t** fwa,
+int gen_grid_device(hipStream_t s, GenScratch& w, int32_t n, double p_bidir, uint64_t seed, int32_t** fwb, int32_t** fwa,
                     int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err);
-int build_csr_device(hipStream_t s, int32_t V, int64_t m, const int32_t* src, const int32_t* dst, int32_t** fwb,
+int build_csr_device(hipStream_t s, GenScratch& w, int32_t V, int64_t m, const int32_t* src, const int32_t* dst, int32_t** fwb,
                      int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err);
 int csr_stable_one(hipStream_t s, int32_t V, int64_t m, const int32_t* key, const int32_t* val, int32_t** beg,
                    int32_t** adj, std::string& err);

@@ -284,50 +284,67 @@ constexpr int kGrid = 4096;
 
 }  // namespace
 
-// keys[0, m) (edge_key form) -> CSR pair.  keys is clobbered.  Only the
-// 2 * bits bits of a key are sorted, in 32-bit keys when they fit (V <= 65536);
-// the kept keys, then in (src, dst) order, are sorted by dst alone for the
+// A builder's scratch: the keys twice, the counts and starts of their chunks,
+// the gaps of one direction, and three counters (gaps of each direction, bad
+// endpoints).
+template <class K>
+struct BuildMem {
+    K *keys, *alt;
+    int32_t* counts;
+    int64_t* start;  // first kept position of every chunk, then their total
+    Gap* gaps;
+    int32_t* n;
+    int64_t chunks;
+
+    BuildMem(void* base, int32_t V, int64_t m, size_t* bytes = nullptr) {
+        chunks = (m + kKeepChunk - 1) / kKeepChunk;
+        size_t off = 0;
+        auto take = [&](size_t size) {
+            char* p = static_cast<char*>(base) + off;
+            off += (size + 255) & ~(size_t)255;
+            return static_cast<void*>(p);
+        };
+        keys = static_cast<K*>(take((size_t)std::max<int64_t>(m, 1) * sizeof(K)));
+        alt = static_cast<K*>(take((size_t)std::max<int64_t>(m, 1) * sizeof(K)));
+        counts = static_cast<int32_t*>(take((size_t)(chunks + 1) * 4));
+        start = static_cast<int64_t*>(take((size_t)(chunks + 1) * 8));
+        gaps = static_cast<Gap*>(take((size_t)gap_capacity(V) * sizeof(Gap)));
+        n = static_cast<int32_t*>(take(12));
+        if (bytes) *bytes = off;
+    }
+};
+
+// M.keys[0, m) (edge_key form) -> CSR pair; M.n is zero.  Only the 2 * bits
+// bits of a key are sorted, in 32-bit keys when they fit (V <= 65536); the
+// kept keys, then in (src, dst) order, are sorted by dst alone for the
 // transposed rows: the sort is stable, so each row stays in src order.  At
 // 2^20 vertices that is 5 + 3 radix passes instead of the 8 + 8 of full 64-bit
 // keys.
 template <class K>
-int csr_from_keys(hipStream_t s, int32_t V, int64_t m, K* keys, int32_t** fwb, int32_t** fwa, int32_t** bwb,
-                  int32_t** bwa, int64_t* E_out, std::string& err) {
+int csr_from_keys(hipStream_t s, Workspace& sort, const BuildMem<K>& M, int32_t V, int64_t m, int32_t** fwb,
+                  int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E_out, std::string& err) {
     int rc = 0;
     const int bits = id_bits(V);
-    const int64_t chunks = (m + kKeepChunk - 1) / kKeepChunk;
+    const int64_t chunks = M.chunks;
     const int keep_grid = (int)std::max<int64_t>(1, std::min<int64_t>(kGrid, (chunks + kKeepWaves - 1) / kKeepWaves));
-    const int64_t gap_bytes = gap_capacity(V) * (int64_t)sizeof(Gap);
-    K* alt = nullptr;
-    void* tmp = nullptr;
-    int32_t* counts = nullptr;
-    int64_t* start = nullptr;  // first kept position of every chunk, then their total
-    size_t tmp_bytes = 0, b1 = 0, b2 = 0;
+    size_t b1 = 0, b2 = 0;
     int64_t E = 0;
-    char* gaps = nullptr;  // two counters, then the gaps of one direction
-    rocprim::double_buffer<K> buf(keys, keys);
-    *fwb = *fwa = *bwb = *bwa = nullptr;
-    GK(hipMalloc(&alt, (size_t)std::max<int64_t>(m, 1) * sizeof(K)));
-    GK(hipMalloc(&start, (size_t)(chunks + 1) * 8));
-    GK(hipMalloc(&counts, (size_t)(chunks + 1) * 4));
-    GK(hipMalloc(&gaps, (size_t)gap_bytes + 16));
-    buf = rocprim::double_buffer<K>(keys, alt);
+    rocprim::double_buffer<K> buf(M.keys, M.alt);
     if (m > 0) {
         GK(rocprim::radix_sort_keys(nullptr, b1, buf, (size_t)m, 0, 2 * bits, s));
-        GK(rocprim::exclusive_scan(nullptr, b2, counts, start, (int64_t)0, (size_t)chunks + 1,
+        GK(rocprim::exclusive_scan(nullptr, b2, M.counts, M.start, (int64_t)0, (size_t)chunks + 1,
                                    rocprim::plus<int64_t>(), s));
-        tmp_bytes = std::max(b1, b2) + 256;
-        GK(hipMalloc(&tmp, tmp_bytes));
-        b1 = b2 = tmp_bytes;
-        GK(rocprim::radix_sort_keys(tmp, b1, buf, (size_t)m, 0, 2 * bits, s));
+        GK(sort.ensure(std::max(b1, b2) + 256));
+        b1 = b2 = sort.cap;
+        GK(rocprim::radix_sort_keys(sort.p, b1, buf, (size_t)m, 0, 2 * bits, s));
         hipLaunchKernelGGL(k_keep_count<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), m, bits,
-                           chunks, counts);
+                           chunks, M.counts);
         GK(hipGetLastError());
         // one entry more than chunks: the last start is the total (the last
         // count is not read into it)
-        GK(rocprim::exclusive_scan(tmp, b2, counts, start, (int64_t)0, (size_t)chunks + 1, rocprim::plus<int64_t>(),
-                                   s));
-        GK(hipMemcpyAsync(&E, start + chunks, 8, hipMemcpyDeviceToHost, s));
+        GK(rocprim::exclusive_scan(sort.p, b2, M.counts, M.start, (int64_t)0, (size_t)chunks + 1,
+                                   rocprim::plus<int64_t>(), s));
+        GK(hipMemcpyAsync(&E, M.start + chunks, 8, hipMemcpyDeviceToHost, s));
         GK(hipStreamSynchronize(s));
     }
     if (E > INT32_MAX) {
@@ -341,27 +358,20 @@ int csr_from_keys(hipStream_t s, int32_t V, int64_t m, K* keys, int32_t** fwb, i
     GK(hipMalloc(bwa, (size_t)std::max<int64_t>(E, 1) * 4));
     if (E > 0) {
         K* kept = buf.alternate();
-        int32_t* n_gaps = reinterpret_cast<int32_t*>(gaps);
-        Rows R{*fwb, reinterpret_cast<Gap*>(gaps + 16), n_gaps};
-        GK(launch_fill_i32(n_gaps, 0, 2, 1, s));
+        Rows R{*fwb, M.gaps, M.n};
         hipLaunchKernelGGL(k_keep<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), m, bits, chunks,
-                           start, kept, *fwa, R, V);
+                           M.start, kept, *fwa, R, V);
         GK(hipGetLastError());
         hipLaunchKernelGGL(k_gaps, dim3(256), dim3(256), 0, s, R);
         GK(hipGetLastError());
         buf = rocprim::double_buffer<K>(kept, buf.current());
         // fewer keys can take another of the sort's methods, with more scratch
         GK(rocprim::radix_sort_keys(nullptr, b1, buf, (size_t)E, 0, bits, s));
-        if (b1 > tmp_bytes) {
-            (void)hipFree(tmp);
-            tmp = nullptr;
-            GK(hipMalloc(&tmp, b1));
-            tmp_bytes = b1;
-        }
-        b1 = tmp_bytes;
-        GK(rocprim::radix_sort_keys(tmp, b1, buf, (size_t)E, 0, bits, s));
+        GK(sort.ensure(b1));
+        b1 = sort.cap;
+        GK(rocprim::radix_sort_keys(sort.p, b1, buf, (size_t)E, 0, bits, s));
         R.beg = *bwb;
-        R.n_gaps = n_gaps + 1;
+        R.n_gaps = M.n + 1;
         hipLaunchKernelGGL(k_transposed<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), E, bits,
                            (E + kKeepChunk - 1) / kKeepChunk, *bwa, R, V);
         GK(hipGetLastError());
@@ -374,14 +384,6 @@ int csr_from_keys(hipStream_t s, int32_t V, int64_t m, K* keys, int32_t** fwb, i
     GK(hipStreamSynchronize(s));
     *E_out = E;
 done:
-    for (void* p : {(void*)alt, tmp, (void*)counts, (void*)start, (void*)gaps})
-        if (p) (void)hipFree(p);
-    if (rc) {
-        for (int32_t** p : {fwb, fwa, bwb, bwa}) {
-            if (*p) (void)hipFree(*p);
-            *p = nullptr;
-        }
-    }
     return rc;
 }
 
@@ -429,27 +431,6 @@ done:
     return rc;
 }
 
-// The key buffer of m edges over V vertices and, on it, `fill` (which writes
-// the keys) and csr_from_keys.
-template <class Fill>
-int csr_from_filled(hipStream_t s, int32_t V, int64_t m, Fill&& fill, int32_t** fwb, int32_t** fwa, int32_t** bwb,
-                    int32_t** bwa, int64_t* E, std::string& err) {
-    void* keys = nullptr;
-    int rc = 0;
-    const bool narrow = 2 * id_bits(V) <= 32;
-    GK(hipMalloc(&keys, (size_t)std::max<int64_t>(m, 1) * (narrow ? 4 : 8)));
-    if (narrow) {
-        rc = fill(static_cast<uint32_t*>(keys));
-        if (!rc) rc = csr_from_keys(s, V, m, static_cast<uint32_t*>(keys), fwb, fwa, bwb, bwa, E, err);
-    } else {
-        rc = fill(static_cast<uint64_t*>(keys));
-        if (!rc) rc = csr_from_keys(s, V, m, static_cast<uint64_t*>(keys), fwb, fwa, bwb, bwa, E, err);
-    }
-done:
-    if (keys) (void)hipFree(keys);
-    return rc;
-}
-
 int launched(std::string& err) {
     const hipError_t e = hipGetLastError();
     if (e == hipSuccess) return 0;
@@ -457,50 +438,83 @@ int launched(std::string& err) {
     return e == hipErrorOutOfMemory ? -3 : -4;
 }
 
-int gen_rmat_device(hipStream_t s, int32_t V, double ef, double a, double b, double c, uint64_t seed, int32_t** fwb,
-                    int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
+// Scratch for m edges over V vertices and, on it, fill(memory) (which writes
+// the keys) and csr_from_keys.
+template <class K, class Fill>
+int csr_from_filled(hipStream_t s, GenScratch& w, int32_t V, int64_t m, Fill&& fill, int32_t** fwb, int32_t** fwa,
+                    int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
+    int rc = 0;
+    size_t bytes = 0;
+    BuildMem<K> size(nullptr, V, m, &bytes);
+    *fwb = *fwa = *bwb = *bwa = nullptr;
+    GK(w.m.ensure(bytes));
+    {
+        const BuildMem<K> M(w.m.p, V, m);
+        GK(launch_fill_i32(M.n, 0, 3, 1, s));
+        rc = fill(M);
+        if (!rc) rc = csr_from_keys<K>(s, w.sort, M, V, m, fwb, fwa, bwb, bwa, E, err);
+    }
+done:
+    if (rc) {
+        (void)hipStreamSynchronize(s);  // nothing queued may outlive what is freed
+        for (int32_t** p : {fwb, fwa, bwb, bwa}) {
+            if (*p) (void)hipFree(*p);
+            *p = nullptr;
+        }
+    }
+    if (w.m.cap > kKeepScratch) w.m.release();
+    if (w.sort.cap > kKeepScratch) w.sort.release();
+    return rc;
+}
+
+template <class Fill>
+int csr_from(hipStream_t s, GenScratch& w, int32_t V, int64_t m, Fill&& fill, int32_t** fwb, int32_t** fwa,
+             int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
+    if (2 * id_bits(V) <= 32) return csr_from_filled<uint32_t>(s, w, V, m, fill, fwb, fwa, bwb, bwa, E, err);
+    return csr_from_filled<uint64_t>(s, w, V, m, fill, fwb, fwa, bwb, bwa, E, err);
+}
+
+int gen_rmat_device(hipStream_t s, GenScratch& w, int32_t V, double ef, double a, double b, double c, uint64_t seed,
+                    int32_t** fwb, int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
     if (V <= 0 || ef < 0 || a < 0 || b < 0 || c < 0 || a + b + c > 1.0) return -1;
     int scale = 0;
     while (((int64_t)1 << scale) < (int64_t)V) ++scale;
     const int64_t m = llround(ef * (double)V);
     const double S = 4294967296.0;
     const uint32_t t1 = (uint32_t)(a * S), t2 = (uint32_t)((a + b) * S), t3 = (uint32_t)((a + b + c) * S);
-    auto fill = [&](auto* keys) {
-        using K = std::remove_pointer_t<decltype(keys)>;
+    auto fill = [&](const auto& M) {
+        using K = std::remove_pointer_t<decltype(M.keys)>;
         hipLaunchKernelGGL(k_rmat<K>, dim3(kGrid), dim3(256), 0, s, V, scale, m, t1, t2, t3, stream_base(seed, 1),
-                           id_bits(V), keys);
+                           id_bits(V), M.keys);
         return launched(err);
     };
-    return csr_from_filled(s, V, m, fill, fwb, fwa, bwb, bwa, E, err);
+    return csr_from(s, w, V, m, fill, fwb, fwa, bwb, bwa, E, err);
 }
 
-int gen_grid_device(hipStream_t s, int32_t n, double p_bidir, uint64_t seed, int32_t** fwb, int32_t** fwa,
-                    int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
+int gen_grid_device(hipStream_t s, GenScratch& w, int32_t n, double p_bidir, uint64_t seed, int32_t** fwb,
+                    int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
     if (n < 2 || (int64_t)n * n > INT32_MAX || p_bidir < 0 || p_bidir > 1) return -1;
     const int64_t L = 2 * (int64_t)n * (n - 1), R = L / 100, m = 2 * L + R;
     const uint32_t tb = (uint32_t)(p_bidir * 4294967296.0);
-    auto fill = [&](auto* keys) {
-        using K = std::remove_pointer_t<decltype(keys)>;
+    auto fill = [&](const auto& M) {
+        using K = std::remove_pointer_t<decltype(M.keys)>;
         hipLaunchKernelGGL(k_grid<K>, dim3(kGrid), dim3(256), 0, s, n, tb, stream_base(seed, 2), stream_base(seed, 3),
-                           id_bits((int64_t)n * n), keys);
+                           id_bits((int64_t)n * n), M.keys);
         return launched(err);
     };
-    return csr_from_filled(s, n * n, m, fill, fwb, fwa, bwb, bwa, E, err);
+    return csr_from(s, w, n * n, m, fill, fwb, fwa, bwb, bwa, E, err);
 }
 
-int build_csr_device(hipStream_t s, int32_t V, int64_t m, const int32_t* src, const int32_t* dst, int32_t** fwb,
-                     int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
+int build_csr_device(hipStream_t s, GenScratch& w, int32_t V, int64_t m, const int32_t* src, const int32_t* dst,
+                     int32_t** fwb, int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E, std::string& err) {
     if (V < 0 || m < 0) return -1;
-    int32_t* d_bad = nullptr;
-    int32_t bad = 0;
-    int rc = 0;
-    auto fill = [&](auto* keys) {
-        using K = std::remove_pointer_t<decltype(keys)>;
-        if (m > 0) {
-            hipLaunchKernelGGL(k_pack<K>, dim3(kGrid), dim3(256), 0, s, src, dst, m, V, id_bits(V), keys, d_bad);
-            if (int e = launched(err)) return e;
-        }
-        if (hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+    auto fill = [&](const auto& M) {
+        using K = std::remove_pointer_t<decltype(M.keys)>;
+        if (m == 0) return 0;
+        int32_t bad = 0;
+        hipLaunchKernelGGL(k_pack<K>, dim3(kGrid), dim3(256), 0, s, src, dst, m, V, id_bits(V), M.keys, M.n + 2);
+        if (int e = launched(err)) return e;
+        if (hipMemcpyAsync(&bad, M.n + 2, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipStreamSynchronize(s) != hipSuccess) {
             err = "reading the edge check failed";
             return -4;
@@ -511,12 +525,7 @@ int build_csr_device(hipStream_t s, int32_t V, int64_t m, const int32_t* src, co
         }
         return 0;
     };
-    GK(hipMalloc(&d_bad, 4));
-    GK(hipMemsetAsync(d_bad, 0, 4, s));
-    rc = csr_from_filled(s, V, m, fill, fwb, fwa, bwb, bwa, E, err);
-done:
-    if (d_bad) (void)hipFree(d_bad);
-    return rc;
+    return csr_from(s, w, V, m, fill, fwb, fwa, bwb, bwa, E, err);
 }
 
 }  // namespace ispan

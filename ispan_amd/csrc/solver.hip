@@ -45,8 +45,11 @@ struct ispan_ctx {
     int64_t nwords = 0;
     int32_t* fw_first = nullptr;  // first out-/in-neighbour per vertex, built at bind
     int32_t* bw_first = nullptr;
+    Workspace first_mem;  // of a bound single graph's first arrays, kept from one graph to the next
+    Workspace gen_mem, gen_sort;  // the graph builders' scratch (gen.hip), kept up to kKeepScratch
 
-    // solve state (capacity cap_V / cap_E)
+    // solve state (capacity cap_V / cap_E), carved from solve_mem
+    void* solve_mem = nullptr;
     int32_t cap_V = -1;
     int64_t cap_E = -1;
     int32_t* lab = nullptr;
@@ -146,33 +149,63 @@ void dfree(T*& p) {
     p = nullptr;
 }
 
-void free_solve_buffers(ispan_ctx* ctx) {
-    dfree(ctx->lab);
-    dfree(ctx->act);
-    dfree(ctx->fvis);
-    dfree(ctx->bvis);
-    for (int i = 0; i < 2; ++i) {
-        dfree(ctx->fq[i]);
-        dfree(ctx->q[i]);
-        dfree(ctx->hub[i]);
+// Buffers placed one after another from base, 256-byte aligned; without a
+// base they are only sized.
+struct Carve {
+    unsigned char* base;
+    size_t off = 0;
+    template <class T>
+    void take(T*& p, size_t bytes) {
+        p = base ? reinterpret_cast<T*>(base + off) : nullptr;
+        off += (bytes + 255) & ~(size_t)255;
     }
-    dfree(ctx->parent);
-    dfree(ctx->stamp);
-    dfree(ctx->keys);
-    dfree(ctx->keys_alt);
-    dfree(ctx->starts);
-    dfree(ctx->qbuf);
-    dfree(ctx->part);
-    dfree(ctx->snap);
-    dfree(ctx->gh[0]);
-    dfree(ctx->gh[1]);
-    dfree(ctx->ghb[0]);
-    dfree(ctx->ghb[1]);
-    dfree(ctx->snapb);
-    dfree(ctx->gdbg);
-    if (ctx->sort_tmp) (void)hipFree(ctx->sort_tmp);
-    ctx->sort_tmp = nullptr;
-    ctx->sort_tmp_bytes = 0;
+};
+
+int64_t hub_capacity(int64_t E) { return 2 * (E / kHubChunk) + 64; }
+
+// The solve state of a graph of V vertices and E edges.
+void carve_solve_state(ispan_ctx* c, Carve& m, int32_t V, int64_t E, size_t sort_bytes) {
+    const size_t nv = (size_t)std::max(V, 1) + 1;
+    const size_t nw = (size_t)((V + 63) / 64) + 1;
+    m.take(c->lab, nv * 4);
+    m.take(c->act, nw * 8);
+    m.take(c->fvis, nw * 8);
+    m.take(c->bvis, nw * 8);
+    for (int i = 0; i < 2; ++i) {
+        // 8 bytes a vertex: the giant kernel's top-down queue entries
+        // (first edge, degree); the other phases queue 4-byte ids in them
+        m.take(c->fq[i], nv * 8);
+        m.take(c->q[i], nv * 8);
+        m.take(c->hub[i], (size_t)hub_capacity(E) * sizeof(HubItem));
+    }
+    m.take(c->parent, nv * 4);
+    m.take(c->stamp, nv * 4);
+    m.take(c->keys, nv * 8);
+    m.take(c->keys_alt, nv * 8);
+    m.take(c->starts, nv * 4);
+    m.take(c->qbuf, nv * 4);
+    m.take(c->part, (size_t)c->grid * sizeof(PivotPart));
+    m.take(c->snap, nw * 8);
+    for (int i = 0; i < 2; ++i) {
+        m.take(c->gh[i], (size_t)giant_hub_capacity(E) * sizeof(HubItem));
+        m.take(c->ghb[i], (size_t)giant_hub_capacity(E) * sizeof(HubItem));
+    }
+    m.take(c->snapb, nw * 8);
+    m.take(c->gdbg, (size_t)2 * std::max(c->coop_grid, 1) * 4);
+    m.take(c->sort_tmp, sort_bytes + 256);
+    c->sort_tmp_bytes = sort_bytes + 256;
+}
+
+// Scratch of the sort of nv WCC keys.
+hipError_t sort_scratch(int32_t V, size_t& bytes, hipStream_t s) {
+    const size_t nv = (size_t)std::max(V, 1) + 1;
+    return rocprim::radix_sort_keys(nullptr, bytes, static_cast<uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr), nv,
+                                    0, 64, s);
+}
+
+void free_solve_buffers(ispan_ctx* ctx) {
+    if (ctx->solve_mem) (void)hipFree(ctx->solve_mem);
+    ctx->solve_mem = nullptr;
     ctx->cap_V = -1;
     ctx->cap_E = -1;
     ctx->have_solution = false;
@@ -219,50 +252,25 @@ void free_workspace(ispan_ctx* ctx) {
 void free_graph(ispan_ctx* ctx) {
     free_batch(ctx);
     for (auto& p : ctx->owned) dfree(p);
-    dfree(ctx->fw_first);
-    dfree(ctx->bw_first);
+    ctx->fw_first = ctx->bw_first = nullptr;
     ctx->fwb = ctx->fwa = ctx->bwb = ctx->bwa = nullptr;
     ctx->V = -1;
     ctx->E = 0;
     ctx->have_solution = false;
 }
 
-int64_t hub_capacity(int64_t E) { return 2 * (E / kHubChunk) + 64; }
-
+// One allocation for all of it: two dozen of their own cost a graph's first
+// solve more than the solve.
 int ensure_buffers(ispan_ctx* ctx, int32_t V, int64_t E) {
     if (V <= ctx->cap_V && E <= ctx->cap_E) return ISPAN_OK;
     free_solve_buffers(ctx);
-    const size_t nv = (size_t)std::max(V, 1) + 1;
-    const size_t nw = (size_t)((V + 63) / 64) + 1;
-    CK(hipMalloc(&ctx->lab, nv * 4));
-    CK(hipMalloc(&ctx->act, nw * 8));
-    CK(hipMalloc(&ctx->fvis, nw * 8));
-    CK(hipMalloc(&ctx->bvis, nw * 8));
-    for (int i = 0; i < 2; ++i) {
-        // 8 bytes a vertex: the giant kernel's top-down queue entries
-        // (first edge, degree); the other phases queue 4-byte ids in them
-        CK(hipMalloc(&ctx->fq[i], nv * 8));
-        CK(hipMalloc(&ctx->q[i], nv * 8));
-        CK(hipMalloc(&ctx->hub[i], (size_t)hub_capacity(E) * sizeof(HubItem)));
-    }
-    CK(hipMalloc(&ctx->parent, nv * 4));
-    CK(hipMalloc(&ctx->stamp, nv * 4));
-    CK(hipMalloc(&ctx->keys, nv * 8));
-    CK(hipMalloc(&ctx->keys_alt, nv * 8));
-    CK(hipMalloc(&ctx->starts, nv * 4));
-    CK(hipMalloc(&ctx->qbuf, nv * 4));
-    CK(hipMalloc(&ctx->part, (size_t)ctx->grid * sizeof(PivotPart)));
-    CK(hipMalloc(&ctx->snap, nw * 8));
-    for (int i = 0; i < 2; ++i) {
-        CK(hipMalloc(&ctx->gh[i], (size_t)giant_hub_capacity(E) * sizeof(HubItem)));
-        CK(hipMalloc(&ctx->ghb[i], (size_t)giant_hub_capacity(E) * sizeof(HubItem)));
-    }
-    CK(hipMalloc(&ctx->snapb, nw * 8));
-    CK(hipMalloc(&ctx->gdbg, (size_t)2 * std::max(ctx->coop_grid, 1) * 4));
     size_t bytes = 0;
-    CK(rocprim::radix_sort_keys(nullptr, bytes, ctx->keys, ctx->keys_alt, (size_t)nv, 0, 64, ctx->stream));
-    CK(hipMalloc(&ctx->sort_tmp, bytes + 256));
-    ctx->sort_tmp_bytes = bytes + 256;
+    CK(sort_scratch(V, bytes, ctx->stream));
+    Carve size{nullptr};
+    carve_solve_state(ctx, size, V, E, bytes);
+    CK(hipMalloc(&ctx->solve_mem, size.off));
+    Carve place{static_cast<unsigned char*>(ctx->solve_mem)};
+    carve_solve_state(ctx, place, V, E, bytes);
     ctx->cap_V = V;
     ctx->cap_E = E;
     return ISPAN_OK;
@@ -882,9 +890,10 @@ int bind_common(ispan_ctx* ctx, int32_t V, int64_t E) {
     ctx->V = V;
     ctx->E = E;
     ctx->nwords = ((int64_t)V + 63) / 64;
-    const size_t nv = (size_t)std::max(V, 1);
-    CK(hipMalloc(&ctx->fw_first, nv * 4));
-    CK(hipMalloc(&ctx->bw_first, nv * 4));
+    const size_t nv = ((size_t)std::max(V, 1) + 63) & ~(size_t)63;
+    CK(ctx->first_mem.ensure(nv * 8));
+    ctx->fw_first = static_cast<int32_t*>(ctx->first_mem.p);
+    ctx->bw_first = ctx->fw_first + nv;
     if (V > 0) {
         CK(launch_first(ctx->fwb, ctx->fwa, V, ctx->fw_first, ctx->grid, ctx->stream));
         CK(launch_first(ctx->bwb, ctx->bwa, V, ctx->bw_first, ctx->grid, ctx->stream));
@@ -1000,6 +1009,9 @@ int ispan_ctx_destroy(ispan_ctx* ctx) {
     free_solve_buffers(ctx);
     free_graph(ctx);
     free_workspace(ctx);
+    ctx->first_mem.release();
+    ctx->gen_mem.release();
+    ctx->gen_sort.release();
     dfree(ctx->ctl);
     dfree(ctx->gstate);
     dfree(ctx->bar);
@@ -1765,52 +1777,16 @@ int scratch_device(int dev, ScratchDevice** out) {
     return ISPAN_OK;
 }
 
-// Places the buffers ensure_buffers would allocate (same sizes), the control
-// block, the giant kernel's state and the first-neighbour arrays of bind
-// one after another from base, 256-byte aligned; with base == nullptr only
-// sizes them.  Returns the bytes used.
-size_t carve_solve_state(ispan_ctx* c, unsigned char* base, int32_t V, int64_t E, size_t sort_bytes) {
-    size_t off = 0;
-    auto take = [&](auto*& p, size_t bytes) {
-        using T = std::remove_reference_t<decltype(p)>;
-        p = base ? reinterpret_cast<T>(base + off) : nullptr;
-        off += (bytes + 255) & ~(size_t)255;
-    };
-    const size_t nv = (size_t)std::max(V, 1) + 1;
-    const size_t nw = (size_t)((V + 63) / 64) + 1;
-    take(c->lab, nv * 4);
-    take(c->act, nw * 8);
-    take(c->fvis, nw * 8);
-    take(c->bvis, nw * 8);
-    for (int i = 0; i < 2; ++i) {
-        take(c->fq[i], nv * 8);
-        take(c->q[i], nv * 8);
-        take(c->hub[i], (size_t)hub_capacity(E) * sizeof(HubItem));
-    }
-    take(c->parent, nv * 4);
-    take(c->stamp, nv * 4);
-    take(c->keys, nv * 8);
-    take(c->keys_alt, nv * 8);
-    take(c->starts, nv * 4);
-    take(c->qbuf, nv * 4);
-    take(c->part, (size_t)c->grid * sizeof(PivotPart));
-    take(c->snap, nw * 8);
-    for (int i = 0; i < 2; ++i) {
-        take(c->gh[i], (size_t)giant_hub_capacity(E) * sizeof(HubItem));
-        take(c->ghb[i], (size_t)giant_hub_capacity(E) * sizeof(HubItem));
-    }
-    take(c->snapb, nw * 8);
-    take(c->gdbg, (size_t)2 * std::max(c->coop_grid, 1) * 4);
-    unsigned char* st = nullptr;
-    take(st, sort_bytes + 256);
-    c->sort_tmp = st;
-    c->sort_tmp_bytes = sort_bytes + 256;
-    take(c->ctl, sizeof(Ctl));
-    take(c->gstate, sizeof(GiantState));
-    take(c->bar, (size_t)kBarBytesPerBlock * std::max(c->coop_grid, 1));
-    take(c->fw_first, (size_t)std::max(V, 1) * 4);
-    take(c->bw_first, (size_t)std::max(V, 1) * 4);
-    return off;
+// Places everything of an allocation-free solve: the solve state, the control
+// block, the giant kernel's state and barrier records, and the
+// first-neighbour arrays of bind.
+void carve_scratch(ispan_ctx* c, Carve& m, int32_t V, int64_t E, size_t sort_bytes) {
+    carve_solve_state(c, m, V, E, sort_bytes);
+    m.take(c->ctl, sizeof(Ctl));
+    m.take(c->gstate, sizeof(GiantState));
+    m.take(c->bar, (size_t)kBarBytesPerBlock * std::max(c->coop_grid, 1));
+    m.take(c->fw_first, (size_t)std::max(V, 1) * 4);
+    m.take(c->bw_first, (size_t)std::max(V, 1) * 4);
 }
 
 }  // namespace
@@ -1839,11 +1815,12 @@ int ispan_scc_detection_noalloc(int32_t V, int64_t E, const int32_t* d_fw_beg, c
     c.coop_grid = sd->coop_grid;
     c.clock_khz = sd->clock_khz;
     size_t sort_bytes = 0;
-    if (rocprim::radix_sort_keys(nullptr, sort_bytes, static_cast<uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr),
-                                 (size_t)std::max(V, 1) + 1, 0, 64, c.stream) != hipSuccess)
-        return ISPAN_ERR_HIP;
-    if (carve_solve_state(&c, nullptr, V, E, sort_bytes) > kScratchBytes) return ISPAN_ERR_SCRATCH;
-    carve_solve_state(&c, sd->ptr, V, E, sort_bytes);
+    if (sort_scratch(V, sort_bytes, c.stream) != hipSuccess) return ISPAN_ERR_HIP;
+    Carve size{nullptr};
+    carve_scratch(&c, size, V, E, sort_bytes);
+    if (size.off > kScratchBytes) return ISPAN_ERR_SCRATCH;
+    Carve place{sd->ptr};
+    carve_scratch(&c, place, V, E, sort_bytes);
     c.cap_V = V;  // the buffers are in place: ensure_buffers allocates nothing
     c.cap_E = E;
     c.h_ctl = &sd->h_ctl;
@@ -1984,7 +1961,8 @@ int ispan_gen_rmat_device(ispan_ctx* ctx, int32_t V, double edge_factor, double 
                           int32_t** d_fw_beg, int32_t** d_fw_adj, int32_t** d_bw_beg, int32_t** d_bw_adj, int64_t* E) {
     if (!ctx || !d_fw_beg || !d_fw_adj || !d_bw_beg || !d_bw_adj || !E) return ISPAN_ERR_ARG;
     CK(hipSetDevice(ctx->device));
-    return gen_rc(gen_rmat_device(ctx->stream, V, edge_factor, a, b, c, seed, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj,
+    GenScratch scratch{ctx->gen_mem, ctx->gen_sort};
+    return gen_rc(gen_rmat_device(ctx->stream, scratch, V, edge_factor, a, b, c, seed, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj,
                                   E, ctx->err));
 }
 
@@ -1992,8 +1970,9 @@ int ispan_gen_grid_device(ispan_ctx* ctx, int32_t n, double p_bidir, uint64_t se
                           int32_t** d_fw_adj, int32_t** d_bw_beg, int32_t** d_bw_adj, int64_t* E) {
     if (!ctx || !d_fw_beg || !d_fw_adj || !d_bw_beg || !d_bw_adj || !E) return ISPAN_ERR_ARG;
     CK(hipSetDevice(ctx->device));
+    GenScratch scratch{ctx->gen_mem, ctx->gen_sort};
     return gen_rc(
-        gen_grid_device(ctx->stream, n, p_bidir, seed, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj, E, ctx->err));
+        gen_grid_device(ctx->stream, scratch, n, p_bidir, seed, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj, E, ctx->err));
 }
 
 int ispan_build_csr_device(ispan_ctx* ctx, int32_t V, int64_t m, const int32_t* d_src, const int32_t* d_dst,
@@ -2002,7 +1981,8 @@ int ispan_build_csr_device(ispan_ctx* ctx, int32_t V, int64_t m, const int32_t* 
     if (!ctx || (m > 0 && (!d_src || !d_dst)) || !d_fw_beg || !d_fw_adj || !d_bw_beg || !d_bw_adj || !E)
         return ISPAN_ERR_ARG;
     CK(hipSetDevice(ctx->device));
-    return gen_rc(build_csr_device(ctx->stream, V, m, d_src, d_dst, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj, E,
+    GenScratch scratch{ctx->gen_mem, ctx->gen_sort};
+    return gen_rc(build_csr_device(ctx->stream, scratch, V, m, d_src, d_dst, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj, E,
                                    ctx->err));
 }
 
@@ -2110,7 +2090,8 @@ int ispan_convert_edge_list(ispan_ctx* ctx, const char* txt_path, const char* ou
         CK(hipMemcpy(d_dst, dst.data(), (size_t)m * 4, hipMemcpyHostToDevice));
     }
     if (clean) {
-        rc = gen_rc(build_csr_device(ctx->stream, V, m, d_src, d_dst, &fb, &fa, &bb, &ba, &E, ctx->err));
+        GenScratch scratch{ctx->gen_mem, ctx->gen_sort};
+        rc = gen_rc(build_csr_device(ctx->stream, scratch, V, m, d_src, d_dst, &fb, &fa, &bb, &ba, &E, ctx->err));
     } else {
         rc = gen_rc(csr_stable_one(ctx->stream, V, m, d_src, d_dst, &fb, &fa, ctx->err));
         if (!rc) rc = gen_rc(csr_stable_one(ctx->stream, V, m, d_dst, d_src, &bb, &ba, ctx->err));
