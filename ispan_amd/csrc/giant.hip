@@ -37,6 +37,7 @@ struct Smem {
     alignas(16) uint32_t bv[kBarWords][kW];  // a barrier's payload per wave
     int64_t tot[2][kBarWords];               // its totals over the grid, per reading wave
     int ok[2];
+    int steps;  // levels a narrow frontier may still take in its block
     int32_t wcnt[2][kW];    // block flushes: per-wave counts and bases of up to two counters
     int32_t wbase[2][kW];
     int32_t hv[kW][kWave];  // per-wave staged hub vertices: id, first edge, degree
@@ -594,6 +595,20 @@ __device__ __forceinline__ void push_found_n(const bool (&claim)[K], const int32
     }
 }
 
+// A frontier that is all in one tile, so in one block, goes on there without
+// grid barriers: the block takes what it claimed as its next tile while that
+// has at most kNarrowBlock edges, and its first wave alone, with no block
+// barriers either, while it has at most kNarrowWave.  A level of a few edges
+// costs 11 us across the grid, nearly all of it barrier and round trips that
+// do no work, and about 4 us in a block and 2 us in a wave.  More edges than
+// a couple of steps of one block go back to the grid, which also bounds how
+// long one block expands a growing region alone.
+constexpr int kNarrowWave = 256;
+constexpr int kNarrowBlock = 2048;
+// Such levels in a row, while the other direction waits at the barrier and
+// when it has finished.
+constexpr int kNarrowShort = 16, kNarrowLong = 4096;
+
 // Top-down to exhaustion (mode 2) without level barriers in the thin parts:
 // a wave expands the vertices it claimed itself, in the same level, instead
 // of publishing them for the next level -- the reference's asynchronous
@@ -607,17 +622,24 @@ __device__ __forceinline__ void push_found_n(const bool (&claim)[K], const int32
 // Claims stay exact (the same wave-combined atomics), so the reach set and
 // the found counts are those of a level-synchronous traversal; only the
 // level at which a vertex is expanded changes.  All lanes call it.
-__device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root, const int32_t* __restrict__ beg,
+//
+// narrow: goes on only while a step takes everything that is pending (at most
+// kWave entries of at most kNarrowWave edges together) and no hub turned up;
+// what is left then stays staged in wq, for the block to go on with.
+// Returns the steps that are left of max_steps.
+__device__ __forceinline__ int expand_local(Ctx& c, PairQueue& wq, int32_t root, const int32_t* __restrict__ beg,
                                              const int32_t* __restrict__ adj, const uint64_t* __restrict__ allow,
                                              uint64_t* vis, uint64_t* qout, int32_t* qn_out, HubStage& hs,
-                                             HubItem* hout, int32_t* hn_out, int64_t& my_found, int max_steps) {
+                                             HubItem* hout, int32_t* hn_out, int64_t& my_found, int max_steps,
+                                             bool narrow) {
     int32_t* off = c.sm.off + c.wave * kWave;  // this wave's slice of the tile arrays
     int32_t* stv = c.sm.start + c.wave * kWave;
     uint64_t* buf = wq.buf;
     constexpr int mask = kPairCap - 1;
     int head = 0, n = wq.n;  // pending: buf[head .. n) modulo kPairCap
     wave_sync();
-    for (int step = 0; n > head && step < max_steps; ++step) {
+    for (; n > head && max_steps > 0; --max_steps) {
+        if (narrow && (n > kWave || hs.n > 0)) break;
         const int k = min(kWave, n - head);
         int32_t st = 0, dg = 0;
         if (c.lane < k) {
@@ -625,9 +647,14 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
             st = qentry_start(q);
             dg = qentry_degree(q);
         }
-        head += k;
         const int incl = wave_incl_scan(dg);
         const int total = lane_get(incl, kWave - 1);
+        if (narrow) {
+            if (total > kNarrowWave) break;
+            head = n = 0;  // all of them are in registers
+        } else {
+            head += k;
+        }
         off[c.lane] = incl - dg;
         stv[c.lane] = st;
         wave_sync();
@@ -663,6 +690,10 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
         }
         wave_sync();  // the queue entries and the slice are rewritten next step
     }
+    if (narrow) {
+        wq.n = n;
+        return max_steps;
+    }
     const int left = n - head;  // the step budget ran out: the next level takes them
     if (left > 0) {
         int base = 0;
@@ -673,6 +704,7 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
     }
     wq.n = 0;
     wave_sync();
+    return max_steps;
 }
 
 // Level-synchronous top-down levels are expanded in place (as in mode 2)
@@ -707,7 +739,7 @@ struct Level {
 // giant SCC is fvis & bvis either way (a path from v to the pivot lies in
 // the forward set when v does), and the two directions then need not wait
 // for each other.
-__device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_t root, Level& lv) {
+__device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_t root, int narrow_steps, Level& lv) {
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
     const bool bw = dir != 0;
@@ -777,10 +809,11 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
         // when both directions' levels are small (fewer tiles than blocks)
         // they run on different blocks at the same time
         const int64_t b0 = bw ? ((int64_t)c.b + c.G / 2) % c.G : c.b;
+        const bool narrow = a.td_local > 0 && mode == 0 && ntiles + nh == 1;  // mode 2 goes on in place below
         for (int64_t u = b0; u < ntiles + nh; u += c.G) {
             // a tile: queue entries on threads 0..tile-1; a hub item is a
             // tile of one entry on thread 0
-            const bool hub = u >= ntiles;
+            bool hub = u >= ntiles;
             int32_t st = 0, dg = 0;
             if (!hub) {
                 const int64_t i = u * tile + c.tid;
@@ -799,33 +832,72 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
                 }
                 dg = min(rchunk, beg[v + 1] - st);
             }
-            int excl, total;
-            block_excl_scan<kW>(dg, excl, total, sm.tmp);
-            sm.off[c.tid] = excl;
-            sm.start[c.tid] = st;
-            if (c.wave == 0) c.edges_td += total;
-            __syncthreads();
-            for (int eb = 0; eb < total; eb += kGBlock) {
-                // the source of edge e is the last j with off[j] <= e
-                // (off[0] = 0, non-decreasing), found by a fixed-depth
-                // search; a hub item's is its one entry
-                const int e = eb + c.tid;
-                int pos = 0;
-                if (!hub) {
-#pragma unroll
-                    for (int sp = kGBlock / 2; sp > 0; sp >>= 1)
-                        if (sm.off[pos + sp] <= e) pos += sp;
+            while (true) {
+                int excl, total;
+                block_excl_scan<kW>(dg, excl, total, sm.tmp);
+                sm.off[c.tid] = excl;
+                sm.start[c.tid] = st;
+                if (c.wave == 0) c.edges_td += total;
+                __syncthreads();
+                for (int eb = 0; eb < total; eb += kGBlock) {
+                    // the source of edge e is the last j with off[j] <= e
+                    // (off[0] = 0, non-decreasing), found by a fixed-depth
+                    // search; a hub item's is its one entry
+                    const int e = eb + c.tid;
+                    int pos = 0;
+                    if (!hub) {
+    #pragma unroll
+                        for (int sp = kGBlock / 2; sp > 0; sp >>= 1)
+                            if (sm.off[pos + sp] <= e) pos += sp;
+                    }
+                    int32_t w[1] = {0};
+                    if (e < total) w[0] = adj[sm.start[pos] + (e - sm.off[pos])];
+                    const bool want[1] = {e < total && w[0] != root};
+                    bool claim[1];
+                    int32_t s0[1], dw[1];
+                    claim_with_degree<1>(want, w, allow, vis, beg, claim, s0, dw);
+                    my_found += claim[0];
+                    push_found_n<1>(claim, w, s0, dw, pq, qout, qn_out, hs, hout, hn_out, fedges);
                 }
-                int32_t w[1] = {0};
-                if (e < total) w[0] = adj[sm.start[pos] + (e - sm.off[pos])];
-                const bool want[1] = {e < total && w[0] != root};
-                bool claim[1];
-                int32_t s0[1], dw[1];
-                claim_with_degree<1>(want, w, allow, vis, beg, claim, s0, dw);
-                my_found += claim[0];
-                push_found_n<1>(claim, w, s0, dw, pq, qout, qn_out, hs, hout, hn_out, fedges);
+                __syncthreads();
+                if (!narrow) break;
+                // the only tile: take what it claimed as the next one
+                if (total <= kWave) {  // only the first wave had edges
+                    if (c.wave == 0) {
+                        narrow_steps = expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out,
+                                                    my_found, narrow_steps, true);
+                        fedges = c.lane < hs.n ? hs.d[c.lane] : 0;
+                        for (int i = c.lane; i < pq.n; i += kWave) fedges += qentry_degree(pq.buf[i]);
+                    }
+                }
+                const int work = wave_sum((int)fedges);
+                if (c.tid == 0) sm.steps = narrow_steps;
+                if (c.lane == 0) {
+                    sm.wcnt[0][c.wave] = pq.n;
+                    sm.wcnt[1][c.wave] = (hs.n > 0 || pq.sent > 0 || hs.sent > 0) ? kNarrowBlock + 1 : min(work, kNarrowBlock + 1);
+                }
+                __syncthreads();
+                const int cnt = sm.wcnt[0][c.lane & 15];
+                const int ci = row_incl(cnt, 0, [](int x, int y) { return x + y; });
+                const int wi = row_incl(sm.wcnt[1][c.lane & 15], 0, [](int x, int y) { return x + y; });
+                const int entries = lane_get(ci, kW - 1), edges = lane_get(wi, kW - 1);
+                const int base = lane_get(ci - cnt, c.wave);
+                narrow_steps = __builtin_amdgcn_readfirstlane(sm.steps) - 1;
+                if (entries == 0 || entries > kGBlock || edges > kNarrowBlock || narrow_steps <= 0) break;
+                wave_sync();
+                for (int i = c.lane; i < pq.n; i += kWave) {
+                    const uint64_t q = pq.buf[i];
+                    sm.off[base + i] = qentry_degree(q);
+                    sm.start[base + i] = qentry_start(q);
+                }
+                pq.n = 0;
+                fedges = 0;
+                __syncthreads();
+                st = c.tid < entries ? sm.start[c.tid] : 0;
+                dg = c.tid < entries ? sm.off[c.tid] : 0;
+                hub = false;
+                __syncthreads();
             }
-            __syncthreads();
         }
         // in place: in top-down to exhaustion, and in any later top-down
         // level whose input gives every wave at least kLocalPerWave
@@ -835,7 +907,7 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
         // expanded so took the 4096^2 grid from 5.09 to 5.8-6.5 ms.
         if (a.td_local > 0 && (mode == 2 || (L > 0 && nh == 0 && n >= kLocalPerWave * total_waves)))
             expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found,
-                             a.td_local);
+                             a.td_local, false);
         block_flush_both(c, pq, qout, qn_out, hs, hout, hn_out);
         lv = Level{(int)my_found, (int)fedges, pq.sent, hs.sent};
     } else {
@@ -1141,7 +1213,7 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
             const Dir d = dir ? b : f;
             if (!d.live) continue;
             Level lv{0, 0, 0, 0};
-            level_work(c, d, dir, root, lv);
+            level_work(c, d, dir, root, (dir ? f.live : b.live) ? kNarrowShort : kNarrowLong, lv);
             lv.found = wave_sum(lv.found);
             lv.edges = wave_sum(lv.edges);
             if (dir) lb = lv;
