@@ -41,7 +41,8 @@ struct alignas(128) Ctl {
     int64_t n_scc;
     int64_t work_edges[3];  // adjacency entries read: 0 top-down, 1 hub items, 2 bottom-up
     int64_t work_found[3];  // vertices reached, same classes
-    int32_t pad[2];
+    int32_t wcc_members;    // members of the WCCs placed so far (mice phase)
+    int32_t pad;
 };
 
 struct PivotPart {
@@ -290,14 +291,18 @@ hipError_t launch_uf_init(const int32_t* fq, int32_t* parent, Ctl* ctl, int sel,
 hipError_t launch_lp_round(const int32_t* fwb, const int32_t* fwa, const int32_t* bwb, const int32_t* bwa,
                            const uint64_t* act, const int32_t* fq, int32_t* color, Ctl* ctl, int sel, int grid,
                            hipStream_t s);
-hipError_t launch_mice_keys(const int32_t* fq, const int32_t* wcc, int32_t* stamp, uint64_t* keys, Ctl* ctl, int sel,
-                            int grid, hipStream_t s);
-hipError_t launch_mice_starts(const uint64_t* keys, int32_t n, int32_t* starts, Ctl* ctl, int grid, hipStream_t s);
-// max_wcc > 0: does nothing when a WCC has more vertices than that
-// (ctl->max_wcc, from launch_mice_starts); the caller labels them otherwise
+// The mice phase's arrays, int32[V] each: per WCC root its size and its first
+// member's place, per vertex its place in its WCC; the WCCs' roots, the
+// members WCC by WCC, and search queues.
+struct MiceBuf {
+    int32_t *cnt, *first, *slot, *roots, *member, *queue;
+};
+// SCCs of the WCCs of fq[0, n) (wcc[v]: the smallest id of v's WCC), one wave
+// each.  max_wcc > 0: labels nothing when a WCC has more vertices than that
+// (ctl->max_wcc, set here); the caller labels them otherwise.
 hipError_t launch_mice(const int32_t* fwb, const int32_t* fwa, const int32_t* bwb, const int32_t* bwa, int32_t* lab,
-                       int32_t* stamp, const uint64_t* keys, int32_t n, const int32_t* starts, Ctl* ctl,
-                       int32_t* qbuf, int32_t max_wcc, int grid, hipStream_t s);
+                       int32_t* stamp, const int32_t* fq, int32_t n, const int32_t* wcc, const MiceBuf& m, Ctl* ctl,
+                       int32_t max_wcc, int grid, hipStream_t s);
 hipError_t launch_count_unlabelled(const int32_t* lab, int32_t V, const uint64_t* sel, Ctl* ctl, int grid,
                                    hipStream_t s);
 hipError_t launch_stats(const int32_t* fwb, const int32_t* bwb, const int32_t* lab, const uint64_t* fvis,

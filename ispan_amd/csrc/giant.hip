@@ -1352,15 +1352,6 @@ __device__ __forceinline__ void trim_sweep(Ctx& c, const int32_t* fin, int64_t n
     block_flush(c, wq, fout, fcount);
 }
 
-__device__ __forceinline__ int32_t uf_root_g(int32_t* parent, int32_t v) {
-    int32_t nx = load_agent(&parent[v]);
-    while (nx != v) {
-        v = nx;
-        nx = load_agent(&parent[v]);
-    }
-    return v;
-}
-
 // ---- small-SCC strategies after the trims (wcc_mode 1 and 2), run by
 // k_tail: a second cooperative launch on the same stream, made only when the
 // giant phase leaves active vertices.  A kernel of their own keeps k_giant's
@@ -1676,8 +1667,8 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
                     if (w == v || !bit_of(a.act, w)) continue;
                     int32_t x = v, y = w;
                     while (true) {
-                        x = uf_root_g(a.parent, x);
-                        y = uf_root_g(a.parent, y);
+                        x = uf_root(a.parent, x);
+                        y = uf_root(a.parent, y);
                         if (x == y) break;
                         if (x < y) {
                             const int32_t t = x;
@@ -1691,7 +1682,7 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
             if (!gsync(c)) return false;
             for (int64_t i = gt; i < n; i += nthreads) {
                 const int32_t v = g[i];
-                st_agent(&a.parent[v], uf_root_g(a.parent, v));
+                st_agent(&a.parent[v], uf_find(a.parent, v));
             }
             wcc = true;
         }

@@ -499,15 +499,6 @@ __global__ __launch_bounds__(kBlock) void k_pattern_commit(const int32_t* __rest
 // root under the smaller one with a CAS, then every vertex jumps to its
 // root, so parent[v] = smallest id of v's WCC.  Out-edges of active vertices
 // cover every active edge once.
-__device__ __forceinline__ int32_t uf_root(int32_t* parent, int32_t v) {
-    int32_t nx = load_agent(&parent[v]);
-    while (nx != v) {
-        v = nx;
-        nx = load_agent(&parent[v]);
-    }
-    return v;
-}
-
 __global__ __launch_bounds__(kBlock) void k_uf_init(const int32_t* __restrict__ fq, int32_t* parent, const Ctl* ctl,
                                                     int sel) {
     const int n = ctl->fq_n[sel];
@@ -545,7 +536,7 @@ __global__ __launch_bounds__(kBlock) void k_uf_compress(const int32_t* __restric
     const int n = ctl->fq_n[sel];
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const int32_t v = fq[i];
-        parent[v] = uf_root(parent, v);
+        parent[v] = uf_find(parent, v);
     }
 }
 
@@ -597,74 +588,257 @@ __global__ __launch_bounds__(kBlock) void k_lp_jump(const int32_t* __restrict__ 
 __global__ void k_clear_changed(Ctl* ctl) { ctl->changed = 0; }
 
 // ------------------------------------------------------------------ mice
-// init_fw_sa + mice_fw_bw (src/fw_bw.h:1548-1691) regrouped: (wcc, v) keys
-// are sorted so each WCC is a contiguous ascending run; one wave owns a WCC
-// and repeatedly takes its smallest unlabelled member as pivot, runs a FW
-// search (visit stamp = pivot) and a BW search inside it, and labels that
-// SCC with the pivot -- its smallest id.
-__global__ __launch_bounds__(kBlock) void k_mice_keys(const int32_t* __restrict__ fq, const int32_t* __restrict__ wcc,
-                                                      int32_t* stamp, uint64_t* keys, const Ctl* ctl, int sel) {
-    const int n = ctl->fq_n[sel];
+// init_fw_sa + mice_fw_bw (src/fw_bw.h:1548-1691) regrouped: the members of
+// each WCC are brought together (k_wcc_*), and one wave owns a WCC.  Grouping
+// is a counting sort by WCC root: a member's place in its WCC is its count on
+// the root's counter, in no particular order.
+
+// The roots' counters cleared.
+__global__ __launch_bounds__(kBlock) void k_wcc_reset(const int32_t* __restrict__ fq, int32_t n,
+                                                      const int32_t* __restrict__ wcc, int32_t* cnt, Ctl* ctl) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->unlabelled = 0;  // counted again after the mice
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const int32_t v = fq[i];
-        keys[i] = ((uint64_t)(uint32_t)wcc[v] << 32) | (uint32_t)v;
-        stamp[v] = -1;
+        if (wcc[v] == v) cnt[v] = 0;
     }
 }
 
-// The start of every WCC in the sorted (WCC, vertex) keys, and the largest
-// WCC's size: a start finds its WCC's end by binary search (keys ascend by
-// WCC in their high half).
-__global__ __launch_bounds__(kBlock) void k_mice_starts(const uint64_t* __restrict__ keys, int32_t n, int32_t* starts,
-                                                        Ctl* ctl) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint64_t w = keys[i] >> 32;
-        if (i == 0 || w != (keys[i - 1] >> 32)) {
-            starts[atomicAdd(&ctl->n_wcc, 1)] = (int32_t)i;
-            int64_t lo = i + 1, hi = n;  // first index past the WCC
-            while (lo < hi) {
-                const int64_t mid = (lo + hi) / 2;
-                if ((keys[mid] >> 32) == w) lo = mid + 1;
-                else hi = mid;
+// slot[v] = v's place in its WCC; cnt[root] = the WCC's size.  The queue is in
+// ascending id order for the most part, so lanes of a wave often share a
+// root: up to kSlotRounds roots are counted once per wave.
+constexpr int kSlotRounds = 4;
+__global__ __launch_bounds__(kBlock) void k_wcc_slots(const int32_t* __restrict__ fq, int32_t n,
+                                                      const int32_t* __restrict__ wcc, int32_t* cnt, int32_t* slot,
+                                                      int32_t* stamp) {
+    const int lane = lane_id();
+    const int64_t waves = (int64_t)gridDim.x * (kBlock / kWave);
+    for (int64_t base = ((int64_t)blockIdx.x * (kBlock / kWave) + wave_id()) * kWave; base < n; base += waves * kWave) {
+        const int64_t i = base + lane;
+        const int32_t v = i < n ? fq[i] : 0;
+        const int32_t r = i < n ? wcc[v] : -1;
+        bool todo = i < n;
+        int32_t at = 0;
+        for (int k = 0; k < kSlotRounds; ++k) {
+            const uint64_t m = __ballot(todo);
+            if (!m) break;
+            const int lead = __ffsll((unsigned long long)m) - 1;
+            const int32_t L = lane_get(r, lead);
+            const uint64_t same = __ballot(todo && r == L);
+            int32_t b = 0;
+            if (lane == lead) b = atomicAdd(&cnt[L], __popcll(same));
+            b = lane_get(b, lead);
+            if (todo && r == L) {
+                at = b + __popcll(same & lanemask_lt());
+                todo = false;
             }
-            atomicMax(&ctl->max_wcc, (int32_t)(lo - i));
+        }
+        if (todo) at = atomicAdd(&cnt[r], 1);
+        if (i < n) {
+            slot[v] = at;
+            stamp[v] = -1;
         }
     }
 }
 
+// Every WCC's range of the member array and its entry in the list of WCCs; the
+// number of WCCs and the largest.  A block takes one piece of the queue, adds
+// up its WCCs first and reserves for all of them with one atomic per counter
+// (one per 256 vertices took 58 us for 318,000: 11 ns each on one address).
+constexpr int kRangeBlocks = 256;
+__global__ __launch_bounds__(kBlock) void k_wcc_ranges(const int32_t* __restrict__ fq, int32_t n,
+                                                       const int32_t* __restrict__ wcc, const int32_t* __restrict__ cnt,
+                                                       int32_t* first, int32_t* roots, Ctl* ctl) {
+    constexpr int NW = kBlock / kWave;
+    __shared__ int s_tmp[NW];
+    __shared__ int s_part[3][NW];
+    __shared__ int s_at[2];
+    const int64_t per = (((int64_t)n + gridDim.x - 1) / gridDim.x + kBlock - 1) / kBlock * kBlock;
+    const int64_t lo = min((int64_t)blockIdx.x * per, (int64_t)n), hi = min(lo + per, (int64_t)n);
+    int members = 0, found = 0, largest = 0;
+    for (int64_t i = lo + threadIdx.x; i < hi; i += kBlock) {
+        const int32_t v = fq[i];
+        if (wcc[v] != v) continue;
+        members += cnt[v];
+        largest = max(largest, cnt[v]);
+        ++found;
+    }
+    members = wave_sum(members);
+    found = wave_sum(found);
+    largest = -wave_min(-largest);
+    if (lane_id() == 0) {
+        s_part[0][wave_id()] = members;
+        s_part[1][wave_id()] = found;
+        s_part[2][wave_id()] = largest;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int m = 0, f = 0, l = 0;
+        for (int w = 0; w < NW; ++w) {
+            m += s_part[0][w];
+            f += s_part[1][w];
+            l = max(l, s_part[2][w]);
+        }
+        if (f) {
+            s_at[0] = atomicAdd(&ctl->wcc_members, m);
+            s_at[1] = atomicAdd(&ctl->n_wcc, f);
+            atomicMax(&ctl->max_wcc, l);
+        }
+    }
+    __syncthreads();
+    int at_m = s_at[0], at_f = s_at[1];  // read only where the block found a WCC
+    for (int64_t base = lo; base < hi; base += kBlock) {
+        const int64_t i = base + threadIdx.x;
+        const int32_t v = i < hi ? fq[i] : 0;
+        const bool root = i < hi && wcc[v] == v;
+        int m, f, all_m, all_f;
+        block_excl_scan(root ? cnt[v] : 0, m, all_m, s_tmp);
+        block_excl_scan(root ? 1 : 0, f, all_f, s_tmp);
+        if (root) {
+            first[v] = at_m + m;
+            roots[at_f + f] = v;
+        }
+        at_m += all_m;
+        at_f += all_f;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_wcc_members(const int32_t* __restrict__ fq, int32_t n,
+                                                        const int32_t* __restrict__ wcc,
+                                                        const int32_t* __restrict__ first,
+                                                        const int32_t* __restrict__ slot, int32_t* member) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const int32_t v = fq[i];
+        member[first[wcc[v]] + slot[v]] = v;
+    }
+}
+
+// SCCs of a WCC of n <= 64 * W vertices by one wave, from the transitive
+// closure of its out-edges: lane l holds the rows of vertices l, l + 64, ..,
+// W words each, in registers.  Active neighbours of a member are members
+// (an edge joins their WCCs), and members are unlabelled until the end here,
+// so an unlabelled neighbour's slot is its column.  Warshall's step k ORs row
+// k into the rows that have bit k: n steps of a few instructions, however long
+// the paths are, where a search per SCC costs a round trip per level (WCCs of
+// 28 vertices in 8 groups: 526 -> 25 us for 12,500 of them).
+constexpr int kLongList = 64;  // a longer list is scanned by the whole wave
+template <int W>
+__device__ __forceinline__ void closure_sccs(const int32_t* __restrict__ fwb, const int32_t* __restrict__ fwa,
+                                             int32_t* lab, const int32_t* __restrict__ slot,
+                                             const int32_t* __restrict__ member, int32_t n, uint64_t* s_row) {
+    const int lane = lane_id();
+    int32_t id[W];
+    uint64_t R[W][W];
+#pragma unroll
+    for (int a = 0; a < W; ++a) {
+        const int32_t i = a * kWave + lane;
+        id[a] = i < n ? member[i] : -1;
+#pragma unroll
+        for (int b = 0; b < W; ++b) R[a][b] = 0;
+        const int32_t p = i < n ? fwb[id[a]] : 0, e = i < n ? fwb[id[a] + 1] : 0;
+        if (e - p <= kLongList) {
+            for (int32_t k = p; k < e; ++k) {
+                const int32_t w = fwa[k];
+                if (load_agent(&lab[w]) != -1) continue;
+                const int32_t j = slot[w];
+#pragma unroll
+                for (int b = 0; b < W; ++b)
+                    if (W == 1 || (j >> 6) == b) R[a][b] |= 1ull << (j & 63);
+            }
+        }
+        uint64_t pend = __ballot(e - p > kLongList);
+        while (pend) {
+            const int l = __ffsll((unsigned long long)pend) - 1;
+            pend &= pend - 1;
+            const int32_t p0 = lane_get(p, l), e0 = lane_get(e, l);
+            if (lane < W) s_row[lane] = 0;
+            wave_sync();
+            for (int32_t k = p0 + lane; k < e0; k += kWave) {
+                const int32_t w = fwa[k];
+                if (load_agent(&lab[w]) != -1) continue;
+                const int32_t j = slot[w];
+                atomicOr(reinterpret_cast<unsigned long long*>(&s_row[j >> 6]), 1ull << (j & 63));
+            }
+            wave_sync();
+            if (lane == l) {
+#pragma unroll
+                for (int b = 0; b < W; ++b) R[a][b] = s_row[b];
+            }
+            wave_sync();
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+        const int m = min(kWave, n - c * kWave);
+        for (int k = 0; k < m; ++k) {
+            uint64_t row[W];
+#pragma unroll
+            for (int b = 0; b < W; ++b) row[b] = lane_get(R[c][b], k);
+#pragma unroll
+            for (int a = 0; a < W; ++a) {
+                const uint64_t take = 0 - ((R[a][c] >> k) & 1ull);
+#pragma unroll
+                for (int b = 0; b < W; ++b) R[a][b] |= row[b] & take;
+            }
+        }
+    }
+    // a vertex's SCC: itself and the members it reaches and that reach it;
+    // the label is the smallest id of them
+    int32_t mn[W];
+#pragma unroll
+    for (int a = 0; a < W; ++a) mn[a] = id[a];
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+        const int m = min(kWave, n - c * kWave);
+        for (int k = 0; k < m; ++k) {
+            const int32_t idk = lane_get(id[c], k);
+            uint64_t row[W];  // whom k reaches
+#pragma unroll
+            for (int b = 0; b < W; ++b) row[b] = lane_get(R[c][b], k);
+#pragma unroll
+            for (int a = 0; a < W; ++a)
+                if (((R[a][c] >> k) & (row[a] >> lane)) & 1ull) mn[a] = min(mn[a], idk);
+        }
+    }
+    // every lane has read the labels it needed: the closure used them all
+#pragma unroll
+    for (int a = 0; a < W; ++a)
+        if (a * kWave + lane < n) st_agent(&lab[id[a]], mn[a]);
+}
+
+// Larger WCCs: the wave repeatedly takes an unlabelled member as pivot, runs a
+// FW search (visit stamp = pivot) and a BW search inside the WCC, whose queue
+// then holds the pivot's SCC, and labels that with its smallest id.
+constexpr int kClosureMax = 256;  // largest WCC taken by its closure (4 words a row)
 __global__ __launch_bounds__(kBlock) void k_mice(const int32_t* __restrict__ fwb, const int32_t* __restrict__ fwa,
                                                  const int32_t* __restrict__ bwb, const int32_t* __restrict__ bwa,
-                                                 int32_t* lab, int32_t* stamp, const uint64_t* __restrict__ keys,
-                                                 int32_t n, const int32_t* __restrict__ starts, const Ctl* ctl,
-                                                 int32_t* qbuf, int32_t max_wcc) {
+                                                 int32_t* lab, int32_t* stamp, const int32_t* __restrict__ roots,
+                                                 const int32_t* __restrict__ cnt, const int32_t* __restrict__ first,
+                                                 const int32_t* __restrict__ slot, const int32_t* __restrict__ member,
+                                                 const Ctl* ctl, int32_t* qbuf, int32_t max_wcc) {
     __shared__ int s_tail[kBlock / kWave];
+    __shared__ uint64_t s_rows[kBlock / kWave][kClosureMax / kWave];
     if (max_wcc > 0 && ctl->max_wcc > max_wcc) return;  // left to the caller's other method
     const int lane = lane_id(), wave = wave_id();
     const int nw = ctl->n_wcc;
     const int waves = gridDim.x * (kBlock / kWave);
     for (int idx = blockIdx.x * (kBlock / kWave) + wave; idx < nw; idx += waves) {
-        const int32_t s = starts[idx];
-        const uint32_t root = (uint32_t)(keys[s] >> 32);
-        // segment end
-        int32_t e = s;
-        for (int32_t b = s; b < n; b += kWave) {
-            const int32_t j = b + lane;
-            const bool other = j >= n || (uint32_t)(keys[j] >> 32) != root;
-            const uint64_t m = __ballot(other);
-            if (m) {
-                e = b + __ffsll((unsigned long long)m) - 1;
-                break;
-            }
-            e = b + kWave;
+        const int32_t root = lane_get(roots[idx], 0);
+        const int32_t s = lane_get(first[root], 0), n = lane_get(cnt[root], 0);
+        if (n <= kClosureMax) {
+            if (n <= kWave) closure_sccs<1>(fwb, fwa, lab, slot, member + s, n, s_rows[wave]);
+            else if (n <= 2 * kWave) closure_sccs<2>(fwb, fwa, lab, slot, member + s, n, s_rows[wave]);
+            else closure_sccs<4>(fwb, fwa, lab, slot, member + s, n, s_rows[wave]);
+            continue;
         }
+        const int32_t e = s + n;
         int32_t* q = qbuf + s;
         int32_t cursor = s;
         while (true) {
-            // next pivot: smallest member still unlabelled
+            // next pivot: the next member still unlabelled
             int32_t pj = -1;
             for (int32_t b = cursor; b < e; b += kWave) {
                 const int32_t j = b + lane;
-                const bool fr = j < e && load_agent(&lab[(int32_t)(uint32_t)keys[j]]) == -1;
+                const bool fr = j < e && load_agent(&lab[member[j]]) == -1;
                 const uint64_t m = __ballot(fr);
                 if (m) {
                     pj = b + __ffsll((unsigned long long)m) - 1;
@@ -673,7 +847,8 @@ __global__ __launch_bounds__(kBlock) void k_mice(const int32_t* __restrict__ fwb
             }
             if (pj < 0) break;
             cursor = pj + 1;
-            const int32_t pv = (int32_t)(uint32_t)keys[pj];
+            const int32_t pv = member[pj];
+            int32_t found = 0;
             for (int phase = 0; phase < 2; ++phase) {
                 const int32_t* beg = phase == 0 ? fwb : bwb;
                 const int32_t* adj = phase == 0 ? fwa : bwa;
@@ -708,7 +883,14 @@ __global__ __launch_bounds__(kBlock) void k_mice(const int32_t* __restrict__ fwb
                     tail = s_tail[wave];
                     wave_sync();
                 }
+                found = tail;
             }
+            int32_t mn = INT32_MAX;
+            for (int32_t i = lane; i < found; i += kWave) mn = min(mn, load_agent(&q[i]));
+            mn = wave_min(mn);
+            if (mn != pv)
+                for (int32_t i = lane; i < found; i += kWave) st_agent(&lab[load_agent(&q[i])], mn);
+            wave_sync();
         }
     }
 }
@@ -1020,19 +1202,18 @@ hipError_t launch_uf_init(const int32_t* fq, int32_t* parent, Ctl* ctl, int sel,
     LAUNCH(k_uf_init, grid, fq, parent, ctl, sel);
 }
 
-hipError_t launch_mice_keys(const int32_t* fq, const int32_t* wcc, int32_t* stamp, uint64_t* keys, Ctl* ctl, int sel,
-                            int grid, hipStream_t s) {
-    LAUNCH(k_mice_keys, grid, fq, wcc, stamp, keys, ctl, sel);
-}
-
-hipError_t launch_mice_starts(const uint64_t* keys, int32_t n, int32_t* starts, Ctl* ctl, int grid, hipStream_t s) {
-    LAUNCH(k_mice_starts, grid, keys, n, starts, ctl);
-}
-
 hipError_t launch_mice(const int32_t* fwb, const int32_t* fwa, const int32_t* bwb, const int32_t* bwa, int32_t* lab,
-                       int32_t* stamp, const uint64_t* keys, int32_t n, const int32_t* starts, Ctl* ctl,
-                       int32_t* qbuf, int32_t max_wcc, int grid, hipStream_t s) {
-    LAUNCH(k_mice, grid, fwb, fwa, bwb, bwa, lab, stamp, keys, n, starts, ctl, qbuf, max_wcc);
+                       int32_t* stamp, const int32_t* fq, int32_t n, const int32_t* wcc, const MiceBuf& m, Ctl* ctl,
+                       int32_t max_wcc, int grid, hipStream_t s) {
+    const int g = (int)std::max<int64_t>(1, std::min<int64_t>(grid, ((int64_t)n + kBlock - 1) / kBlock));
+    hipLaunchKernelGGL(k_wcc_reset, dim3(g), dim3(kBlock), 0, s, fq, n, wcc, m.cnt, ctl);
+    hipLaunchKernelGGL(k_wcc_slots, dim3(g), dim3(kBlock), 0, s, fq, n, wcc, m.cnt, m.slot, stamp);
+    hipLaunchKernelGGL(k_wcc_ranges, dim3(std::min(g, kRangeBlocks)), dim3(kBlock), 0, s, fq, n, wcc, m.cnt, m.first, m.roots, ctl);
+    hipLaunchKernelGGL(k_wcc_members, dim3(g), dim3(kBlock), 0, s, fq, n, wcc, m.first, m.slot, m.member);
+    // a wave per WCC, of which there are at most n
+    const int gm = (int)std::max<int64_t>(1, std::min<int64_t>(grid, ((int64_t)n + kBlock / kWave - 1) / (kBlock / kWave)));
+    LAUNCH(k_mice, gm, fwb, fwa, bwb, bwa, lab, stamp, m.roots, m.cnt, m.first, m.slot, m.member, ctl, m.queue,
+           max_wcc);
 }
 
 hipError_t launch_count_unlabelled(const int32_t* lab, int32_t V, const uint64_t* sel, Ctl* ctl, int grid,

@@ -6,7 +6,6 @@
 
 #include <cstring>
 #include <hip/hip_runtime.h>
-#include <rocprim/rocprim.hpp>
 
 #include <stdio.h>
 #include <stdlib.h>
@@ -67,8 +66,6 @@ struct ispan_ctx {
     int32_t* qbuf = nullptr;
     PivotPart* part = nullptr;
     Ctl* ctl = nullptr;
-    void* sort_tmp = nullptr;
-    size_t sort_tmp_bytes = 0;
     Ctl* h_ctl = nullptr;  // pinned
     // cooperative giant-phase kernel
     int coop_grid = 0;
@@ -164,7 +161,7 @@ struct Carve {
 int64_t hub_capacity(int64_t E) { return 2 * (E / kHubChunk) + 64; }
 
 // The solve state of a graph of V vertices and E edges.
-void carve_solve_state(ispan_ctx* c, Carve& m, int32_t V, int64_t E, size_t sort_bytes) {
+void carve_solve_state(ispan_ctx* c, Carve& m, int32_t V, int64_t E) {
     const size_t nv = (size_t)std::max(V, 1) + 1;
     const size_t nw = (size_t)((V + 63) / 64) + 1;
     m.take(c->lab, nv * 4);
@@ -192,15 +189,6 @@ void carve_solve_state(ispan_ctx* c, Carve& m, int32_t V, int64_t E, size_t sort
     }
     m.take(c->snapb, nw * 8);
     m.take(c->gdbg, (size_t)2 * std::max(c->coop_grid, 1) * 4);
-    m.take(c->sort_tmp, sort_bytes + 256);
-    c->sort_tmp_bytes = sort_bytes + 256;
-}
-
-// Scratch of the sort of nv WCC keys.
-hipError_t sort_scratch(int32_t V, size_t& bytes, hipStream_t s) {
-    const size_t nv = (size_t)std::max(V, 1) + 1;
-    return rocprim::radix_sort_keys(nullptr, bytes, static_cast<uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr), nv,
-                                    0, 64, s);
 }
 
 void free_solve_buffers(ispan_ctx* ctx) {
@@ -264,13 +252,11 @@ void free_graph(ispan_ctx* ctx) {
 int ensure_buffers(ispan_ctx* ctx, int32_t V, int64_t E) {
     if (V <= ctx->cap_V && E <= ctx->cap_E) return ISPAN_OK;
     free_solve_buffers(ctx);
-    size_t bytes = 0;
-    CK(sort_scratch(V, bytes, ctx->stream));
     Carve size{nullptr};
-    carve_solve_state(ctx, size, V, E, bytes);
+    carve_solve_state(ctx, size, V, E);
     CK(hipMalloc(&ctx->solve_mem, size.off));
     Carve place{static_cast<unsigned char*>(ctx->solve_mem)};
-    carve_solve_state(ctx, place, V, E, bytes);
+    carve_solve_state(ctx, place, V, E);
     ctx->cap_V = V;
     ctx->cap_E = E;
     return ISPAN_OK;
@@ -767,28 +753,24 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
             CK(launch_wcc_uf(ctx->fwb, ctx->fwa, ctx->act, ctx->fq[sel], ctx->parent, ctx->ctl, sel, G, s));
         }
         rec(ctx, P, 8);
-        // P13-P14 mice: group by WCC, FW-BW per WCC
-        CK(launch_mice_keys(ctx->fq[sel], ctx->parent, ctx->stamp, ctx->keys, ctx->ctl, sel, G, s));
-        int end_bit = 32;
-        while (end_bit < 64 && ((int64_t)1 << (end_bit - 32)) < (int64_t)V) ++end_bit;
-        size_t bytes = ctx->sort_tmp_bytes;
-        CK(rocprim::radix_sort_keys(ctx->sort_tmp, bytes, ctx->keys, ctx->keys_alt, (size_t)n, 0, (unsigned)end_bit,
-                                    s));
-        CK(launch_mice_starts(ctx->keys_alt, (int32_t)n, ctx->starts, ctx->ctl, G, s));
-        // FW-BW per WCC costs a long WCC of small SCCs its size per SCC (each
-        // search runs down the rest of it): on engine 0, past
+        // P13-P14 mice: group by WCC, then each WCC's SCCs.  A long WCC of
+        // small SCCs would cost its size per SCC: on engine 0, past
         // ISPAN_MICE_MAX_WCC vertices k_mice leaves everything to the
         // colouring method, launched after the readback below shows it
-        CK(launch_mice(ctx->fwb, ctx->fwa, ctx->bwb, ctx->bwa, ctx->lab, ctx->stamp, ctx->keys_alt, (int32_t)n,
-                       ctx->starts, ctx->ctl, ctx->qbuf, coop ? ISPAN_MICE_MAX_WCC : 0, G, s));
+        int32_t* k0 = reinterpret_cast<int32_t*>(ctx->keys);      // 2 int32 a vertex
+        int32_t* k1 = reinterpret_cast<int32_t*>(ctx->keys_alt);  // and here
+        const size_t nv = (size_t)std::max(V, 1) + 1;
+        const MiceBuf mb{k0, k0 + nv, k1, ctx->starts, k1 + nv, ctx->qbuf};
+        CK(launch_mice(ctx->fwb, ctx->fwa, ctx->bwb, ctx->bwa, ctx->lab, ctx->stamp, ctx->fq[sel], (int32_t)n,
+                       ctx->parent, mb, ctx->ctl, coop ? ISPAN_MICE_MAX_WCC : 0, G, s));
         local.mice = n;
     } else if (!coop) {
         rec(ctx, P, 8);
     }
     if (!coop || host_tail) rec(ctx, P, 9);
     if (!counted) {
-        CK(launch_fill_i32(&ctx->ctl->unlabelled, 0, 1, 1, s));
-        CK(launch_count_unlabelled(ctx->lab, V, ctx->batch_sel, ctx->ctl, G, s));
+        // engine 0 gave every vertex outside the set it left in snap a label
+        CK(launch_count_unlabelled(ctx->lab, V, coop ? ctx->snap : nullptr, ctx->ctl, G, s));
         if ((rc = readback(ctx, &syncs))) return rc;
     }
     if (host_tail) local.max_wcc = ctx->h_ctl->max_wcc;
@@ -1780,8 +1762,8 @@ int scratch_device(int dev, ScratchDevice** out) {
 // Places everything of an allocation-free solve: the solve state, the control
 // block, the giant kernel's state and barrier records, and the
 // first-neighbour arrays of bind.
-void carve_scratch(ispan_ctx* c, Carve& m, int32_t V, int64_t E, size_t sort_bytes) {
-    carve_solve_state(c, m, V, E, sort_bytes);
+void carve_scratch(ispan_ctx* c, Carve& m, int32_t V, int64_t E) {
+    carve_solve_state(c, m, V, E);
     m.take(c->ctl, sizeof(Ctl));
     m.take(c->gstate, sizeof(GiantState));
     m.take(c->bar, (size_t)kBarBytesPerBlock * std::max(c->coop_grid, 1));
@@ -1814,13 +1796,11 @@ int ispan_scc_detection_noalloc(int32_t V, int64_t E, const int32_t* d_fw_beg, c
     c.grid = sd->grid;
     c.coop_grid = sd->coop_grid;
     c.clock_khz = sd->clock_khz;
-    size_t sort_bytes = 0;
-    if (sort_scratch(V, sort_bytes, c.stream) != hipSuccess) return ISPAN_ERR_HIP;
     Carve size{nullptr};
-    carve_scratch(&c, size, V, E, sort_bytes);
+    carve_scratch(&c, size, V, E);
     if (size.off > kScratchBytes) return ISPAN_ERR_SCRATCH;
     Carve place{sd->ptr};
-    carve_scratch(&c, place, V, E, sort_bytes);
+    carve_scratch(&c, place, V, E);
     c.cap_V = V;  // the buffers are in place: ensure_buffers allocates nothing
     c.cap_E = E;
     c.h_ctl = &sd->h_ctl;
