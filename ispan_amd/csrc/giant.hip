@@ -632,8 +632,6 @@ __device__ __forceinline__ int expand_local(Ctx& c, PairQueue& wq, int32_t root,
                                              uint64_t* vis, uint64_t* qout, int32_t* qn_out, HubStage& hs,
                                              HubItem* hout, int32_t* hn_out, int64_t& my_found, int max_steps,
                                              bool narrow) {
-    int32_t* off = c.sm.off + c.wave * kWave;  // this wave's slice of the tile arrays
-    int32_t* stv = c.sm.start + c.wave * kWave;
     uint64_t* buf = wq.buf;
     constexpr int mask = kPairCap - 1;
     int head = 0, n = wq.n;  // pending: buf[head .. n) modulo kPairCap
@@ -655,19 +653,27 @@ __device__ __forceinline__ int expand_local(Ctx& c, PairQueue& wq, int32_t root,
         } else {
             head += k;
         }
-        off[c.lane] = incl - dg;
-        stv[c.lane] = st;
-        wave_sync();
+        const int off = incl - dg;  // this entry's first edge of the step
+        wave_sync();  // the queue entries are read: their places may be written
         for (int eb = 0; eb < total; eb += kWave) {
-            // the source of edge e: the last j < k with off[j] <= e
+            // The source of edge e is the last entry j with off_j <= e.  Every
+            // entry has an edge, so that is the number of entries that begin
+            // at or before e, less one: those before the chunk, and those whose
+            // bit is set up to e's in the chunk's word of beginnings (an OR
+            // over the wave by DPP).  A binary search of the offsets in LDS is
+            // six dependent reads.
+            const int rel = off - eb;
+            const bool valid = c.lane < k;
+            const int before = __popcll(__ballot(valid && rel < 0));
+            uint64_t begins = row_incl((uint64_t)(valid && rel >= 0 && rel < kWave ? 1ull << rel : 0ull), (uint64_t)0,
+                                       [](uint64_t x, uint64_t y) { return x | y; });
+            begins = lane_get(begins, 15) | lane_get(begins, 31) | lane_get(begins, 47) | lane_get(begins, 63);
             const int e = eb + c.lane;
-            int pos = 0;
-#pragma unroll
-            for (int sp = kWave / 2; sp > 0; sp >>= 1)
-                if (pos + sp < k && off[pos + sp] <= e) pos += sp;
+            const int pos = before + __popcll(begins & (lanemask_lt() | (1ull << c.lane))) - 1;
+            const int32_t src = __shfl(st - off, pos, kWave);  // adj index of the entry's edge 0, less its offset
             bool want[1];
             int32_t w[1];
-            w[0] = e < total ? adj[stv[pos] + (e - off[pos])] : 0;
+            w[0] = e < total ? adj[src + e] : 0;
             want[0] = e < total && w[0] != root;
             bool claim[1];
             int32_t s0[1], d[1];
@@ -688,7 +694,7 @@ __device__ __forceinline__ int expand_local(Ctx& c, PairQueue& wq, int32_t root,
                 if (keep) st_agent(&qout[base + __popcll(m & lanemask_lt())], qentry(s0[0], d[0]));
             }
         }
-        wave_sync();  // the queue entries and the slice are rewritten next step
+        wave_sync();  // the entries pushed are read next step
     }
     if (narrow) {
         wq.n = n;
