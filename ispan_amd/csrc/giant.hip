@@ -1918,9 +1918,13 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
     const int64_t giant = lane_get(sm.tot[0][1], 0);
     const int64_t w0 = sm.tot[0][3], w1 = sm.tot[0][4], w2 = sm.tot[0][5], w3 = sm.tot[0][6];
     if (a.trace && c.tid == 0) atomicMax((unsigned long long*)&gs->post_cp[1], (unsigned long long)wall_clock64());
-    // the labels: one word per lane, the wave loads 64 words at once (its own
+    // the labels, here and in the caller's array when it gave one (a copy of
+    // its own after the launch reads and writes them once more and costs
+    // another host wait: R-MAT s24 403 -> 387 us, 700 K vertices 203 -> 190 us):
+    // one word per lane, the wave loads 64 words at once (its own
     // block's, narrowed above), then writes them four words at a time, four
     // consecutive labels a lane (coalesced 1 KB stores, no loads in the loop)
+    const bool wide2 = a.lab2 && (reinterpret_cast<uintptr_t>(a.lab2) & 15) == 0;
     for (int64_t base = wb + (int64_t)c.wave * kWave; base < we; base += (int64_t)kW * kWave) {
         const int64_t w = base + c.lane;
         uint64_t ac = 0, g = 0, sw = 0;
@@ -1947,10 +1951,16 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
             }
             if (all) {
                 st_agent4(&a.lab[v0], l[0], l[1], l[2], l[3]);
+                if (wide2) st_agent4(&a.lab2[v0], l[0], l[1], l[2], l[3]);
             } else {
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
                     if (v0 + k < a.V && ((sj >> (q + k)) & 1ull)) st_agent(&a.lab[v0 + k], l[k]);
+            }
+            if (a.lab2 && !(all && wide2)) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (v0 + k < a.V && ((sj >> (q + k)) & 1ull)) st_agent(&a.lab2[v0 + k], l[k]);
             }
         }
     }
@@ -2007,7 +2017,9 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
                 uint64_t m = a.snap[w];
                 while (m) {
                     const int64_t v = w * 64 + __ffsll((unsigned long long)m) - 1;
-                    left += a.lab[v] < 0;
+                    const int32_t l = a.lab[v];
+                    left += l < 0;
+                    if (a.lab2) st_agent(&a.lab2[v], l);  // the rest phase's labels
                     m &= m - 1;
                 }
             }

@@ -433,6 +433,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
     int32_t root = -1;
     bool rest_done = false;
     double giant_phase_ms[4] = {0, 0, 0, 0};  // engine 0: trim-1-first+pivot, FW, BW+relabel, trims+WCC
+    bool copied = false;   // d_labels holds the labels already
     bool counted = false;  // ctl->unlabelled holds the count of the finished labelling
     GiantArgs ga_tail{};   // engine 0: the giant kernel's arguments, for a colouring tail
     if (coop) {
@@ -447,6 +448,16 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
         ga.V = V;
         ga.nwords = ctx->nwords;
         ga.lab = ctx->lab;
+        // the caller's array in this device's memory is written along with
+        // the context's; any other kind gets a copy at the end
+        if (d_labels && d_labels != ctx->lab) {
+            hipPointerAttribute_t at{};
+            if (hipPointerGetAttributes(&at, d_labels) == hipSuccess) {
+                if (at.type == hipMemoryTypeDevice && at.device == ctx->device) ga.lab2 = d_labels;
+            } else {
+                (void)hipGetLastError();
+            }
+        }
         ga.act = ctx->act;
         ga.fvis = ctx->fvis;
         ga.bvis = ctx->bvis;
@@ -627,6 +638,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
             // k_tail's labels are counted by the scan after it; otherwise the
             // kernel's own check counts when nothing was left for the host
             counted = tail ? gs.n_final == 0 : gs.unl_checked != 0;
+            copied = !tail && gs.unl_checked != 0 && ga.lab2 != nullptr;
             ctx->prof.edges[0] = gs.work[0];
             ctx->prof.edges[2] = gs.work[1];
             ctx->prof.found[0] = gs.work[2];
@@ -799,7 +811,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
         ctx->err = std::to_string(ctx->h_ctl->unlabelled) + " vertices left unlabelled";
         return ISPAN_ERR_UNLABELLED;
     }
-    if (d_labels && d_labels != ctx->lab) {
+    if (d_labels && d_labels != ctx->lab && !copied) {
         CK(hipMemcpyAsync(d_labels, ctx->lab, (size_t)V * 4, hipMemcpyDeviceToDevice, s));
         CK(hipStreamSynchronize(s));
     }
