@@ -27,7 +27,20 @@ static_assert(kBarWords * 2 * 8 == kBarBytesPerBlock, "two record buffers of 8-b
 constexpr int kGBlock = 1024;
 constexpr int kW = kGBlock / kWave;
 
+// Per-direction state of the joint traversal (the same in every block).
+struct Dir {
+    int32_t mode;     // 0 top-down, 1 bottom-up, 2 top-down to exhaustion
+    int32_t L;        // levels done
+    int32_t visited;  // vertices claimed, the roots excluded
+    int32_t nq, nh;   // next level's queue entries and hub work items
+};
+// What the traversal goes on with (Smem::flow): which directions are still
+// traversing; which had a bottom-up level last and have a top-down one next.
+constexpr int kLive = 1, kGather = 4, kFailed = 16;  // of direction d: kLive << d, kGather << d
+
 struct Smem {
+    Dir dir[2];
+    int flow;
     int32_t off[kGBlock];    // top-down tile: exclusive degree prefix, first edge
     int32_t start[kGBlock];
     int tmp[kW];
@@ -488,13 +501,6 @@ __device__ __forceinline__ void push_next(bool claim, int32_t w, const int32_t* 
     pq_push(pq, claim && d > 0 && d < kGiantHubDeg, qentry(s0, d), qout, qn_out);
 }
 
-// The acquire of a barrier with ACQ, for a block that passed a barrier
-// without it.
-__device__ __forceinline__ void block_acquire() {
-    if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    __syncthreads();
-}
-
 // Claims K targets per lane, each as wave_try_claim does, and loads the
 // offsets of every candidate while the claim atomics are in flight: a
 // claimed vertex's degree costs no round trip of its own.  All lanes call it.
@@ -719,16 +725,6 @@ __device__ __forceinline__ int expand_local(Ctx& c, PairQueue& wq, int32_t root,
 // flat).
 constexpr int kLocalPerWave = 8;
 
-// Per-direction state of the joint traversal (the same in every block).
-struct Dir {
-    int mode;         // 0 top-down, 1 bottom-up, 2 top-down to exhaustion
-    int64_t L;        // levels done
-    int64_t visited;  // vertices claimed, the roots excluded
-    bool live;        // still traversing
-    bool gather;      // its last level was bottom-up and its next is top-down
-    int64_t nq, nh;   // next level's queue entries and hub work items
-};
-
 // What a wave's part of a level came to: per-thread counts and wave-uniform
 // queue totals.
 struct Level {
@@ -745,7 +741,8 @@ struct Level {
 // giant SCC is fvis & bvis either way (a path from v to the pivot lies in
 // the forward set when v does), and the two directions then need not wait
 // for each other.
-__device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_t root, int narrow_steps, Level& lv) {
+__device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t nq, int32_t nh_in, int dir, int32_t root,
+                                           int narrow_steps, Level& lv) {
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
     const bool bw = dir != 0;
@@ -765,8 +762,6 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
     PairQueue pq{c.stage(), 0};    // top-down: staged next-level entries
     WaveQueue wq{c.stage32(), 0};  // bottom-up: the same LDS, parked misses (ids)
     HubStage hs{sm.hv[c.wave], sm.hs[c.wave], sm.hd[c.wave], 0};
-    const int mode = d.mode;
-    const int64_t L = d.L;
     const int64_t total_waves = (int64_t)c.G * kW;
     const int64_t gwave = (int64_t)c.b * kW + c.wave;
     auto is_vis = [vis](int32_t u, int32_t) { return bit_of(vis, u); };
@@ -795,8 +790,8 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
             rchunk = min(rchunk, kGiantChunk);
             nh = (rdeg + rchunk - 1) / rchunk;
         } else {
-            n = d.nq;
-            nh = d.nh;
+            n = nq;
+            nh = nh_in;
             if (n < 0 || n > a.V || nh < 0 || nh > a.hub_cap) {  // cannot happen with exact claims
                 if (c.tid == 0) atomicOr(&gs->err.v, 4);
                 n = 0;
@@ -1090,7 +1085,7 @@ __device__ __forceinline__ void level_work(Ctx& c, const Dir& d, int dir, int32_
 // The gather of a direction that switches from bottom-up back to top-down:
 // the last level's finds (vis & ~snap) become the next level's queue and hub
 // items.  Each wave loads 64 words at once, then expands the non-empty ones.
-__device__ __forceinline__ void gather_finds(Ctx& c, const Dir& d, int dir, uint32_t& nq, uint32_t& nh) {
+__device__ __forceinline__ void gather_finds(Ctx& c, int32_t L, int dir, uint32_t& nq, uint32_t& nh) {
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
     GiantState* gs = a.gs;
@@ -1098,10 +1093,10 @@ __device__ __forceinline__ void gather_finds(Ctx& c, const Dir& d, int dir, uint
     const int32_t* beg = bw ? a.bwb : a.fwb;
     const uint64_t* vis = bw ? a.bvis : a.fvis;
     const uint64_t* snap = bw ? a.snapb : a.snap;
-    uint64_t* q_next = (d.L & 1) ? (bw ? a.qb1 : a.q1) : (bw ? a.qb0 : a.q0);
-    HubItem* h_next = (d.L & 1) ? (bw ? a.hb1 : a.h1) : (bw ? a.hb0 : a.h0);
-    int32_t* qn_next = &gs->qn[dir][d.L % 3].v;
-    int32_t* hn_next = &gs->hn[dir][d.L % 3].v;
+    uint64_t* q_next = (L & 1) ? (bw ? a.qb1 : a.q1) : (bw ? a.qb0 : a.q0);
+    HubItem* h_next = (L & 1) ? (bw ? a.hb1 : a.h1) : (bw ? a.hb0 : a.h0);
+    int32_t* qn_next = &gs->qn[dir][L % 3].v;
+    int32_t* hn_next = &gs->hn[dir][L % 3].v;
     PairQueue wq{c.stage(), 0};
     HubStage hs{sm.hv[c.wave], sm.hs[c.wave], sm.hd[c.wave], 0};
     const int64_t total_waves = (int64_t)c.G * kW;
@@ -1133,14 +1128,19 @@ __device__ __forceinline__ void gather_finds(Ctx& c, const Dir& d, int dir, uint
 // (src/fw_bw.h:576-624) with set_size the active count for both; a
 // direction that has finished idles while the other goes on.  Returns false
 // after a failed barrier.  With a.n_roots > 0 every listed root seeds both
-// directions (*seeded_out of them).
-__device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set_size, Dir& f, Dir& b,
-                                               int64_t* seeded_out) {
+// directions (*seeded_out of them).  The directions' state is in sm.dir.
+//
+// Wave 0 alone takes the decisions after a barrier and leaves them in LDS: the
+// block's 16 waves share four SIMDs, so a few hundred instructions that all of
+// them execute take four times as long (2.8 us a level against 1.0).
+__device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set_size, int64_t* seeded_out) {
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
     GiantState* gs = a.gs;
-    f = Dir{0, 0, 0, true, false, 0, 0};
-    b = Dir{0, 0, 0, true, false, 0, 0};
+    if (c.tid == 0) {
+        sm.dir[0] = sm.dir[1] = Dir{0, 0, 0, 0, 0};
+        sm.flow = kLive | kLive << 1;
+    }
     *seeded_out = 1;
     if (a.n_roots > 0) {
         // level-0 input of both directions: every graph's root, marked
@@ -1171,80 +1171,78 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
         if (!gsync_sum<8, true>(c, {(uint32_t)wave_sum(seeded), 0, cnt[0], cnt[1], 0, 0, cnt[2], cnt[3]}, r))
             return false;
         *seeded_out = r[0];
-        f.nq = r[2];
-        f.nh = r[3];
-        b.nq = r[6];
-        b.nh = r[7];
+        if (c.tid == 0) {
+            sm.dir[0].nq = (int32_t)r[2];
+            sm.dir[0].nh = (int32_t)r[3];
+            sm.dir[1].nq = (int32_t)r[6];
+            sm.dir[1].nh = (int32_t)r[7];
+        }
     }
-    while (f.live || b.live) {
-        if (f.gather || b.gather) {
+    __syncthreads();
+    while (true) {
+        const int flow = lane_get(sm.flow, 0);
+        if (!(flow & (kLive | kLive << 1))) break;
+        if (flow & (kGather | kGather << 1)) {
             // the visited bits were made exact after the level's barrier
-            uint32_t fq = 0, fh = 0, bq = 0, bh = 0;
+            uint32_t cnt[4] = {0, 0, 0, 0};
 #pragma unroll 1
             for (int dir = 0; dir < 2; ++dir) {
-                const Dir d = dir ? b : f;
                 uint32_t nq = 0, nh = 0;
-                if (d.gather) gather_finds(c, d, dir, nq, nh);
+                if (flow & (kGather << dir)) gather_finds(c, lane_get(sm.dir[dir].L, 0), dir, nq, nh);
                 if (dir) {
-                    bq = nq;
-                    bh = nh;
+                    cnt[2] = nq;
+                    cnt[3] = nh;
                 } else {
-                    fq = nq;
-                    fh = nh;
+                    cnt[0] = nq;
+                    cnt[1] = nh;
                 }
             }
             // the top-down level reads the queues coherently and visited bits
             // only as hints: no L2 invalidation
             int64_t r[4];
-            if (!gsync_sum<4, false>(c, {fq, fh, bq, bh}, r)) return false;
-            if (f.gather) {
-                f.nq = r[0];
-                f.nh = r[1];
+            if (!gsync_sum<4, false>(c, cnt, r)) return false;
+            if (c.tid == 0) {
+                for (int dir = 0; dir < 2; ++dir)
+                    if (flow & (kGather << dir)) {
+                        sm.dir[dir].nq = (int32_t)(dir ? r[2] : r[0]);
+                        sm.dir[dir].nh = (int32_t)(dir ? r[3] : r[1]);
+                    }
             }
-            if (b.gather) {
-                b.nq = r[2];
-                b.nh = r[3];
-            }
-            f.gather = b.gather = false;
+            __syncthreads();
         }
-        const bool tdf = f.mode != 1, tdb = b.mode != 1;
-        const int64_t edges0 = c.edges_td + c.edges_bu;  // thread 0's are the block's
         const bool tr = a.trace != 0;
         const int64_t tl0 = tr ? (int64_t)wall_clock64() : 0;
         // One copy of the level's code serves both directions: the
         // instruction cache (64 KB for two CUs) does not hold two.
-        Level lf{0, 0, 0, 0}, lb{0, 0, 0, 0};
+        uint32_t pay[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll 1
         for (int dir = 0; dir < 2; ++dir) {
-            const Dir d = dir ? b : f;
-            if (!d.live) continue;
+            if (!(flow & (kLive << dir))) continue;
+            const int mode = lane_get(sm.dir[dir].mode, 0);
+            const int32_t L = lane_get(sm.dir[dir].L, 0);
+            const int64_t edges0 = c.edges_td;
             Level lv{0, 0, 0, 0};
-            level_work(c, d, dir, root, (dir ? f.live : b.live) ? kNarrowShort : kNarrowLong, lv);
+            level_work(c, mode, L, lane_get(sm.dir[dir].nq, 0), lane_get(sm.dir[dir].nh, 0), dir, root,
+                       (flow & (kLive << (dir ^ 1))) ? kNarrowShort : kNarrowLong, lv);
             lv.found = wave_sum(lv.found);
             lv.edges = wave_sum(lv.edges);
-            if (dir) lb = lv;
-            else lf = lv;
-        }
-        // this wave's part of the work counters
-        auto wave_counts = [&](const Dir& d, const Level& lv, bool td, int dir) {
+            // this wave's part of the work counters
+            const bool td = mode != 1;
             if (td) {
                 c.found_td += (uint32_t)lv.found;
             } else {
                 c.found_bu += (uint32_t)lv.found;
                 c.edges_bu += (uint32_t)lv.edges;
             }
-            if (tr && d.L < kLevelTrace) {
-                const int64_t scan = c.edges_td + c.edges_bu - edges0;
-                if (c.lane == 0)
-                    atomicAdd(reinterpret_cast<unsigned long long*>(&gs->lv_edges[dir][d.L]),
-                              (unsigned long long)(td ? scan : (int64_t)(uint32_t)lv.edges));
+            if (tr && L < kLevelTrace && c.lane == 0) {
+                using ull = unsigned long long;
+                atomicAdd(reinterpret_cast<ull*>(&gs->lv_edges[dir][L]),
+                          (ull)(td ? c.edges_td - edges0 : (int64_t)(uint32_t)lv.edges));
                 if (c.tid == 0) {  // wave 0 of each block
-                    if (!td)
-                        atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_cp[dir][d.L][0]),
-                                  (unsigned long long)(uint32_t)lv.edges);
-                    const unsigned long long wt = (unsigned long long)((int64_t)wall_clock64() - tl0);
-                    atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_wmax[dir][d.L]), wt);
-                    atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_wmin[dir][d.L]), ~wt);
+                    const ull wt = (ull)((int64_t)wall_clock64() - tl0);
+                    if (!td) atomicMax(reinterpret_cast<ull*>(&gs->lv_cp[dir][L][0]), (ull)(uint32_t)lv.edges);
+                    atomicMax(reinterpret_cast<ull*>(&gs->lv_wmax[dir][L]), wt);
+                    atomicMax(reinterpret_cast<ull*>(&gs->lv_wmin[dir][L]), ~wt);
                     if (!td && dir == 0 && c.b < 1024 && gs->bu1_scan[c.b] == 0) {
                         gs->bu1_scan[c.b] = (uint32_t)lv.edges + 1;
                         gs->bu1_work[c.b] = (int64_t)wt;
@@ -1254,64 +1252,81 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
             // counters of level L+2: last read at the start of level L-1,
             // first written in level L+1 (reset here, before the barrier)
             if (c.b == 0 && c.tid == 0) {
-                __hip_atomic_store(&gs->qn[dir][(d.L + 2) % 3].v, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&gs->hn[dir][(d.L + 2) % 3].v, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                st_agent(&gs->qn[dir][(L + 2) % 3].v, 0);
+                st_agent(&gs->hn[dir][(L + 2) % 3].v, 0);
             }
-        };
-        if (f.live) wave_counts(f, lf, tdf, 0);
-        if (b.live) wave_counts(b, lb, tdb, 1);
+            if (dir) {
+                pay[4] = (uint32_t)lv.found;
+                pay[5] = (uint32_t)lv.edges;
+                pay[6] = lv.nq;
+                pay[7] = lv.nh;
+            } else {
+                pay[0] = (uint32_t)lv.found;
+                pay[1] = (uint32_t)lv.edges;
+                pay[2] = lv.nq;
+                pay[3] = lv.nh;
+            }
+        }
         // Top-down levels read what other blocks wrote in the level before
         // through coherent loads (queue entries, hub items, counts), a
         // candidate bitmap that is fixed during the traversal, and visited
         // bits only as a hint for the claim atomics: their barriers skip the
         // L2 invalidation (the acquire below catches up where needed).
-        int64_t r[8];
-        if (!gsync_sum<8, false>(c,
-                                 {(uint32_t)lf.found, (uint32_t)lf.edges, lf.nq, lf.nh, (uint32_t)lb.found,
-                                  (uint32_t)lb.edges, lb.nq, lb.nh},
-                                 r))
-            return false;
-        // per direction: the level's totals, the end test and the switches
-        bool acquire = false, failed = false;
-        auto decide = [&](Dir& d, int64_t found, int64_t next_edges, int64_t nq, int64_t nh, bool td, int dir) {
-            // next_edges: top-down levels, the exact work of the next level
-            d.nq = nq;
-            d.nh = nh;
-            if (c.b == 0 && c.tid == 0 && d.L < kLevelTrace) {
-                gs->lv_ts[dir][d.L] = wall_clock64();
-                gs->lv_found[dir][d.L] = found;
-                gs->lv_mode[dir][d.L] = td ? 0 : 1;
+        stage_words<8>(c, pay);
+        SumFold<8> fold;
+        if (!gsync_with<8, false>(c, [&c]() { return staged_sum(c.sm, c.lane); }, fold)) return false;
+        if (c.wave == 0) {
+            // per direction: the level's totals, the end test and the switches
+            bool acquire = false;
+            int next = 0;
+#pragma unroll 1
+            for (int dir = 0; dir < 2; ++dir) {
+                if (!(flow & (kLive << dir))) continue;
+                auto total = [&](int w) {
+                    return lane_get(sm.tot[0][4 * dir + w], 0) + lane_get(sm.tot[1][4 * dir + w], 0);
+                };
+                const int64_t found = total(0);
+                const int64_t next_edges = total(1);  // top-down levels: exact work of the next level
+                const int32_t nq = (int32_t)total(2), nh = (int32_t)total(3);
+                int mode = lane_get(sm.dir[dir].mode, 0);
+                const int32_t L = lane_get(sm.dir[dir].L, 0) + 1;  // levels done now
+                const int64_t visited = lane_get(sm.dir[dir].visited, 0) + found;
+                const bool td = mode != 1;
+                if (c.b == 0 && c.lane == 0 && L <= kLevelTrace) {
+                    gs->lv_ts[dir][L - 1] = wall_clock64();
+                    gs->lv_found[dir][L - 1] = found;
+                    gs->lv_mode[dir][L - 1] = td ? 0 : 1;
+                }
+                int bits = 0;
+                if (found == 0 ||
+                    (td && a.td_local > 0 && nq == 0 && nh == 0)) {  // the waves expanded everything they found
+                    acquire = true;  // what follows reads the visited bits exactly
+                    if (dir == 0 && c.b == 0 && c.lane == 0) gs->ts[2] = wall_clock64();  // the forward one's end
+                } else if ((int64_t)L > (int64_t)a.V + 2) {
+                    if (c.lane == 0) atomicOr(&gs->err.v, 2);
+                    bits = kFailed;
+                } else {
+                    bits = kLive << dir;
+                    if (mode == 0) {
+                        const double ef = a.switch_rule ? (double)next_edges : (double)found * a.avg_degree;
+                        const double er = (double)(set_size - visited) * a.avg_degree;
+                        if (er / a.alpha < ef) mode = 1;
+                    }
+                    // bottom-up levels and the gather read visited bits exactly
+                    if (!td || mode == 1) acquire = true;
+                    if (!td && ((set_size * 1.0 / a.beta) > found || L - 1 > a.gamma)) {  // this level was bottom-up
+                        mode = 2;
+                        bits |= kGather << dir;
+                    }
+                }
+                next |= bits;
+                if (c.lane == 0) sm.dir[dir] = Dir{mode, L, (int32_t)visited, nq, nh};
             }
-            d.visited += found;
-            ++d.L;
-            if (found == 0 ||
-                (td && a.td_local > 0 && nq == 0 && nh == 0)) {  // the waves expanded everything they found
-                d.live = false;
-                acquire = true;  // what follows reads the visited bits exactly
-                if (dir == 0 && c.b == 0 && c.tid == 0) gs->ts[2] = wall_clock64();  // the forward one's end
-                return;
-            }
-            if (d.L > (int64_t)a.V + 2) {
-                if (c.tid == 0) atomicOr(&gs->err.v, 2);
-                failed = true;
-                return;
-            }
-            if (d.mode == 0) {
-                const double ef = a.switch_rule ? (double)next_edges : (double)found * a.avg_degree;
-                const double er = (double)(set_size - d.visited) * a.avg_degree;
-                if (er / a.alpha < ef) d.mode = 1;
-            }
-            // bottom-up levels and the gather read visited bits exactly
-            if (!td || d.mode == 1) acquire = true;
-            if (!td && ((set_size * 1.0 / a.beta) > found || d.L - 1 > a.gamma)) {  // this level was bottom-up
-                d.mode = 2;
-                d.gather = true;
-            }
-        };
-        if (f.live) decide(f, r[0], r[1], r[2], r[3], tdf, 0);
-        if (b.live) decide(b, r[4], r[5], r[6], r[7], tdb, 1);
-        if (failed) return false;
-        if (acquire) block_acquire();
+            if (acquire) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // as a barrier with ACQ does
+            if (c.lane == 0) sm.flow = next;
+        }
+        __syncthreads();
+        if (lane_get(sm.flow, 0) & kFailed) return false;
     }
     return true;
 }
@@ -1715,20 +1730,17 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
     GiantState* gs = a.gs;
     // Block 0 clears the state and the control block.  No other block writes
     // either before the first barrier (whose records are not part of them),
-    // so none has to wait for it.
+    // so none has to wait for it, and the barrier waits for the stores.
     if (c.b == 0) {
         int64_t* p = reinterpret_cast<int64_t*>(gs);
         for (int i = c.tid; i < a.state_words; i += kGBlock) st_agent(&p[i], (int64_t)0);
         int64_t* q = reinterpret_cast<int64_t*>(a.ctl);
         for (int i = c.tid; i < a.ctl_words; i += kGBlock) st_agent(&q[i], (int64_t)0);
-        wait_vm();
-        __syncthreads();
     }
     const int64_t total_waves = (int64_t)c.G * kW;
     const int64_t gwave = (int64_t)c.b * kW + c.wave;
     const bool stamp = c.b == 0 && c.tid == 0;  // phase timestamps (constant-rate clock)
-    if (stamp) gs->ts[0] = wall_clock64();
-    const unsigned long long t_begin = a.trace ? wall_clock64() : 0;  // launch ramp: when each block started
+    const unsigned long long t_begin = wall_clock64();  // launch ramp: when each block started
 
     // ---- phase A: trim-1-first (raw degree 0 either way), act bitmap,
     // cleared traversal bitmaps, pivot = largest out*in (lowest id on ties).
@@ -1850,7 +1862,10 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
         atomicMax(reinterpret_cast<ull*>(&gs->t_arrive[1]), t_arrive);
     }
     const int32_t root = (a.n_roots == 0 && bestp > 0 && besti < a.V) ? besti : -1;
-    if (stamp) gs->ts[1] = wall_clock64();
+    if (stamp) {
+        gs->ts[0] = (int64_t)t_begin;
+        gs->ts[1] = wall_clock64();
+    }
 
     int64_t fw_count = 0, bw_reach = 0, fw_levels = 0, bw_levels = 0;
     int32_t gmin = root;
@@ -1858,12 +1873,11 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
     const bool traversed = multi || root >= 0;
     if (traversed) {
         int64_t seeded = 0;
-        Dir f, b;
-        if (!traverse_joint(c, root, fq0, f, b, &seeded)) return;
-        fw_count = f.visited + seeded;
-        bw_reach = b.visited + seeded;
-        fw_levels = f.L;
-        bw_levels = b.L;
+        if (!traverse_joint(c, root, fq0, &seeded)) return;
+        fw_count = sm.dir[0].visited + seeded;
+        bw_reach = sm.dir[1].visited + seeded;
+        fw_levels = sm.dir[0].L;
+        bw_levels = sm.dir[1].L;
     }
     if (stamp) {
         if (!traversed) gs->ts[2] = wall_clock64();
