@@ -1236,9 +1236,9 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
             }
             if (tr && L < kLevelTrace && c.lane == 0) {
                 using ull = unsigned long long;
-                atomicAdd(reinterpret_cast<ull*>(&gs->lv_edges[dir][L]),
-                          (ull)(td ? c.edges_td - edges0 : (int64_t)(uint32_t)lv.edges));
                 if (c.tid == 0) {  // wave 0 of each block
+                    if (c.edges_td > edges0)
+                        atomicAdd(reinterpret_cast<ull*>(&gs->lv_edges[dir][L]), (ull)(c.edges_td - edges0));
                     const ull wt = (ull)((int64_t)wall_clock64() - tl0);
                     if (!td) atomicMax(reinterpret_cast<ull*>(&gs->lv_cp[dir][L][0]), (ull)(uint32_t)lv.edges);
                     atomicMax(reinterpret_cast<ull*>(&gs->lv_wmax[dir][L]), wt);
@@ -1296,6 +1296,7 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
                     gs->lv_ts[dir][L - 1] = wall_clock64();
                     gs->lv_found[dir][L - 1] = found;
                     gs->lv_mode[dir][L - 1] = td ? 0 : 1;
+                    if (!td) gs->lv_edges[dir][L - 1] = next_edges;
                 }
                 int bits = 0;
                 if (found == 0 ||
