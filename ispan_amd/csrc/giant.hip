@@ -35,7 +35,8 @@ struct Dir {
     int32_t nq, nh;   // next level's queue entries and hub work items
 };
 // What the traversal goes on with (Smem::flow): which directions are still
-// traversing; which had a bottom-up level last and have a top-down one next.
+// traversing; which had a bottom-up level last and have a top-down one next,
+// which starts from the bitmaps instead of a queue.
 constexpr int kLive = 1, kGather = 4, kFailed = 16;  // of direction d: kLive << d, kGather << d
 
 struct Smem {
@@ -742,7 +743,7 @@ struct Level {
 // the forward set when v does), and the two directions then need not wait
 // for each other.
 __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t nq, int32_t nh_in, int dir, int32_t root,
-                                           int narrow_steps, bool half, Level& lv) {
+                                           int narrow_steps, bool half, bool gather, Level& lv) {
     const GiantArgs& a = c.a;
     Smem& sm = c.sm;
     const bool bw = dir != 0;
@@ -778,7 +779,31 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
     const bool topdown = mode != 1;
     const bool tr = a.trace && L < kLevelTrace;
     const int64_t tl0 = tr ? (int64_t)wall_clock64() : 0;
-    if (topdown) {
+    if (topdown && gather) {
+        // ---- the first top-down level after bottom-up ones: each wave takes
+        // the last level's finds (vis & ~snap) of its words, 64 words at a
+        // time, and goes on from them in place.  No queue and no barrier lie
+        // between the finds and their expansion (a gather pass that queued
+        // them for a level of their own: 29 us for both at R-MAT s24).
+        for (int64_t wb = gwave * kWave; wb < a.nwords; wb += total_waves * kWave) {
+            const int64_t w = wb + c.lane;
+            uint64_t nw = 0;
+            if (w < a.nwords) nw = vis[w] & ~snap[w];
+            uint64_t busy = __ballot(nw != 0);
+            while (busy) {
+                const int l = __ffsll((unsigned long long)busy) - 1;
+                busy &= busy - 1;
+                const uint64_t m = lane_get(nw, l);
+                const int32_t v = (int32_t)((wb + l) * 64 + c.lane);
+                push_next((m >> c.lane) & 1ull, v, beg, pq, qout, qn_out, hs, hout, hn_out, fedges);
+            }
+        }
+        if (a.td_local > 0)
+            expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found, a.td_local,
+                         false);
+        block_flush_both(c, pq, qout, qn_out, hs, hout, hn_out);
+        lv = Level{(int)my_found, (int)fedges, pq.sent, hs.sent};
+    } else if (topdown) {
         // ---- top-down: tiles of the queue, then hub work items; level 0
         // expands the root's list in kGiantChunk-edge pieces.
         int64_t n = 0, nh = 0;
@@ -1084,44 +1109,6 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
     }
 }
 
-// The gather of a direction that switches from bottom-up back to top-down:
-// the last level's finds (vis & ~snap) become the next level's queue and hub
-// items.  Each wave loads 64 words at once, then expands the non-empty ones.
-__device__ __forceinline__ void gather_finds(Ctx& c, int32_t L, int dir, uint32_t& nq, uint32_t& nh) {
-    const GiantArgs& a = c.a;
-    Smem& sm = c.sm;
-    GiantState* gs = a.gs;
-    const bool bw = dir != 0;
-    const int32_t* beg = bw ? a.bwb : a.fwb;
-    const uint64_t* vis = bw ? a.bvis : a.fvis;
-    const uint64_t* snap = bw ? a.snapb : a.snap;
-    uint64_t* q_next = (L & 1) ? (bw ? a.qb1 : a.q1) : (bw ? a.qb0 : a.q0);
-    HubItem* h_next = (L & 1) ? (bw ? a.hb1 : a.h1) : (bw ? a.hb0 : a.h0);
-    int32_t* qn_next = &gs->qn[dir][L % 3].v;
-    int32_t* hn_next = &gs->hn[dir][L % 3].v;
-    PairQueue wq{c.stage(), 0};
-    HubStage hs{sm.hv[c.wave], sm.hs[c.wave], sm.hd[c.wave], 0};
-    const int64_t total_waves = (int64_t)c.G * kW;
-    const int64_t gwave = (int64_t)c.b * kW + c.wave;
-    int64_t unused = 0;
-    for (int64_t wb = gwave * kWave; wb < a.nwords; wb += total_waves * kWave) {
-        const int64_t w = wb + c.lane;
-        uint64_t nw = 0;
-        if (w < a.nwords) nw = vis[w] & ~snap[w];
-        uint64_t busy = __ballot(nw != 0);
-        while (busy) {
-            const int l = __ffsll((unsigned long long)busy) - 1;
-            busy &= busy - 1;
-            const uint64_t m = lane_get(nw, l);
-            const int32_t v = (int32_t)((wb + l) * 64 + c.lane);
-            push_next((m >> c.lane) & 1ull, v, beg, wq, q_next, qn_next, hs, h_next, hn_next, unused);
-        }
-    }
-    block_flush_both(c, wq, q_next, qn_next, hs, h_next, hn_next);
-    nq = wq.sent;
-    nh = hs.sent;
-}
-
 // The giant's traversals: forward and backward in the same levels, one grid
 // barrier per level for both (fw_bfs_fq_queue, src/fw_bw.h:396-698, and
 // bw_bfs_fq_queue, :944-1248, which the reference runs one after the
@@ -1184,34 +1171,6 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
     while (true) {
         const int flow = lane_get(sm.flow, 0);
         if (!(flow & (kLive | kLive << 1))) break;
-        if (flow & (kGather | kGather << 1)) {
-            // the visited bits were made exact after the level's barrier
-            uint32_t cnt[4] = {0, 0, 0, 0};
-#pragma unroll 1
-            for (int dir = 0; dir < 2; ++dir) {
-                uint32_t nq = 0, nh = 0;
-                if (flow & (kGather << dir)) gather_finds(c, lane_get(sm.dir[dir].L, 0), dir, nq, nh);
-                if (dir) {
-                    cnt[2] = nq;
-                    cnt[3] = nh;
-                } else {
-                    cnt[0] = nq;
-                    cnt[1] = nh;
-                }
-            }
-            // the top-down level reads the queues coherently and visited bits
-            // only as hints: no L2 invalidation
-            int64_t r[4];
-            if (!gsync_sum<4, false>(c, cnt, r)) return false;
-            if (c.tid == 0) {
-                for (int dir = 0; dir < 2; ++dir)
-                    if (flow & (kGather << dir)) {
-                        sm.dir[dir].nq = (int32_t)(dir ? r[2] : r[0]);
-                        sm.dir[dir].nh = (int32_t)(dir ? r[3] : r[1]);
-                    }
-            }
-            __syncthreads();
-        }
         const bool tr = a.trace != 0;
         const int64_t tl0 = tr ? (int64_t)wall_clock64() : 0;
         // One copy of the level's code serves both directions: the
@@ -1233,7 +1192,7 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
             const int64_t edges0 = c.edges_td;
             Level lv{0, 0, 0, 0};
             level_work(c, mode, L, lane_get(sm.dir[dir].nq, 0), lane_get(sm.dir[dir].nh, 0), dir, root,
-                       both ? kNarrowShort : kNarrowLong, half, lv);
+                       both ? kNarrowShort : kNarrowLong, half, (flow & (kGather << dir)) != 0, lv);
             lv.found = wave_sum(lv.found);
             lv.edges = wave_sum(lv.edges);
             // this wave's part of the work counters
@@ -1310,8 +1269,10 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
                     if (!td) gs->lv_edges[dir][L - 1] = next_edges;
                 }
                 int bits = 0;
-                if (found == 0 ||
-                    (td && a.td_local > 0 && nq == 0 && nh == 0)) {  // the waves expanded everything they found
+                // a top-down level ends the traversal when it hands nothing on
+                // (it may have found something and expanded it in place, or
+                // only handed on what it gathered)
+                if (td ? nq == 0 && nh == 0 && (found == 0 || a.td_local > 0) : found == 0) {
                     acquire = true;  // what follows reads the visited bits exactly
                     if (dir == 0 && c.b == 0 && c.lane == 0) gs->ts[2] = wall_clock64();  // the forward one's end
                 } else if ((int64_t)L > (int64_t)a.V + 2) {
