@@ -68,8 +68,20 @@ static_assert(kWaveBuf * 4 <= kPairCap * 8, "the id view fits the staging");
 static_assert((kPairCap & (kPairCap - 1)) == 0, "the in-place ring indexes with a mask");
 extern __shared__ uint64_t stage_lds[];
 
+// The launch's arguments, read from the kernel argument segment.  args()
+// hides where the address comes from, so that what a phase reads of them is
+// loaded in that phase: read once at the start they take more scalar
+// registers than there are, and every use of a spilled one is a move from a
+// vector register's lane.
+typedef const GiantArgs __attribute__((address_space(4))) KernelArgs;
+__device__ __forceinline__ KernelArgs& kernel_args() {
+    KernelArgs* p = (KernelArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *p;
+}
+
 struct Ctx {
-    const GiantArgs& a;
+    __device__ KernelArgs& args() const { return kernel_args(); }
     int G, b, tid, lane, wave;
     Smem& sm;
     uint32_t nbar;  // barriers this launch has passed (the same in every block)
@@ -141,15 +153,16 @@ __device__ __forceinline__ bool gsync_with(Ctx& c, Src src, Fold& fold) {
     wait_vm();  // this wave's writes for other blocks have completed
     __syncthreads();
     if (c.wave < kReaders) {
-        const uint32_t tag = c.a.bar_base + nb;
-        uint64_t* rec = c.a.bar + (int64_t)(tag & 1) * c.G * kBarWords;
+        KernelArgs& a = c.args();
+        const uint32_t tag = a.bar_base + nb;
+        uint64_t* rec = a.bar + (int64_t)(tag & 1) * c.G * kBarWords;
         if (c.wave == 0) {
             const uint32_t mine = src();  // by every lane
             if (c.lane < NW) st_agent(&rec[c.b * NW + c.lane], ((uint64_t)tag << 32) | mine);
         }
         if (c.tid == 0) {  // diagnostics: barriers arrived at, and passed
-            c.a.dbg[c.b] = (int32_t)nb;
-            c.a.dbg[c.G + c.b] = (int32_t)nb - 1;
+            a.dbg[c.b] = (int32_t)nb;
+            a.dbg[c.G + c.b] = (int32_t)nb - 1;
         }
         constexpr int K = 16;  // loads a lane has in flight
         const int words = c.G * NW;
@@ -173,7 +186,7 @@ __device__ __forceinline__ bool gsync_with(Ctx& c, Src src, Fold& fold) {
                 if (!__ballot(todo != 0)) break;
                 __builtin_amdgcn_s_sleep(1);
                 if (++spins > kSpinCap) {
-                    if (c.lane == 0) atomicOr(&c.a.gs->err.v, 1);
+                    if (c.lane == 0) atomicOr(&a.gs->err.v, 1);
                     ok = 0;
                     break;
                 }
@@ -744,7 +757,7 @@ struct Level {
 // for each other.
 __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t nq, int32_t nh_in, int dir, int32_t root,
                                            int narrow_steps, bool half, bool gather, Level& lv) {
-    const GiantArgs& a = c.a;
+    KernelArgs& a = c.args();
     Smem& sm = c.sm;
     const bool bw = dir != 0;
     const int32_t* beg = bw ? a.bwb : a.fwb;  // expansion (top-down) direction
@@ -1123,7 +1136,7 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
 // block's 16 waves share four SIMDs, so a few hundred instructions that all of
 // them execute take four times as long (2.8 us a level against 1.0).
 __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set_size, int64_t* seeded_out) {
-    const GiantArgs& a = c.a;
+    KernelArgs& a = c.args();
     Smem& sm = c.sm;
     GiantState* gs = a.gs;
     if (c.tid == 0) {
@@ -1313,7 +1326,7 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
 // itself, so no barrier has to make other blocks' entries visible first.
 __device__ __forceinline__ void trim_sweep(Ctx& c, const int32_t* fin, int64_t n, int32_t* fout, int32_t* fcount,
                                            int64_t lo, int& trimmed, int& kept) {
-    const GiantArgs& a = c.a;
+    KernelArgs& a = c.args();
     WaveQueue wq{c.stage32(), 0};
     const uint64_t* act = a.act;
     auto live = [act](int32_t w, int32_t self) { return w != self && bit_of(act, w); };
@@ -1356,7 +1369,7 @@ __device__ __forceinline__ void trim_sweep(Ctx& c, const int32_t* fin, int64_t n
 // the largest id).  The count of changed vertices rides on the barrier, so
 // every block leaves after the same sweep.
 __device__ __forceinline__ bool lp_wcc(Ctx& c, const int32_t* q, int64_t n, int64_t& rounds) {
-    const GiantArgs& a = c.a;
+    KernelArgs& a = c.args();
     const int64_t nthreads = (int64_t)c.G * kGBlock;
     const int64_t gt = (int64_t)c.b * kGBlock + c.tid;
     int32_t* col = a.parent;
@@ -1415,7 +1428,7 @@ __device__ __forceinline__ int32_t key_colour(uint64_t k) { return (int32_t)(uin
 // round with their own keys again (color_init, :262-290).  Each round labels
 // at least the SCC of the largest key of every weakly connected piece.
 __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, int64_t& rounds, int64_t& sccs) {
-    const GiantArgs& a = c.a;
+    KernelArgs& a = c.args();
     GiantState* gs = a.gs;
     const int64_t nthreads = (int64_t)c.G * kGBlock;
     const int64_t gt = (int64_t)c.b * kGBlock + c.tid;
@@ -1552,7 +1565,7 @@ constexpr int kPatternLong = 32;
 // taken when no sweep comes first).
 __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64_t own_lo, int64_t own_n,
                                            int64_t& n_left) {
-    const GiantArgs& a = c.a;
+    KernelArgs& a = c.args();
     GiantState* gs = a.gs;
     int cur = 1, s = 0;
     auto buf = [&a](int k) { return k ? a.fq : a.fq_alt; };
@@ -1727,9 +1740,10 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
 
 }  // namespace
 
-__global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
+__global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs) {
+    KernelArgs& a = kernel_args();
     __shared__ Smem sm;
-    Ctx c{a, (int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, lane_id(), wave_id(), sm, 0, 0, 0, 0, 0};
+    Ctx c{(int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, lane_id(), wave_id(), sm, 0, 0, 0, 0, 0};
     GiantState* gs = a.gs;
     // Block 0 clears the state and the control block.  No other block writes
     // either before the first barrier (whose records are not part of them),
@@ -2051,14 +2065,15 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs a) {
     if (stamp) gs->bar_next = a.bar_base + c.nbar;
 }
 
-__global__ __launch_bounds__(kGBlock) void k_tail(const GiantArgs a) {
+__global__ __launch_bounds__(kGBlock) void k_tail(const GiantArgs) {
+    KernelArgs& a = kernel_args();
     __shared__ Smem sm;
     GiantState* gs = a.gs;
     if (gs->err.v != 0) return;  // k_giant failed; the host reports its error
     const int64_t n = gs->n_final;
     int cur = (int)gs->final_sel;
     if (n == 0) return;
-    Ctx c{a, (int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, lane_id(), wave_id(), sm, 0, 0, 0, 0, 0};
+    Ctx c{(int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, lane_id(), wave_id(), sm, 0, 0, 0, 0, 0};
     const bool lead = c.b == 0 && c.tid == 0;
     int64_t rounds = 0, sccs = 0;
     if (a.wcc_mode == 1) {  // P12 by label propagation: parent = smallest id of the WCC
