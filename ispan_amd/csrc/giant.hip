@@ -620,7 +620,7 @@ __device__ __forceinline__ void push_found_n(const bool (&claim)[K], const int32
 // has at most kNarrowBlock edges, and its first wave alone, with no block
 // barriers either, while it has at most kNarrowWave.  A level of a few edges
 // costs 11 us across the grid, nearly all of it barrier and round trips that
-// do no work, and about 4 us in a block and 2 us in a wave.  More edges than
+// do no work, and about 4 us in a block and under 1 us in a wave.  More edges than
 // a couple of steps of one block go back to the grid, which also bounds how
 // long one block expands a growing region alone.
 constexpr int kNarrowWave = 256;
@@ -628,6 +628,24 @@ constexpr int kNarrowBlock = 2048;
 // Such levels in a row, while the other direction waits at the barrier and
 // when it has finished.
 constexpr int kNarrowShort = 16, kNarrowLong = 4096;
+
+// The adj index of this lane's edge, less the edge's number eb + lane, for
+// edges eb to eb + kWave - 1 of up to kWave entries, one a lane, that begin at
+// edge `off` (ascending) and at adj index `st`; a lane past the last edge gets
+// some value.  The source of edge e is the last entry j with off_j <= e.
+// Every entry has an edge, so that is the number of entries that begin at or
+// before e, less one: those before the chunk, and those whose bit is set up to
+// e's in the chunk's word of beginnings (an OR over the wave by DPP).  A
+// binary search of the offsets in LDS is six dependent reads.
+__device__ __forceinline__ int32_t edge_entry(bool valid, int off, int32_t st, int eb) {
+    const int rel = off - eb;
+    const int before = __popcll(__ballot(valid && rel < 0));
+    uint64_t begins = row_incl((uint64_t)(valid && rel >= 0 && rel < kWave ? 1ull << rel : 0ull), (uint64_t)0,
+                               [](uint64_t x, uint64_t y) { return x | y; });
+    begins = lane_get(begins, 15) | lane_get(begins, 31) | lane_get(begins, 47) | lane_get(begins, 63);
+    const int pos = before + __popcll(begins & (lanemask_lt() | (1ull << lane_id()))) - 1;
+    return __shfl(st - off, pos, kWave);
+}
 
 // Top-down to exhaustion (mode 2) without level barriers in the thin parts:
 // a wave expands the vertices it claimed itself, in the same level, instead
@@ -642,22 +660,15 @@ constexpr int kNarrowShort = 16, kNarrowLong = 4096;
 // Claims stay exact (the same wave-combined atomics), so the reach set and
 // the found counts are those of a level-synchronous traversal; only the
 // level at which a vertex is expanded changes.  All lanes call it.
-//
-// narrow: goes on only while a step takes everything that is pending (at most
-// kWave entries of at most kNarrowWave edges together) and no hub turned up;
-// what is left then stays staged in wq, for the block to go on with.
-// Returns the steps that are left of max_steps.
-__device__ __forceinline__ int expand_local(Ctx& c, PairQueue& wq, int32_t root, const int32_t* __restrict__ beg,
+__device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root, const int32_t* __restrict__ beg,
                                              const int32_t* __restrict__ adj, const uint64_t* __restrict__ allow,
                                              uint64_t* vis, uint64_t* qout, int32_t* qn_out, HubStage& hs,
-                                             HubItem* hout, int32_t* hn_out, int64_t& my_found, int max_steps,
-                                             bool narrow) {
+                                             HubItem* hout, int32_t* hn_out, int64_t& my_found, int max_steps) {
     uint64_t* buf = wq.buf;
     constexpr int mask = kPairCap - 1;
     int head = 0, n = wq.n;  // pending: buf[head .. n) modulo kPairCap
     wave_sync();
     for (; n > head && max_steps > 0; --max_steps) {
-        if (narrow && (n > kWave || hs.n > 0)) break;
         const int k = min(kWave, n - head);
         int32_t st = 0, dg = 0;
         if (c.lane < k) {
@@ -667,30 +678,12 @@ __device__ __forceinline__ int expand_local(Ctx& c, PairQueue& wq, int32_t root,
         }
         const int incl = wave_incl_scan(dg);
         const int total = lane_get(incl, kWave - 1);
-        if (narrow) {
-            if (total > kNarrowWave) break;
-            head = n = 0;  // all of them are in registers
-        } else {
-            head += k;
-        }
+        head += k;
         const int off = incl - dg;  // this entry's first edge of the step
         wave_sync();  // the queue entries are read: their places may be written
         for (int eb = 0; eb < total; eb += kWave) {
-            // The source of edge e is the last entry j with off_j <= e.  Every
-            // entry has an edge, so that is the number of entries that begin
-            // at or before e, less one: those before the chunk, and those whose
-            // bit is set up to e's in the chunk's word of beginnings (an OR
-            // over the wave by DPP).  A binary search of the offsets in LDS is
-            // six dependent reads.
-            const int rel = off - eb;
-            const bool valid = c.lane < k;
-            const int before = __popcll(__ballot(valid && rel < 0));
-            uint64_t begins = row_incl((uint64_t)(valid && rel >= 0 && rel < kWave ? 1ull << rel : 0ull), (uint64_t)0,
-                                       [](uint64_t x, uint64_t y) { return x | y; });
-            begins = lane_get(begins, 15) | lane_get(begins, 31) | lane_get(begins, 47) | lane_get(begins, 63);
             const int e = eb + c.lane;
-            const int pos = before + __popcll(begins & (lanemask_lt() | (1ull << c.lane))) - 1;
-            const int32_t src = __shfl(st - off, pos, kWave);  // adj index of the entry's edge 0, less its offset
+            const int32_t src = edge_entry(c.lane < k, off, st, eb);
             bool want[1];
             int32_t w[1];
             w[0] = e < total ? adj[src + e] : 0;
@@ -716,10 +709,6 @@ __device__ __forceinline__ int expand_local(Ctx& c, PairQueue& wq, int32_t root,
         }
         wave_sync();  // the entries pushed are read next step
     }
-    if (narrow) {
-        wq.n = n;
-        return max_steps;
-    }
     const int left = n - head;  // the step budget ran out: the next level takes them
     if (left > 0) {
         int base = 0;
@@ -730,6 +719,156 @@ __device__ __forceinline__ int expand_local(Ctx& c, PairQueue& wq, int32_t root,
     }
     wq.n = 0;
     wave_sync();
+}
+
+// The frontier of a narrow region in one wave: expand_local for at most kWave
+// entries of at most kNarrowWave edges together at a time, and only while
+// that is everything that is pending and no hub turned up; what is left then
+// stays staged in wq, for the block to go on with.  Returns the steps that
+// are left of max_steps.
+//
+// Such a step is one serial chain of round trips and dependent instructions,
+// so it is cut to what a step cannot do without.  Nobody else claims in this
+// direction meanwhile (the frontier is all in this wave, the other blocks
+// wait at the grid's barrier), so the claims are made in LDS, on copies of the
+// visited words: kSets of them, by word number modulo kSets, each beside what
+// it was in memory, which gets the new bits when another word takes the place
+// and at the end.  That leaves two round trips a step, the list and the
+// offsets of what it names, mostly cache hits, where there are four with the
+// visited bits read and then claimed in memory.  While a step's edges fit the
+// wave, the entries stay in the registers of the lanes that claimed them, and
+// no lane branches except where a word is missing or a hub turns up.  A
+// chain of 10^4 levels of about two vertices: 1.6 us a level in expand_local,
+// 0.94 with the copies, 0.74 with both.  The copies lie in the other waves'
+// staging, which is empty while they wait at the block's barrier.
+__device__ __forceinline__ int expand_wave(Ctx& c, PairQueue& wq, int32_t root, const int32_t* __restrict__ beg,
+                                           const int32_t* __restrict__ adj, const uint64_t* __restrict__ allow,
+                                           uint64_t* vis, HubStage& hs, HubItem* hout, int32_t* hn_out,
+                                           int64_t& my_found, int max_steps) {
+    constexpr int kSets = 256, kStep = kWave - 1;
+    static_assert(2 * kSets <= kPairCap && kSets % kWave == 0 && kW >= 3, "the copies fit two waves' staging");
+    static_assert(kNarrowWave <= kPairCap, "a step's claims fit the staging");
+    uint64_t* buf = wq.buf;
+    unsigned long long* seen = reinterpret_cast<unsigned long long*>(buf + kPairCap);  // visited, or not to be visited
+    unsigned long long* had = seen + kSets;                                            // the same as it is in memory
+    int32_t* word = reinterpret_cast<int32_t*>(buf + 2 * kPairCap);                    // the word's number
+    unsigned long long* mem = reinterpret_cast<unsigned long long*>(vis);
+    if (wq.n > kWave || hs.n > 0) return max_steps;
+    for (int i = c.lane; i < kSets; i += kWave) {
+        word[i] = -1;
+        seen[i] = 0;
+        had[i] = 0;
+    }
+    int32_t st = 0, dg = 0;  // an entry a lane, in any lane; dg = 0 is none
+    if (c.lane < wq.n) {
+        const uint64_t q = buf[c.lane];
+        st = qentry_start(q);
+        dg = qentry_degree(q);
+    }
+    wave_sync();
+    int staged = 0;  // entries in buf, when they are too many for the lanes
+    for (; max_steps > 0; --max_steps) {
+        const int incl = wave_incl_scan(dg);
+        const int total = lane_get(incl, kWave - 1);
+        if (total == 0 || total > kNarrowWave) break;
+        const int off = incl - dg;
+        int n = 0;
+        for (int eb = 0; eb < total; eb += kStep) {
+            // Edges eb to eb + kStep - 1, one a lane.  An entry sends where
+            // its list lies, less its offset, to the lane of its first edge;
+            // an edge's entry is then at the last such lane up to its own,
+            // or began before the chunk.  (The last lane has no edge: what is
+            // not to be sent goes there.  kBias keeps a sent value from 0.)
+            constexpr int kBias = kNarrowWave + 1;
+            const int rel = off - eb;
+            const bool starts = dg > 0 && rel >= 0 && rel < kStep;
+            const int got = __builtin_amdgcn_ds_permute((starts ? rel : kStep) * 4, st - off + kBias);
+            const uint64_t at = __ballot(got != 0 && c.lane < kStep) & ((2ull << c.lane) - 1);
+            int32_t src = __shfl(got, 63 - __clzll((long long)(at | 1)), kWave) - kBias;
+            if (eb) {
+                const uint64_t before = __ballot(dg > 0 && rel < 0);
+                const int32_t cur = lane_get(st - off, 63 - __clzll((long long)before));
+                src = at ? src : cur;
+            }
+            const int e = eb + c.lane;
+            const bool edge = c.lane < kStep && e < total;
+            const int32_t w = adj[edge ? src + e : lane_get(src, 0) + eb];
+            const int32_t s0 = beg[w], d = beg[w + 1] - s0;
+            const bool cand = edge && w != root;
+            const int32_t wd = w >> 6;
+            const int set = wd & (kSets - 1);
+            const unsigned long long bit = 1ull << (w & 63);
+            bool here = word[set] == wd;
+            unsigned long long old = ~0ull;
+            if (__ballot(cand && !here)) {
+                wait_vm();  // what earlier words left is in memory
+                const bool miss = cand && !here;
+                unsigned long long now = 0, left = 0;
+                int32_t from = 0;
+                if (miss) {
+                    now = load_agent(&vis[wd]) | ~allow[wd];
+                    from = word[set];
+                    left = seen[set] & ~had[set];
+                }
+                wave_sync();
+                if (miss) word[set] = wd;
+                wave_sync();
+                if (miss && word[set] == wd) {  // of several words for one place, one has it
+                    if (left) atomicOr(mem + from, left);
+                    seen[set] = now;
+                    had[set] = now;
+                }
+                wave_sync();
+                here = word[set] == wd;
+                if (__ballot(cand && !here)) {  // the others, and a word that was here until now, in memory
+                    wait_vm();
+                    if (cand && !here && (allow[wd] & bit)) old = atomicOr(mem + wd, bit);
+                    wait_vm();
+                }
+            }
+            const unsigned long long was = atomicOr(&seen[set], cand && here ? bit : 0ull);
+            old = here ? was : old;
+            const bool claim = cand && !(old & bit);
+            my_found += claim;
+            hub_push(hs, claim && d >= kGiantHubDeg, w, s0, d, hout, hn_out);
+            const bool keep = claim && d > 0 && d < kGiantHubDeg;
+            if (total <= kStep) {
+                st = s0;
+                dg = keep ? d : 0;
+            } else {
+                const uint64_t m = __ballot(keep);
+                if (keep) buf[n + __popcll(m & lanemask_lt())] = qentry(s0, d);
+                n += __popcll(m);
+            }
+        }
+        if (total > kStep) {
+            wave_sync();
+            uint64_t q = 0;
+            if (n > kWave)
+                staged = n;
+            else if (c.lane < n)
+                q = buf[c.lane];
+            st = qentry_start(q);
+            dg = qentry_degree(q);
+            wave_sync();
+        }
+        if (staged || hs.n > 0) {
+            --max_steps;
+            break;
+        }
+    }
+    if (staged == 0) {
+        const uint64_t m = __ballot(dg > 0);
+        if (dg > 0) buf[__popcll(m & lanemask_lt())] = qentry(st, dg);
+        staged = __popcll(m);
+    }
+    wave_sync();
+    for (int i = c.lane; i < kSets; i += kWave) {
+        const unsigned long long left = seen[i] & ~had[i];
+        if (left) atomicOr(mem + word[i], left);
+    }
+    wait_vm();  // the other waves claim from memory
+    wq.n = staged;
     return max_steps;
 }
 
@@ -812,8 +951,7 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
             }
         }
         if (a.td_local > 0)
-            expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found, a.td_local,
-                         false);
+            expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found, a.td_local);
         block_flush_both(c, pq, qout, qn_out, hs, hout, hn_out);
         lv = Level{(int)my_found, (int)fedges, pq.sent, hs.sent};
     } else if (topdown) {
@@ -905,8 +1043,8 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
                 // the only tile: take what it claimed as the next one
                 if (total <= kWave) {  // only the first wave had edges
                     if (c.wave == 0) {
-                        narrow_steps = expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out,
-                                                    my_found, narrow_steps, true);
+                        narrow_steps = expand_wave(c, pq, root, beg, adj, allow, vis, hs, hout, hn_out, my_found,
+                                                   narrow_steps);
                         fedges = c.lane < hs.n ? hs.d[c.lane] : 0;
                         for (int i = c.lane; i < pq.n; i += kWave) fedges += qentry_degree(pq.buf[i]);
                     }
@@ -948,7 +1086,7 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
         // expanded so took the 4096^2 grid from 5.09 to 5.8-6.5 ms.
         if (a.td_local > 0 && (mode == 2 || (L > 0 && nh == 0 && n >= kLocalPerWave * total_waves)))
             expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found,
-                             a.td_local, false);
+                         a.td_local);
         block_flush_both(c, pq, qout, qn_out, hs, hout, hn_out);
         lv = Level{(int)my_found, (int)fedges, pq.sent, hs.sent};
     } else {

@@ -48,3 +48,33 @@ def test_narrow_frontiers(widths, path, tail, flip):
             assert np.array_equal(s.labels(), want), local
             got[local] = (st.fw_size, st.bw_reach, st.giant_size, st.pivot)
         assert got[64] == got[0]
+
+
+@pytest.mark.parametrize("ids", ["one place", "two places", "any place"])
+@pytest.mark.parametrize("widths,path,tail", [([1, 2, 3], 60, 20), ([60, 20, 60], 30, 5), ([33] * 12, 4, 200)],
+                         ids=lambda x: str(x)[:20])
+def test_narrow_words_that_share_a_place(widths, path, tail, ids):
+    """One wave keeps copies of 256 visited words, by word number modulo 256:
+    vertices whose words want the same one or two places, each word with one
+    or two of the graph's vertices, and vertices anywhere among many words."""
+    g = bursts(widths, path, tail, 7)
+    n, V = g.V, 1 << 24
+    rng = np.random.default_rng(8)
+    if ids == "any place":
+        at = rng.choice(V, n, replace=False)
+    else:
+        k = 1 if ids == "one place" else 2
+        word = (np.arange(n) // 2) // k * 256 + (np.arange(n) // 2) % k
+        at = rng.permutation(word * 64 + np.arange(n) % 2 * 37)
+    V = int(at.max()) + 1
+    src = np.repeat(at, np.diff(g.fw_beg)).astype(np.int32)
+    g = O.build_csr(V, src, at[g.fw_adj].astype(np.int32))
+    want = O.tarjan(g)
+    with I.Solver(0) as s:
+        s.upload(I.HostGraph(g.fw_beg, g.fw_adj, g.bw_beg, g.bw_adj))
+        got = {}
+        for local in (64, 0):
+            st = s.solve(I.default_params(td_local=local))
+            assert np.array_equal(s.labels(), want), local
+            got[local] = (st.fw_size, st.bw_reach, st.giant_size, st.pivot)
+        assert got[64] == got[0]
