@@ -744,7 +744,7 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
 __device__ __forceinline__ int expand_wave(Ctx& c, PairQueue& wq, int32_t root, const int32_t* __restrict__ beg,
                                            const int32_t* __restrict__ adj, const uint64_t* __restrict__ allow,
                                            uint64_t* vis, HubStage& hs, HubItem* hout, int32_t* hn_out,
-                                           int64_t& my_found, int max_steps) {
+                                           int32_t nwords, int64_t& my_found, int max_steps) {
     constexpr int kSets = 256, kStep = kWave - 1;
     static_assert(2 * kSets <= kPairCap && kSets % kWave == 0 && kW >= 3, "the copies fit two waves' staging");
     static_assert(kNarrowWave <= kPairCap, "a step's claims fit the staging");
@@ -783,12 +783,12 @@ __device__ __forceinline__ int expand_wave(Ctx& c, PairQueue& wq, int32_t root, 
             const int rel = off - eb;
             const bool starts = dg > 0 && rel >= 0 && rel < kStep;
             const int got = __builtin_amdgcn_ds_permute((starts ? rel : kStep) * 4, st - off + kBias);
-            const uint64_t at = __ballot(got != 0 && c.lane < kStep) & ((2ull << c.lane) - 1);
-            int32_t src = __shfl(got, 63 - __clzll((long long)(at | 1)), kWave) - kBias;
+            const uint64_t heads = __ballot(got != 0 && c.lane < kStep) & ((2ull << c.lane) - 1);
+            int32_t src = __shfl(got, 63 - __clzll((long long)(heads | 1)), kWave) - kBias;
             if (eb) {
                 const uint64_t before = __ballot(dg > 0 && rel < 0);
                 const int32_t cur = lane_get(st - off, 63 - __clzll((long long)before));
-                src = at ? src : cur;
+                src = heads ? src : cur;
             }
             const int e = eb + c.lane;
             const bool edge = c.lane < kStep && e < total;
@@ -802,21 +802,29 @@ __device__ __forceinline__ int expand_wave(Ctx& c, PairQueue& wq, int32_t root, 
             unsigned long long old = ~0ull;
             if (__ballot(cand && !here)) {
                 wait_vm();  // what earlier words left is in memory
+                // the missing words, and in the other lanes the words around
+                // the first of them: vertices that follow each other along a
+                // path mostly have ids close together
+                const uint64_t missing = __ballot(cand && !here);
+                const int32_t near = lane_get(wd, __ffsll((unsigned long long)missing) - 1) + c.lane - kWave / 2;
                 const bool miss = cand && !here;
+                const int32_t take = miss ? wd : near;
+                const int at = take & (kSets - 1);
+                const bool fill = miss || (near >= 0 && near < nwords && word[at] != near);
                 unsigned long long now = 0, left = 0;
                 int32_t from = 0;
-                if (miss) {
-                    now = load_agent(&vis[wd]) | ~allow[wd];
-                    from = word[set];
-                    left = seen[set] & ~had[set];
+                if (fill) {
+                    now = load_agent(&vis[take]) | ~allow[take];
+                    from = word[at];
+                    left = seen[at] & ~had[at];
                 }
                 wave_sync();
-                if (miss) word[set] = wd;
+                if (fill) word[at] = take;
                 wave_sync();
-                if (miss && word[set] == wd) {  // of several words for one place, one has it
+                if (fill && word[at] == take) {  // of several words for one place, one has it
                     if (left) atomicOr(mem + from, left);
-                    seen[set] = now;
-                    had[set] = now;
+                    seen[at] = now;
+                    had[at] = now;
                 }
                 wave_sync();
                 here = word[set] == wd;
@@ -1043,8 +1051,8 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
                 // the only tile: take what it claimed as the next one
                 if (total <= kWave) {  // only the first wave had edges
                     if (c.wave == 0) {
-                        narrow_steps = expand_wave(c, pq, root, beg, adj, allow, vis, hs, hout, hn_out, my_found,
-                                                   narrow_steps);
+                        narrow_steps = expand_wave(c, pq, root, beg, adj, allow, vis, hs, hout, hn_out, (int32_t)a.nwords,
+                                                   my_found, narrow_steps);
                         fedges = c.lane < hs.n ? hs.d[c.lane] : 0;
                         for (int i = c.lane; i < pq.n; i += kWave) fedges += qentry_degree(pq.buf[i]);
                     }
