@@ -739,7 +739,7 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
 // wave, the entries stay in the registers of the lanes that claimed them, and
 // no lane branches except where a word is missing or a hub turns up.  A
 // chain of 10^4 levels of about two vertices: 1.6 us a level in expand_local,
-// 0.94 with the copies, 0.74 with both.  The copies lie in the other waves'
+// 0.94 with the copies, 0.71 with both.  The copies lie in the other waves'
 // staging, which is empty while they wait at the block's barrier.
 __device__ __forceinline__ int expand_wave(Ctx& c, PairQueue& wq, int32_t root, const int32_t* __restrict__ beg,
                                            const int32_t* __restrict__ adj, const uint64_t* __restrict__ allow,
@@ -1560,6 +1560,44 @@ __device__ __forceinline__ bool lp_wcc(Ctx& c, const int32_t* q, int64_t n, int6
 
 __device__ __forceinline__ int32_t key_colour(uint64_t k) { return (int32_t)(uint32_t)k; }
 
+// Sweeps of a fixed-point iteration by one block over its own vertices, until
+// one of them changes nothing there or kBlockSweeps are done: between two
+// grid barriers, so what came from other blocks goes as far as it can.  A
+// block's vertices are neighbours in the queue, which is ascending, so most
+// edges of a graph with local ids stay inside it.  sweep() returns what this
+// thread changed; the sum over the sweeps comes back.
+constexpr int kBlockSweeps = 16;
+template <class Sweep>
+__device__ __forceinline__ int block_sweeps(Ctx& c, bool one, Sweep sweep) {
+    int all = 0;
+    for (int k = 0; k < kBlockSweeps; ++k) {
+        const int changed = sweep();
+        all += changed;
+        wait_vm();  // the other waves' next sweep reads it
+        if (!__syncthreads_or(changed)) return one ? 0 : all;  // alone: that was the fixed point
+    }
+    return all;
+}
+
+// colour_scc's barrier, with the sum of x over the threads: of the grid, or
+// of one block while the others have left.
+template <bool ACQ>
+__device__ __forceinline__ bool colour_sync(Ctx& c, bool one, int x, int64_t& sum) {
+    if (!one) {
+        int64_t r[4];
+        if (!gsync_sum<4, ACQ>(c, {(uint32_t)wave_sum(x), 0, 0, 0}, r)) return false;
+        sum = r[0];
+        return true;
+    }
+    wait_vm();
+    sum = block_sum(x, c.sm);
+    if (ACQ) {
+        if (c.wave == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        __syncthreads();
+    }
+    return true;
+}
+
 // The colouring SCC method (graph_color, src/color_propagation.h:9-467).  A
 // vertex's priority is (active out-degree + 5) x active in-degree
 // (degree_rank, :9-58; clipped to 31 bits here, which can only change ties:
@@ -1573,6 +1611,13 @@ __device__ __forceinline__ int32_t key_colour(uint64_t k) { return (int32_t)(uin
 // with their smallest id and leave the active set; the rest start the next
 // round with their own keys again (color_init, :262-290).  Each round labels
 // at least the SCC of the largest key of every weakly connected piece.
+//
+// Nearly all of it is barriers and round trips: about 25 sweeps a round over
+// a chain of 20,000 SCCs.  So blocks sweep on their own between barriers,
+// barriers within a round skip the acquire (keys, stamps and minima are read
+// coherently), entries are read four at a time, and a rest of at most a block's
+// threads is left to one block: k_tail 924 -> 590 us there, 300 SCCs
+// 400 -> 283.
 __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, int64_t& rounds, int64_t& sccs) {
     KernelArgs& a = c.args();
     GiantState* gs = a.gs;
@@ -1580,6 +1625,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
     const int64_t gt = (int64_t)c.b * kGBlock + c.tid;
     auto buf = [&a](int k) { return k ? a.fq : a.fq_alt; };
     using ull = unsigned long long;
+    constexpr int kAhead = 4;  // list entries whose keys or stamps are read together
     {  // degree rank, once, into parent
         const int32_t* q = buf(cur);
         for (int64_t i = gt; i < n; i += nthreads) {
@@ -1592,6 +1638,8 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
     }
     sccs = 0;
     for (rounds = 1;; ++rounds) {
+        const bool one = n <= kGBlock;
+        if (one && c.b != 0) return true;
         const int32_t* q = buf(cur);
         int32_t* qn = buf(cur ^ 1);
         int32_t* cnt = &gs->fqn[s % 3].v;  // last read three rounds (or sweeps) ago
@@ -1601,31 +1649,41 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
             st_agent(&a.ckey[v], ((uint64_t)(uint32_t)load_agent(&a.parent[v]) << 32) | (uint32_t)v);
             st_agent(&a.stamp[v], -1);
         }
-        if (!gsync(c)) return false;
+        int64_t got;
+        if (!colour_sync<false>(c, one, 0, got)) return false;
         for (int64_t it = 0;; ++it) {  // largest key among the vertices that reach v
-            int changed = 0;
-            for (int64_t i = gt; i < n; i += nthreads) {
-                const int32_t v = q[i];
-                const uint64_t k0 = load_agent(&a.ckey[v]);
-                uint64_t k = k0;
-                const int32_t end = a.bwb[v + 1];
-                for (int32_t e = a.bwb[v]; e < end; ++e) {
-                    const int32_t w = a.bwa[e];
-                    if (w != v && bit_of(a.act, w)) k = max(k, load_agent(&a.ckey[w]));
+            const int changed = block_sweeps(c, one, [&]() {
+                int ch = 0;
+                for (int64_t i = gt; i < n; i += nthreads) {
+                    const int32_t v = q[i];
+                    const uint64_t k0 = load_agent(&a.ckey[v]);
+                    uint64_t k = k0;
+                    const int32_t end = a.bwb[v + 1];
+                    for (int32_t e = a.bwb[v]; e < end; e += kAhead) {
+                        int32_t w[kAhead];
+                        uint64_t kw[kAhead];
+#pragma unroll
+                        for (int j = 0; j < kAhead; ++j) w[j] = a.bwa[min(e + j, end - 1)];
+#pragma unroll
+                        for (int j = 0; j < kAhead; ++j) kw[j] = load_agent(&a.ckey[w[j]]);
+#pragma unroll
+                        for (int j = 0; j < kAhead; ++j)
+                            if (w[j] != v && bit_of(a.act, w[j])) k = max(k, kw[j]);
+                    }
+                    for (int hop = 0; hop < 100; ++hop) {  // the colour's own key, and so on
+                        const uint64_t kc = load_agent(&a.ckey[key_colour(k)]);
+                        if (kc <= k) break;
+                        k = kc;
+                    }
+                    if (k > k0) {
+                        atomicMax(reinterpret_cast<ull*>(&a.ckey[v]), (ull)k);
+                        ++ch;
+                    }
                 }
-                for (int hop = 0; hop < 100; ++hop) {  // the colour's own key, and so on
-                    const uint64_t kc = load_agent(&a.ckey[key_colour(k)]);
-                    if (kc <= k) break;
-                    k = kc;
-                }
-                if (k > k0) {
-                    atomicMax(reinterpret_cast<ull*>(&a.ckey[v]), (ull)k);
-                    ++changed;
-                }
-            }
-            int64_t r[4];
-            if (!gsync_sum<4, true>(c, {(uint32_t)wave_sum(changed), 0, 0, 0}, r)) return false;
-            if (r[0] == 0) break;
+                return ch;
+            });
+            if (!colour_sync<false>(c, one, changed, got)) return false;
+            if (got == 0) break;
             if (it > (int64_t)a.V + 2) {
                 if (c.tid == 0) atomicOr(&gs->err.v, 2);
                 return false;
@@ -1638,26 +1696,36 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
                 st_agent(&a.aux[v], v);
             }
         }
-        if (!gsync(c)) return false;
+        if (!colour_sync<false>(c, one, 0, got)) return false;
         for (int64_t it = 0;; ++it) {  // v joins its colour's SCC through an out-neighbour in it
-            int changed = 0;
-            for (int64_t i = gt; i < n; i += nthreads) {
-                const int32_t v = q[i];
-                if (load_agent(&a.stamp[v]) >= 0) continue;
-                const int32_t r = key_colour(load_agent(&a.ckey[v]));
-                const int32_t end = a.fwb[v + 1];
-                for (int32_t e = a.fwb[v]; e < end; ++e) {
-                    const int32_t u = a.fwa[e];
-                    if (u != v && bit_of(a.act, u) && load_agent(&a.stamp[u]) == r) {
-                        st_agent(&a.stamp[v], r);
-                        ++changed;
-                        break;
+            const int changed = block_sweeps(c, one, [&]() {
+                int ch = 0;
+                for (int64_t i = gt; i < n; i += nthreads) {
+                    const int32_t v = q[i];
+                    if (load_agent(&a.stamp[v]) >= 0) continue;
+                    const int32_t r = key_colour(load_agent(&a.ckey[v]));
+                    const int32_t end = a.fwb[v + 1];
+                    for (int32_t e = a.fwb[v]; e < end; e += kAhead) {
+                        int32_t u[kAhead], su[kAhead];
+#pragma unroll
+                        for (int j = 0; j < kAhead; ++j) u[j] = a.fwa[min(e + j, end - 1)];
+#pragma unroll
+                        for (int j = 0; j < kAhead; ++j) su[j] = load_agent(&a.stamp[u[j]]);
+                        bool join = false;
+#pragma unroll
+                        for (int j = 0; j < kAhead; ++j)
+                            join = join || (su[j] == r && u[j] != v && bit_of(a.act, u[j]));
+                        if (join) {
+                            st_agent(&a.stamp[v], r);
+                            ++ch;
+                            break;
+                        }
                     }
                 }
-            }
-            int64_t r[4];
-            if (!gsync_sum<4, true>(c, {(uint32_t)wave_sum(changed), 0, 0, 0}, r)) return false;
-            if (r[0] == 0) break;
+                return ch;
+            });
+            if (!colour_sync<false>(c, one, changed, got)) return false;
+            if (got == 0) break;
             if (it > (int64_t)a.V + 2) {
                 if (c.tid == 0) atomicOr(&gs->err.v, 2);
                 return false;
@@ -1668,7 +1736,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
             const int32_t r = load_agent(&a.stamp[v]);
             if (r >= 0 && r != v) atomicMin(&a.aux[r], v);
         }
-        if (!gsync(c)) return false;
+        if (!colour_sync<false>(c, one, 0, got)) return false;
         // label the SCCs found, take them out of the active set, queue the rest
         WaveQueue wq{c.stage32(), 0};
         int found = 0;
@@ -1687,9 +1755,8 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
             wq_push<true>(wq, i < n && r < 0, v, qn, cnt);
         }
         block_flush(c, wq, qn, cnt);
-        int64_t r[4];
-        if (!gsync_sum<4, true>(c, {(uint32_t)wave_sum(found), 0, 0, 0}, r)) return false;
-        sccs += r[0];
+        if (!colour_sync<true>(c, one, found, got)) return false;  // the active set and the queue are read plainly
+        sccs += got;
         n = load_agent(cnt);
         cur ^= 1;
         ++s;
