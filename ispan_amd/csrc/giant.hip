@@ -518,7 +518,15 @@ __device__ __forceinline__ void push_next(bool claim, int32_t w, const int32_t* 
 // Claims K targets per lane, each as wave_try_claim does, and loads the
 // offsets of every candidate while the claim atomics are in flight: a
 // claimed vertex's degree costs no round trip of its own.  All lanes call it.
-template <int K>
+//
+// FEW: without the allowed bits.  What a traversal reaches over an edge is
+// allowed exactly if its own list in that direction is not empty (the edge is
+// in its other list, and only vertices with both are active), so the offsets
+// say it too, read before the claim and only for targets not yet visited.
+// That is one more round trip and a third fewer requests: for a chip full of
+// waves that expand in place, which random requests bound (this card: 27 G/s
+// atomics, 65 G/s loads past the L2), 4096^2 grid 3.72 -> 3.62 ms.
+template <int K, bool FEW = false>
 __device__ __forceinline__ void claim_with_degree(const bool (&want)[K], const int32_t (&w)[K],
                                                   const uint64_t* __restrict__ allow, uint64_t* vis,
                                                   const int32_t* __restrict__ beg, bool (&claim)[K],
@@ -530,13 +538,30 @@ __device__ __forceinline__ void claim_with_degree(const bool (&want)[K], const i
         al[k] = 0;
         vi[k] = 0;
         if (want[k]) {
-            al[k] = allow[w[k] >> 6];
+            al[k] = FEW ? ~0ull : allow[w[k] >> 6];
             vi[k] = vis[w[k] >> 6];
         }
     }
     bool cand[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) cand[k] = want[k] && ((al[k] & ~vi[k]) >> (w[k] & 63)) & 1ull;
+    int32_t e1[K];
+    auto load_offsets = [&]() {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            s0[k] = 0;
+            e1[k] = 0;
+            if (cand[k]) {
+                s0[k] = beg[w[k]];
+                e1[k] = beg[w[k] + 1];
+            }
+        }
+    };
+    if (FEW) {
+        load_offsets();
+#pragma unroll
+        for (int k = 0; k < K; ++k) cand[k] = cand[k] && e1[k] > s0[k];
+    }
     uint64_t incl[K], excl[K];
     int end[K];
 #pragma unroll
@@ -584,16 +609,7 @@ __device__ __forceinline__ void claim_with_degree(const bool (&want)[K], const i
         if (lane == end[k] && incl[k])
             old[k] = atomicOr(reinterpret_cast<unsigned long long*>(vis + (w[k] >> 6)), (unsigned long long)incl[k]);
     }
-    int32_t e1[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        s0[k] = 0;
-        e1[k] = 0;
-        if (cand[k]) {
-            s0[k] = beg[w[k]];
-            e1[k] = beg[w[k] + 1];
-        }
-    }
+    if (!FEW) load_offsets();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const uint64_t o = __shfl(old[k], end[k], kWave);
@@ -690,7 +706,7 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
             want[0] = e < total && w[0] != root;
             bool claim[1];
             int32_t s0[1], d[1];
-            claim_with_degree<1>(want, w, allow, vis, beg, claim, s0, d);
+            claim_with_degree<1, true>(want, w, allow, vis, beg, claim, s0, d);
             my_found += claim[0];
             hub_push(hs, claim[0] && d[0] >= kGiantHubDeg, w[0], s0[0], d[0], hout, hn_out);
             const bool keep = claim[0] && d[0] > 0 && d[0] < kGiantHubDeg;
