@@ -343,6 +343,7 @@ struct HubStage {
     int32_t* d;
     int n;              // wave-uniform fill
     uint32_t sent = 0;  // work items written so far (wave-uniform)
+    int chunk = kGiantChunk;  // edges per work item
 };
 
 __device__ __forceinline__ void hub_flush(HubStage& hs, HubItem* hout, int32_t* hn_out) {
@@ -353,7 +354,7 @@ __device__ __forceinline__ void hub_flush(HubStage& hs, HubItem* hout, int32_t* 
     if (lane < hs.n) {
         v = hs.v[lane];
         s0 = hs.s[lane];
-        nch = (hs.d[lane] + kGiantChunk - 1) / kGiantChunk;
+        nch = (hs.d[lane] + hs.chunk - 1) / hs.chunk;
     }
     const int incl = wave_incl_scan(nch);
     int base = 0;
@@ -362,7 +363,7 @@ __device__ __forceinline__ void hub_flush(HubStage& hs, HubItem* hout, int32_t* 
     hs.sent += (uint32_t)lane_get(incl, kWave - 1);
     for (int k = 0; k < nch; ++k) {
         st_agent(&hout[base + k].v, v);
-        st_agent(&hout[base + k].start, s0 + k * kGiantChunk);
+        st_agent(&hout[base + k].start, s0 + k * hs.chunk);
     }
     hs.n = 0;
     wave_sync();
@@ -481,7 +482,7 @@ __device__ __forceinline__ void block_flush_both(Ctx& c, PairQueue& pq, uint64_t
     if (c.lane < hs.n) {
         v = hs.v[c.lane];
         s0 = hs.s[c.lane];
-        nch = (hs.d[c.lane] + kGiantChunk - 1) / kGiantChunk;
+        nch = (hs.d[c.lane] + hs.chunk - 1) / hs.chunk;
     }
     const int incl = wave_incl_scan(nch);
     int qb, hb;
@@ -490,7 +491,7 @@ __device__ __forceinline__ void block_flush_both(Ctx& c, PairQueue& pq, uint64_t
     hb += incl - nch;
     for (int k = 0; k < nch; ++k) {
         st_agent(&hout[hb + k].v, v);
-        st_agent(&hout[hb + k].start, s0 + k * kGiantChunk);
+        st_agent(&hout[hb + k].start, s0 + k * hs.chunk);
     }
     pq.sent += (uint32_t)pq.n;
     hs.sent += (uint32_t)lane_get(incl, kWave - 1);
@@ -504,15 +505,16 @@ __device__ __forceinline__ void block_flush_both(Ctx& c, PairQueue& pq, uint64_t
 // the queue (degree-0 vertices have nothing to expand).  All lanes call it.
 __device__ __forceinline__ void push_next(bool claim, int32_t w, const int32_t* __restrict__ beg, PairQueue& pq,
                                           uint64_t* qout, int32_t* qn_out, HubStage& hs, HubItem* hout,
-                                          int32_t* hn_out, int64_t& pushed_edges) {
+                                          int32_t* hn_out, int64_t& pushed_edges,
+                                          int32_t hub_deg = kGiantHubDeg) {
     int32_t d = 0, s0 = 0;
     if (claim) {
         s0 = beg[w];
         d = beg[w + 1] - s0;
         pushed_edges += d;
     }
-    hub_push(hs, claim && d >= kGiantHubDeg, w, s0, d, hout, hn_out);
-    pq_push(pq, claim && d > 0 && d < kGiantHubDeg, qentry(s0, d), qout, qn_out);
+    hub_push(hs, claim && d >= hub_deg, w, s0, d, hout, hn_out);
+    pq_push(pq, claim && d > 0 && d < hub_deg, qentry(s0, d), qout, qn_out);
 }
 
 // Claims K targets per lane, each as wave_try_claim does, and loads the
@@ -902,6 +904,15 @@ __device__ __forceinline__ int expand_wave(Ctx& c, PairQueue& wq, int32_t root, 
 // flat).
 constexpr int kLocalPerWave = 8;
 
+// A batch's roots, the vertices of most edges of its graphs, are the whole
+// level 0: their lists are cut into items of a block's step, from kSeedHubDeg
+// edges on where the items' room allows.  With kGiantChunk edges an item and
+// up to 64 lists of less than kGiantHubDeg in a tile a few blocks had most of
+// the level (400 graphs, 660 K edges a direction: the level 97 -> 64 us).
+constexpr int kSeedChunk = kGBlock;
+constexpr int kSeedHubDeg = kWave;
+static_assert(kSeedChunk >= 2 * kGiantHubDeg, "giant_hub_capacity holds such items");
+
 // What a wave's part of a level came to: per-thread counts and wave-uniform
 // queue totals.
 struct Level {
@@ -994,6 +1005,7 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
         } else {
             n = nq;
             nh = nh_in;
+            if (L == 0) rchunk = kSeedChunk;
             if (n < 0 || n > a.V || nh < 0 || nh > a.hub_cap) {  // cannot happen with exact claims
                 if (c.tid == 0) atomicOr(&gs->err.v, 4);
                 n = 0;
@@ -1313,19 +1325,21 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
         uint32_t cnt[4];
         for (int dir = 0; dir < 2; ++dir) {
             PairQueue wq{c.stage(), 0};
-            HubStage hs{sm.hv[c.wave], sm.hs[c.wave], sm.hd[c.wave], 0};
+            HubStage hs{sm.hv[c.wave], sm.hs[c.wave], sm.hd[c.wave], 0, 0, kSeedChunk};
             const int32_t* beg = dir ? a.bwb : a.fwb;
             uint64_t* vis = dir ? a.bvis : a.fvis;
             uint64_t* q0 = dir ? a.qb0 : a.q0;
             HubItem* h0 = dir ? a.hb0 : a.h0;
             int64_t unused = 0;
+            const bool fits = a.n_roots + beg[a.V] / kSeedChunk <= a.hub_cap;
             for (int64_t ib = (int64_t)c.b * kGBlock + c.wave * kWave; ib < a.n_roots; ib += (int64_t)c.G * kGBlock) {
                 const int64_t i = ib + c.lane;
                 const int32_t r = i < a.n_roots ? a.roots[i] : -1;
                 const bool ok = r >= 0 && r < a.V;
                 if (ok) atomicOr(reinterpret_cast<unsigned long long*>(vis + (r >> 6)), 1ull << (r & 63));
                 if (dir == 0) seeded += ok;
-                push_next(ok, r, beg, wq, q0, &gs->qn[dir][0].v, hs, h0, &gs->hn[dir][0].v, unused);
+                push_next(ok, r, beg, wq, q0, &gs->qn[dir][0].v, hs, h0, &gs->hn[dir][0].v, unused,
+                          fits ? kSeedHubDeg : kGiantHubDeg);
             }
             block_flush_both(c, wq, q0, &gs->qn[dir][0].v, hs, h0, &gs->hn[dir][0].v);
             cnt[2 * dir] = wq.sent;
