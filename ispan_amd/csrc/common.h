@@ -313,8 +313,15 @@ hipError_t launch_stats(const int32_t* fwb, const int32_t* bwb, const int32_t* l
 // out[kHistSlots]: 64 log2 bins, largest, counts of sizes 1-3, SCC count.
 constexpr int kHistSlots = 69;
 hipError_t launch_scc_histogram(const int32_t* lab, int32_t V, int32_t* size, int64_t* out, hipStream_t s);
-hipError_t launch_check_csr(const int32_t* beg, const int32_t* adj, int32_t V, int64_t E, Ctl* ctl, int grid,
-                            hipStream_t s);
+// Both directions of a graph, out-edges then in-edges; first[d] may be null.
+struct CsrPair {
+    const int32_t* beg[2];
+    const int32_t* adj[2];
+    int32_t* first[2];  // every list's first entry
+};
+// Adds the pair's violations to ctl->bad_csr; fills first[d] where given (of no
+// use when there are any).
+hipError_t launch_check_csr(const CsrPair& pair, int32_t V, int64_t E, Ctl* ctl, int grid, hipStream_t s);
 
 // ---- graph building (gen.hip).  Return 0, -1 bad argument, -2 bad edge,
 // -3 out of memory, -4 HIP error (message in err).

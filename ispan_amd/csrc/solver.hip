@@ -383,12 +383,15 @@ float ev_ms(ispan_ctx* ctx, int a, int b) {
     return ms;
 }
 
-int check_bound(ispan_ctx* ctx, const ispan_params* P) {
+// The check that P asks for; with `first`, the bound graph's first entries come
+// with it.
+int check_bound(ispan_ctx* ctx, const ispan_params* P, bool first = false) {
     if (!P || !P->validate) return ISPAN_OK;
     CK(launch_reset_ctl(ctx->ctl, ctx->stream));
     if (ctx->V > 0) {
-        CK(launch_check_csr(ctx->fwb, ctx->fwa, ctx->V, ctx->E, ctx->ctl, ctx->grid, ctx->stream));
-        CK(launch_check_csr(ctx->bwb, ctx->bwa, ctx->V, ctx->E, ctx->ctl, ctx->grid, ctx->stream));
+        const CsrPair pair{{ctx->fwb, ctx->bwb}, {ctx->fwa, ctx->bwa},
+                           {first ? ctx->fw_first : nullptr, first ? ctx->bw_first : nullptr}};
+        CK(launch_check_csr(pair, ctx->V, ctx->E, ctx->ctl, ctx->grid, ctx->stream));
     }
     int rc = readback(ctx, nullptr);
     if (rc) return rc;
@@ -880,7 +883,8 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
     return ISPAN_OK;
 }
 
-int bind_common(ispan_ctx* ctx, int32_t V, int64_t E) {
+// The graph whose arrays ctx holds by now: its check and its first entries.
+int bind_common(ispan_ctx* ctx, int32_t V, int64_t E, const ispan_params* P) {
     ctx->V = V;
     ctx->E = E;
     ctx->nwords = ((int64_t)V + 63) / 64;
@@ -888,6 +892,8 @@ int bind_common(ispan_ctx* ctx, int32_t V, int64_t E) {
     CK(ctx->first_mem.ensure(nv * 8));
     ctx->fw_first = static_cast<int32_t*>(ctx->first_mem.p);
     ctx->bw_first = ctx->fw_first + nv;
+    if (int rc = check_bound(ctx, P, true)) return rc;
+    if (P && P->validate) return ISPAN_OK;
     if (V > 0) {
         CK(launch_first(ctx->fwb, ctx->fwa, V, ctx->fw_first, ctx->grid, ctx->stream));
         CK(launch_first(ctx->bwb, ctx->bwa, V, ctx->bw_first, ctx->grid, ctx->stream));
@@ -1066,10 +1072,7 @@ int ispan_graph_upload(ispan_ctx* ctx, int32_t V, int64_t E, const int32_t* fw_b
     ctx->bwa = ctx->owned[3];
     ispan_params d;
     ispan_default_params(&d);
-    ctx->V = V;
-    ctx->E = E;
-    int rc = check_bound(ctx, params ? params : &d);
-    if (!rc) rc = bind_common(ctx, V, E);
+    int rc = bind_common(ctx, V, E, params ? params : &d);
     if (rc) free_graph(ctx);
     return rc;
 }
@@ -1084,12 +1087,9 @@ int ispan_graph_bind_device(ispan_ctx* ctx, int32_t V, int64_t E, const int32_t*
     ctx->fwa = d_fw_adj;
     ctx->bwb = d_bw_beg;
     ctx->bwa = d_bw_adj;
-    ctx->V = V;
-    ctx->E = E;
     ispan_params d;
     ispan_default_params(&d);
-    int rc = check_bound(ctx, params ? params : &d);
-    if (!rc) rc = bind_common(ctx, V, E);
+    int rc = bind_common(ctx, V, E, params ? params : &d);
     if (rc) free_graph(ctx);
     return rc;
 }
@@ -1431,9 +1431,9 @@ int check_csr_device(int32_t V, int64_t E, const int32_t* fwb, const int32_t* fw
     int dev = 0, cu = 1;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev);
+    const CsrPair pair{{fwb, bwb}, {fwa, bwa}, {nullptr, nullptr}};
     if (launch_reset_ctl(d, s) != hipSuccess ||
-        (V > 0 && (launch_check_csr(fwb, fwa, V, E, d, cu * 8, s) != hipSuccess ||
-                   launch_check_csr(bwb, bwa, V, E, d, cu * 8, s) != hipSuccess)) ||
+        (V > 0 && launch_check_csr(pair, V, E, d, cu * 8, s) != hipSuccess) ||
         hipMemcpyAsync(&h, d, sizeof(Ctl), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         rc = ISPAN_ERR_HIP;
@@ -1824,14 +1824,14 @@ int ispan_scc_detection_noalloc(int32_t V, int64_t E, const int32_t* d_fw_beg, c
     c.fwa = d_fw_adj;
     c.bwb = d_bw_beg;
     c.bwa = d_bw_adj;
-    if ((rc = check_bound(&c, &P))) return rc;
+    if ((rc = check_bound(&c, &P, true))) return rc;
     if (V > 0) {
         // the barrier records sit wherever this call's layout puts them: they
         // must not hold a tag a barrier is still to use
         if (launch_fill_i32(reinterpret_cast<int32_t*>(c.bar), 0, (int64_t)kBarBytesPerBlock / 4 * c.coop_grid, 32,
                             c.stream) != hipSuccess ||
-            launch_first(c.fwb, c.fwa, V, c.fw_first, c.grid, c.stream) != hipSuccess ||
-            launch_first(c.bwb, c.bwa, V, c.bw_first, c.grid, c.stream) != hipSuccess)
+            (!P.validate && (launch_first(c.fwb, c.fwa, V, c.fw_first, c.grid, c.stream) != hipSuccess ||
+                             launch_first(c.bwb, c.bwa, V, c.bw_first, c.grid, c.stream) != hipSuccess)))
             return ISPAN_ERR_HIP;
     }
     return solve_impl(&c, &P, d_labels, stats);
