@@ -314,6 +314,18 @@ struct BuildMem {
     }
 };
 
+// How keys are sorted.  By radix passes from 2^18 keys on: the library's own
+// line, 2^20, has merges up to there, whose time steps up with the size (64-bit
+// keys, 40 / 17 bits: 200,000 keys 67 / 63 us merged, 99 / 63 by passes; 400,000
+// keys 123 / 118 and 106 / 68; a million 177 / 170 and 123 / 80).  And 1024
+// threads of 8 keys a block, which for 64-bit keys is faster than its choice
+// from 2.5 M keys on (16 M keys of 40 bits 547 -> 510 us) and otherwise equal.
+using KeySort = rocprim::radix_sort_config<
+    rocprim::default_config, rocprim::default_config,
+    rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 8>, rocprim::kernel_config<1024, 8>, 8,
+                                        rocprim::block_radix_rank_algorithm::match>,
+    1 << 18>;
+
 // M.keys[0, m) (edge_key form) -> CSR pair; M.n is zero.  Only the 2 * bits
 // bits of a key are sorted, in 32-bit keys when they fit (V <= 65536); the
 // kept keys, then in (src, dst) order, are sorted by dst alone for the
@@ -331,12 +343,12 @@ int csr_from_keys(hipStream_t s, Workspace& sort, const BuildMem<K>& M, int32_t 
     int64_t E = 0;
     rocprim::double_buffer<K> buf(M.keys, M.alt);
     if (m > 0) {
-        GK(rocprim::radix_sort_keys(nullptr, b1, buf, (size_t)m, 0, 2 * bits, s));
+        GK(rocprim::radix_sort_keys<KeySort>(nullptr, b1, buf, (size_t)m, 0, 2 * bits, s));
         GK(rocprim::exclusive_scan(nullptr, b2, M.counts, M.start, (int64_t)0, (size_t)chunks + 1,
                                    rocprim::plus<int64_t>(), s));
         GK(sort.ensure(std::max(b1, b2) + 256));
         b1 = b2 = sort.cap;
-        GK(rocprim::radix_sort_keys(sort.p, b1, buf, (size_t)m, 0, 2 * bits, s));
+        GK(rocprim::radix_sort_keys<KeySort>(sort.p, b1, buf, (size_t)m, 0, 2 * bits, s));
         hipLaunchKernelGGL(k_keep_count<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), m, bits,
                            chunks, M.counts);
         GK(hipGetLastError());
@@ -366,10 +378,10 @@ int csr_from_keys(hipStream_t s, Workspace& sort, const BuildMem<K>& M, int32_t 
         GK(hipGetLastError());
         buf = rocprim::double_buffer<K>(kept, buf.current());
         // fewer keys can take another of the sort's methods, with more scratch
-        GK(rocprim::radix_sort_keys(nullptr, b1, buf, (size_t)E, 0, bits, s));
+        GK(rocprim::radix_sort_keys<KeySort>(nullptr, b1, buf, (size_t)E, 0, bits, s));
         GK(sort.ensure(b1));
         b1 = sort.cap;
-        GK(rocprim::radix_sort_keys(sort.p, b1, buf, (size_t)E, 0, bits, s));
+        GK(rocprim::radix_sort_keys<KeySort>(sort.p, b1, buf, (size_t)E, 0, bits, s));
         R.beg = *bwb;
         R.n_gaps = M.n + 1;
         hipLaunchKernelGGL(k_transposed<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), E, bits,

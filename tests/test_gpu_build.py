@@ -63,3 +63,12 @@ def test_build_csr_rejects_an_id_outside():
         with I.Solver(0) as S, pytest.raises(I.IspanError) as e:
             S.build_csr(7, 2, a.ptr, b.ptr)
         assert e.value.code == -2
+
+
+@pytest.mark.parametrize("kind", ["uniform", "skewed"])
+@pytest.mark.parametrize("V", [40000, 70000])
+@pytest.mark.parametrize("m", [(1 << 18) - 1, 1 << 18, (1 << 18) + 1, 262143 + 8192, 600_000])
+def test_build_csr_where_the_sorts_change(V, m, kind):
+    """Around the size from which keys are sorted by radix passes, where the
+    second sort, of the fewer kept keys, still merges."""
+    test_build_csr(V, m, kind)
