@@ -402,6 +402,18 @@ int check_bound(ispan_ctx* ctx, const ispan_params* P, bool first = false) {
     return ISPAN_OK;
 }
 
+// Blocks of a solve's cooperative kernels: half of the CUs' for a small graph,
+// whose levels are barriers and round trips either way, and a barrier of half
+// as many blocks is shorter.  Half against all blocks: R-MAT of 1,000, 20,000,
+// 120,000 and 700,000 vertices 100 / 108, 104 / 113, 111 / 119 and 140 / 138 us,
+// islands of 35,000, 70,000 and 350,000 vertices 171 / 183, 180 / 191 and
+// 304 / 263 us, lattices of 200^2, 500^2 and 1000^2 492 / 515, 589 / 581 and
+// 991 / 902 us.  A quarter is no shorter again.
+constexpr int32_t kHalfGridV = 1 << 17;
+int coop_blocks(const ispan_ctx* ctx) {
+    return ctx->V <= kHalfGridV ? std::max(ctx->coop_grid / 2, 1) : ctx->coop_grid;
+}
+
 int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_stats* st) {
     const double t0 = wall_ms();
     hipStream_t s = ctx->stream;
@@ -414,6 +426,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
     ctx->have_solution = false;
     const double avg_degree = V > 0 ? (double)E / V : 0.0;
     const int G = ctx->grid;
+    const int blocks = coop_blocks(ctx);
 
     ctx->recs.clear();
     ctx->pool_used = 0;
@@ -500,7 +513,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
         ga.fq_n_ctl = ctx->ctl->fq_n;
         ga.dbg = ctx->gdbg;
         ga.trace = ctx->level_trace ? 1 : 0;
-        ga.bu_mult = giant_bu_mult(ctx->coop_grid);
+        ga.bu_mult = giant_bu_mult(blocks);
         ga.wcc_mode = P->wcc_mode;
         ga.trim_scope = P->trim_scope;
         ga.td_local = std::max(P->td_local, 0);
@@ -509,7 +522,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
         ga_tail = ga;
         hipEvent_t ga0 = nullptr, ga1 = nullptr;
         if (P->timing >= 2 && (ga0 = pool_event(ctx)) && (ga1 = pool_event(ctx))) ctx->recs.push_back({3, ga0, ga1});
-        const hipError_t le = launch_giant(ga, ctx->ctl, ctx->coop_grid, s, ga0);
+        const hipError_t le = launch_giant(ga, ctx->ctl, blocks, s, ga0);
         if (le == hipErrorCooperativeLaunchTooLarge || le == hipErrorIllegalState || le == hipErrorNotSupported ||
             le == hipErrorLaunchOutOfResources) {
             (void)hipGetLastError();
@@ -538,7 +551,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
                 // the colouring SCC method, on the device (one more launch
                 // and wait, as the mice phase would take)
                 ga.bar_base = ctx->bar_base;
-                CK(launch_tail(ga, ctx->coop_grid, s));
+                CK(launch_tail(ga, blocks, s));
                 CK(hipMemcpyAsync(ctx->h_gstate, ctx->gstate,
                                   ctx->level_trace ? sizeof(GiantState) : kGiantStateHead, hipMemcpyDeviceToHost, s));
                 CK(launch_fill_i32(&ctx->ctl->unlabelled, 0, 1, 1, s));
@@ -553,18 +566,18 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
                 CK(launch_fill_i32(reinterpret_cast<int32_t*>(ctx->bar), 0,
                                    (int64_t)kBarBytesPerBlock / 4 * ctx->coop_grid, 1, s));
                 if (gs.err.v & 1) {  // where did the blocks stop?
-                    std::vector<int32_t> d((size_t)2 * ctx->coop_grid);
+                    std::vector<int32_t> d((size_t)2 * blocks);
                     if (hipMemcpy(d.data(), ctx->gdbg, d.size() * 4, hipMemcpyDeviceToHost) == hipSuccess) {
                         int amin = INT32_MAX, amax = 0, pmin = INT32_MAX, pmax = 0, zero = 0;
-                        for (int b = 0; b < ctx->coop_grid; ++b) {
+                        for (int b = 0; b < blocks; ++b) {
                             amin = std::min(amin, d[b]);
                             amax = std::max(amax, d[b]);
-                            pmin = std::min(pmin, d[ctx->coop_grid + b]);
-                            pmax = std::max(pmax, d[ctx->coop_grid + b]);
+                            pmin = std::min(pmin, d[blocks + b]);
+                            pmax = std::max(pmax, d[blocks + b]);
                             zero += d[b] == 0;
                         }
                         fprintf(stderr, "[ispan] barrier timeout: grid %d, arrived min %d max %d (blocks at 0: %d), "
-                                "passed min %d max %d\n", ctx->coop_grid, amin, amax, zero, pmin, pmax);
+                                "passed min %d max %d\n", blocks, amin, amax, zero, pmin, pmax);
                     }
                 }
                 ctx->err = gs.err.v & 1   ? "giant phase: grid barrier timed out"
@@ -604,7 +617,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
                             (gs.post_cp[0] - gs.ts[3]) * k, (gs.post_cp[1] - gs.ts[3]) * k,
                             (gs.post_cp[2] - gs.ts[3]) * k);
                 if (gs.bu1_scan[0]) {  // first forward bottom-up level, per block and by XCC (block % 8)
-                    const int nb = std::min(ctx->coop_grid, 1024);
+                    const int nb = std::min(blocks, 1024);
                     double xs[8] = {0}, xw[8] = {0}, xmax[8] = {0};
                     int xn[8] = {0};
                     for (int b = 0; b < nb; ++b) {
@@ -794,7 +807,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
         GiantArgs gc = ga_tail;
         gc.wcc_mode = 2;
         gc.bar_base = ctx->bar_base;
-        CK(launch_tail(gc, ctx->coop_grid, s));
+        CK(launch_tail(gc, blocks, s));
         CK(hipMemcpyAsync(ctx->h_gstate, ctx->gstate, kGiantStateHead, hipMemcpyDeviceToHost, s));
         CK(launch_fill_i32(&ctx->ctl->unlabelled, 0, 1, 1, s));
         CK(launch_count_unlabelled(ctx->lab, V, ctx->batch_sel, ctx->ctl, G, s));

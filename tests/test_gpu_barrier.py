@@ -38,3 +38,23 @@ def test_launches_of_different_lengths_in_turn(order):
                 for wcc in (0, 1):
                     s.solve(I.default_params(wcc_mode=wcc))
                     assert np.array_equal(s.labels(), want[n]), (rep, n, wcc)
+
+
+@pytest.mark.parametrize("wcc", [0, 1, 2])
+def test_half_the_blocks_and_all_in_turn(wcc):
+    """Graphs at the size up to which half of the blocks are launched, just
+    past it, and small ones between, on the same records."""
+    made = [O.rmat(17, 4.0, 1), O.grid(363, 0.5, 2), O.rmat(9, 8.0, 3), G.cycle_chain(400, 5)]
+    for extra in (0, 1):  # 2^17 vertices, and one isolated vertex more
+        V = (1 << 17) + extra
+        src = np.repeat(np.arange(made[0].V), np.diff(made[0].fw_beg)).astype(np.int32)
+        made.append(O.build_csr(V, src, made[0].fw_adj.astype(np.int32)))
+    want = [O.tarjan(g) for g in made]
+    with I.Solver(0) as s:
+        for _ in range(2):
+            for i in (4, 5, 0, 2, 1, 3, 5, 4, 2):
+                g = made[i]
+                s.upload(I.HostGraph(g.fw_beg, g.fw_adj, g.bw_beg, g.bw_adj))
+                st = s.solve(I.default_params(wcc_mode=wcc))
+                assert st.engine_used == 0
+                assert np.array_equal(s.labels(), want[i]), i
