@@ -644,8 +644,11 @@ __device__ __forceinline__ void push_found_n(const bool (&claim)[K], const int32
 constexpr int kNarrowWave = 256;
 constexpr int kNarrowBlock = 2048;
 // Such levels in a row, while the other direction waits at the barrier and
-// when it has finished.
-constexpr int kNarrowShort = 16, kNarrowLong = 4096;
+// when it has finished: counted as levels of a wave, one of a block as the
+// kNarrowCost wave levels whose time it takes.  128, 64 and 16 with every
+// level counted as one gave lattices of 60^2 192, 281 and 358 us and of 2000^2
+// 1.46, 1.45 and 1.68 ms; 256 and 512 gave what 128 gives.
+constexpr int kNarrowShort = 128, kNarrowLong = 16384, kNarrowCost = 4;
 
 // The adj index of this lane's edge, less the edge's number eb + lane, for
 // edges eb to eb + kWave - 1 of up to kWave entries, one a lane, that begin at
@@ -899,10 +902,11 @@ __device__ __forceinline__ int expand_wave(Ctx& c, PairQueue& wq, int32_t root, 
 }
 
 // Level-synchronous top-down levels are expanded in place (as in mode 2)
-// once their input gives every wave at least this many vertices (grid 4096:
-// 2, 4, 8, 16 and 32 measured 4.30, 4.19, 4.01, 4.09 and 4.30 ms; R-MAT
-// flat).
-constexpr int kLocalPerWave = 8;
+// once their input gives every wave at least this many vertices.  Five
+// 4096^2 lattices: 3.65 ms on average with 12, 3.70 with 11, 3.72 with 10 and
+// 3.69 with 14 (8 and 16: three of them, 3.88 and 3.89), smaller ones alike;
+// R-MAT flat.
+constexpr int kLocalPerWave = 12;
 
 // A batch's roots, the vertices of most edges of its graphs, are the whole
 // level 0: their lists are cut into items of a block's step, from kSeedHubDeg
@@ -1099,7 +1103,7 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
                 const int wi = row_incl(sm.wcnt[1][c.lane & 15], 0, [](int x, int y) { return x + y; });
                 const int entries = lane_get(ci, kW - 1), edges = lane_get(wi, kW - 1);
                 const int base = lane_get(ci - cnt, c.wave);
-                narrow_steps = __builtin_amdgcn_readfirstlane(sm.steps) - 1;
+                narrow_steps = __builtin_amdgcn_readfirstlane(sm.steps) - kNarrowCost;
                 if (entries == 0 || entries > kGBlock || edges > kNarrowBlock || narrow_steps <= 0) break;
                 wave_sync();
                 for (int i = c.lane; i < pq.n; i += kWave) {
