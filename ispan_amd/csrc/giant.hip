@@ -1597,16 +1597,23 @@ __device__ __forceinline__ bool lp_wcc(Ctx& c, const int32_t* q, int64_t n, int6
 __device__ __forceinline__ int32_t key_colour(uint64_t k) { return (int32_t)(uint32_t)k; }
 
 // Sweeps of a fixed-point iteration by one block over its own vertices, until
-// one of them changes nothing there or kBlockSweeps are done: between two
+// one of them changes nothing there or `most` are done: between two
 // grid barriers, so what came from other blocks goes as far as it can.  A
 // block's vertices are neighbours in the queue, which is ascending, so most
 // edges of a graph with local ids stay inside it.  sweep() returns what this
 // thread changed; the sum over the sweeps comes back.
 constexpr int kBlockSweeps = 16;
+// From this many edges a vertex a block sweeps once: its sweep takes longer
+// than a grid barrier, and most of what it waits for is in other blocks.
+// Once against up to 16 times, random DAGs: of 20,000 vertices and 34, 50 and
+// 198 edges each 21.0 / 21.9, 37.4 / 39.0 and 308 / 337 ms, of 5,000 and 59
+// 25.6 / 27.0; with at most 30 edges no block is held to one.  A limit on a
+// sweep's time instead (30 us) took 16.0 ms for 8.6 with 20 edges.
+constexpr int kBlockSweepsDeg = 32;
 template <class Sweep>
-__device__ __forceinline__ int block_sweeps(Ctx& c, bool one, Sweep sweep) {
+__device__ __forceinline__ int block_sweeps(Ctx& c, bool one, int most, Sweep sweep) {
     int all = 0;
-    for (int k = 0; k < kBlockSweeps; ++k) {
+    for (int k = 0; k < most; ++k) {
         const int changed = sweep();
         all += changed;
         wait_vm();  // the other waves' next sweep reads it
@@ -1662,6 +1669,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
     auto buf = [&a](int k) { return k ? a.fq : a.fq_alt; };
     using ull = unsigned long long;
     constexpr int kAhead = 4;  // list entries whose keys or stamps are read together
+    const bool dense = a.fwb[a.V] >= (int64_t)kBlockSweepsDeg * a.V;
     {  // degree rank, once, into parent
         const int32_t* q = buf(cur);
         for (int64_t i = gt; i < n; i += nthreads) {
@@ -1676,6 +1684,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
     for (rounds = 1;; ++rounds) {
         const bool one = n <= kGBlock;
         if (one && c.b != 0) return true;
+        const int most = dense && !one ? 1 : kBlockSweeps;
         const int32_t* q = buf(cur);
         int32_t* qn = buf(cur ^ 1);
         int32_t* cnt = &gs->fqn[s % 3].v;  // last read three rounds (or sweeps) ago
@@ -1688,7 +1697,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
         int64_t got;
         if (!colour_sync<false>(c, one, 0, got)) return false;
         for (int64_t it = 0;; ++it) {  // largest key among the vertices that reach v
-            const int changed = block_sweeps(c, one, [&]() {
+            const int changed = block_sweeps(c, one, most, [&]() {
                 int ch = 0;
                 for (int64_t i = gt; i < n; i += nthreads) {
                     const int32_t v = q[i];
@@ -1734,7 +1743,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
         }
         if (!colour_sync<false>(c, one, 0, got)) return false;
         for (int64_t it = 0;; ++it) {  // v joins its colour's SCC through an out-neighbour in it
-            const int changed = block_sweeps(c, one, [&]() {
+            const int changed = block_sweeps(c, one, most, [&]() {
                 int ch = 0;
                 for (int64_t i = gt; i < n; i += nthreads) {
                     const int32_t v = q[i];

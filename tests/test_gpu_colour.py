@@ -48,3 +48,29 @@ def test_colouring_by_one_block_and_by_all(n, links, shuffle):
             s.upload(I.HostGraph(h.fw_beg, h.fw_adj, h.bw_beg, h.bw_adj))
             s.solve(I.default_params(wcc_mode=2))
             assert np.array_equal(s.labels(), want)
+
+
+@pytest.mark.parametrize("seed", [0, 1])
+@pytest.mark.parametrize("n", [40, 700, 1040, 3001])
+@pytest.mark.parametrize("more", [-1, 0])  # one edge short of 32 a vertex, and 32
+def test_colouring_at_the_dense_line(n, more, seed):
+    """Lists so long that a block sweeps once between grid barriers, and one
+    edge short of that: cycles with extra edges forward (and back
+    where the ids are too few for that)."""
+    rng = np.random.default_rng(100 * n + seed)
+    base = cycles(n, 2, n + seed, False)
+    src = np.repeat(np.arange(n), np.diff(base.fw_beg))
+    have = np.unique(src * n + base.fw_adj)
+    room = np.setdiff1d(np.flatnonzero(np.triu(np.ones((n, n), bool), 1).ravel()), have)
+    extra = rng.permutation(room)[:32 * n + more - have.size]
+    if extra.size < 32 * n + more - have.size:  # 40 vertices: past the upper triangle too
+        low = np.setdiff1d(np.flatnonzero(np.tril(np.ones((n, n), bool), -1).ravel()), have)
+        extra = np.concatenate([extra, rng.permutation(low)[:32 * n + more - have.size - extra.size]])
+    e = np.concatenate([have, extra])
+    g = O.build_csr(n, (e // n).astype(np.int32), (e % n).astype(np.int32))
+    assert g.fw_adj.size == 32 * n + more
+    want = O.tarjan(g)
+    with I.Solver(0) as s:
+        s.upload(I.HostGraph(g.fw_beg, g.fw_adj, g.bw_beg, g.bw_adj))
+        s.solve(I.default_params(wcc_mode=2))
+        assert np.array_equal(s.labels(), want)
