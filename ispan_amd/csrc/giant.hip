@@ -52,6 +52,7 @@ struct Smem {
     int64_t tot[2][kBarWords];               // its totals over the grid, per reading wave
     int ok[2];
     int steps;  // levels a narrow frontier may still take in its block
+    int32_t narrow[2][kW];  // the same: every wave's staged entries, and their edges
     int32_t wcnt[2][kW];    // block flushes: per-wave counts and bases of up to two counters
     int32_t wbase[2][kW];
     int32_t hv[kW][kWave];  // per-wave staged hub vertices: id, first edge, degree
@@ -1091,16 +1092,21 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
                         for (int i = c.lane; i < pq.n; i += kWave) fedges += qentry_degree(pq.buf[i]);
                     }
                 }
+                // Every wave decides by itself from all waves' counts.  They have
+                // arrays of their own: a wave that leaves writes its flush
+                // counts (wcnt) with no barrier in between, while others may
+                // still be reading these.  They are written again only after
+                // the barriers of another round, or after the grid's.
                 const int work = wave_sum((int)fedges);
                 if (c.tid == 0) sm.steps = narrow_steps;
                 if (c.lane == 0) {
-                    sm.wcnt[0][c.wave] = pq.n;
-                    sm.wcnt[1][c.wave] = (hs.n > 0 || pq.sent > 0 || hs.sent > 0) ? kNarrowBlock + 1 : min(work, kNarrowBlock + 1);
+                    sm.narrow[0][c.wave] = pq.n;
+                    sm.narrow[1][c.wave] = (hs.n > 0 || pq.sent > 0 || hs.sent > 0) ? kNarrowBlock + 1 : min(work, kNarrowBlock + 1);
                 }
                 __syncthreads();
-                const int cnt = sm.wcnt[0][c.lane & 15];
+                const int cnt = sm.narrow[0][c.lane & 15];
                 const int ci = row_incl(cnt, 0, [](int x, int y) { return x + y; });
-                const int wi = row_incl(sm.wcnt[1][c.lane & 15], 0, [](int x, int y) { return x + y; });
+                const int wi = row_incl(sm.narrow[1][c.lane & 15], 0, [](int x, int y) { return x + y; });
                 const int entries = lane_get(ci, kW - 1), edges = lane_get(wi, kW - 1);
                 const int base = lane_get(ci - cnt, c.wave);
                 narrow_steps = __builtin_amdgcn_readfirstlane(sm.steps) - kNarrowCost;
