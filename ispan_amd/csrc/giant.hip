@@ -701,6 +701,7 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
         const int incl = wave_incl_scan(dg);
         const int total = lane_get(incl, kWave - 1);
         head += k;
+        c.edges_td += total;
         const int off = incl - dg;  // this entry's first edge of the step
         wave_sync();  // the queue entries are read: their places may be written
         for (int eb = 0; eb < total; eb += kWave) {
@@ -793,6 +794,7 @@ __device__ __forceinline__ int expand_wave(Ctx& c, PairQueue& wq, int32_t root, 
         const int incl = wave_incl_scan(dg);
         const int total = lane_get(incl, kWave - 1);
         if (total == 0 || total > kNarrowWave) break;
+        c.edges_td += total;
         const int off = incl - dg;
         int n = 0;
         for (int eb = 0; eb < total; eb += kStep) {
@@ -1406,9 +1408,9 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
             }
             if (tr && L < kLevelTrace && c.lane == 0) {
                 using ull = unsigned long long;
+                if (c.edges_td > edges0)
+                    atomicAdd(reinterpret_cast<ull*>(&gs->lv_edges[dir][L]), (ull)(c.edges_td - edges0));
                 if (c.tid == 0) {  // wave 0 of each block
-                    if (c.edges_td > edges0)
-                        atomicAdd(reinterpret_cast<ull*>(&gs->lv_edges[dir][L]), (ull)(c.edges_td - edges0));
                     const ull wt = (ull)((int64_t)wall_clock64() - tl0);
                     if (!td) atomicMax(reinterpret_cast<ull*>(&gs->lv_cp[dir][L][0]), (ull)(uint32_t)lv.edges);
                     atomicMax(reinterpret_cast<ull*>(&gs->lv_wmax[dir][L]), wt);
