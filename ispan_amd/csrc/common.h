@@ -142,7 +142,8 @@ struct GiantArgs {
     uint64_t* act;
     uint64_t* fvis;
     uint64_t* bvis;
-    uint64_t* snap;           // forward bottom-up: visited words before the level
+    uint64_t* snap;           // forward: visited words before the last bottom-up level, and the visited
+                              // words from the first top-down level after it on
     uint64_t* snapb;          // backward
     uint64_t* q0;             // forward top-down queues (ping-pong by level): (first edge << 32) | degree
     uint64_t* q1;

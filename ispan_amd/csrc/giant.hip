@@ -522,14 +522,16 @@ __device__ __forceinline__ void push_next(bool claim, int32_t w, const int32_t* 
 // offsets of every candidate while the claim atomics are in flight: a
 // claimed vertex's degree costs no round trip of its own.  All lanes call it.
 //
-// FEW: without the allowed bits.  What a traversal reaches over an edge is
-// allowed exactly if its own list in that direction is not empty (the edge is
-// in its other list, and only vertices with both are active), so the offsets
-// say it too, read before the claim and only for targets not yet visited.
-// That is one more round trip and a third fewer requests: for a chip full of
-// waves that expand in place, which random requests bound (this card: 27 G/s
-// atomics, 65 G/s loads past the L2), 4096^2 grid 3.72 -> 3.62 ms.
-template <int K, bool FEW = false>
+// kAskListed: without the allowed bits.  What a traversal reaches over an edge
+// is allowed exactly if its own list in that direction is not empty (the edge
+// is in its other list, and only vertices with both are active), so the
+// offsets say it too, read before the claim and only for targets not yet
+// visited.  That is one more round trip and a third fewer requests: for a chip
+// full of waves that expand in place, which random requests bound (this card:
+// 27 G/s atomics, 65 G/s loads past the L2), 4096^2 grid 3.72 -> 3.62 ms.
+// kAskFresh: the same, and `allow` holds vertices that are not to be claimed.
+enum { kAskAllowed, kAskListed, kAskFresh };
+template <int K, int ASK = kAskAllowed>
 __device__ __forceinline__ void claim_with_degree(const bool (&want)[K], const int32_t (&w)[K],
                                                   const uint64_t* __restrict__ allow, uint64_t* vis,
                                                   const int32_t* __restrict__ beg, bool (&claim)[K],
@@ -541,7 +543,8 @@ __device__ __forceinline__ void claim_with_degree(const bool (&want)[K], const i
         al[k] = 0;
         vi[k] = 0;
         if (want[k]) {
-            al[k] = FEW ? ~0ull : allow[w[k] >> 6];
+            al[k] = ASK == kAskListed ? ~0ull : allow[w[k] >> 6];
+            if (ASK == kAskFresh) al[k] = ~al[k];
             vi[k] = vis[w[k] >> 6];
         }
     }
@@ -560,7 +563,7 @@ __device__ __forceinline__ void claim_with_degree(const bool (&want)[K], const i
             }
         }
     };
-    if (FEW) {
+    if (ASK != kAskAllowed) {
         load_offsets();
 #pragma unroll
         for (int k = 0; k < K; ++k) cand[k] = cand[k] && e1[k] > s0[k];
@@ -612,7 +615,7 @@ __device__ __forceinline__ void claim_with_degree(const bool (&want)[K], const i
         if (lane == end[k] && incl[k])
             old[k] = atomicOr(reinterpret_cast<unsigned long long*>(vis + (w[k] >> 6)), (unsigned long long)incl[k]);
     }
-    if (!FEW) load_offsets();
+    if (ASK == kAskAllowed) load_offsets();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const uint64_t o = __shfl(old[k], end[k], kWave);
@@ -681,9 +684,11 @@ __device__ __forceinline__ int32_t edge_entry(bool valid, int off, int32_t st, i
 // one wave holds is shared again -- entries go to the next level's queue.
 // Claims stay exact (the same wave-combined atomics), so the reach set and
 // the found counts are those of a level-synchronous traversal; only the
-// level at which a vertex is expanded changes.  All lanes call it.
+// level at which a vertex is expanded changes.  With FRESH, what is in `before`
+// is not claimed, besides what is in vis.  All lanes call it.
+template <bool FRESH>
 __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root, const int32_t* __restrict__ beg,
-                                             const int32_t* __restrict__ adj, const uint64_t* __restrict__ allow,
+                                             const int32_t* __restrict__ adj, const uint64_t* __restrict__ before,
                                              uint64_t* vis, uint64_t* qout, int32_t* qn_out, HubStage& hs,
                                              HubItem* hout, int32_t* hn_out, int64_t& my_found, int max_steps) {
     uint64_t* buf = wq.buf;
@@ -713,7 +718,7 @@ __device__ __forceinline__ void expand_local(Ctx& c, PairQueue& wq, int32_t root
             want[0] = e < total && w[0] != root;
             bool claim[1];
             int32_t s0[1], d[1];
-            claim_with_degree<1, true>(want, w, allow, vis, beg, claim, s0, d);
+            claim_with_degree<1, FRESH ? kAskFresh : kAskListed>(want, w, before, vis, beg, claim, s0, d);
             my_found += claim[0];
             hub_push(hs, claim[0] && d[0] >= kGiantHubDeg, w[0], s0[0], d[0], hout, hn_out);
             const bool keep = claim[0] && d[0] > 0 && d[0] < kGiantHubDeg;
@@ -947,8 +952,10 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
     const int32_t* radj = bw ? a.fwa : a.bwa;
     const int32_t* rfirst = bw ? a.fw_first : a.bw_first;
     const uint64_t* allow = a.act;
-    uint64_t* vis = bw ? a.bvis : a.fvis;
     uint64_t* snap = bw ? a.snapb : a.snap;
+    // what is visited: from the gathering level on, the bitmap that the
+    // bottom-up levels left in snap
+    uint64_t* vis = mode == 2 ? snap : bw ? a.bvis : a.fvis;
     uint64_t* q0 = bw ? a.qb0 : a.q0;
     uint64_t* q1 = bw ? a.qb1 : a.q1;
     HubItem* h0 = bw ? a.hb0 : a.h0;
@@ -975,16 +982,27 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
     const int64_t tl0 = tr ? (int64_t)wall_clock64() : 0;
     if (topdown && gather) {
         // ---- the first top-down level after bottom-up ones: each wave takes
-        // the last level's finds (vis & ~snap) of its words, an even share of
-        // up to 64 at a time, and goes on from them in place (64 whatever the
-        // size left a lattice of 500^2 to 61 waves, 0.56 ms a direction).  No queue and no barrier lie
-        // between the finds and their expansion (a gather pass that queued
-        // them for a level of their own: 29 us for both at R-MAT s24).
+        // the last level's finds of its words, an even share of up to 64 at a
+        // time, and goes on from them in place (64 whatever the size left a
+        // lattice of 500^2 to 61 waves, 0.56 ms a direction).  No queue and no
+        // barrier lie between the finds and their expansion (a gather pass
+        // that queued them for a level of their own: 29 us for both at R-MAT
+        // s24).
+        // Some waves expand while others still gather, so the claims must not
+        // show among the finds: a vertex queued by both would be one entry
+        // more than the queues and hub lists have room for.  The bitmap that
+        // the finds were made in (`found`) therefore stays as it is, and
+        // claims, of vertices outside it, go into snap (what was visited
+        // before the last level), to which each wave adds the finds it takes.
+        // After the level snap holds all that is visited, and the later levels
+        // and the phases after them go by it.
+        const uint64_t* found = bw ? a.bvis : a.fvis;
         const int64_t share = min((a.nwords + total_waves - 1) / total_waves, (int64_t)kWave);
         for (int64_t wb = gwave * share; wb < a.nwords; wb += total_waves * share) {
             const int64_t w = wb + c.lane;
             uint64_t nw = 0;
-            if (c.lane < share && w < a.nwords) nw = vis[w] & ~snap[w];
+            if (c.lane < share && w < a.nwords) nw = found[w] & ~vis[w];
+            if (nw) atomicOr(reinterpret_cast<unsigned long long*>(vis + w), (unsigned long long)nw);
             uint64_t busy = __ballot(nw != 0);
             while (busy) {
                 const int l = __ffsll((unsigned long long)busy) - 1;
@@ -995,7 +1013,8 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
             }
         }
         if (a.td_local > 0)
-            expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found, a.td_local);
+            expand_local<true>(c, pq, root, beg, adj, found, vis, qout, qn_out, hs, hout, hn_out, my_found,
+                               a.td_local);
         block_flush_both(c, pq, qout, qn_out, hs, hout, hn_out);
         lv = Level{(int)my_found, (int)fedges, pq.sent, hs.sent};
     } else if (topdown) {
@@ -1135,8 +1154,8 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
         // growing region alone: levels of up to 256-65536 entries
         // expanded so took the 4096^2 grid from 5.09 to 5.8-6.5 ms.
         if (a.td_local > 0 && (mode == 2 || (L > 0 && nh == 0 && n >= kLocalPerWave * total_waves)))
-            expand_local(c, pq, root, beg, adj, allow, vis, qout, qn_out, hs, hout, hn_out, my_found,
-                         a.td_local);
+            expand_local<false>(c, pq, root, beg, adj, nullptr, vis, qout, qn_out, hs, hout, hn_out, my_found,
+                                a.td_local);
         block_flush_both(c, pq, qout, qn_out, hs, hout, hn_out);
         lv = Level{(int)my_found, (int)fedges, pq.sent, hs.sent};
     } else {
@@ -1145,7 +1164,7 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
         // words in this level.  Each stage issues its kU loads (first
         // in-neighbours, their visited bits) before any result is used.
         // Nothing is queued: each word's visited bits before the level go
-        // to `snap`, and a switch back to top-down gathers vis & ~snap.
+        // to `snap`, and a switch back to top-down takes vis & ~snap.
         constexpr int kU = 8;       // dense words per group
         constexpr int kSparse = 8;  // at most this many candidates: a lane's own work
         constexpr int kS = 4;       // sparse candidates per lane per step
@@ -2176,15 +2195,19 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs) {
     const int64_t per = (a.nwords + c.G - 1) / c.G;
     const int64_t wb = min((int64_t)c.b * per, a.nwords), we = min(wb + per, a.nwords);
     const bool want_min = traversed && !multi;
+    // a direction that ended top-down after bottom-up levels has its visited
+    // bits in its snapshot
+    const bool fsnap = traversed && sm.dir[0].mode == 2, bsnap = traversed && sm.dir[1].mode == 2;
     int64_t cnt = 0, gcnt = 0;
     int32_t mn = INT32_MAX;
     for (int64_t w = wb + c.tid; w < we; w += kGBlock) {
         const uint64_t a0 = a.act[w];
         uint64_t g = 0;
         if (traversed) {  // the giant: reached both ways; bvis keeps only it
-            const uint64_t bw = a.bvis[w];
-            g = a.fvis[w] & bw;
-            if (g != bw) st_agent(&a.bvis[w], g);
+            const uint64_t fw = fsnap ? a.snap[w] : a.fvis[w], bw = bsnap ? a.snapb[w] : a.bvis[w];
+            g = fw & bw;
+            if (fsnap) st_agent(&a.fvis[w], fw);
+            if (bsnap || g != bw) st_agent(&a.bvis[w], g);
         }
         if (g) st_agent(&a.act[w], a0 & ~g);
         // the vertices left at -1 below: only they can still be unlabelled at
