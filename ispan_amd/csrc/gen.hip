@@ -274,6 +274,7 @@ __global__ void k_beg_from_keys(const uint64_t* __restrict__ keys, int64_t m, in
     do {                                                                     \
         hipError_t e_ = (call);                                              \
         if (e_ != hipSuccess) {                                              \
+            (void)hipGetLastError(); /* or the next launch reports it */     \
             err = std::string(#call) + ": " + hipGetErrorString(e_);         \
             rc = e_ == hipErrorOutOfMemory ? -3 : -4;                        \
             goto done;                                                       \

@@ -135,6 +135,7 @@ double wall_ms() {
     do {                                                                                          \
         hipError_t e_ = (call);                                                                   \
         if (e_ != hipSuccess) {                                                                   \
+            (void)hipGetLastError(); /* or the next launch reports it again */                    \
             ctx->err = std::string(#call) + ": " + hipGetErrorString(e_);                         \
             return e_ == hipErrorOutOfMemory ? ISPAN_ERR_NOMEM : ISPAN_ERR_HIP;                   \
         }                                                                                         \
