@@ -175,7 +175,9 @@ int ispan_graph_bind_device(ispan_ctx* ctx, int32_t V, int64_t E, const int32_t*
 
 /* One SCC solve of the bound graph (scc_detection, src/scc_core.cpp:27-1094).
  * Labels stay on the device; d_labels (int32[V], device) receives them when
- * not NULL.  stats may be NULL. */
+ * not NULL and the solve succeeds.  It may lie over the bound graph's arrays,
+ * which are read no more by then (a later solve needs the graph bound again).
+ * stats may be NULL. */
 int ispan_solve(ispan_ctx* ctx, const ispan_params* params, int32_t* d_labels, ispan_stats* stats);
 /* Copy the labels of the last solve to host memory (int32[V]). */
 int ispan_labels_download(ispan_ctx* ctx, int32_t* labels);

@@ -137,8 +137,8 @@ struct GiantArgs {
     int32_t V;
     int64_t nwords;
     int32_t* lab;
-    int32_t* lab2;            // optional second copy of the labels (the caller's array), complete when the
-                              // launch leaves nothing for the host (unl_checked)
+    int32_t* lab2;            // optional second copy of the labels (the caller's array), written when the
+                              // launch leaves nothing for the host (unl_checked), else untouched
     uint64_t* act;
     uint64_t* fvis;
     uint64_t* bvis;

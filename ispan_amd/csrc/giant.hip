@@ -2023,6 +2023,64 @@ __device__ __forceinline__ bool rest_phase(Ctx& c, int64_t fq0, int64_t n, int64
     return true;
 }
 
+// Labels of words [wb, we), the block's own: the giant's from its bitmap, the
+// vertices' own ids elsewhere, and for the vertices the giant phase left (a.act
+// then, a.snap later) -1 into the context's array, or, FINAL, what the
+// context's array says by then into the caller's.  One word per lane: a wave
+// loads its share of the words, up to 64 at once, then writes them four words
+// at a time, four consecutive labels a lane (coalesced 1 KB stores, no loads in
+// the loop but for the vertices left).  (64 whatever there are left the 43
+// words a block of 700 K vertices to one wave: 162 us a solve against 154.)
+//
+// The caller's array is written at the very end, when no barrier is left that
+// could fail and nobody reads the graph any more: it stays as it was if the
+// solve fails, and may lie over the graph's arrays.  (A copy after the launch
+// instead reads and writes the labels once more and costs another host wait:
+// R-MAT s24 403 -> 387 us, 700 K vertices 203 -> 190 us.)
+template <bool FINAL>
+__device__ __forceinline__ void write_labels(Ctx& c, int64_t wb, int64_t we, bool traversed, int32_t gmin) {
+    KernelArgs& a = c.args();
+    const bool multi = a.n_roots > 0;
+    int32_t* lab = FINAL ? a.lab2 : a.lab;
+    const uint64_t* left = FINAL ? a.snap : a.act;
+    const bool wide = (reinterpret_cast<uintptr_t>(lab) & 15) == 0;
+    const int share = (int)min(((we - wb + kW - 1) / kW + 3) & ~(int64_t)3, (int64_t)kWave);
+    for (int64_t base = wb + (int64_t)c.wave * share; base < we; base += (int64_t)kW * share) {
+        const int64_t w = base + c.lane;
+        uint64_t ac = 0, g = 0, sw = 0;
+        if (w < we) {
+            ac = left[w];
+            g = traversed ? a.bvis[w] : 0ull;
+            sw = a.sel ? a.sel[w] : ~0ull;  // unselected vertices keep whatever label they had
+        }
+        const int nw = (int)min<int64_t>(share, we - base);
+        const int q = (c.lane & 15) * 4;  // this lane's first bit in its word
+        for (int j = 0; j < nw; j += 4) {
+            const int src = j + (c.lane >> 4);  // this lane's word in the group of four
+            const uint64_t aj = lane_from(ac, src), gj = lane_from(g, src), sj = lane_from(sw, src);
+            if (src >= nw) continue;
+            const int64_t v0 = (base + src) * 64 + q;
+            int32_t l[4];
+            bool all = v0 + 3 < a.V;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int64_t v = v0 + k;
+                const bool gi = (gj >> (q + k)) & 1ull, rest = (aj >> (q + k)) & 1ull;
+                l[k] = gi ? (multi ? (int32_t)v : gmin) : (rest ? -1 : (int32_t)v);
+                if (FINAL && !gi && rest) l[k] = a.lab[v];
+                all = all && ((sj >> (q + k)) & 1ull);
+            }
+            if (all && wide) {
+                st_agent4(&lab[v0], l[0], l[1], l[2], l[3]);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (v0 + k < a.V && ((sj >> (q + k)) & 1ull)) st_agent(&lab[v0 + k], l[k]);
+            }
+        }
+    }
+}
+
 }  // namespace
 
 __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs) {
@@ -2238,52 +2296,8 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs) {
     const int64_t giant = lane_get(sm.tot[0][1], 0);
     const int64_t w0 = sm.tot[0][3], w1 = sm.tot[0][4], w2 = sm.tot[0][5], w3 = sm.tot[0][6];
     if (a.trace && c.tid == 0) atomicMax((unsigned long long*)&gs->post_cp[1], (unsigned long long)wall_clock64());
-    // the labels, here and in the caller's array when it gave one (a copy of
-    // its own after the launch reads and writes them once more and costs
-    // another host wait: R-MAT s24 403 -> 387 us, 700 K vertices 203 -> 190 us):
-    // one word per lane, the wave loads 64 words at once (its own
-    // block's, narrowed above), then writes them four words at a time, four
-    // consecutive labels a lane (coalesced 1 KB stores, no loads in the loop)
-    const bool wide2 = a.lab2 && (reinterpret_cast<uintptr_t>(a.lab2) & 15) == 0;
-    for (int64_t base = wb + (int64_t)c.wave * kWave; base < we; base += (int64_t)kW * kWave) {
-        const int64_t w = base + c.lane;
-        uint64_t ac = 0, g = 0, sw = 0;
-        if (w < we) {
-            ac = a.act[w];
-            g = traversed ? a.bvis[w] : 0ull;
-            sw = a.sel ? a.sel[w] : ~0ull;  // unselected vertices keep whatever label they had
-        }
-        const int nw = (int)min<int64_t>(kWave, we - base);
-        const int q = (c.lane & 15) * 4;  // this lane's first bit in its word
-        for (int j = 0; j < nw; j += 4) {
-            const int src = j + (c.lane >> 4);  // this lane's word in the group of four
-            const uint64_t aj = lane_from(ac, src), gj = lane_from(g, src), sj = lane_from(sw, src);
-            if (src >= nw) continue;
-            const int64_t v0 = (base + src) * 64 + q;
-            int32_t l[4];
-            bool all = v0 + 3 < a.V;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int64_t v = v0 + k;
-                const bool gi = (gj >> (q + k)) & 1ull, act_v = (aj >> (q + k)) & 1ull;
-                l[k] = gi ? (multi ? (int32_t)v : gmin) : (act_v ? -1 : (int32_t)v);
-                all = all && ((sj >> (q + k)) & 1ull);
-            }
-            if (all) {
-                st_agent4(&a.lab[v0], l[0], l[1], l[2], l[3]);
-                if (wide2) st_agent4(&a.lab2[v0], l[0], l[1], l[2], l[3]);
-            } else {
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (v0 + k < a.V && ((sj >> (q + k)) & 1ull)) st_agent(&a.lab[v0 + k], l[k]);
-            }
-            if (a.lab2 && !(all && wide2)) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (v0 + k < a.V && ((sj >> (q + k)) & 1ull)) st_agent(&a.lab2[v0 + k], l[k]);
-            }
-        }
-    }
+    // the labels; the vertices left get theirs later
+    write_labels<false>(c, wb, we, traversed, gmin);
     // this block's slice of the queue, the active vertices of its own words.
     // The first trim sweep takes it alone (no barrier before it): a sweep
     // clears act bits only of the vertices it sweeps, so no block's sweep
@@ -2337,9 +2351,7 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs) {
                 uint64_t m = a.snap[w];
                 while (m) {
                     const int64_t v = w * 64 + __ffsll((unsigned long long)m) - 1;
-                    const int32_t l = a.lab[v];
-                    left += l < 0;
-                    if (a.lab2) st_agent(&a.lab2[v], l);  // the rest phase's labels
+                    left += a.lab[v] < 0;
                     m &= m - 1;
                 }
             }
@@ -2348,6 +2360,7 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs) {
                 if (left) atomicAdd(reinterpret_cast<unsigned long long*>(&gs->unlabelled), (unsigned long long)left);
                 if (c.b == 0) gs->unl_checked = 1;
             }
+            if (a.lab2) write_labels<true>(c, wb, we, traversed, gmin);
         }
         if (stamp) gs->ts[5] = wall_clock64();
     }

@@ -415,6 +415,23 @@ int coop_blocks(const ispan_ctx* ctx) {
     return ctx->V <= kHalfGridV ? std::max(ctx->coop_grid / 2, 1) : ctx->coop_grid;
 }
 
+// May a kernel write V labels at p?  Memory of this device, aligned, and known
+// to go on for V labels.  Any other array gets a copy at the end, which the
+// runtime checks.
+bool holds_labels(const ispan_ctx* ctx, int32_t* p, int32_t V) {
+    if (!p || (reinterpret_cast<uintptr_t>(p) & 3)) return false;
+    hipPointerAttribute_t at{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess || at.type != hipMemoryTypeDevice || at.device != ctx->device ||
+        hipMemGetAddressRange(&base, &size, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const size_t before = (size_t)(reinterpret_cast<char*>(p) - static_cast<char*>(base));
+    return before <= size && (size_t)V * 4 <= size - before;
+}
+
 int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_stats* st) {
     const double t0 = wall_ms();
     hipStream_t s = ctx->stream;
@@ -465,16 +482,7 @@ int solve_impl(ispan_ctx* ctx, const ispan_params* P, int32_t* d_labels, ispan_s
         ga.V = V;
         ga.nwords = ctx->nwords;
         ga.lab = ctx->lab;
-        // the caller's array in this device's memory is written along with
-        // the context's; any other kind gets a copy at the end
-        if (d_labels && d_labels != ctx->lab) {
-            hipPointerAttribute_t at{};
-            if (hipPointerGetAttributes(&at, d_labels) == hipSuccess) {
-                if (at.type == hipMemoryTypeDevice && at.device == ctx->device) ga.lab2 = d_labels;
-            } else {
-                (void)hipGetLastError();
-            }
-        }
+        if (d_labels != ctx->lab && holds_labels(ctx, d_labels, V)) ga.lab2 = d_labels;
         ga.act = ctx->act;
         ga.fvis = ctx->fvis;
         ga.bvis = ctx->bvis;
