@@ -160,7 +160,7 @@ __device__ __forceinline__ void begin_rows(const Rows& R, int32_t r0, int32_t r1
         const int32_t lo = __builtin_amdgcn_readlane(r0, l) + 1 + kLaneRows, hi = __builtin_amdgcn_readlane(r1, l);
         const int32_t p = __builtin_amdgcn_readlane(pos, l);
         if (hi - lo < kGapRows) {
-            for (int32_t v = lo + lane; v <= hi; v += 64) R.beg[v] = p;
+            for (int32_t k = lane; k <= hi - lo; k += 64) R.beg[lo + k] = p;  // hi + 64 may be past int32
         } else if (lane == 0) {
             const int32_t pieces = (int32_t)(((int64_t)hi - lo + kGapRows) / kGapRows);
             const int32_t at = atomicAdd(R.n_gaps, pieces);
