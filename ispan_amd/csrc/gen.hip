@@ -131,9 +131,14 @@ __global__ void k_pack(const int32_t* __restrict__ src, const int32_t* __restric
 // bound by its scattered probes: 60 us for 2^20 rows over 16 M keys, twice a
 // build.)  A lane writes up to kLaneRows rows itself, the wave the rest of a
 // gap, and a gap of more than kGapRows rows is cut into pieces that k_gaps
-// fills, one block each, so that a hole in the ids does not hold up one wave.
+// fills, one block each, so that a hole in the ids does not hold up one wave:
+// of kGapRows rows, or in a large gap of so many that there are kGapPieces.
+// (2 x 10^9 rows, one key: 36.0 ms of kernels with one lane listing 490,000
+// pieces, 3.3 now; a search per row took 3.2.  Of 1,000 keys: 33.8, 5.1, 17.9.)
 constexpr int kLaneRows = 4;
 constexpr int kGapRows = 4096;
+constexpr int kGapPieces = 8192;
+constexpr int kGapBlocks = 2048;
 struct Gap {
     int32_t lo, n, pos;
 };
@@ -161,11 +166,15 @@ __device__ __forceinline__ void begin_rows(const Rows& R, int32_t r0, int32_t r1
         const int32_t p = __builtin_amdgcn_readlane(pos, l);
         if (hi - lo < kGapRows) {
             for (int32_t k = lane; k <= hi - lo; k += 64) R.beg[lo + k] = p;  // hi + 64 may be past int32
-        } else if (lane == 0) {
-            const int32_t pieces = (int32_t)(((int64_t)hi - lo + kGapRows) / kGapRows);
-            const int32_t at = atomicAdd(R.n_gaps, pieces);
-            for (int32_t k = 0; k < pieces; ++k)
-                R.gaps[at + k] = Gap{lo + k * kGapRows, min(kGapRows, hi - lo + 1 - k * kGapRows), p};
+        } else {
+            const int32_t rows = hi - lo + 1;
+            const int32_t size = max(kGapRows, (rows / kGapPieces | 63) + 1);
+            const int32_t pieces = (int32_t)(((int64_t)rows + size - 1) / size);
+            int32_t at = 0;
+            if (lane == 0) at = atomicAdd(R.n_gaps, pieces);
+            at = __builtin_amdgcn_readfirstlane(at);
+            for (int32_t k = lane; k < pieces; k += 64)
+                R.gaps[at + k] = Gap{lo + k * size, min(size, rows - k * size), p};
         }
     }
 }
@@ -174,24 +183,40 @@ __global__ void k_gaps(Rows R) {
     const int32_t n = *R.n_gaps;
     for (int32_t g = blockIdx.x; g < n; g += gridDim.x) {
         const Gap x = R.gaps[g];
-        for (int32_t k = threadIdx.x; k < x.n; k += blockDim.x) R.beg[x.lo + k] = x.pos;
+        const int32_t head = min(x.n, (4 - (x.lo & 3)) & 3), quads = (x.n - head) / 4, tail = head + quads * 4;
+        int32_t* beg = R.beg + x.lo;
+        int4* wide = reinterpret_cast<int4*>(beg + head);  // the array starts aligned
+        const int t = threadIdx.x;
+        if (t < head) beg[t] = x.pos;
+        if (t < x.n - tail) beg[tail + t] = x.pos;
+        for (int32_t k = t; k < quads; k += blockDim.x) wide[k] = int4{x.pos, x.pos, x.pos, x.pos};
     }
 }
 
 // Sorted keys -> kept keys (the first of equal ones, no self-loops).  A wave
-// owns kKeepChunk consecutive keys; k_keep_count counts what each keeps, and
+// owns a chunk of consecutive keys; k_keep_count counts what each keeps, and
 // after a prefix sum over the chunks k_keep writes them in order, with their
 // low halves as the adjacency, and the row offsets.  Bound by memory: two
 // reads of the keys and one write.
+//
+// A chunk has kKeepChunk keys, or fewer (in whole steps of 64) where that would
+// be less than kKeepFull chunks: with few keys over many rows the waves are
+// needed for the rows (2^24 rows, 70,000 keys: 777 us of kernels with 1024
+// keys a wave, 201 with 64, 463 with a search per row).
 constexpr int kKeepChunk = 1024;
+constexpr int kKeepFull = 2048;
 constexpr int kKeepWaves = 4;
+int keep_chunk(int64_t m) {
+    return (int)std::max<int64_t>(64, std::min<int64_t>(kKeepChunk, (m / kKeepFull + 63) & ~(int64_t)63));
+}
 
 // f(valid, key, keep, previous key) for the 64 keys of every step.
 template <class K, class F>
-__device__ __forceinline__ void each_key(const K* __restrict__ keys, int64_t m, int bits, int64_t chunk, F&& f) {
+__device__ __forceinline__ void each_key(const K* __restrict__ keys, int64_t m, int bits, int per, int64_t chunk,
+                                         F&& f) {
     const int lane = threadIdx.x & 63;
     const K low = ((K)1 << bits) - 1;
-    const int64_t i0 = chunk * kKeepChunk, i1 = min(i0 + kKeepChunk, m);
+    const int64_t i0 = chunk * per, i1 = min(i0 + per, m);
     for (int64_t ib = i0; ib < i1; ib += 64) {
         const int64_t i = ib + lane;
         const bool valid = i < i1;
@@ -201,17 +226,17 @@ __device__ __forceinline__ void each_key(const K* __restrict__ keys, int64_t m, 
 }
 
 template <class K>
-__global__ __launch_bounds__(64 * kKeepWaves) void k_keep_count(const K* __restrict__ keys, int64_t m, int bits,
+__global__ __launch_bounds__(64 * kKeepWaves) void k_keep_count(const K* __restrict__ keys, int64_t m, int bits, int per,
                                                                 int64_t chunks, int32_t* __restrict__ counts) {
     for (int64_t c = (int64_t)blockIdx.x * kKeepWaves + threadIdx.x / 64; c < chunks; c += (int64_t)gridDim.x * kKeepWaves) {
         int n = 0;
-        each_key<K>(keys, m, bits, c, [&](int64_t, bool, K, bool keep, K) { n += __popcll(__ballot(keep)); });
+        each_key<K>(keys, m, bits, per, c, [&](int64_t, bool, K, bool keep, K) { n += __popcll(__ballot(keep)); });
         if ((threadIdx.x & 63) == 0) counts[c] = n;
     }
 }
 
 template <class K>
-__global__ __launch_bounds__(64 * kKeepWaves) void k_keep(const K* __restrict__ keys, int64_t m, int bits,
+__global__ __launch_bounds__(64 * kKeepWaves) void k_keep(const K* __restrict__ keys, int64_t m, int bits, int per,
                                                           int64_t chunks, const int64_t* __restrict__ start,
                                                           K* __restrict__ kept, int32_t* __restrict__ adj, Rows R,
                                                           int32_t V) {
@@ -219,7 +244,7 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(const K* __restrict__ 
     const K low = ((K)1 << bits) - 1;
     for (int64_t c = (int64_t)blockIdx.x * kKeepWaves + threadIdx.x / 64; c < chunks; c += (int64_t)gridDim.x * kKeepWaves) {
         int64_t p = start[c];
-        each_key<K>(keys, m, bits, c, [&](int64_t i, bool valid, K k, bool keep, K before) {
+        each_key<K>(keys, m, bits, per, c, [&](int64_t i, bool valid, K k, bool keep, K before) {
             const uint64_t mask = __ballot(keep);
             const int64_t q = p + __popcll(mask & ((1ull << lane) - 1));
             if (keep) {
@@ -237,12 +262,12 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(const K* __restrict__ 
 
 // Kept keys in (dst, src) order -> the transposed rows.
 template <class K>
-__global__ __launch_bounds__(64 * kKeepWaves) void k_transposed(const K* __restrict__ keys, int64_t E, int bits,
+__global__ __launch_bounds__(64 * kKeepWaves) void k_transposed(const K* __restrict__ keys, int64_t E, int bits, int per,
                                                                 int64_t chunks, int32_t* __restrict__ adj, Rows R,
                                                                 int32_t V) {
     const K low = ((K)1 << bits) - 1;
     for (int64_t c = (int64_t)blockIdx.x * kKeepWaves + threadIdx.x / 64; c < chunks; c += (int64_t)gridDim.x * kKeepWaves)
-        each_key<K>(keys, E, bits, c, [&](int64_t i, bool valid, K k, bool, K before) {
+        each_key<K>(keys, E, bits, per, c, [&](int64_t i, bool valid, K k, bool, K before) {
             if (valid) adj[i] = (int32_t)(k >> bits);
             const int32_t row = (int32_t)(k & low);
             begin_rows(R, i == 0 ? -1 : (int32_t)(before & low), valid ? row : -1, (int32_t)i);
@@ -295,10 +320,12 @@ struct BuildMem {
     int64_t* start;  // first kept position of every chunk, then their total
     Gap* gaps;
     int32_t* n;
+    int per;  // keys a chunk
     int64_t chunks;
 
     BuildMem(void* base, int32_t V, int64_t m, size_t* bytes = nullptr) {
-        chunks = (m + kKeepChunk - 1) / kKeepChunk;
+        per = keep_chunk(m);
+        chunks = (m + per - 1) / per;
         size_t off = 0;
         auto take = [&](size_t size) {
             char* p = static_cast<char*>(base) + off;
@@ -338,6 +365,7 @@ int csr_from_keys(hipStream_t s, Workspace& sort, const BuildMem<K>& M, int32_t 
                   int32_t** fwa, int32_t** bwb, int32_t** bwa, int64_t* E_out, std::string& err) {
     int rc = 0;
     const int bits = id_bits(V);
+    const int per = M.per;
     const int64_t chunks = M.chunks;
     const int keep_grid = (int)std::max<int64_t>(1, std::min<int64_t>(kGrid, (chunks + kKeepWaves - 1) / kKeepWaves));
     size_t b1 = 0, b2 = 0;
@@ -351,7 +379,7 @@ int csr_from_keys(hipStream_t s, Workspace& sort, const BuildMem<K>& M, int32_t 
         b1 = b2 = sort.cap;
         GK(rocprim::radix_sort_keys<KeySort>(sort.p, b1, buf, (size_t)m, 0, 2 * bits, s));
         hipLaunchKernelGGL(k_keep_count<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), m, bits,
-                           chunks, M.counts);
+                           per, chunks, M.counts);
         GK(hipGetLastError());
         // one entry more than chunks: the last start is the total (the last
         // count is not read into it)
@@ -372,10 +400,10 @@ int csr_from_keys(hipStream_t s, Workspace& sort, const BuildMem<K>& M, int32_t 
     if (E > 0) {
         K* kept = buf.alternate();
         Rows R{*fwb, M.gaps, M.n};
-        hipLaunchKernelGGL(k_keep<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), m, bits, chunks,
+        hipLaunchKernelGGL(k_keep<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), m, bits, per, chunks,
                            M.start, kept, *fwa, R, V);
         GK(hipGetLastError());
-        hipLaunchKernelGGL(k_gaps, dim3(256), dim3(256), 0, s, R);
+        hipLaunchKernelGGL(k_gaps, dim3(kGapBlocks), dim3(256), 0, s, R);
         GK(hipGetLastError());
         buf = rocprim::double_buffer<K>(kept, buf.current());
         // fewer keys can take another of the sort's methods, with more scratch
@@ -385,10 +413,10 @@ int csr_from_keys(hipStream_t s, Workspace& sort, const BuildMem<K>& M, int32_t 
         GK(rocprim::radix_sort_keys<KeySort>(sort.p, b1, buf, (size_t)E, 0, bits, s));
         R.beg = *bwb;
         R.n_gaps = M.n + 1;
-        hipLaunchKernelGGL(k_transposed<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), E, bits,
-                           (E + kKeepChunk - 1) / kKeepChunk, *bwa, R, V);
+        hipLaunchKernelGGL(k_transposed<K>, dim3(keep_grid), dim3(64 * kKeepWaves), 0, s, buf.current(), E, bits, per,
+                           (E + per - 1) / per, *bwa, R, V);
         GK(hipGetLastError());
-        hipLaunchKernelGGL(k_gaps, dim3(256), dim3(256), 0, s, R);
+        hipLaunchKernelGGL(k_gaps, dim3(kGapBlocks), dim3(256), 0, s, R);
         GK(hipGetLastError());
     } else {
         GK(launch_fill_i32(*fwb, 0, (int64_t)V + 1, kGrid, s));
