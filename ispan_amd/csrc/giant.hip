@@ -1630,13 +1630,16 @@ __device__ __forceinline__ int32_t key_colour(uint64_t k) { return (int32_t)(uin
 // edges of a graph with local ids stay inside it.  sweep() returns what this
 // thread changed; the sum over the sweeps comes back.
 constexpr int kBlockSweeps = 16;
-// From this many edges a vertex a block sweeps once: its sweep takes longer
-// than a grid barrier, and most of what it waits for is in other blocks.
-// Once against up to 16 times, random DAGs: of 20,000 vertices and 34, 50 and
-// 198 edges each 21.0 / 21.9, 37.4 / 39.0 and 308 / 337 ms, of 5,000 and 59
-// 25.6 / 27.0; with at most 30 edges no block is held to one.  A limit on a
-// sweep's time instead (30 us) took 16.0 ms for 8.6 with 20 edges.
-constexpr int kBlockSweepsDeg = 32;
+// With more vertices than this for each thread of the grid, a block sweeps
+// once: its sweep takes longer than the grid barrier it saves, and with many
+// vertices most edges lead out of the block's slices.  Up to 16 times against
+// once: random DAGs of 4-cycles, 3 M vertices 67 / 46 ms, 1 M with 6 edges each
+// 55 / 46, 200,000 with 20 edges 96 / 96; edges to the next 12 ids, 4 M vertices
+// 1.81 / 1.15 s, 1 M 0.27 / 0.18, 300,000 34.9 / 46.2 ms, 20,000 with 2 edges
+// 1.95 / 2.11.  The rule is the same for all blocks on purpose: where some
+// sweep once and some 16 times (by their own lists, or by a time limit), the
+// former wait for the latter, 20,000 vertices with 20 edges each 86 for 46 ms.
+constexpr int kBlockSweepsPer = 2;
 template <class Sweep>
 __device__ __forceinline__ int block_sweeps(Ctx& c, bool one, int most, Sweep sweep) {
     int all = 0;
@@ -1695,8 +1698,12 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
     const int64_t gt = (int64_t)c.b * kGBlock + c.tid;
     auto buf = [&a](int k) { return k ? a.fq : a.fq_alt; };
     using ull = unsigned long long;
-    constexpr int kAhead = 4;  // list entries whose keys or stamps are read together
-    const bool dense = a.fwb[a.V] >= (int64_t)kBlockSweepsDeg * a.V;
+    // List entries whose keys or stamps are read together.  They come from past
+    // the L2, the active bits mostly from it, and after the first rounds most
+    // entries are active no more: only those that are get read.  (All of them
+    // at once, which saves the bits' round trip: random DAGs of 20,000 and 1 M
+    // vertices with 20 and 6 edges each 46 and 73 ms, 39 and 47 this way.)
+    constexpr int kAhead = 4;
     {  // degree rank, once, into parent
         const int32_t* q = buf(cur);
         for (int64_t i = gt; i < n; i += nthreads) {
@@ -1711,7 +1718,7 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
     for (rounds = 1;; ++rounds) {
         const bool one = n <= kGBlock;
         if (one && c.b != 0) return true;
-        const int most = dense && !one ? 1 : kBlockSweeps;
+        const int most = n > kBlockSweepsPer * nthreads ? 1 : kBlockSweeps;
         const int32_t* q = buf(cur);
         int32_t* qn = buf(cur ^ 1);
         int32_t* cnt = &gs->fqn[s % 3].v;  // last read three rounds (or sweeps) ago
@@ -1733,14 +1740,16 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
                     const int32_t end = a.bwb[v + 1];
                     for (int32_t e = a.bwb[v]; e < end; e += kAhead) {
                         int32_t w[kAhead];
+                        bool on[kAhead];
                         uint64_t kw[kAhead];
 #pragma unroll
                         for (int j = 0; j < kAhead; ++j) w[j] = a.bwa[min(e + j, end - 1)];
 #pragma unroll
-                        for (int j = 0; j < kAhead; ++j) kw[j] = load_agent(&a.ckey[w[j]]);
+                        for (int j = 0; j < kAhead; ++j) on[j] = e + j < end && w[j] != v && bit_of(a.act, w[j]);
 #pragma unroll
-                        for (int j = 0; j < kAhead; ++j)
-                            if (w[j] != v && bit_of(a.act, w[j])) k = max(k, kw[j]);
+                        for (int j = 0; j < kAhead; ++j) kw[j] = on[j] ? load_agent(&a.ckey[w[j]]) : 0;
+#pragma unroll
+                        for (int j = 0; j < kAhead; ++j) k = max(k, kw[j]);
                     }
                     for (int hop = 0; hop < 100; ++hop) {  // the colour's own key, and so on
                         const uint64_t kc = load_agent(&a.ckey[key_colour(k)]);
@@ -1779,14 +1788,16 @@ __device__ __forceinline__ bool colour_scc(Ctx& c, int& cur, int64_t n, int s, i
                     const int32_t end = a.fwb[v + 1];
                     for (int32_t e = a.fwb[v]; e < end; e += kAhead) {
                         int32_t u[kAhead], su[kAhead];
+                        bool on[kAhead];
 #pragma unroll
                         for (int j = 0; j < kAhead; ++j) u[j] = a.fwa[min(e + j, end - 1)];
 #pragma unroll
-                        for (int j = 0; j < kAhead; ++j) su[j] = load_agent(&a.stamp[u[j]]);
+                        for (int j = 0; j < kAhead; ++j) on[j] = e + j < end && u[j] != v && bit_of(a.act, u[j]);
+#pragma unroll
+                        for (int j = 0; j < kAhead; ++j) su[j] = on[j] ? load_agent(&a.stamp[u[j]]) : -1;
                         bool join = false;
 #pragma unroll
-                        for (int j = 0; j < kAhead; ++j)
-                            join = join || (su[j] == r && u[j] != v && bit_of(a.act, u[j]));
+                        for (int j = 0; j < kAhead; ++j) join = join || su[j] == r;
                         if (join) {
                             st_agent(&a.stamp[v], r);
                             ++ch;
