@@ -306,8 +306,8 @@ struct PivotFold {
 };
 
 // Totals of every word but word 2, whose largest value is taken, into
-// sm.tot[0][0..6], and into sm.tot[0][7] the sum of word 0 over the blocks before
-// this one (word 7 carries nothing).
+// sm.tot[0], and into sm.tot[1][0] the sum of word 0 over the blocks before
+// this one.
 struct PostFold {
     int b;
     uint64_t s = 0, pre = 0;
@@ -319,8 +319,8 @@ struct PostFold {
         const bool mx = (lane_id() & 7) == 2;
         s = fold_lanes<8>(s, [mx](uint64_t p, uint64_t q) { return mx ? max(p, q) : p + q; });
         pre = fold_lanes<8>(pre, [](uint64_t p, uint64_t q) { return p + q; });
-        if (lane_id() < 7) sm.tot[0][lane_id()] = (int64_t)s;
-        if (lane_id() == 0) sm.tot[0][7] = (int64_t)pre;
+        if (lane_id() < 8) sm.tot[0][lane_id()] = (int64_t)s;
+        if (lane_id() == 0) sm.tot[1][0] = (int64_t)pre;
     }
 };
 
@@ -2289,8 +2289,12 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs) {
     const int wmn = wave_min(mn);
     const uint32_t key = wmn < INT32_MAX ? (uint32_t)(INT32_MAX - wmn) : 0u;
     if (a.trace && c.tid == 0) atomicMax((unsigned long long*)&gs->post_cp[0], (unsigned long long)wall_clock64());
+    // (vertices, and entries read top-down, once each: a block's fit 32 bits;
+    // bottom-up levels read lists again and again, so that count goes in two)
+    constexpr int kLowBits = 20;
     stage_words<8>(c, {(uint32_t)wave_sum((int)cnt), (uint32_t)wave_sum((int)gcnt), key, (uint32_t)c.edges_td,
-                       (uint32_t)c.edges_bu, (uint32_t)c.found_td, (uint32_t)c.found_bu, 0});
+                       (uint32_t)c.edges_bu & ((1u << kLowBits) - 1), (uint32_t)c.found_td, (uint32_t)c.found_bu,
+                       (uint32_t)(c.edges_bu >> kLowBits)});
     {
         PostFold f{c.b};
         auto src = [&]() {
@@ -2302,10 +2306,9 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs) {
         if (!gsync_with<8, true>(c, src, f)) return;
     }
     if (want_min) gmin = (int32_t)((int64_t)INT32_MAX - lane_get(sm.tot[0][2], 0));
-    int64_t off = lane_get(sm.tot[0][7], 0);  // active vertices of the blocks before this one
+    int64_t off = lane_get(sm.tot[1][0], 0);  // active vertices of the blocks before this one
     const int64_t tot = lane_get(sm.tot[0][0], 0);
     const int64_t giant = lane_get(sm.tot[0][1], 0);
-    const int64_t w0 = sm.tot[0][3], w1 = sm.tot[0][4], w2 = sm.tot[0][5], w3 = sm.tot[0][6];
     if (a.trace && c.tid == 0) atomicMax((unsigned long long*)&gs->post_cp[1], (unsigned long long)wall_clock64());
     // the labels; the vertices left get theirs later
     write_labels<false>(c, wb, we, traversed, gmin);
@@ -2340,10 +2343,10 @@ __global__ __launch_bounds__(kGBlock) void k_giant(const GiantArgs) {
             gs->fq_n = tot;
             gs->fw_levels = fw_levels;
             gs->bw_levels = bw_levels;
-            gs->work[0] = w0;
-            gs->work[1] = w1;
-            gs->work[2] = w2;
-            gs->work[3] = w3;
+            gs->work[0] = sm.tot[0][3];
+            gs->work[1] = sm.tot[0][4] + (sm.tot[0][7] << kLowBits);
+            gs->work[2] = sm.tot[0][5];
+            gs->work[3] = sm.tot[0][6];
             *a.fq_n_out = (int32_t)tot;
             gs->ts[4] = wall_clock64();
         }
