@@ -978,7 +978,9 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
     int32_t* qn_out = &gs->qn[dir][(L + 1) % 3].v;
     int32_t* hn_out = &gs->hn[dir][(L + 1) % 3].v;
     const bool topdown = mode != 1;
-    const bool tr = a.trace && L < kLevelTrace;
+    // the level trace is kept by one thread of the block: of its part that has
+    // this direction, where each direction has half of the waves
+    const bool tr = a.trace && L < kLevelTrace && c.tid % (wpb * kWave) == 0;
     const int64_t tl0 = tr ? (int64_t)wall_clock64() : 0;
     if (topdown && gather) {
         // ---- the first top-down level after bottom-up ones: each wave takes
@@ -1278,7 +1280,7 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
                     my_found += hit;
                 }
             }
-            if (tr && c.tid == 0 && cb == 0)
+            if (tr && cb == 0)
                 atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_cp[dir][L][3]),
                           (unsigned long long)((int64_t)wall_clock64() - tl0));
             // sparse words: each lane works through its own word's
@@ -1318,11 +1320,11 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
             if (fm_lane) atomicOr(reinterpret_cast<unsigned long long*>(vis + wl), (unsigned long long)fm_lane);
             if (wl < a.nwords) st_agent(&snap[wl], lvw);  // the gather's "visited before this level"
         }
-        if (tr && c.tid == 0)  // wave 0 of each block
+        if (tr)
             atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_cp[dir][L][1]),
                       (unsigned long long)((int64_t)wall_clock64() - tl0));
         scan_misses();
-        if (tr && c.tid == 0)
+        if (tr)
             atomicMax(reinterpret_cast<unsigned long long*>(&gs->lv_cp[dir][L][2]),
                       (unsigned long long)((int64_t)wall_clock64() - tl0));
         lv = Level{(int)my_found, scanned, 0, 0};  // bottom-up pushes nothing
@@ -1429,7 +1431,7 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
                 using ull = unsigned long long;
                 if (c.edges_td > edges0)
                     atomicAdd(reinterpret_cast<ull*>(&gs->lv_edges[dir][L]), (ull)(c.edges_td - edges0));
-                if (c.tid == 0) {  // wave 0 of each block
+                if (c.wave % (half ? kW / 2 : kW) == 0) {  // the direction's first wave of each block
                     const ull wt = (ull)((int64_t)wall_clock64() - tl0);
                     if (!td) atomicMax(reinterpret_cast<ull*>(&gs->lv_cp[dir][L][0]), (ull)(uint32_t)lv.edges);
                     atomicMax(reinterpret_cast<ull*>(&gs->lv_wmax[dir][L]), wt);
