@@ -75,7 +75,8 @@ struct Workspace {
         cap = 0;
     }
 };
-// A graph builder's scratch beyond this is given back when the call ends.
+// A graph builder's scratch (keys and sort together) beyond this is given back
+// when the call ends, and what is kept when another allocation finds no room.
 constexpr size_t kKeepScratch = (size_t)1 << 30;
 
 // ---- cooperative giant-phase kernel (giant.hip) --------------------------

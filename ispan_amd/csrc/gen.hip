@@ -503,8 +503,10 @@ done:
             *p = nullptr;
         }
     }
-    if (w.m.cap > kKeepScratch) w.m.release();
-    if (w.sort.cap > kKeepScratch) w.sort.release();
+    if (w.m.cap + w.sort.cap > kKeepScratch) {
+        w.m.release();
+        w.sort.release();
+    }
     return rc;
 }
 

@@ -44,8 +44,8 @@ struct ispan_ctx {
     int64_t nwords = 0;
     int32_t* fw_first = nullptr;  // first out-/in-neighbour per vertex, built at bind
     int32_t* bw_first = nullptr;
-    Workspace first_mem;  // of a bound single graph's first arrays, kept from one graph to the next
-    Workspace gen_mem, gen_sort;  // the graph builders' scratch (gen.hip), kept up to kKeepScratch
+    Workspace first_mem;  // of a bound single graph's first arrays, kept from one single graph to the next
+    Workspace gen_mem, gen_sort;  // the graph builders' scratch (gen.hip), together kept up to kKeepScratch
 
     // solve state (capacity cap_V / cap_E), carved from solve_mem
     void* solve_mem = nullptr;
@@ -145,6 +145,45 @@ template <class T>
 void dfree(T*& p) {
     if (p) (void)hipFree((void*)p);
     p = nullptr;
+}
+
+// Gives back what the context only keeps for a later builder call; was there
+// anything?
+bool give_back(ispan_ctx* ctx) {
+    const bool some = ctx->gen_mem.p || ctx->gen_sort.p;
+    ctx->gen_mem.release();
+    ctx->gen_sort.release();
+    return some;
+}
+
+// A device allocation that fails only if there is no room without that either.
+template <class T>
+hipError_t dmalloc(ispan_ctx* ctx, T** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && give_back(ctx)) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
+int gen_rc(int rc) {
+    return rc == 0 ? ISPAN_OK : rc == -1 ? ISPAN_ERR_ARG : rc == -2 ? ISPAN_ERR_CSR : rc == -3 ? ISPAN_ERR_NOMEM
+                                                                                               : ISPAN_ERR_HIP;
+}
+
+// A builder's call on the scratch that the context keeps; once more without it
+// where that left too little room.
+template <class F>
+int with_scratch(ispan_ctx* ctx, F&& build) {
+    GenScratch w{ctx->gen_mem, ctx->gen_sort};
+    const bool kept = w.m.p || w.sort.p;
+    int rc = gen_rc(build(w));
+    if (rc == ISPAN_ERR_NOMEM && kept) {
+        give_back(ctx);
+        rc = gen_rc(build(w));
+    }
+    return rc;
 }
 
 // Buffers placed one after another from base, 256-byte aligned; without a
@@ -248,6 +287,12 @@ void free_graph(ispan_ctx* ctx) {
     ctx->have_solution = false;
 }
 
+// The same, and nothing is kept for a next single graph.
+void drop_graph(ispan_ctx* ctx) {
+    free_graph(ctx);
+    ctx->first_mem.release();
+}
+
 // One allocation for all of it: two dozen of their own cost a graph's first
 // solve more than the solve.
 int ensure_buffers(ispan_ctx* ctx, int32_t V, int64_t E) {
@@ -255,7 +300,7 @@ int ensure_buffers(ispan_ctx* ctx, int32_t V, int64_t E) {
     free_solve_buffers(ctx);
     Carve size{nullptr};
     carve_solve_state(ctx, size, V, E);
-    CK(hipMalloc(&ctx->solve_mem, size.off));
+    CK(dmalloc(ctx, &ctx->solve_mem, size.off));
     Carve place{static_cast<unsigned char*>(ctx->solve_mem)};
     carve_solve_state(ctx, place, V, E);
     ctx->cap_V = V;
@@ -911,7 +956,12 @@ int bind_common(ispan_ctx* ctx, int32_t V, int64_t E, const ispan_params* P) {
     ctx->E = E;
     ctx->nwords = ((int64_t)V + 63) / 64;
     const size_t nv = ((size_t)std::max(V, 1) + 63) & ~(size_t)63;
-    CK(ctx->first_mem.ensure(nv * 8));
+    hipError_t e = ctx->first_mem.ensure(nv * 8);
+    if (e == hipErrorOutOfMemory && give_back(ctx)) {
+        (void)hipGetLastError();
+        e = ctx->first_mem.ensure(nv * 8);
+    }
+    CK(e);
     ctx->fw_first = static_cast<int32_t*>(ctx->first_mem.p);
     ctx->bw_first = ctx->fw_first + nv;
     if (int rc = check_bound(ctx, P, true)) return rc;
@@ -1029,11 +1079,9 @@ int ispan_ctx_destroy(ispan_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     free_solve_buffers(ctx);
-    free_graph(ctx);
+    drop_graph(ctx);
     free_workspace(ctx);
-    ctx->first_mem.release();
-    ctx->gen_mem.release();
-    ctx->gen_sort.release();
+    give_back(ctx);
     dfree(ctx->ctl);
     dfree(ctx->gstate);
     dfree(ctx->bar);
@@ -1077,10 +1125,10 @@ int ispan_graph_upload(ispan_ctx* ctx, int32_t V, int64_t E, const int32_t* fw_b
     CK(hipSetDevice(ctx->device));
     free_graph(ctx);
     const size_t nb = ((size_t)V + 1) * 4, na = (size_t)std::max<int64_t>(E, 1) * 4;
-    CK(hipMalloc(&ctx->owned[0], nb));
-    CK(hipMalloc(&ctx->owned[1], na));
-    CK(hipMalloc(&ctx->owned[2], nb));
-    CK(hipMalloc(&ctx->owned[3], na));
+    CK(dmalloc(ctx, &ctx->owned[0], nb));
+    CK(dmalloc(ctx, &ctx->owned[1], na));
+    CK(dmalloc(ctx, &ctx->owned[2], nb));
+    CK(dmalloc(ctx, &ctx->owned[3], na));
     CK(hipMemcpyAsync(ctx->owned[0], fw_beg, nb, hipMemcpyHostToDevice, ctx->stream));
     CK(hipMemcpyAsync(ctx->owned[2], bw_beg, nb, hipMemcpyHostToDevice, ctx->stream));
     if (E > 0) {
@@ -1095,7 +1143,7 @@ int ispan_graph_upload(ispan_ctx* ctx, int32_t V, int64_t E, const int32_t* fw_b
     ispan_params d;
     ispan_default_params(&d);
     int rc = bind_common(ctx, V, E, params ? params : &d);
-    if (rc) free_graph(ctx);
+    if (rc) drop_graph(ctx);
     return rc;
 }
 
@@ -1112,7 +1160,7 @@ int ispan_graph_bind_device(ispan_ctx* ctx, int32_t V, int64_t E, const int32_t*
     ispan_params d;
     ispan_default_params(&d);
     int rc = bind_common(ctx, V, E, params ? params : &d);
-    if (rc) free_graph(ctx);
+    if (rc) drop_graph(ctx);
     return rc;
 }
 
@@ -1224,9 +1272,9 @@ int ranges_upload(ispan_ctx* ctx, BatchRanges& r, int32_t* capN, int64_t* capC, 
         dfree(r.vb);  // vb owns the packed block: vb, ve, cstart, out
         dfree(r.roots);
         dfree(r.gmin);
-        CK(hipMalloc(&r.vb, bytes));
-        CK(hipMalloc(&r.roots, m * 4));
-        CK(hipMalloc(&r.gmin, m * 4));
+        CK(dmalloc(ctx, &r.vb, bytes));
+        CK(dmalloc(ctx, &r.roots, m * 4));
+        CK(dmalloc(ctx, &r.gmin, m * 4));
         if (capN) *capN = n;
     }
     r.ve = r.vb + m;
@@ -1236,8 +1284,8 @@ int ranges_upload(ispan_ctx* ctx, BatchRanges& r, int32_t* capN, int64_t* capC, 
         dfree(r.cp);
         dfree(r.ci);
         const size_t c = (size_t)std::max<int64_t>(nc, 1);
-        CK(hipMalloc(&r.cp, c * 8));
-        CK(hipMalloc(&r.ci, c * 4));
+        CK(dmalloc(ctx, &r.cp, c * 8));
+        CK(dmalloc(ctx, &r.ci, c * 4));
         if (capC) *capC = nc;
     }
     CK(hipMemcpyAsync(r.vb, h, bytes, hipMemcpyHostToDevice, ctx->stream));
@@ -1307,8 +1355,8 @@ int batch_build(ispan_ctx* ctx, int32_t n, const int64_t* v_off, const int64_t* 
         }
         return rc == ISPAN_OK;
     };
-    if (!hip(hipMalloc(&d_off, (size_t)2 * (n + 1) * 8), "hipMalloc") ||
-        !hip(hipMalloc(&d_bad, 4), "hipMalloc") ||
+    if (!hip(dmalloc(ctx, &d_off, (size_t)2 * (n + 1) * 8), "hipMalloc") ||
+        !hip(dmalloc(ctx, &d_bad, 4), "hipMalloc") ||
         !hip(hipMemcpyAsync(d_off, v_off, (size_t)(n + 1) * 8, hipMemcpyHostToDevice, s), "hipMemcpyAsync") ||
         !hip(hipMemcpyAsync(d_off + n + 1, e_off, (size_t)(n + 1) * 8, hipMemcpyHostToDevice, s), "hipMemcpyAsync") ||
         !hip(hipMemsetAsync(d_bad, 0, 4, s), "hipMemsetAsync")) {
@@ -1316,7 +1364,7 @@ int batch_build(ispan_ctx* ctx, int32_t n, const int64_t* v_off, const int64_t* 
         dfree(d_bad);
         return rc;
     }
-    hip(hipMalloc(&ctx->batch_labels, (size_t)std::max<int64_t>(v_off[n], 1) * 4), "hipMalloc");
+    hip(dmalloc(ctx, &ctx->batch_labels, (size_t)std::max<int64_t>(v_off[n], 1) * 4), "hipMalloc");
     std::vector<int32_t> order(n);
     for (int32_t g = 0; g < n; ++g) order[g] = g;
     auto cls_of = [&](int32_t g) { return size_class(v_off[g + 1] - v_off[g]); };
@@ -1356,10 +1404,10 @@ int batch_build(ispan_ctx* ctx, int32_t n, const int64_t* v_off, const int64_t* 
             big = std::max(big, v_off[g + 1] - v_off[g]);
         }
         G.cls = size_class(big);
-        if (!hip(hipMalloc(&G.csr[0], nb), "hipMalloc") || !hip(hipMalloc(&G.csr[1], na), "hipMalloc") ||
-            !hip(hipMalloc(&G.csr[2], nb), "hipMalloc") || !hip(hipMalloc(&G.csr[3], na), "hipMalloc") ||
-            !hip(hipMalloc(&G.first[0], (size_t)std::max(G.V, 1) * 4), "hipMalloc") ||
-            !hip(hipMalloc(&G.first[1], (size_t)std::max(G.V, 1) * 4), "hipMalloc"))
+        if (!hip(dmalloc(ctx, &G.csr[0], nb), "hipMalloc") || !hip(dmalloc(ctx, &G.csr[1], na), "hipMalloc") ||
+            !hip(dmalloc(ctx, &G.csr[2], nb), "hipMalloc") || !hip(dmalloc(ctx, &G.csr[3], na), "hipMalloc") ||
+            !hip(dmalloc(ctx, &G.first[0], (size_t)std::max(G.V, 1) * 4), "hipMalloc") ||
+            !hip(dmalloc(ctx, &G.first[1], (size_t)std::max(G.V, 1) * 4), "hipMalloc"))
             break;
         if (contiguous) {
             if (!hip(launch_batch_union(fwb_cat, fwa_cat, bwb_cat, bwa_cat, d_off, d_off + n + 1, G.g0, G.ng, G.V,
@@ -1384,7 +1432,7 @@ int batch_build(ispan_ctx* ctx, int32_t n, const int64_t* v_off, const int64_t* 
             }
             // the previous group's union is built (its check below waited)
             dfree(d_perm);
-            if (!hip(hipMalloc(&d_perm, tab.size() * 8), "hipMalloc") ||
+            if (!hip(dmalloc(ctx, &d_perm, tab.size() * 8), "hipMalloc") ||
                 !hip(hipMemcpyAsync(d_perm, tab.data(), tab.size() * 8, hipMemcpyHostToDevice, s), "hipMemcpyAsync") ||
                 !hip(launch_batch_union_perm(fwb_cat, fwa_cat, bwb_cat, bwa_cat, d_perm, d_perm + m + 1,
                                              d_perm + 2 * (m + 1), d_perm + 3 * (m + 1),
@@ -1474,13 +1522,13 @@ int64_t solve_state_bytes(int64_t V, int64_t E) {
 int solve_arena(ispan_ctx* ctx, const ArenaView& av, int32_t n, const int64_t* vb, const int64_t* ve,
                 int32_t* const* out, const ispan_params* P, ispan_stats* st) {
     if (!ctx || n < 1 || av.V < 0) return ISPAN_ERR_ARG;
-    if (ctx->batch_n >= 0 || ctx->V >= 0) free_graph(ctx);
+    if (ctx->batch_n >= 0 || ctx->V >= 0) drop_graph(ctx);
     int rc = ranges_upload(ctx, ctx->ws_rb, &ctx->ws_capN, &ctx->ws_capC, n, vb, ve, out);
     if (rc) return rc;
     const int64_t nwords = ((int64_t)av.V + 63) / 64;
     if (nwords > ctx->sel_cap) {
         dfree(ctx->sel);
-        CK(hipMalloc(&ctx->sel, (size_t)std::max<int64_t>(nwords, 1) * 8));
+        CK(dmalloc(ctx, &ctx->sel, (size_t)std::max<int64_t>(nwords, 1) * 8));
         ctx->sel_cap = nwords;
     }
     CK(launch_batch_select(ctx->ws_rb, ctx->sel, nwords, ctx->stream));
@@ -1507,7 +1555,7 @@ int ispan_batch_bind_device(ispan_ctx* ctx, int32_t n_graphs, const int64_t* h_v
     }
     if (h_e_off[n_graphs] > 0 && (!d_fw_adj || !d_bw_adj)) return ISPAN_ERR_ARG;
     CK(hipSetDevice(ctx->device));
-    free_graph(ctx);
+    drop_graph(ctx);
     ispan_params d;
     ispan_default_params(&d);
     const int64_t cap = max_group_edges > 0 ? std::min<int64_t>(max_group_edges, INT32_MAX) : INT32_MAX;
@@ -1945,7 +1993,7 @@ int ispan_scc_histogram(ispan_ctx* ctx, int64_t* bins, int32_t n_bins, ispan_sum
     int64_t h[kHistSlots] = {0};
     if (ctx->V > 0) {
         CK(hipSetDevice(ctx->device));
-        if (!ctx->hist) CK(hipMalloc(&ctx->hist, sizeof(h)));
+        if (!ctx->hist) CK(dmalloc(ctx, &ctx->hist, sizeof(h)));
         // the mice queue buffer (int32[V + 1]) holds the sizes: the solve is over
         CK(launch_scc_histogram(ctx->lab, ctx->V, ctx->qbuf, ctx->hist, ctx->stream));
         CK(hipMemcpyAsync(h, ctx->hist, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
@@ -1966,27 +2014,23 @@ int ispan_scc_histogram(ispan_ctx* ctx, int64_t* bins, int32_t n_bins, ispan_sum
     return ISPAN_OK;
 }
 
-static int gen_rc(int rc) {
-    return rc == 0 ? ISPAN_OK : rc == -1 ? ISPAN_ERR_ARG : rc == -2 ? ISPAN_ERR_CSR : rc == -3 ? ISPAN_ERR_NOMEM
-                                                                                               : ISPAN_ERR_HIP;
-}
-
 int ispan_gen_rmat_device(ispan_ctx* ctx, int32_t V, double edge_factor, double a, double b, double c, uint64_t seed,
                           int32_t** d_fw_beg, int32_t** d_fw_adj, int32_t** d_bw_beg, int32_t** d_bw_adj, int64_t* E) {
     if (!ctx || !d_fw_beg || !d_fw_adj || !d_bw_beg || !d_bw_adj || !E) return ISPAN_ERR_ARG;
     CK(hipSetDevice(ctx->device));
-    GenScratch scratch{ctx->gen_mem, ctx->gen_sort};
-    return gen_rc(gen_rmat_device(ctx->stream, scratch, V, edge_factor, a, b, c, seed, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj,
-                                  E, ctx->err));
+    return with_scratch(ctx, [&](GenScratch& w) {
+        return gen_rmat_device(ctx->stream, w, V, edge_factor, a, b, c, seed, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj, E,
+                               ctx->err);
+    });
 }
 
 int ispan_gen_grid_device(ispan_ctx* ctx, int32_t n, double p_bidir, uint64_t seed, int32_t** d_fw_beg,
                           int32_t** d_fw_adj, int32_t** d_bw_beg, int32_t** d_bw_adj, int64_t* E) {
     if (!ctx || !d_fw_beg || !d_fw_adj || !d_bw_beg || !d_bw_adj || !E) return ISPAN_ERR_ARG;
     CK(hipSetDevice(ctx->device));
-    GenScratch scratch{ctx->gen_mem, ctx->gen_sort};
-    return gen_rc(
-        gen_grid_device(ctx->stream, scratch, n, p_bidir, seed, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj, E, ctx->err));
+    return with_scratch(ctx, [&](GenScratch& w) {
+        return gen_grid_device(ctx->stream, w, n, p_bidir, seed, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj, E, ctx->err);
+    });
 }
 
 int ispan_build_csr_device(ispan_ctx* ctx, int32_t V, int64_t m, const int32_t* d_src, const int32_t* d_dst,
@@ -1995,9 +2039,9 @@ int ispan_build_csr_device(ispan_ctx* ctx, int32_t V, int64_t m, const int32_t* 
     if (!ctx || (m > 0 && (!d_src || !d_dst)) || !d_fw_beg || !d_fw_adj || !d_bw_beg || !d_bw_adj || !E)
         return ISPAN_ERR_ARG;
     CK(hipSetDevice(ctx->device));
-    GenScratch scratch{ctx->gen_mem, ctx->gen_sort};
-    return gen_rc(build_csr_device(ctx->stream, scratch, V, m, d_src, d_dst, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj, E,
-                                   ctx->err));
+    return with_scratch(ctx, [&](GenScratch& w) {
+        return build_csr_device(ctx->stream, w, V, m, d_src, d_dst, d_fw_beg, d_fw_adj, d_bw_beg, d_bw_adj, E, ctx->err);
+    });
 }
 
 int ispan_kernel_profile_get(const ispan_ctx* ctx, ispan_kernel_profile* out) {
@@ -2097,16 +2141,18 @@ int ispan_convert_edge_list(ispan_ctx* ctx, const char* txt_path, const char* ou
     int32_t *d_src = nullptr, *d_dst = nullptr, *fb = nullptr, *fa = nullptr, *bb = nullptr, *ba = nullptr;
     int64_t E = m;
     std::vector<int32_t> h[4];
-    CK(hipMalloc(&d_src, (size_t)std::max<int64_t>(m, 1) * 4));
-    CK(hipMalloc(&d_dst, (size_t)std::max<int64_t>(m, 1) * 4));
+    CK(dmalloc(ctx, &d_src, (size_t)std::max<int64_t>(m, 1) * 4));
+    CK(dmalloc(ctx, &d_dst, (size_t)std::max<int64_t>(m, 1) * 4));
     if (m) {
         CK(hipMemcpy(d_src, src.data(), (size_t)m * 4, hipMemcpyHostToDevice));
         CK(hipMemcpy(d_dst, dst.data(), (size_t)m * 4, hipMemcpyHostToDevice));
     }
     if (clean) {
-        GenScratch scratch{ctx->gen_mem, ctx->gen_sort};
-        rc = gen_rc(build_csr_device(ctx->stream, scratch, V, m, d_src, d_dst, &fb, &fa, &bb, &ba, &E, ctx->err));
+        rc = with_scratch(ctx, [&](GenScratch& w) {
+            return build_csr_device(ctx->stream, w, V, m, d_src, d_dst, &fb, &fa, &bb, &ba, &E, ctx->err);
+        });
     } else {
+        give_back(ctx);  // it takes memory of its own
         rc = gen_rc(csr_stable_one(ctx->stream, V, m, d_src, d_dst, &fb, &fa, ctx->err));
         if (!rc) rc = gen_rc(csr_stable_one(ctx->stream, V, m, d_dst, d_src, &bb, &ba, ctx->err));
     }
