@@ -1,6 +1,8 @@
 """What a context keeps between calls: the builders' scratch up to 1 GiB in
 all, given back when something else needs the room, and nothing of a single
 graph once a batch is bound or a binding fails."""
+import time
+
 import numpy as np
 import pytest
 
@@ -13,8 +15,17 @@ MB = 1 << 20
 
 
 def free():
+    """Free device memory, once it has stopped growing: the driver clears what
+    was freed before it counts as free again."""
     H.synchronize()
-    return H.mem_info()[0]
+    last, since = H.mem_info()[0], time.monotonic()
+    end = since + 10
+    while time.monotonic() < min(since + 0.3, end):
+        time.sleep(0.02)
+        now = H.mem_info()[0]
+        if now != last:
+            last, since = now, time.monotonic()
+    return last
 
 
 def edges(V, m):
@@ -74,7 +85,7 @@ def test_kept_scratch_makes_room():
         a.free()
         a, b = edges(V, 1000)
         try:
-            for _ in range(30):  # in pieces; the runtime may hand back some of its own on the way
+            for _ in range(16):
                 room = free() - 600 * MB
                 if room > 50 * MB:
                     hogs.append(H.malloc(min(room, 32 << 30)))
