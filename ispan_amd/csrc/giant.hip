@@ -19,7 +19,9 @@ using namespace dev;
 
 namespace {
 
-constexpr int kSpinCap = 1 << 24;  // barrier wait bound (~1 s); beyond it the kernel aborts
+// Polls that a barrier waits at most, each a round trip past the L2 and a short
+// sleep (10 s and more in all); beyond them the kernel aborts.
+constexpr int kSpinCap = 1 << 24;
 constexpr int kBarWords = 8;       // payload words a barrier can carry per block
 static_assert(kBarWords * 2 * 8 == kBarBytesPerBlock, "two record buffers of 8-byte words");
 // One 1024-thread block per CU: every block invalidates its caches after a
@@ -1091,7 +1093,7 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
                     const int e = eb + c.tid;
                     int pos = 0;
                     if (!hub) {
-    #pragma unroll
+#pragma unroll
                         for (int sp = kGBlock / 2; sp > 0; sp >>= 1)
                             if (sm.off[pos + sp] <= e) pos += sp;
                     }
@@ -1218,7 +1220,9 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
         // permutation: with plain indices a block's runs would share
         // fixed bits of their vertex ids, and in graphs whose degrees
         // follow id bits (R-MAT) the blocks' work would differ severalfold.
-        // (bu_mult < total_waves <= 65536: the product fits 32 bits)
+        // (gwave and bu_mult are less than all waves of the grid, at most
+        // 65536, also where a direction has half of them: the product fits
+        // 32 bits, and bu_mult, coprime to all of them, is so to the half)
         const int64_t pg = (int64_t)(((uint32_t)gwave * (uint32_t)a.bu_mult) % (uint32_t)total_waves);
         for (int64_t cb = 0; cb < nruns; cb += total_waves * (kWave / kBUrun)) {
             // lane j loads one word; then only words with candidates are
@@ -2414,11 +2418,6 @@ __global__ __launch_bounds__(kGBlock) void k_tail(const GiantArgs) {
         gs->bar_next = a.bar_base + c.nbar;
         gs->ts[5] = wall_clock64();
     }
-}
-
-__global__ void k_zero_i64(int64_t* p, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = 0;
 }
 
 // first[v] = the first entry of v's list (-1 if empty): the bottom-up sweep's
