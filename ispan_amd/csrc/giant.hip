@@ -34,7 +34,7 @@ struct Dir {
     int32_t mode;     // 0 top-down, 1 bottom-up, 2 top-down to exhaustion
     int32_t L;        // levels done
     int32_t visited;  // vertices claimed, the roots excluded
-    int32_t nq, nh;   // next level's queue entries and hub work items
+    int32_t nq, nh;   // next level's queue entries and hub work items (nq: the finds to gather, before a gathering level)
 };
 // What the traversal goes on with (Smem::flow): which directions are still
 // traversing; which had a bottom-up level last and have a top-down one next,
@@ -918,6 +918,16 @@ __device__ __forceinline__ int expand_wave(Ctx& c, PairQueue& wq, int32_t root, 
 // R-MAT flat.
 constexpr int kLocalPerWave = 12;
 
+// The first top-down level after bottom-up ones goes on from the finds in place
+// while there are at most this many for each wave, and else queues them for the
+// next level: a wave's words have what they have, and where the finds are many
+// some waves have most of their edges (R-MAT's degrees follow the id bits).
+// With the defaults few are left.  Always in place, and by this rule: beta = 1 on
+// 3 M vertices at edge factor 3 2.38 / 0.50 ms, on R-MAT of 700 K and 8 M vertices
+// 0.63 / 0.31 and 2.9 / 1.38; with 8, 32 or 64 the same.  Never in place: by the
+// defaults 700 K vertices 151 us against 137, a lattice of 500^2 623 against 577.
+constexpr int kGatherLocal = 16;
+
 // A batch's roots, the vertices of most edges of its graphs, are the whole
 // level 0: their lists are cut into items of a block's step, from kSeedHubDeg
 // edges on where the items' room allows.  With kGiantChunk edges an item and
@@ -1016,7 +1026,7 @@ __device__ __forceinline__ void level_work(Ctx& c, int mode, int32_t L, int32_t 
                 push_next((m >> c.lane) & 1ull, v, beg, pq, qout, qn_out, hs, hout, hn_out, fedges);
             }
         }
-        if (a.td_local > 0)
+        if (a.td_local > 0 && nq <= kGatherLocal * total_waves)
             expand_local<true>(c, pq, root, beg, adj, found, vis, qout, qn_out, hs, hout, hn_out, my_found,
                                a.td_local);
         block_flush_both(c, pq, qout, qn_out, hs, hout, hn_out);
@@ -1521,7 +1531,9 @@ __device__ __forceinline__ bool traverse_joint(Ctx& c, int32_t root, int64_t set
                     }
                 }
                 next |= bits;
-                if (c.lane == 0) sm.dir[dir] = Dir{mode, L, (int32_t)visited, nq, nh};
+                const int32_t finds = (int32_t)found;
+                if (c.lane == 0)
+                    sm.dir[dir] = Dir{mode, L, (int32_t)visited, (bits & (kGather << dir)) ? finds : nq, nh};
             }
             if (acquire) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // as a barrier with ACQ does
             if (c.lane == 0) sm.flow = next;
