@@ -15,8 +15,8 @@ MB = 1 << 20
 
 
 def free():
-    """Free device memory, once it has stopped growing: the driver clears what
-    was freed before it counts as free again."""
+    """Free device memory, once it has stopped growing: memory is cleared after
+    it was freed, and only then counts as free."""
     H.synchronize()
     last, since = H.mem_info()[0], time.monotonic()
     end = since + 10
